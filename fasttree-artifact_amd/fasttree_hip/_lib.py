@@ -80,6 +80,24 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_binding = None
+
+
+def binding():
+    """The compiled binding of the per-layer calls (csrc/fasttree_torch.cpp), loaded once."""
+    global _binding
+    if _binding is None:
+        load()   # (torch first, then the C-ABI library the binding links to)
+        try:
+            from . import _torch_binding
+        except ImportError as e:
+            raise FastTreeLibraryError(
+                f"the compiled binding of {LIB_PATH} is missing or does not load ({e}): build it with "
+                "`python -c 'import __graft_entry__ as g; g.build()'`. There is no fallback path.") from e
+        _binding = _torch_binding
+    return _binding
+
+
 def check(code: int, what: str) -> None:
     if code == 0:
         return

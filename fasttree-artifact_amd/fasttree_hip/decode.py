@@ -1,4 +1,6 @@
-"""Python entry points of the decode path: thin argument marshalling over the C ABI.
+"""Python entry points of the decode path: thin argument marshalling over the C ABI.  The calls a
+serving loop makes once per layer (``fasttree_decode``, ``store_kv_cache``) marshal and check their
+arguments in the compiled binding (csrc/fasttree_torch.cpp), the others here.
 
 ``fasttree_decode`` keeps the reference's positional signature
 (kernel_bench/fasttree.py:582-604; called positionally at kernel_bench/benchmark.py:115-124
@@ -75,52 +77,12 @@ def fasttree_decode(
 
     ``logit_cap`` is accepted and ignored, as in the reference (fasttree.py:603).
     """
-    assert q.shape[-1] == k_buffer.shape[-1]          # fasttree.py:437-438
-    _need_gpu(q, k_buffer, v_buffer, o, mid_o, mid_lse, vnode_to_kv_entries)
-    _need_inner_contiguous(q, k_buffer, v_buffer, o, mid_o, mid_lse)
-    _need_i32(vnode_to_kv_entries, vnode_to_kv_offs, vnode_to_kv_lens, vnode_to_q_entries, vnode_to_q_offs,
-              vnode_to_q_lens, req_to_vnode_entries, req_to_vnode_offs, req_to_vnode_lens)
-    if k_buffer.dtype != q.dtype or v_buffer.dtype != q.dtype or o.dtype != q.dtype:
-        raise _lib.FastTreeLibraryError("q, k, v and o must share one dtype")
-    if mid_o.dtype != torch.float32 or mid_lse.dtype != torch.float32:
-        raise _lib.FastTreeLibraryError("mid_o and mid_lse must be float32")
-    lib = _lib.load()
-    programs = getattr(phase_node_nums, "prog_table", None)
-    narrow_table = _narrow_table_ptr(phase_node_nums)
-    if (programs is not None or narrow_table is not None) and q.shape[-1] >= 32:
-        # the launch was arranged as block programs (launch_schedule.block_programs)
-        rc = lib.ft_decode_programs(
-            q.data_ptr(), k_buffer.data_ptr(), v_buffer.data_ptr(), o.data_ptr(),
-            q.stride(0), q.stride(1), k_buffer.stride(0), k_buffer.stride(1),
-            v_buffer.stride(0), v_buffer.stride(1), o.stride(0), o.stride(1),
-            vnode_to_kv_entries.data_ptr(), vnode_to_kv_offs.data_ptr(), vnode_to_kv_lens.data_ptr(),
-            vnode_to_q_entries.data_ptr(), vnode_to_q_offs.data_ptr(), vnode_to_q_lens.data_ptr(),
-            req_to_vnode_entries.data_ptr(), req_to_vnode_offs.data_ptr(), req_to_vnode_lens.data_ptr(),
-            mid_o.data_ptr(), mid_o.stride(0), mid_o.stride(1), mid_lse.data_ptr(), mid_lse.stride(0),
-            _lib.int32_pair(phase_node_nums), _lib.int32_pair(phase_node_offsets),
-            programs.data_ptr() if programs is not None else None,
-            int(phase_node_nums.num_programs) if programs is not None else 0,
-            int(phase_node_nums.narrow_in_programs) if programs is not None else 0, narrow_table,
-            _prog_records_ptr(phase_node_nums), _req_table_ptr(phase_node_nums),
-            q.shape[0], q.shape[1], k_buffer.shape[1], q.shape[-1],
-            float(sm_scale), _dtype_code(q), _stream_handle(q),
-        )
-        _lib.check(rc, "ft_decode_programs")
-        return
-    rc = lib.ft_decode(
-        q.data_ptr(), k_buffer.data_ptr(), v_buffer.data_ptr(), o.data_ptr(),
-        q.stride(0), q.stride(1), k_buffer.stride(0), k_buffer.stride(1),
-        v_buffer.stride(0), v_buffer.stride(1), o.stride(0), o.stride(1),
-        vnode_to_kv_entries.data_ptr(), vnode_to_kv_offs.data_ptr(), vnode_to_kv_lens.data_ptr(),
-        vnode_to_q_entries.data_ptr(), vnode_to_q_offs.data_ptr(), vnode_to_q_lens.data_ptr(),
-        req_to_vnode_entries.data_ptr(), req_to_vnode_offs.data_ptr(), req_to_vnode_lens.data_ptr(),
-        mid_o.data_ptr(), mid_o.stride(0), mid_o.stride(1), mid_lse.data_ptr(), mid_lse.stride(0),
-        _lib.int32_pair(phase_node_nums), _lib.int32_pair(phase_node_offsets),
-        _lib.int32_pair(phase_q_tile_sizes), _lib.int32_pair(phase_kv_tile_sizes),
-        q.shape[0], q.shape[1], k_buffer.shape[1], q.shape[-1],
-        float(sm_scale), _dtype_code(q), _stream_handle(q),
-    )
-    _lib.check(rc, "ft_decode")
+    rc = _lib.binding().decode(
+        q, k_buffer, v_buffer, o, vnode_to_kv_entries, vnode_to_kv_offs, vnode_to_kv_lens, vnode_to_q_entries, vnode_to_q_offs,
+        vnode_to_q_lens, req_to_vnode_entries, req_to_vnode_offs, req_to_vnode_lens, mid_o, mid_lse, phase_node_nums,
+        phase_node_offsets, phase_q_tile_sizes, phase_kv_tile_sizes, sm_scale)
+    if rc:
+        _lib.check(rc, "fasttree_decode")
 
 
 def fasttree_decode_static(q, k_buffer, v_buffer, o, vnode_to_kv_entries, vnode_to_kv_offs, vnode_to_kv_lens,
@@ -267,28 +229,6 @@ def store_kv_cache(cache_k, cache_v, out_cache_loc, k_buffer, v_buffer):
     ``cache_k`` / ``cache_v`` are ``[tokens, Hkv, D]`` (or ``[tokens, Hkv * D]``), ``out_cache_loc``
     int32 or int64 pool slots.  A slot outside the pool is skipped, not wrapped.
     """
-    import torch
-
-    _need_gpu(cache_k, cache_v, out_cache_loc, k_buffer, v_buffer)
-    hkv, d = k_buffer.shape[1], k_buffer.shape[2]
-    if v_buffer.shape[1:] != k_buffer.shape[1:] or v_buffer.dtype != k_buffer.dtype:
-        raise _lib.FastTreeLibraryError("k_buffer and v_buffer must have the same heads, head size and dtype")
-    cache_k = cache_k.view(-1, hkv, d)
-    cache_v = cache_v.view(-1, hkv, d)
-    if cache_k.dtype != k_buffer.dtype or cache_v.dtype != k_buffer.dtype:
-        raise _lib.FastTreeLibraryError("the new rows must have the pools' dtype")
-    _need_inner_contiguous(cache_k, cache_v, k_buffer, v_buffer)
-    n = cache_k.shape[0]
-    if cache_v.shape[0] != n or out_cache_loc.numel() != n:
-        raise _lib.FastTreeLibraryError("cache_k, cache_v and out_cache_loc must name the same number of tokens")
-    if out_cache_loc.dtype not in (torch.int32, torch.int64) or not out_cache_loc.is_contiguous():
-        raise _lib.FastTreeLibraryError("out_cache_loc must be a contiguous int32 or int64 tensor")
-    lib = _lib.load()
-    rc = lib.ft_store_kv(
-        cache_k.data_ptr(), cache_v.data_ptr(), cache_k.stride(0), cache_k.stride(1), cache_v.stride(0), cache_v.stride(1),
-        out_cache_loc.data_ptr(), int(out_cache_loc.dtype == torch.int64), n,
-        k_buffer.data_ptr(), v_buffer.data_ptr(), k_buffer.stride(0), k_buffer.stride(1),
-        v_buffer.stride(0), v_buffer.stride(1), min(k_buffer.shape[0], v_buffer.shape[0]), hkv, d,
-        _dtype_code(k_buffer), _stream_handle(k_buffer),
-    )
-    _lib.check(rc, "ft_store_kv")
+    rc = _lib.binding().store_kv(cache_k, cache_v, out_cache_loc, k_buffer, v_buffer)
+    if rc:
+        _lib.check(rc, "ft_store_kv")

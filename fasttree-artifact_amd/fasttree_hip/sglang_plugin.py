@@ -25,6 +25,8 @@ from typing import Dict, List, Optional, Sequence, Tuple
 import numpy as np
 import torch
 
+from . import _lib
+
 
 class FastTreeMetadata:
     """Planner hyper-parameters plus the device buffers one decode step reads (metadata.py:5-66).
@@ -117,35 +119,24 @@ def decode_forward_fasttree(self, q, k, v, input_metadata):
     the metadata bound to ``input_metadata.fasttree``.  The output shape for ``qk_head_dim != v_head_dim``
     follows the reference literally (plugin.py:22-23).
     """
-    from .decode import fasttree_decode, store_kv_cache
-
+    meta = input_metadata.fasttree
+    pool = input_metadata.token_to_kv_pool
+    k_buffer, v_buffer = pool.get_key_buffer(self.layer_id), pool.get_value_buffer(self.layer_id)
     if self.qk_head_dim != self.v_head_dim:
         o = q.new_empty((q.shape[-1], self.tp_q_head_num * self.v_head_dim))
     else:
         o = torch.empty_like(q)
-    meta = input_metadata.fasttree
+    native = _lib.binding()
     if getattr(meta, "fused_store", False):
-        store_kv_cache(k, v, input_metadata.out_cache_loc,
-                       input_metadata.token_to_kv_pool.get_key_buffer(self.layer_id),
-                       input_metadata.token_to_kv_pool.get_value_buffer(self.layer_id))
+        rc = native.store_kv(k, v, input_metadata.out_cache_loc, k_buffer, v_buffer)
+        if rc:
+            _lib.check(rc, "ft_store_kv")
     else:
         self.store_kv_cache(k, v, input_metadata)
-
-    fasttree_decode(
-        q.view(-1, self.tp_q_head_num, self.qk_head_dim),
-        input_metadata.token_to_kv_pool.get_key_buffer(self.layer_id),
-        input_metadata.token_to_kv_pool.get_value_buffer(self.layer_id),
-        o.view(-1, self.tp_q_head_num, self.v_head_dim),
-        input_metadata.req_to_token_pool.req_to_token,
-        meta.vnode_to_kv_offs, meta.vnode_to_kv_lens,
-        meta.vnode_to_q_entries, meta.vnode_to_q_offs, meta.vnode_to_q_lens,
-        meta.req_to_vnode_entries, meta.req_to_vnode_offs, meta.req_to_vnode_lens,
-        meta.mid_o, meta.mid_lse,
-        meta.phase_node_nums, meta.phase_node_offsets,
-        meta.phase_q_tile_sizes, meta.phase_kv_tile_sizes,
-        sm_scale=self.scaling,
-        logit_cap=self.logit_cap,
-    )
+    rc = native.decode_layer(q, o, k_buffer, v_buffer, input_metadata.req_to_token_pool.req_to_token, meta,
+                             self.tp_q_head_num, self.qk_head_dim, self.v_head_dim, self.scaling)
+    if rc:
+        _lib.check(rc, "fasttree_decode")
     return o
 
 

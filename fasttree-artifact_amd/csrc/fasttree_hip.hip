@@ -105,6 +105,15 @@ __device__ __forceinline__ float xor32_max(float x) { LanePair h = halves32(x); 
 __device__ __forceinline__ float xor16_sum(float x) { LanePair h = halves16(x); return h.lo + h.hi; }
 __device__ __forceinline__ float xor32_sum(float x) { LanePair h = halves32(x); return h.lo + h.hi; }
 __device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
+// The lane's number, opaque to the compiler: what is derived from it stays where it is used.  (In a
+// kernel whose loops hold several kinds of work the compiler would otherwise compute every kind's
+// lane addresses ahead of all of them and spill them: scratch reloads inside a stream of direct
+// loads wait for the stream.)
+__device__ __forceinline__ int lane_here() {
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
 // Orders this wave's LDS traffic around a point where lanes read what other lanes of the
 // same wave wrote.  LDS executes one wave's instructions in order, so no wait is needed;
 // the fences only stop the compiler from moving accesses across.
@@ -168,6 +177,18 @@ struct VnodeView {
   int kv_len;      // tokens in the run
   int64_t kv_base; // tree mode: index into kv_entries; gathered mode: first cache row
 };
+
+// A view that every lane of the wave holds alike (read from LDS, say) as scalars: loops over it then
+// are scalar loops.
+__device__ __forceinline__ VnodeView uniform(const VnodeView& w) {
+  VnodeView u;
+  u.q_off = __builtin_amdgcn_readfirstlane(w.q_off);
+  u.q_len = __builtin_amdgcn_readfirstlane(w.q_len);
+  u.kv_len = __builtin_amdgcn_readfirstlane(w.kv_len);
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)w.kv_base), hi = __builtin_amdgcn_readfirstlane((unsigned)(w.kv_base >> 32));
+  u.kv_base = (int64_t)(((uint64_t)hi << 32) | lo);
+  return u;
+}
 
 template <bool GATHERED>
 __device__ __forceinline__ VnodeView load_vnode(const Stage1Args& a, int vnode) {
@@ -411,15 +432,15 @@ __device__ __forceinline__ void wave_attend(const Stage1Args& a, const VnodeView
 
 template <int D, int NQB>
 __device__ __forceinline__ void write_partials(const Stage1Args& a, const VnodeView& vn, int kvh, int row0,
-                                               const WaveState<D, NQB>& st) {
+                                               const WaveState<D, NQB>& st, int ngroups = NQB) {
   constexpr int DB = D / 16;
-  const int lane = threadIdx.x & 63;
+  const int lane = lane_here();
   const int p = lane & 15, c = lane >> 4;
   const int rows_total = vn.q_len * a.g;
 #pragma unroll
   for (int qb = 0; qb < NQB; ++qb) {
     const int r = row0 + 16 * qb + p;
-    if (r >= rows_total) continue;
+    if (qb >= ngroups || r >= rows_total) continue;
     const int ri = r / a.g, rj = r - ri * a.g;
     const int64_t row = vn.q_off + ri;
     const int head = kvh * a.g + rj;
@@ -511,20 +532,30 @@ __global__ void __launch_bounds__(kBlock) stage1_kernel(Stage1Args a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Wide vnodes: 32x32x16 MFMA tiles (twice the rate of 16x16x32 on this part), four waves per
-// block with 32 query rows each and two blocks per compute unit, so that two waves share a SIMD
-// and one wave's waits are filled by the other's instructions.  (Within a wave a tile step is one
-// dependent chain, scores -> soft-max -> P.V; the matrix instructions of one wave overlap the
-// vector instructions of the other about half of the time.)
+// Wide vnodes: four waves per block and two blocks per compute unit, so that two waves share a
+// SIMD and one wave's waits are filled by the other's instructions.
+//
+// What bounds the loop is the energy of the matrix instructions: on rows resident in LDS the tile
+// step runs at 1.2 PFLOP/s with one, two or three waves per SIMD alike (the clock drops from 2.3
+// to 1.8 GHz), the rate of a large library matrix product on this part.  16x16x32 instructions
+// draw less than 32x32x16 at the same rate per cycle (32 x 32 scores and their P.V: 430 against
+// 450 ns per SIMD with 32 rows a wave), and 48 query rows per wave read a K or V operand from LDS
+// once for three row groups and spread a tile's loads and barrier over 1.5 times the rows (407 ns).
+// 48 rows take 96 accumulator and 48 query registers of the 256 a wave has.
 // ---------------------------------------------------------------------------------------
 constexpr int kWideWaves = 4;
 constexpr int kWideBlock = kWave * kWideWaves;
-constexpr int kWideRows = 32 * kWideWaves;        // query rows one pass of a block serves
 constexpr int kWaveSlotsPerCu = 8;                // waves of these kernels a compute unit holds
+// 16-row groups a wave serves per pass, and query rows a block does
+template <int D> struct WideRows {
+  static constexpr int kGroups = D <= 128 ? 3 : 2;
+  static constexpr int kBlock = 16 * kGroups * kWideWaves;
+};
+constexpr int kDeftRows = 32 * kWideWaves;        // (the comparison engine's kernel: 32 rows per wave)
 
 // LDS layout of the wide kernel: rows of 2*D bytes back to back (no padding), 64-token super
-// tiles of two 32-token tiles, a ring of kBufs buffers, then a staging area for the run's slot
-// indices.  A row's 16-byte chunks are stored XOR-permuted: chunk c of row r sits in slot
+// tiles of two 32-token tiles, a ring of kBufs buffers, then the rings of slot indices and a
+// program's record.  A row's 16-byte chunks are stored XOR-permuted: chunk c of row r sits in slot
 // c ^ swz(r).  swz swaps the two low bit pairs of r, which makes both read patterns conflict free
 // for 256-byte rows: the K operand read (16 different rows, same chunk) and the transposed V
 // read (4 consecutive rows x 4 consecutive chunks).  Loads go global -> LDS directly; one wave
@@ -535,7 +566,6 @@ template <int D> struct WideGeom {
   static constexpr int kSub = 2;
   static constexpr int kTokens = kSub * kTileTokens;     // 64
   static constexpr int kBufs = 2;
-  static constexpr int kAhead = kBufs - 1;               // super tiles in flight beyond the current one
   static constexpr int kTileBytes = kTileTokens * kRowBytes;
   static constexpr int kBytesK = kTokens * kRowBytes;
   static constexpr int kBytes = 2 * kBytesK;             // K + V of one buffer
@@ -544,13 +574,13 @@ template <int D> struct WideGeom {
   static constexpr int kGroups = kTokens / kGroupRows;   // groups per matrix and super tile
   static constexpr int kUnits = 2 * kGroups / kWideWaves;                       // loads per wave and super tile
   static constexpr int kSlots = kGroups >= kWideWaves ? kGroups / kWideWaves : 1;  // distinct rows among them
-  static constexpr int kIdxCap = 2048;                    // slot indices staged at a time (tokens)
-  static constexpr int kRecord = kRing + 4 * kIdxCap;    // byte offset of the program's record (kProgRecord ints)
+  static constexpr int kIdxBytes = kWideWaves * 4 * 4 * kTokens;                   // per wave: the slot indices of four super tiles
+  static constexpr int kRecord = kRing + kIdxBytes;      // byte offset of the program's record (kProgRecord ints)
   static constexpr int kLds = kRecord + 1024;
   static __device__ __forceinline__ int swz(int row) { return (((row & 3) << 2) | ((row >> 2) & 3)) & (kChunks - 1); }
 };
 
-// State of one wave for its 32 query rows.  o[db][j] = O[row lane%32][dim 32*db + 8*(j/4) +
+// State of one wave for 32 query rows (32x32x16 tiles).  o[db][j] = O[row lane%32][dim 32*db + 8*(j/4) +
 // 4*(lane/32) + j%4]; m = soft-max reference (scaled scores, log2 domain); l = this lane's own
 // share of the row sum until finish_state().
 template <int D> struct WideState {
@@ -575,7 +605,7 @@ __device__ __forceinline__ void reset_state(WideState<D>& st) {
 // zero past the vnode (src == nullptr).
 // The record of a block program (kProgRecord ints, one thread of the block each): entries 0..3 are
 // kv_off, kv_len, q_off and q_len of the program's first wide vnode, entry 4 says whether the rest is
-// there (the vnode exists and has at most kWideRows query rows), entries kProgRecRequests.. the
+// there (the vnode exists, fits one pass of a block and has at most 128 requests), entries kProgRecRequests.. the
 // requests of its scratch rows, entries kProgRecSlots.. the pool slots of its first 64 tokens (the
 // last token repeated past the end of a shorter run).  With it a block knows after one memory round
 // trip what it otherwise learns in three (its table entry, the vnode's list entries, the request
@@ -597,6 +627,19 @@ __device__ __forceinline__ const char* q_row_address32(const Stage1Args& a, cons
   const int64_t entry = GATHERED ? (int64_t)(vn.q_off / a.nsplit)
                                  : (int64_t)(requests ? requests[ri] : a.q_entries[vn.q_off + ri]);
   return a.q + 2 * (entry * a.sq0 + (int64_t)(kvh * a.g + rj) * a.sq1 + 8 * h);
+}
+// The same for 16-row groups: row row0 + lane%16, fragment ks: dims 32*ks + 8*(lane/16) .. +7.
+template <bool GATHERED>
+__device__ __forceinline__ const char* q_row_address16(const Stage1Args& a, const VnodeView& vn, int kvh, int row0,
+                                                       const int* requests = nullptr) {
+  const int lane = lane_here();
+  const int r = row0 + (lane & 15), c = lane >> 4;
+  if (r >= vn.q_len * a.g) return nullptr;
+  const int ri = r / a.g;
+  const int rj = r - ri * a.g;
+  const int64_t entry = GATHERED ? (int64_t)(vn.q_off / a.nsplit)
+                                 : (int64_t)(requests ? requests[ri] : a.q_entries[vn.q_off + ri]);
+  return a.q + 2 * (entry * a.sq0 + (int64_t)(kvh * a.g + rj) * a.sq1 + 8 * c);
 }
 template <int D>
 __device__ __forceinline__ void load_q_frags32(const char* src, u32x4 (&qf)[D / 16]) {
@@ -648,6 +691,10 @@ __device__ __forceinline__ void load_direct16(const char* src, unsigned lds_base
   // (M0 holds the LDS address: bound as an operand, so the compiler writes it and knows it is live)
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "{m0}"(lds_base) : "memory");
 }
+// The same for 4 bytes per lane at base + offset (base wave uniform), landing at lds_base + 4 * lane.
+__device__ __forceinline__ void load_direct4(const void* base, unsigned offset, unsigned lds_base) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(offset), "s"(base), "{m0}"(lds_base) : "memory");
+}
 // Wait until at most N of this wave's vector-memory operations are still in flight (they finish
 // in order).
 template <int N>
@@ -657,6 +704,9 @@ __device__ __forceinline__ void wait_direct_loads() {
 
 __device__ __forceinline__ u32x4 lds_read16(unsigned addr) {
   return *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>((uintptr_t)addr);
+}
+__device__ __forceinline__ unsigned lds_read4(unsigned addr) {
+  return *reinterpret_cast<const __attribute__((address_space(3))) unsigned*>((uintptr_t)addr);
 }
 __device__ __forceinline__ u32x2 lds_read_tr8(unsigned addr) {
   const i16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
@@ -803,210 +853,355 @@ __device__ __forceinline__ void write_partials32(const Stage1Args& a, const Vnod
   if (h == 0) a.mid_lse[row * a.sl0 + head] = st.l > 0.f ? (__builtin_amdgcn_logf(st.l) + st.m) * kLn2 : -INFINITY;
 }
 
-// Merge of the TG waves that hold the same rows (token groups 0..TG-1 of row group rg) into
-// token group 0, pairwise through LDS.  Every wave of the block must call this.
+// Per-lane LDS byte addresses of a wave's 16x16x32 operand reads inside a 32-token tile (of a wide
+// block's ring: tile 0 of the first buffer), for contraction step / dim block 0.  The XOR layout makes the address for step ks
+// (dim block db) the base with 64*ks (32*db) XOR-ed in; the second 16 tokens of a tile, the second
+// tile of a super tile and the second buffer are constant offsets away.
+struct WideLane16 {
+  unsigned k;   // K operand: token lane%16, chunk lane/16 (step ks: chunk 4*ks + lane/16)
+  unsigned v;   // transposed V read: tokens 4*(lane/16) .. +3, dims 4*(lane%4) .. +3
+};
 template <int D>
-__device__ __forceinline__ void merge_token_groups(float* xchg, WideState<D>& st, int rg, int tg, int tgroups, bool active) {
-  constexpr int NV = (D / 32) * 16 + 2;
+__device__ __forceinline__ WideLane16 init_lane16(unsigned k_tile, unsigned v_tile) {
+  using W = WideGeom<D>;
+  const int lane = lane_here(), p = lane & 15, c = lane >> 4;
+  const int vr = 4 * c + (p >> 2);
+  return WideLane16{k_tile + p * W::kRowBytes + 16 * ((c & (W::kChunks - 1)) ^ W::swz(p)),
+                    v_tile + vr * W::kRowBytes + 16 * ((((p & 3) >> 1) & (W::kChunks - 1)) ^ W::swz(vr)) + 8 * (p & 1)};
+}
+
+// A 32-token step for a wave's NQ 16-row groups, in three parts.
+//
+// Scores: S^T = K Q^T: A = K rows (token lane%16, 8 dims per lane), B = Q; s[tb][qb][j] of a lane is
+// the score of token 16*tb + 4*(lane/16) + j and row 16*qb + lane%16, so the eight scores of a
+// row group are exactly the k-slots the lane feeds to the P.V contraction: probabilities never
+// leave registers.  kb: the lane's K address in the tile (see WideLane16).
+template <typename E, int D, int NQ>
+__device__ __forceinline__ void tile_scores(unsigned kb, const u32x4 (&qf)[NQ][D / 32], f32x4 (&s)[2][NQ]) {
+  using W = WideGeom<D>;
+  constexpr int KS = D / 32;
+  constexpr int KB = KS < 4 ? KS : 4;     // contraction steps whose K operands are requested together
+#pragma unroll
+  for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+    for (int qb = 0; qb < NQ; ++qb) s[tb][qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k0 = 0; k0 < KS; k0 += KB) {
+    u32x4 kf[KB][2];
+#pragma unroll
+    for (int ks = 0; ks < KB; ++ks)
+#pragma unroll
+      for (int tb = 0; tb < 2; ++tb) kf[ks][tb] = lds_read16((kb ^ (64u * (k0 + ks))) + tb * 16 * W::kRowBytes);
+    // (keeps the scheduler from sinking each read next to its use, which would expose the full
+    // LDS latency time and again)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < KB; ++ks)
+#pragma unroll
+      for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+        for (int qb = 0; qb < NQ; ++qb) s[tb][qb] = E::mfma(kf[ks][tb], qf[qb][k0 + ks], s[tb][qb]);
+  }
+}
+
+// The V^T operands of the dim blocks d0 .. of a tile: two transposed LDS reads of 4 consecutive tokens each.
+template <int D> struct VOperands {
+  static constexpr int kBatch = D / 16 < 8 ? D / 16 : 8;     // dim blocks requested together
+  u32x4 f[kBatch];
+  __device__ __forceinline__ void request(unsigned vb, int d0) {
+#pragma unroll
+    for (int db = 0; db < kBatch; ++db) {
+      const u32x2 lo = lds_read_tr8(vb ^ (32u * (d0 + db)));
+      const u32x2 hi = lds_read_tr8((vb ^ (32u * (d0 + db))) + 16 * WideGeom<D>::kRowBytes);
+      f[db] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+};
+
+// Scores to probabilities, online.  valid < 32 only on a run's last, partial tile.  The check whether a
+// row's soft-max reference has to move (see kSlack) needs no exchange between the four lanes that
+// share the row: each compares its own eight scores, and only when some lane of the wave finds one
+// too large are the maxima exchanged and the accumulators rescaled.
+template <typename E, int D, int NQ>
+__device__ __forceinline__ void tile_softmax(f32x4 (&s)[2][NQ], int valid, float sc, WaveState<D, NQ>& st, u32x4 (&pf)[NQ]) {
+  if (valid < kTileTokens) {  // wave uniform
+    asm volatile("" ::: "memory");  // keeps this a branch: as selects it would run on every tile
+    const int c = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int tb = 0; tb < 2; ++tb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int qb = 0; qb < NQ; ++qb) s[tb][qb][j] = (16 * tb + 4 * c + j >= valid) ? -INFINITY : s[tb][qb][j];
+  }
+  float mx[NQ];
+  bool grow = false;
+#pragma unroll
+  for (int qb = 0; qb < NQ; ++qb) {
+    mx[qb] = max3(s[0][qb][0], s[0][qb][1], s[0][qb][2]);
+    mx[qb] = max3(mx[qb], s[0][qb][3], s[1][qb][0]);
+    mx[qb] = max3(mx[qb], s[1][qb][1], s[1][qb][2]);
+    mx[qb] = fmaxf(mx[qb], s[1][qb][3]);
+    grow |= mx[qb] * sc > st.m[qb] + kSlack;   // sc > 0; true on a run's first tile (m = -inf)
+  }
+  if (__builtin_amdgcn_ballot_w64(grow)) {
+#pragma unroll
+    for (int qb = 0; qb < NQ; ++qb) {
+      const float top = xor32_max(xor16_max(mx[qb])) * sc;   // finite: the tile holds at least one token
+      const float m_new = top > st.m[qb] + kSlack ? top : st.m[qb];
+      const float alpha = __builtin_amdgcn_exp2f(st.m[qb] - m_new);
+      st.l[qb] *= alpha;
+#pragma unroll
+      for (int db = 0; db < D / 16; ++db) st.o[qb][db] *= alpha;
+      st.m[qb] = m_new;
+    }
+  }
+#pragma unroll
+  for (int qb = 0; qb < NQ; ++qb) {
+    const float neg_m = -st.m[qb];
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j >> 2][qb][j & 3], sc, neg_m));
+    st.l[qb] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
+    pf[qb] = u32x4{E::pack2(x[0], x[1]), E::pack2(x[2], x[3]), E::pack2(x[4], x[5]), E::pack2(x[6], x[7])};
+  }
+}
+
+// O^T += V^T P^T; `v` holds the operands of the first dim blocks.
+template <typename E, int D, int NQ>
+__device__ __forceinline__ void tile_pv(unsigned vb, VOperands<D>& v, const u32x4 (&pf)[NQ], WaveState<D, NQ>& st) {
+  constexpr int DB = D / 16, VB = VOperands<D>::kBatch;
+#pragma unroll
+  for (int d0 = 0; d0 < DB; d0 += VB) {
+    if (d0 > 0) v.request(vb, d0);
+#pragma unroll
+    for (int db = 0; db < VB; ++db)
+#pragma unroll
+      for (int qb = 0; qb < NQ; ++qb) st.o[qb][d0 + db] = E::mfma(v.f[db], pf[qb], st.o[qb][d0 + db]);
+  }
+}
+
+// What the waves of a block share in one pass over a KV run, and what a wave does in it.
+struct WidePass {
+  int kvh;
+  int row0;            // the wave's first query row
+  int groups;          // its 16-row groups (0: it only loads)
+  int set, tg, tgroups;  // its row set, its token group, token groups of the pass
+  const int* record;   // the program's record in LDS, or null
+};
+
+// Merge of the waves that hold the same rows (the token groups of a row set) into token group 0,
+// pairwise through LDS.  Every wave of the block must call this.
+template <int D, int NG>
+__device__ __forceinline__ void merge_token_groups(float* xchg, WaveState<D, NG>& st, const WidePass& p) {
+  constexpr int NV = (D / 16) * 4 + 2;   // floats of state per lane and row group
   const int lane = threadIdx.x & 63;
-  for (int half = tgroups >> 1; half >= 1; half >>= 1) {
+  for (int half = p.tgroups >> 1; half >= 1; half >>= 1) {
     __syncthreads();
-    if (active && tg >= half && tg < 2 * half) {
-      float* dst = xchg + (size_t)(rg * half + tg - half) * NV * kWave + lane;
-      int n = 0;
-      dst[(n++) * kWave] = st.m;
-      dst[(n++) * kWave] = st.l;
+    if (p.tg >= half && p.tg < 2 * half) {
+      float* dst = xchg + (size_t)(p.set * half + p.tg - half) * WideRows<D>::kGroups * NV * kWave + lane;
 #pragma unroll
-      for (int db = 0; db < D / 32; ++db)
+      for (int qb = 0; qb < NG; ++qb) {
+        int n = qb * NV;
+        dst[(n++) * kWave] = st.m[qb];
+        dst[(n++) * kWave] = st.l[qb];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) dst[(n++) * kWave] = st.o[db][j];
+        for (int db = 0; db < D / 16; ++db)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) dst[(n++) * kWave] = st.o[qb][db][j];
+      }
     }
     __syncthreads();
-    if (active && tg < half) {
-      const float* src = xchg + (size_t)(rg * half + tg) * NV * kWave + lane;
-      int n = 0;
-      const float m2 = src[(n++) * kWave];
-      const float l2 = src[(n++) * kWave];
-      const float m = fmaxf(st.m, m2);
-      const float a1 = scale_from(st.m, m), a2 = scale_from(m2, m);
-      st.l = st.l * a1 + l2 * a2;
-      st.m = m;
+    if (p.tg < half) {
+      const float* src = xchg + (size_t)(p.set * half + p.tg) * WideRows<D>::kGroups * NV * kWave + lane;
 #pragma unroll
-      for (int db = 0; db < D / 32; ++db)
+      for (int qb = 0; qb < NG; ++qb) {
+        int n = qb * NV;
+        const float m2 = src[(n++) * kWave];
+        const float l2 = src[(n++) * kWave];
+        const float m = fmaxf(st.m[qb], m2);
+        const float a1 = scale_from(st.m[qb], m), a2 = scale_from(m2, m);
+        st.l[qb] = st.l[qb] * a1 + l2 * a2;
+        st.m[qb] = m;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) st.o[db][j] = st.o[db][j] * a1 + src[(n++) * kWave] * a2;
+        for (int db = 0; db < D / 16; ++db)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) st.o[qb][db][j] = st.o[qb][db][j] * a1 + src[(n++) * kWave] * a2;
+      }
     }
   }
 }
 
-// One block (kWideWaves waves) serves the row pieces chunk, chunk + chunks, ... (kWideRows query
-// rows each) of a vnode for one kv head.  The block
-// streams the vnode's KV run through a ring of kBufs 64-token LDS buffers with direct
-// global->LDS loads, kBufs - 1 super tiles ahead of the one being consumed; the run's slot
-// indices are staged in LDS first so that nothing but those loads is in flight in the loop.
-// Per pass over the run the waves form RG row groups of 32 query rows x TG token groups
-// (RG * TG = kWideWaves): a wave consumes the 32-token tiles t with t % TG == tg for the rows of
-// its row group, and the TG states of a row group are merged at the end.
-template <typename E, int D, bool GATHERED>
-__device__ __forceinline__ void wide_block(const Stage1Args& a, char* smem, const VnodeView& vn, int kvh, int chunk,
-                                           int chunks, const int* record = nullptr) {
+// One wave's pass over a vnode's KV run for NG row groups (p.groups <= NG of them exist).  The block
+// streams the run through a ring of two 64-token LDS buffers with direct global->LDS loads, one
+// super tile ahead of the one being consumed.  The slot indices travel the same way, two super
+// tiles further ahead, into a ring of the wave's own (it reads the indices of the 16 rows it
+// loads): nothing the compiler tracks is in flight in the loop, no register holds an index longer
+// than one super tile, and runs of any length need no staging step.
+template <typename E, int D, int NG, bool GATHERED>
+__device__ __forceinline__ void wide_pass(const Stage1Args& a, char* smem, const VnodeView& vn, const WidePass& p) {
   using W = WideGeom<D>;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int rows_total = vn.q_len * a.g;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_here();
   const int nsuper = (vn.kv_len + W::kTokens - 1) / W::kTokens;
+  const unsigned ring = lds_offset(smem);
+  const unsigned idx_ring = ring + W::kRing + wave * (4 * 4 * W::kTokens);   // four super tiles of indices
+  const int32_t* entries = GATHERED ? nullptr : a.kv_entries + vn.kv_base;
 
   // loader role of this lane: 16-byte slot `pos` of row `grp_row` in each 1 KB group it fills
   const int grp_row = lane / W::kChunks, pos = lane % W::kChunks;
-  const char* kbase = a.k + 2 * ((int64_t)kvh * a.sk1);
-  const char* vbase = a.v + 2 * ((int64_t)kvh * a.sv1);
+  const char* kbase = a.k + 2 * ((int64_t)p.kvh * a.sk1);
+  const char* vbase = a.v + 2 * ((int64_t)p.kvh * a.sv1);
   const unsigned k_stride = (unsigned)(2 * a.sk0), v_stride = (unsigned)(2 * a.sv0);  // bytes, < 2^32 (checked by the host)
-  int* idx_lds = reinterpret_cast<int*>(smem + W::kRing);
-  const unsigned ring = lds_offset(smem);
+  auto group_of = [&](int u) { return W::kGroups >= kWideWaves ? u * kWideWaves + wave : wave % W::kGroups; };
 
-  // this block's pieces of kWideRows rows: chunk, chunk + chunks, ...
-  for (int piece = chunk; piece * kWideRows < rows_total; piece += chunks) {
-  const int rows_end = min((piece + 1) * kWideRows, rows_total);
-  for (int row0 = piece * kWideRows; row0 < rows_end;) {
-    // waves as rgroups row groups x tgroups token groups: halve the row groups (down to a token
-    // split of four) while the rows left in the piece leave half of them without rows
-    const int groups = (rows_end - row0 + 31) >> 5;   // 32-row groups still to serve
-    int rgroups = kWideWaves, tgroups = 1;
-    while (tgroups < 4 && 2 * groups <= rgroups) {
-      rgroups >>= 1;
-      tgroups <<= 1;
+  // indices of super tile j, requested into the wave's ring; those of the rows this wave loads, read back.
+  // Tokens past the run repeat its last token: the scores of such rows are masked and their V rows are finite.
+  auto issue_indices = [&](int j) {
+    if constexpr (!GATHERED) {
+      if (j < nsuper) load_direct4(entries, 4u * (unsigned)min(j * W::kTokens + lane, vn.kv_len - 1), idx_ring + (j & 3) * (4 * W::kTokens));
     }
-    const int rg = wave / tgroups, tg = wave % tgroups;
-    const int my_row0 = row0 + 32 * rg;
-    const bool active = rg < rgroups && my_row0 < rows_end;
+  };
+  unsigned srow[W::kSlots];
+  auto read_rows = [&](int j) {
+    if (j >= nsuper) return;
+#pragma unroll
+    for (int u = 0; u < W::kSlots; ++u) {
+      const int row = group_of(u) * W::kGroupRows + grp_row;
+      if constexpr (GATHERED) srow[u] = (unsigned)(vn.kv_base + min(j * W::kTokens + row, vn.kv_len - 1));
+      else srow[u] = lds_read4(idx_ring + (j & 3) * (4 * W::kTokens) + 4 * row);
+    }
+  };
+  // rows of super tile j -> ring buffer j % 2
+  auto issue_rows = [&](int j) {
+    if (j >= nsuper) return;
+    const unsigned buf = ring + (unsigned)(j & 1) * W::kBytes;
+#pragma unroll
+    for (int u = 0; u < W::kUnits; ++u) {
+      // unit u of this wave: K groups first, then V groups
+      const bool is_v = W::kGroups >= kWideWaves ? u >= W::kSlots : wave >= W::kGroups;
+      const int sl = u % W::kSlots, grp = group_of(sl);
+      const int row = grp * W::kGroupRows + grp_row;
+      const char* src = (is_v ? vbase : kbase) + (uint64_t)srow[sl] * (is_v ? v_stride : k_stride);
+      load_direct16(src + 16 * (pos ^ W::swz(row)), buf + (is_v ? W::kBytesK : 0) + grp * 1024);
+    }
+  };
 
-    // start-up chain: [request ids of the rows, slot indices] -> [Q fragments, first K/V rows]
-    // (the program's record covers the vnode's first kWideRows rows: its first piece, one pass)
-    // (not at head_dim 256, where the step has no register to spare)
-    const int* rec = (!GATHERED && D <= 128 && piece == 0) ? record : nullptr;   // block uniform
-    const char* q_src = q_row_address32<GATHERED>(a, vn, kvh, active ? my_row0 : rows_total,
-                                                  rec ? rec + kProgRecRequests : nullptr);
-    u32x4 qf[D / 16];
-    WideState<D> st;
-    reset_state<D>(st);
-    WideLane la0;
-    init_lane<D>(la0, ring);
-    unsigned cur = 0;  // byte offset of the ring buffer that holds the current super tile
-
-    // slot indices of tokens [idx_base, idx_base + kIdxCap) of the run, staged by the whole block
-    int idx_base = 0;
-    auto stage_indices = [&](int base) {
-      if constexpr (!GATHERED) {
-        idx_base = base;
-        // (branch free, so that the loads are in flight together; entries past the run repeat its last)
-        int e[W::kIdxCap / kWideBlock];
+  // start-up chain: [request ids of the rows, slot indices] -> [Q fragments, first K/V rows]; with the
+  // program's record the first super tile's rows are requested at once
+  if (nsuper > 0) {
+    if (!GATHERED && p.record) {
 #pragma unroll
-        for (int i = 0; i < W::kIdxCap / kWideBlock; ++i)
-          e[i] = a.kv_entries[vn.kv_base + min(base + kWideBlock * i + (int)threadIdx.x, vn.kv_len - 1)];
-#pragma unroll
-        for (int i = 0; i < W::kIdxCap / kWideBlock; ++i) idx_lds[kWideBlock * i + threadIdx.x] = e[i];
-        __syncthreads();
-      }
-    };
-    // rows of super tile j -> ring buffer j % kBufs, in two steps: read_rows(j) takes the slot
-    // indices of the rows this wave loads out of LDS (one super tile ahead of the loads, so that
-    // the LDS round trip is hidden by a tile step), issue_rows(j) requests the rows.  Tokens past
-    // the run repeat its last token: the scores of such rows are masked and their V rows are finite.
-    unsigned srow[W::kSlots];
-    auto read_rows = [&](int j) {
-      if (j >= nsuper) return;
-      if constexpr (!GATHERED) {
-        if (j * W::kTokens >= idx_base + W::kIdxCap) {  // block uniform
-          __syncthreads();                              // every wave has read the indices it needed
-          stage_indices(idx_base + W::kIdxCap);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < W::kSlots; ++u) {
-        const int grp = W::kGroups >= kWideWaves ? u * kWideWaves + wave : wave % W::kGroups;
-        const int row = grp * W::kGroupRows + grp_row;
-        const int t = min(j * W::kTokens + row, vn.kv_len - 1);
-        srow[u] = GATHERED ? (unsigned)(vn.kv_base + t) : (unsigned)idx_lds[t - idx_base];
-      }
-    };
-    auto issue_rows = [&](int j) {
-      if (j >= nsuper) return;
-      const unsigned buf = ring + (unsigned)(j % W::kBufs) * W::kBytes;
-#pragma unroll
-      for (int u = 0; u < W::kUnits; ++u) {
-        // unit u of this wave: K groups first, then V groups
-        const bool is_v = W::kGroups >= kWideWaves ? u >= W::kSlots : wave >= W::kGroups;
-        const int sl = u % W::kSlots;
-        const int grp = W::kGroups >= kWideWaves ? sl * kWideWaves + wave : wave % W::kGroups;
-        const int row = grp * W::kGroupRows + grp_row;
-        const char* src = (is_v ? vbase : kbase) + (uint64_t)srow[sl] * (is_v ? v_stride : k_stride);
-        load_direct16(src + 16 * (pos ^ W::swz(row)), buf + (is_v ? W::kBytesK : 0) + grp * 1024);
-      }
-    };
-    static_assert(W::kAhead == 1, "the record path below requests exactly the first super tile");
-    if (rec && nsuper > 0) {
-      // the first super tile's slots come with the record: its rows are requested before the
-      // run's index list has been read at all
-#pragma unroll
-      for (int u = 0; u < W::kSlots; ++u) {
-        const int grp = W::kGroups >= kWideWaves ? u * kWideWaves + wave : wave % W::kGroups;
-        srow[u] = (unsigned)rec[kProgRecSlots + grp * W::kGroupRows + grp_row];
-      }
+      for (int u = 0; u < W::kSlots; ++u) srow[u] = (unsigned)p.record[kProgRecSlots + group_of(u) * W::kGroupRows + grp_row];
       issue_rows(0);
-      stage_indices(0);
     } else {
-      if (nsuper > 0) stage_indices(0);  // block uniform
-#pragma unroll
-      for (int j = 0; j < W::kAhead; ++j) {
-        read_rows(j);
-        issue_rows(j);
-      }
+      issue_indices(0);
     }
-    read_rows(W::kAhead);
-    load_q_frags32<D>(q_src, qf);
-    // nothing the compiler itself tracks (the Q fragments) may still be in flight in the loop:
-    // a wait for it there would also wait for every direct load
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    // (and the compiler must see the fragments as complete, or it keeps a wait for them in the loop)
-#pragma unroll
-    for (int ks = 0; ks < D / 16; ++ks) asm volatile("" : "+v"(qf[ks]));
-    for (int super = 0; super < nsuper; ++super) {
-      // publish super tile `super` to the block; the ones after it may stay in flight
-      const int behind = min(nsuper - 1 - super, W::kAhead - 1);
-      if (behind >= 2) wait_direct_loads<2 * W::kUnits>();
-      else if (behind == 1) wait_direct_loads<W::kUnits>();
-      else wait_direct_loads<0>();
-      __syncthreads();
-      // the buffer consumed before that barrier is free: refill it
-      issue_rows(super + W::kAhead);
-      read_rows(super + W::kAhead + 1);
-      if (active) {
-        const WideLane la = at_buffer(la0, cur);
-#pragma unroll 1
-        for (int sub = 0; sub < W::kSub; ++sub) {
-          const int tile = super * W::kSub + sub;
-          if ((tile & (tgroups - 1)) != tg) continue;
-          const int valid = vn.kv_len - tile * kTileTokens;
-          if (valid > 0) tile_step32<E, D>(la, sub * W::kTileBytes, valid, a.scale_log2, qf, st);
-        }
-      }
-      cur = cur + W::kBytes == W::kRing ? 0u : cur + W::kBytes;
-    }
-    finish_state<D>(st);
-    if (tgroups > 1) merge_token_groups<D>(reinterpret_cast<float*>(smem), st, rg, tg, tgroups, active);
-    if (active && tg == 0) write_partials32<D>(a, vn, kvh, my_row0, st);
-    __syncthreads();  // staging LDS is reused by the next pass over the run
-    row0 += 32 * rgroups;
+    issue_indices(1);
+    issue_indices(2);
   }
+  u32x4 qf[NG][D / 32];
+#pragma unroll
+  for (int qb = 0; qb < NG; ++qb) {
+    const char* src = q_row_address16<GATHERED>(a, vn, p.kvh, qb < p.groups ? p.row0 + 16 * qb : vn.q_len * a.g,
+                                                p.record ? p.record + kProgRecRequests : nullptr);
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ++ks) {
+      u32x4 z = {0u, 0u, 0u, 0u};
+      qf[qb][ks] = src ? *reinterpret_cast<const u32x4*>(src + 64 * ks) : z;
+    }
+  }
+  if (!p.record && nsuper > 0) {
+    wait_direct_loads<0>();
+    read_rows(0);
+    issue_rows(0);
+  }
+  // nothing the compiler itself tracks (the Q fragments) may still be in flight in the loop:
+  // a wait for it there would also wait for every direct load
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  // (and the compiler must see the fragments as complete, or it keeps a wait for them in the loop)
+#pragma unroll
+  for (int qb = 0; qb < NG; ++qb)
+#pragma unroll
+    for (int ks = 0; ks < D / 32; ++ks) asm volatile("" : "+v"(qf[qb][ks]));
+  WaveState<D, NG> st;
+  reset_state<D, NG>(st);
+  const WideLane16 la = init_lane16<D>(ring, ring + W::kBytesK);
+  read_rows(1);
+
+  for (int super = 0; super < nsuper; ++super) {
+    wait_direct_loads<0>();
+    __syncthreads();   // publishes super tile `super` to the block; the buffer consumed before it is free
+    issue_rows(super + 1);
+    issue_indices(super + 3);
+    read_rows(super + 2);
+#pragma unroll 1
+    for (int sub = 0; sub < W::kSub; ++sub) {
+      const int tile = super * W::kSub + sub;
+      const int valid = vn.kv_len - tile * kTileTokens;
+      if ((tile & (p.tgroups - 1)) != p.tg || valid <= 0 || p.groups == 0) continue;
+      const unsigned off = (super & 1) * W::kBytes + sub * W::kTileBytes;
+      f32x4 sc[2][NG];
+      u32x4 pf[NG];
+      VOperands<D> v;
+      tile_scores<E, D, NG>(la.k + off, qf, sc);
+      // the V operands do not depend on the probabilities: requested now, they arrive under the soft-max
+      // arithmetic (and take the registers the K operands just left)
+      v.request(la.v + off, 0);
+      tile_softmax<E, D, NG>(sc, valid, a.scale_log2, st, pf);
+      tile_pv<E, D, NG>(la.v + off, v, pf, st);
+    }
+  }
+  finish_state<D, NG>(st);
+  if (p.tgroups > 1) merge_token_groups<D, NG>(reinterpret_cast<float*>(smem), st, p);
+  if (p.tg == 0) write_partials<D, NG>(a, vn, p.kvh, p.row0, st, p.groups);
+  __syncthreads();  // the ring is reused by the next pass
+}
+
+// One block (kWideWaves waves) serves the row pieces chunk, chunk + chunks, ... (WideRows<D>::kBlock
+// query rows each) of a vnode for one kv head.  Per pass over the run the waves form row sets x
+// token groups: a wave consumes the 32-token tiles t with t % tgroups == tg for its row set's 16-row
+// groups, and the states of the token groups of a row set are merged at the end.
+template <typename E, int D, bool GATHERED>
+__device__ __forceinline__ void wide_block(const Stage1Args& a, char* smem, const VnodeView& view, int kvh, int chunk,
+                                           int chunks, const int* record) {
+  const VnodeView vn = uniform(view);
+  constexpr int NQ = WideRows<D>::kGroups, kRows = WideRows<D>::kBlock;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rows_total = vn.q_len * a.g;
+  for (int piece = chunk; piece * kRows < rows_total; piece += chunks) {
+    const int row0 = piece * kRows;
+    const int groups = (min(row0 + kRows, rows_total) - row0 + 15) >> 4;
+    // as many token groups (up to four) as leave every wave at most NQ row groups: fewer waves then
+    // read the same K/V operands from LDS
+    int tgroups = 1;
+    while (tgroups < 4 && groups * 2 * tgroups <= NQ * kWideWaves) tgroups <<= 1;
+    const int sets = kWideWaves / tgroups;
+    WidePass p;
+    p.kvh = kvh;
+    p.set = wave / tgroups;
+    p.tg = wave % tgroups;
+    p.tgroups = tgroups;
+    const int share = groups / sets, extra = groups - share * sets;     // row groups per set: share, one more in the first `extra`
+    p.groups = share + (p.set < extra ? 1 : 0);
+    p.row0 = row0 + 16 * (p.set * share + min(p.set, extra));
+    p.record = !GATHERED && piece == 0 ? record : nullptr;               // (the record covers the vnode's first kRows rows)
+    // (wave uniform; every path has the same block barriers)
+    if (NQ >= 3 && p.groups == 3) wide_pass<E, D, NQ, GATHERED>(a, smem, vn, p);
+    else if (p.groups == 2) wide_pass<E, D, 2, GATHERED>(a, smem, vn, p);
+    else wide_pass<E, D, 1, GATHERED>(a, smem, vn, p);
   }
 }
 
 // ---------------------------------------------------------------------------------------
-// Narrow vnodes (at most 16 query rows): one wave per (vnode, kv head) streams the run through
-// a wave-private LDS tile of 32 tokens with direct global->LDS loads, in the same unpadded XOR
-// layout as the wide kernel.  K and V have one tile each: the K rows of the next tile are
-// requested as soon as the scores of the current one are out of LDS, its V rows as soon as the
-// current P.V is, so a leaf vnode of a few dozen tokens costs little more than its two memory
-// round trips (slot indices, rows).  Slot indices are staged 256 tokens at a time.
+// Narrow vnodes: one wave per (vnode, kv head) streams the run through a wave-private LDS tile of 32
+// tokens with direct global->LDS loads, in the same unpadded XOR layout as the wide kernel, and serves up
+// to NarrowGeom<D>::kGroups 16-row groups on it per pass.  K and V have one tile each: the K rows of
+// the next tile are requested as soon as the scores of the current one are out of LDS, its V rows
+// as soon as the current P.V is, so eight waves of a compute unit keep up to 128 KB of rows in flight
+// and no barrier holds one wave's loads back for another's arithmetic.  A leaf vnode of a few dozen
+// tokens costs little more than its two memory round trips (record, rows).  Slot indices travel the
+// same way, two tiles ahead.
 // ---------------------------------------------------------------------------------------
 template <int D> struct NarrowGeom {
   static constexpr int kRowBytes = 2 * D;
@@ -1014,9 +1209,10 @@ template <int D> struct NarrowGeom {
   static constexpr int kBytesK = kTileTokens * kRowBytes;
   static constexpr int kBytes = 2 * kBytesK;
   static constexpr int kGroupRows = kWave / kChunks;            // rows per 1 KB load
-  static constexpr int kGroups = kTileTokens / kGroupRows;      // loads per matrix and tile
-  static constexpr int kIdxCap = 256;
-  static constexpr int kLds = kBytes + 4 * kIdxCap;             // per wave; a multiple of the row size
+  static constexpr int kLoads = kTileTokens / kGroupRows;       // loads per matrix and tile
+  static constexpr int kIdxSlot = 4 * kWave;                    // bytes of one tile's indices (32, and the 32 after them)
+  static constexpr int kLds = kBytes + 4 * kIdxSlot;            // per wave; a multiple of the row size
+  static constexpr int kGroups = 2;                             // 16-row groups per pass (three spill beside the wide path's code)
   static __device__ __forceinline__ int swz(int row) { return (((row & 3) << 2) | ((row >> 2) & 3)) & (kChunks - 1); }
 };
 
@@ -1027,283 +1223,238 @@ constexpr int kNarrowRecord = 64;
 constexpr int kNarrowRecRequests = 16;
 constexpr int kNarrowRecSlots = 4 + kNarrowRecRequests;
 
-// One wave's share of a narrow vnode for the 16 query rows from row0: the tiles tile0,
+// One wave's share of a narrow vnode for the NG 16-row groups from row0: the tiles tile0,
 // tile0 + tstride, ... of the run, staged in the wave's own LDS area at lds0.  `rec` is the lane's
 // int of the vnode's record when `inlined` (else unused).
-template <typename E, int D, bool GATHERED>
+template <typename E, int D, int NG, bool GATHERED>
 __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeView& vn, char* smem, unsigned lds0,
-                                              int kvh, int row0, int tile0, int tstride, WaveState<D, 1>& st,
-                                              int rec = 0, bool inlined = false) {
+                                              int kvh, int row0, int tile0, int tstride, WaveState<D, NG>& st,
+                                              int rec, bool inlined) {
   using N = NarrowGeom<D>;
-  constexpr int KS = D / 32, DB = D / 16;
-  constexpr float kSlackN = 8.f;
-  const int lane = threadIdx.x & 63;
+  constexpr int KS = D / 32;
+  const int lane = lane_here();
   const int p = lane & 15, c = lane >> 4;
   const int ntiles = (vn.kv_len + kTileTokens - 1) / kTileTokens;
-  int* idx_lds = reinterpret_cast<int*>(smem + lds0 + N::kBytes);
-  const unsigned tile0_addr = lds_offset(smem) + lds0;  // the wave's K tile; its V tile follows
+  const unsigned tile_addr = lds_offset(smem) + lds0;  // the wave's K tile; its V tile follows, then the index ring
+  const unsigned idx_ring = tile_addr + N::kBytes;
+  const int32_t* entries = GATHERED ? nullptr : a.kv_entries + vn.kv_base;
 
-  // loader role: 16-byte slot `pos` of row `grp_row` in each 1 KB group
-  const int grp_row = lane / N::kChunks, pos = lane % N::kChunks;
   const char* kbase = a.k + 2 * ((int64_t)kvh * a.sk1);
   const char* vbase = a.v + 2 * ((int64_t)kvh * a.sv1);
   const unsigned k_stride = (unsigned)(2 * a.sk0), v_stride = (unsigned)(2 * a.sv0);  // bytes, < 2^32 (checked by the host)
 
-  // operand read addresses: K row 16*tb + p, chunk c (contraction step ks: chunk 4*ks + c);
-  // V tokens 4*c + p/4 (+16), chunk 2*db + (p%4)/2, half p%2
-  unsigned k_addr[2], v_addr[2];
+  // the slot indices of the wave's i-th tile -> ring slot i % 4
+  auto issue_indices = [&](int i, int tile) {
+    if constexpr (!GATHERED) load_direct4(entries, 4u * (unsigned)min(tile * kTileTokens + lane, vn.kv_len - 1), idx_ring + (i & 3) * N::kIdxSlot);
+  };
+  // K (or V) rows of the wave's i-th tile -> its K (V) tile.  Tokens past the run repeat its last token
+  // (their scores are masked, their V rows are finite).
+  auto issue = [&](int i, int tile, bool is_v) {
+    // loader role: 16-byte slot `pos` of row `grp_row` in each 1 KB group
+    const int grp_row = lane / N::kChunks, pos = lane % N::kChunks;
+    // (all index reads first: a load instruction is a fence for the compiler, so reads placed
+    // between the loads would each be waited for on its own)
+    unsigned srow[N::kLoads];
 #pragma unroll
-  for (int tb = 0; tb < 2; ++tb) {
-    const int kr = 16 * tb + p, vr = 16 * tb + 4 * c + (p >> 2);
-    k_addr[tb] = tile0_addr + kr * N::kRowBytes + 16 * ((c & (N::kChunks - 1)) ^ N::swz(kr));
-    v_addr[tb] = tile0_addr + N::kBytesK + vr * N::kRowBytes + 16 * ((((p & 3) >> 1) & (N::kChunks - 1)) ^ N::swz(vr)) + 8 * (p & 1);
-  }
+    for (int g = 0; g < N::kLoads; ++g) {
+      const int row = g * N::kGroupRows + grp_row;
+      if constexpr (GATHERED) srow[g] = (unsigned)(vn.kv_base + min(tile * kTileTokens + row, vn.kv_len - 1));
+      else srow[g] = lds_read4(idx_ring + (i & 3) * N::kIdxSlot + 4 * row);
+    }
+#pragma unroll
+    for (int g = 0; g < N::kLoads; ++g) {
+      const int row = g * N::kGroupRows + grp_row;
+      const char* src = (is_v ? vbase : kbase) + (uint64_t)srow[g] * (is_v ? v_stride : k_stride) + 16 * (pos ^ N::swz(row));
+      load_direct16(src, tile_addr + (is_v ? N::kBytesK : 0) + g * 1024);
+    }
+  };
 
-  // start-up chain: [request id of the lane's row, slot indices] -> [Q fragments, first K/V rows].
-  // Fragment ks of a lane: row row0 + p, dims 32*ks + 8*c .. +7; zero past the vnode.
-  const char* q_src = nullptr;
-  {
-    const int r = min(row0 + p, max(vn.q_len * a.g - 1, 0)), ri = r / a.g, rj = r - ri * a.g;
-    // (the record holds the requests of the first rows; every lane takes part in the exchange)
-    const bool from_record = inlined && vn.q_len <= kNarrowRecRequests;
-    const int listed = from_record ? __shfl(rec, 4 + ri) : 0;
-    if (row0 + p < vn.q_len * a.g) {
-      const int64_t entry = GATHERED ? (int64_t)(vn.q_off / a.nsplit)
-                                     : (from_record ? (int64_t)listed : (int64_t)a.q_entries[vn.q_off + ri]);
-      q_src = a.q + 2 * (entry * a.sq0 + (int64_t)(kvh * a.g + rj) * a.sq1 + 8 * c);
-    }
-  }
-  u32x4 qf[1][KS];
-  reset_state<D, 1>(st);
+  reset_state<D, NG>(st);
   if (tile0 < ntiles) {
-    // slot indices of tokens [idx_base, idx_base + kIdxCap) of the run
-    int idx_base = 0;
-    auto stage_indices = [&](int base) {
-      if constexpr (!GATHERED) {
-        idx_base = base;
-        // (branch free, so that the loads are in flight together; entries past the run repeat its last)
-        int e[N::kIdxCap / kWave];
-#pragma unroll
-        for (int i = 0; i < N::kIdxCap / kWave; ++i)
-          e[i] = a.kv_entries[vn.kv_base + min(base + kWave * i + lane, vn.kv_len - 1)];
-#pragma unroll
-        for (int i = 0; i < N::kIdxCap / kWave; ++i) idx_lds[kWave * i + lane] = e[i];
-        wave_lds_fence();
-      }
-    };
-    // K (or V) rows of `tile` -> the wave's K (V) tile.  Tokens past the run repeat its last
-    // token (their scores are masked, their V rows are finite).  The slot indices are read
-    // from the staged window each time rather than kept in registers between the two calls.
-    auto issue = [&](int tile, bool is_v) {
-      if constexpr (!GATHERED) {
-        if (tile * kTileTokens >= idx_base + N::kIdxCap) stage_indices(tile * kTileTokens);
-      }
-      // (all index reads first: a load instruction is a fence for the compiler, so reads placed
-      // between the loads would each be waited for on its own)
-      unsigned srow[N::kGroups];
-#pragma unroll
-      for (int g = 0; g < N::kGroups; ++g) {
-        const int t = min(tile * kTileTokens + g * N::kGroupRows + grp_row, vn.kv_len - 1);
-        srow[g] = GATHERED ? (unsigned)(vn.kv_base + t) : (unsigned)idx_lds[t - idx_base];
-      }
-#pragma unroll
-      for (int g = 0; g < N::kGroups; ++g) {
-        const int row = g * N::kGroupRows + grp_row;
-        const char* src = (is_v ? vbase : kbase) + (uint64_t)srow[g] * (is_v ? v_stride : k_stride) + 16 * (pos ^ N::swz(row));
-        load_direct16(src, tile0_addr + (is_v ? N::kBytesK : 0) + g * 1024);
-      }
-    };
-    // With the vnode's record at hand and the run's first tile to serve, the first 32 slot
-    // indices are already here: the rows are requested at once, and the rest of the window (if
-    // the run is longer than a tile) arrives beside them.
+    // start-up chain: [requests of the rows, slot indices] -> [Q fragments, first K/V rows].  With the
+    // vnode's record at hand and the run's first tile to serve, the first 32 slot indices are already
+    // here: the rows are requested at once.
     const bool from_record = !GATHERED && inlined && tile0 == 0;
-    int rest[N::kIdxCap / kWave];
     if (from_record) {
-      if (lane >= kNarrowRecSlots && lane < kNarrowRecSlots + kTileTokens) idx_lds[lane - kNarrowRecSlots] = rec;
+      if (lane >= kNarrowRecSlots && lane < kNarrowRecSlots + kTileTokens)
+        *reinterpret_cast<int*>(smem + lds0 + N::kBytes + 4 * (lane - kNarrowRecSlots)) = rec;
       wave_lds_fence();
-      idx_base = 0;
-      issue(0, false);
-      issue(0, true);
-      if (vn.kv_len > kTileTokens) {
-#pragma unroll
-        for (int i = 0; i < N::kIdxCap / kWave; ++i)
-          rest[i] = a.kv_entries[vn.kv_base + min(kWave * i + lane, vn.kv_len - 1)];
-      }
+      issue(0, 0, false);
+      issue(0, 0, true);
     } else {
-      stage_indices(tile0 * kTileTokens);
-      issue(tile0, false);
-      issue(tile0, true);
+      issue_indices(0, tile0);
     }
+    issue_indices(1, tile0 + tstride);
+    // Fragment ks of a lane: row row0 + 16*qb + p, dims 32*ks + 8*c .. +7; zero past the vnode.
+    u32x4 qf[NG][KS];
+    const bool listed_in_record = inlined && vn.q_len <= kNarrowRecRequests;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      u32x4 z = {0u, 0u, 0u, 0u};
-      qf[0][ks] = q_src ? *reinterpret_cast<const u32x4*>(q_src + 64 * ks) : z;
+    for (int qb = 0; qb < NG; ++qb) {
+      const int r = row0 + 16 * qb + p, rc = min(r, max(vn.q_len * a.g - 1, 0)), ri = rc / a.g, rj = rc - ri * a.g;
+      const int listed = listed_in_record ? __shfl(rec, 4 + ri) : 0;   // (every lane takes part in the exchange)
+      const char* src = nullptr;
+      if (r < vn.q_len * a.g) {
+        const int64_t entry = GATHERED ? (int64_t)(vn.q_off / a.nsplit)
+                                       : (listed_in_record ? (int64_t)listed : (int64_t)a.q_entries[vn.q_off + ri]);
+        src = a.q + 2 * (entry * a.sq0 + (int64_t)(kvh * a.g + rj) * a.sq1 + 8 * c);
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        u32x4 z = {0u, 0u, 0u, 0u};
+        qf[qb][ks] = src ? *reinterpret_cast<const u32x4*>(src + 64 * ks) : z;
+      }
+    }
+    if (!from_record) {
+      wait_direct_loads<0>();
+      issue(0, tile0, false);
+      issue(0, tile0, true);
     }
     // nothing the compiler itself tracks may still be in flight below: a wait for it would
     // also wait for every direct load
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    if (from_record && vn.kv_len > kTileTokens) {
-      // (the first tile's rows were requested with the record's indices, which these repeat)
-#pragma unroll
-      for (int i = 0; i < N::kIdxCap / kWave; ++i) idx_lds[kWave * i + lane] = rest[i];
-      wave_lds_fence();
-    }
     // (and the compiler must see the fragments as complete, or it keeps a wait for them in the loop)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[0][ks]));
-    for (int tile = tile0; tile < ntiles; tile += tstride) {
+    for (int qb = 0; qb < NG; ++qb)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[qb][ks]));
+    const WideLane16 la = init_lane16<D>(tile_addr, tile_addr + N::kBytesK);
+    constexpr int kIdxLoads = GATHERED ? 0 : 1;
+    for (int i = 0, tile = tile0; tile < ntiles; ++i, tile += tstride) {
       const int next = tile + tstride;
       const bool more = next < ntiles;
-      const int valid = vn.kv_len - tile * kTileTokens;
-      // ---- S^T = K Q^T : s[tb][j] = score(token 16*tb + 4*c + j, row p)
-      wait_direct_loads<N::kGroups>();  // K landed; V may still be in flight
-      f32x4 s[2];
-#pragma unroll
-      for (int tb = 0; tb < 2; ++tb) {
-        s[tb] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) s[tb] = E::mfma(lds_read16(k_addr[tb] ^ (64u * ks)), qf[0][ks], s[tb]);
-      }
+      f32x4 sc[2][NG];
+      u32x4 pf[NG];
+      VOperands<D> v;
+      wait_direct_loads<N::kLoads>();  // K (and the next tile's indices) landed; V may still be in flight
+      tile_scores<E, D, NG>(la.k, qf, sc);
       if (more) {
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the K tile has been read
-        issue(next, false);
+        issue(i + 1, next, false);
+        issue_indices(i + 2, next + tstride);
       }
-      if (valid < kTileTokens) {
-#pragma unroll
-        for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            if (16 * tb + 4 * c + j >= valid) s[tb][j] = -INFINITY;
-      }
-      // online soft-max with a lazily updated reference (see tile_step)
-      float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])),
-                       fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
-      mx = xor32_max(xor16_max(mx)) * a.scale_log2;
-      const bool grow = mx > st.m[0] + kSlackN;
-      if (__builtin_amdgcn_ballot_w64(grow)) {
-        const float m_new = grow ? mx : st.m[0];
-        const float alpha = __builtin_amdgcn_exp2f(st.m[0] - m_new);
-        st.l[0] *= alpha;
-#pragma unroll
-        for (int db = 0; db < DB; ++db) st.o[0][db] *= alpha;
-        st.m[0] = m_new;
-      }
-      const float neg_m = -st.m[0];
-      float x[8];
-      float sum = 0.f;
-#pragma unroll
-      for (int tb = 0; tb < 2; ++tb)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          x[4 * tb + j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[tb][j], a.scale_log2, neg_m));
-          sum += x[4 * tb + j];
-        }
-      st.l[0] += sum;
-      const u32x4 pf = {E::pack2(x[0], x[1]), E::pack2(x[2], x[3]), E::pack2(x[4], x[5]), E::pack2(x[6], x[7])};
-      // ---- O^T += V^T P^T
-      if (more) wait_direct_loads<N::kGroups>();  // V landed; the next K may be in flight
+      tile_softmax<E, D, NG>(sc, vn.kv_len - tile * kTileTokens, a.scale_log2, st, pf);
+      if (more) wait_direct_loads<N::kLoads + kIdxLoads>();  // V landed; the next K and indices may be in flight
       else wait_direct_loads<0>();
-#pragma unroll
-      for (int db = 0; db < DB; ++db) {
-        const u32x2 lo = lds_read_tr8(v_addr[0] ^ (32u * db));
-        const u32x2 hi = lds_read_tr8(v_addr[1] ^ (32u * db));
-        const u32x4 vf = {lo[0], lo[1], hi[0], hi[1]};
-        st.o[0][db] = E::mfma(vf, pf, st.o[0][db]);
-      }
+      v.request(la.v, 0);
+      tile_pv<E, D, NG>(la.v, v, pf, st);
       if (more) {
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the V tile has been read
-        issue(next, true);
+        issue(i + 1, next, true);
       }
     }
   }
-  finish_state<D, 1>(st);
+  finish_state<D, NG>(st);
 }
 
 // Merge of the `share` waves of one narrow vnode (same rows, interleaved tiles) into the first of
 // them, pairwise through LDS at xchg.  Every wave of the block calls this (block barriers).
-template <int D>
-__device__ __forceinline__ void merge_shares(float* xchg, WaveState<D, 1>& st, int w, int share) {
-  constexpr int NV = (D / 16) * 4 + 2;  // floats of state per lane
+template <int D, int NG>
+__device__ __forceinline__ void merge_shares(float* xchg, WaveState<D, NG>& st, int w, int share) {
+  constexpr int NV = (D / 16) * 4 + 2;  // floats of state per lane and row group
+  static_assert(2 * NG * NV * 4 * kWave <= 4 * NarrowGeom<D>::kLds && NG * NV * 4 * kWave <= 2 * NarrowGeom<D>::kLds,
+                "half of the waves' states fit the LDS areas of all of them");
   const int lane = threadIdx.x & 63;
   for (int half = share >> 1; half >= 1; half >>= 1) {
     __syncthreads();
     if (w >= half && w < 2 * half) {
-      float* dst = xchg + (size_t)(w - half) * NV * kWave + lane;
+      float* dst = xchg + (size_t)(w - half) * NG * NV * kWave + lane;
       int n = 0;
-      dst[(n++) * kWave] = st.m[0];
-      dst[(n++) * kWave] = st.l[0];
 #pragma unroll
-      for (int db = 0; db < D / 16; ++db)
+      for (int qb = 0; qb < NG; ++qb) {
+        dst[(n++) * kWave] = st.m[qb];
+        dst[(n++) * kWave] = st.l[qb];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) dst[(n++) * kWave] = st.o[0][db][j];
+        for (int db = 0; db < D / 16; ++db)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) dst[(n++) * kWave] = st.o[qb][db][j];
+      }
     }
     __syncthreads();
     if (w < half) {
-      const float* src = xchg + (size_t)w * NV * kWave + lane;
+      const float* src = xchg + (size_t)w * NG * NV * kWave + lane;
       int n = 0;
-      const float m2 = src[(n++) * kWave];
-      const float l2 = src[(n++) * kWave];
-      const float m = fmaxf(st.m[0], m2);
-      const float a1 = scale_from(st.m[0], m), a2 = scale_from(m2, m);
-      st.l[0] = st.l[0] * a1 + l2 * a2;
-      st.m[0] = m;
 #pragma unroll
-      for (int db = 0; db < D / 16; ++db)
+      for (int qb = 0; qb < NG; ++qb) {
+        const float m2 = src[(n++) * kWave];
+        const float l2 = src[(n++) * kWave];
+        const float m = fmaxf(st.m[qb], m2);
+        const float a1 = scale_from(st.m[qb], m), a2 = scale_from(m2, m);
+        st.l[qb] = st.l[qb] * a1 + l2 * a2;
+        st.m[qb] = m;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) st.o[0][db][j] = st.o[0][db][j] * a1 + src[(n++) * kWave] * a2;
+        for (int db = 0; db < D / 16; ++db)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) st.o[qb][db][j] = st.o[qb][db][j] * a1 + src[(n++) * kWave] * a2;
+      }
     }
   }
+}
+
+// What one wave does for a narrow vnode in one pass (NG row groups from row0; none if row0 is past
+// its rows, and then the wave only keeps the block's barriers company).
+struct NarrowPass {
+  int kvh, row0, w, share, rec;
+  bool inlined;
+  unsigned lds0;      // byte offset of the wave's area in the block's LDS segment
+  unsigned xchg;      // and of the areas of the waves that share the vnode
+};
+template <typename E, int D, int NG, bool GATHERED>
+__device__ __forceinline__ void narrow_pass(const Stage1Args& a, char* smem, const VnodeView& vn, const NarrowPass& p) {
+  WaveState<D, NG> st;
+  const bool rows = p.row0 < vn.q_len * a.g;
+  if (rows) narrow_attend<E, D, NG, GATHERED>(a, vn, smem, p.lds0, p.kvh, p.row0, p.w, p.share, st, p.rec, p.inlined);
+  else reset_state<D, NG>(st);
+  if (p.share > 1) merge_shares<D, NG>(reinterpret_cast<float*>(smem + p.xchg), st, p.w, p.share);
+  if (rows && p.w == 0) write_partials<D, NG>(a, vn, p.kvh, p.row0, st);
 }
 
 // A narrow vnode served by `share` consecutive waves of a block (share = 1, 2 or 4, the same
 // for the whole launch; the host picks more than one when there are fewer vnodes than wave
 // slots): wave w of the vnode takes the tiles w, w + share, ..., and the shares are merged
 // through LDS.  `slot` is the wave's index in the block; a wave without a vnode (exists ==
-// false) only keeps the block's barriers company.
+// false) only keeps the block's barriers company.  More rows than a pass holds take several passes, as
+// even as possible.
 template <typename E, int D, bool GATHERED>
 __device__ __forceinline__ void narrow_item(const Stage1Args& a, char* smem, int slot, int share, bool exists,
                                             int vnode, int kvh) {
   using N = NarrowGeom<D>;
-  const unsigned lds0 = (unsigned)slot * N::kLds;  // byte offset of the wave's area in the block's LDS segment
   VnodeView vn{0, 0, 0, 0};
-  int rec = 0;
-  const bool inlined = !GATHERED && a.narrow_table != nullptr;   // launch uniform
-  if (inlined) {
-    if (exists) rec = a.narrow_table[(int64_t)(vnode - a.narrow_begin) * kNarrowRecord + (threadIdx.x & 63)];
-    vn.kv_base = __builtin_amdgcn_readlane(rec, 0);
-    vn.kv_len = __builtin_amdgcn_readlane(rec, 1);
-    vn.q_off = __builtin_amdgcn_readlane(rec, 2);
-    vn.q_len = __builtin_amdgcn_readlane(rec, 3);
+  NarrowPass p;
+  p.kvh = kvh;
+  p.share = share;
+  p.w = slot & (share - 1);
+  p.lds0 = (unsigned)slot * N::kLds;
+  p.xchg = (unsigned)(slot - p.w) * N::kLds;
+  p.rec = 0;
+  p.inlined = !GATHERED && a.narrow_table != nullptr;   // launch uniform
+  if (p.inlined) {
+    if (exists) p.rec = a.narrow_table[(int64_t)(vnode - a.narrow_begin) * kNarrowRecord + (threadIdx.x & 63)];
+    vn.kv_base = __builtin_amdgcn_readlane(p.rec, 0);
+    vn.kv_len = __builtin_amdgcn_readlane(p.rec, 1);
+    vn.q_off = __builtin_amdgcn_readlane(p.rec, 2);
+    vn.q_len = __builtin_amdgcn_readlane(p.rec, 3);
   } else if (exists) {
-    vn = load_vnode<GATHERED>(a, vnode);
+    vn = uniform(load_vnode<GATHERED>(a, vnode));
   }
-  const int rows_total = vn.q_len * a.g;
-  if (share == 1) {
-    for (int row0 = 0; row0 < rows_total; row0 += 16) {
-      WaveState<D, 1> st;
-      narrow_attend<E, D, GATHERED>(a, vn, smem, lds0, kvh, row0, 0, 1, st, rec, inlined);
-      write_partials<D, 1>(a, vn, kvh, row0, st);
-    }
-    return;
+  int groups = (vn.q_len * a.g + 15) >> 4;
+  if (share > 1) {
+    // every wave of the block makes the same passes (block barriers inside): the most row groups any of
+    // its vnodes has, agreed on through one word of each wave's LDS area
+    const int nwaves = blockDim.x >> 6;
+    *reinterpret_cast<volatile int*>(smem + p.lds0) = groups;
+    __syncthreads();
+    for (int i = 0; i < nwaves; ++i) groups = max(groups, *reinterpret_cast<volatile int*>(smem + (size_t)i * N::kLds));
+    groups = __builtin_amdgcn_readfirstlane(groups);
+    __syncthreads();
   }
-  const int w = slot & (share - 1);
-  float* xchg = reinterpret_cast<float*>(smem + (size_t)(slot - w) * N::kLds);
-  // every wave of the block makes the same number of passes (block barriers inside): the most
-  // any of its vnodes needs, agreed on through one word of each wave's LDS area
-  const int nwaves = blockDim.x >> 6;
-  *reinterpret_cast<volatile int*>(smem + lds0) = (rows_total + 15) >> 4;
-  __syncthreads();
-  int passes = 0;
-  for (int i = 0; i < nwaves; ++i) passes = max(passes, *reinterpret_cast<volatile int*>(smem + (size_t)i * N::kLds));
-  __syncthreads();
-  for (int pass = 0; pass < passes; ++pass) {
-    const int row0 = 16 * pass;
-    WaveState<D, 1> st;
-    if (row0 < rows_total) narrow_attend<E, D, GATHERED>(a, vn, smem, lds0, kvh, row0, w, share, st, rec, inlined);
-    else reset_state<D, 1>(st);
-    merge_shares<D>(xchg, st, w, share);
-    if (w == 0 && row0 < rows_total) write_partials<D, 1>(a, vn, kvh, row0, st);
-    __syncthreads();  // the exchange area is the staging area of the next pass
+  const int passes = (groups + N::kGroups - 1) / N::kGroups;
+  for (int pass = 0, done = 0; pass < passes; ++pass) {
+    const int ng = (groups - done + passes - pass - 1) / (passes - pass);
+    p.row0 = 16 * done;
+    done += ng;
+    if (ng == 2) narrow_pass<E, D, 2, GATHERED>(a, smem, vn, p);
+    else narrow_pass<E, D, 1, GATHERED>(a, smem, vn, p);
+    if (share > 1) __syncthreads();  // the exchange area is the staging area of the next pass
   }
 }
 
@@ -1311,7 +1462,7 @@ __device__ __forceinline__ void narrow_item(const Stage1Args& a, char* smem, int
 // waves: the footprint of one LDS tile per wave instead of a wide block's ring, so that more of
 // these latency-bound waves share a compute unit.
 template <typename E, int D, bool GATHERED>
-__global__ void __launch_bounds__(kWideBlock) stage1_narrow_kernel(Stage1Args a) {
+__global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 2) stage1_narrow_kernel(Stage1Args a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int local_vnode = blockIdx.x / a.hkv;
@@ -1331,7 +1482,7 @@ __global__ void __launch_bounds__(kWideBlock) stage1_narrow_kernel(Stage1Args a)
 // run twice.  The first vnode of a group carries the group; the others become empty items.
 constexpr int kMaxRanked = kWideBlock;
 template <bool GATHERED>
-__device__ __forceinline__ int wide_vnode_of_rank(const Stage1Args& a, char* smem, int target, VnodeView& view) {
+__device__ __forceinline__ int wide_vnode_of_rank(const Stage1Args& a, char* smem, int target, int rows, VnodeView& view) {
   const int n = a.vnode_count;
   if (n < 2 || n > kMaxRanked) {
     view = load_vnode<GATHERED>(a, a.vnode_begin + target);
@@ -1380,7 +1531,7 @@ __device__ __forceinline__ int wide_vnode_of_rank(const Stage1Args& a, char* sme
       }
     }
     // groups of m vnodes from the start of the chain; the chain's first vnode is a full query tile
-    const long long cap = (long long)kWideRows * a.wide_chunks;
+    const long long cap = (long long)rows * a.wide_chunks;
     const long long tile_rows = max(1LL, (long long)views[first].q_len * a.g);
     const int m = (int)max(1LL, cap / tile_rows);
     const int head = first + (tid - first) / m * m;
@@ -1426,70 +1577,84 @@ __device__ __forceinline__ int wide_vnode_of_rank(const Stage1Args& a, char* sme
 // Launch order of the fused kernel.  Wide blocks come rank-major, then row chunk, kv head fastest
 // (blocks that stream the same KV run are launched together and share it in L2); the narrow
 // blocks follow and fill the machine while the wide blocks drain.
-template <typename E, int D, bool GATHERED>
+// PROGRAMS: the wide vnodes come as block programs (Stage1Args::prog_table), else as the planner's list.
+template <typename E, int D, bool GATHERED, bool PROGRAMS>
 __global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 512 / kWideBlock) stage1_fused_kernel(Stage1Args a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int wide_blocks = a.prog_table ? a.num_programs * a.hkv : a.vnode_count * a.wide_chunks * a.hkv;
-  const int wide_index = blockIdx.x, narrow_index = (int)blockIdx.x - wide_blocks;
-  const bool is_wide = (int)blockIdx.x < wide_blocks;
-  if (is_wide && a.prog_table) {
+  const int wide_blocks = PROGRAMS ? a.num_programs * a.hkv : a.vnode_count * a.wide_chunks * a.hkv;
+  const int narrow_index = (int)blockIdx.x - wide_blocks;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // this block's wide vnodes [wide_first, wide_end) and, per wave, its narrow vnodes: item, item + step, .. below
+  // item_end, numbered vnode-major with hkv items each
+  int wide_first = 0, wide_end = 0, kvh = 0, chunk = 0, chunks = 1;
+  int share = 1, item = 0, item_end = 0, step = kWideWaves;
+  bool narrow_first = false;
+  int* record = nullptr;
+  VnodeView vn{0, 0, 0, 0};
+  if (narrow_index < 0 && PROGRAMS) {
     // A block program written by the host, for one kv head (kv head fastest: the eight blocks of
     // a program land on the eight XCDs, and a head's K/V only ever enters one XCD's L2): its wide
     // vnodes one after the other, and its narrow vnodes, one wave each, before or after them.
     // Of the two blocks that share a compute unit one starts with its narrow vnodes and the
     // other ends with them, so that the memory-bound narrow vnodes of one run under the
     // arithmetic-bound wide vnodes of the other.
-    const int program = wide_index / a.hkv;
-    const int kvh = wide_index - program * a.hkv;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wide_first = a.prog_table[4 * program], wide_end = a.prog_table[4 * program + 1];
-    const int narrow_first = a.prog_table[4 * program + 2], narrow_signed = a.prog_table[4 * program + 3];
-    const int narrow_count = narrow_signed < 0 ? -narrow_signed : narrow_signed;
-    auto narrow_vnodes = [&]() {
-      for (int i = wave; i < narrow_count; i += kWideWaves)
-        narrow_item<E, D, GATHERED>(a, smem, wave, 1, true, a.narrow_begin + narrow_first + i, kvh);
-      __syncthreads();  // the waves' tiles become the ring of the next wide vnode
-    };
+    const int program = (int)blockIdx.x / a.hkv;
+    kvh = (int)blockIdx.x - program * a.hkv;
+    wide_first = a.prog_table[4 * program];
+    wide_end = a.prog_table[4 * program + 1];
+    const int first = a.prog_table[4 * program + 2], count = a.prog_table[4 * program + 3];
+    narrow_first = count < 0;
+    item = first + wave;
+    item_end = first + (count < 0 ? -count : count);
     // the program's record, requested together with its table entry
-    int* record = reinterpret_cast<int*>(smem + WideGeom<D>::kRecord);
-    const bool with_records = !GATHERED && D <= 128 && a.prog_records != nullptr;   // launch uniform
-    if (with_records) {
+    if (!GATHERED && a.prog_records != nullptr) {   // launch uniform
+      record = reinterpret_cast<int*>(smem + WideGeom<D>::kRecord);
       record[threadIdx.x] = a.prog_records[(int64_t)program * kProgRecord + threadIdx.x];
       __syncthreads();
+      if (narrow_first || __builtin_amdgcn_readfirstlane(record[4]) == 0) record = nullptr;   // block uniform
     }
-    if (narrow_signed < 0) narrow_vnodes();
-    for (int v = wide_first; v < wide_end; ++v) {
-      if (with_records && narrow_signed >= 0 && v == wide_first && record[4] != 0) {
-        const VnodeView vn{record[2], record[3], record[1], (int64_t)record[0]};
-        wide_block<E, D, GATHERED>(a, smem, vn, kvh, 0, 1, record);
-      } else {
-        const VnodeView vn = load_vnode<GATHERED>(a, a.vnode_begin + v);
-        wide_block<E, D, GATHERED>(a, smem, vn, kvh, 0, 1);
-      }
-    }
-    if (narrow_signed > 0) narrow_vnodes();
-  } else if (is_wide) {
+  } else if (narrow_index < 0) {
     const int per_rank = a.wide_chunks * a.hkv;
-    const int rank = wide_index / per_rank;
-    const int rest = wide_index - rank * per_rank;
+    const int rank = (int)blockIdx.x / per_rank;
+    const int rest = (int)blockIdx.x - rank * per_rank;
     // Launch slot `rest / hkv` of a rank serves chunk (slot + rank / 2) % chunks.  Consecutive
     // blocks of one kv head go round robin to the four shader engines of an XCD, strictly in
     // order (a block waits for its engine even when others have room); without the rotation an
     // engine would only ever get first chunks, which run longer than last ones.
     const int slot = rest / a.hkv;
-    const int chunk = (slot + (rank >> 1)) % a.wide_chunks;
-    VnodeView vn;
-    (void)wide_vnode_of_rank<GATHERED>(a, smem, rank, vn);
-    wide_block<E, D, GATHERED>(a, smem, vn, rest - slot * a.hkv, chunk, a.wide_chunks);
+    kvh = rest - slot * a.hkv;
+    chunks = a.wide_chunks;
+    chunk = (slot + (rank >> 1)) % chunks;
+    (void)wide_vnode_of_rank<GATHERED>(a, smem, rank, WideRows<D>::kBlock, vn);
+    wide_end = 1;
   } else {
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int share = a.narrow_share;
-    const int item = narrow_index * (kWideWaves / share) + wave / share + a.narrow_in_programs * a.hkv;
-    const bool exists = item < a.narrow_count * a.hkv;
-    if (share == 1 && !exists) return;  // whole wave; no block barrier below in this mode
-    const int local_vnode = item / a.hkv;
-    const int kvh = item - local_vnode * a.hkv;
-    narrow_item<E, D, GATHERED>(a, smem, wave, share, exists, a.narrow_begin + local_vnode, kvh);
+    share = a.narrow_share;
+    item = narrow_index * (kWideWaves / share) + wave / share + a.narrow_in_programs * a.hkv;
+    item_end = a.narrow_count * a.hkv;
+    step = 1 << 30;   // one item (item + step stays below 2^31: the host bounds the items)
+  }
+  // (one call each, in either order, so that the kernel holds one copy of the code)
+#pragma unroll 1
+  for (int turn = 0; turn < 2; ++turn) {
+    if ((turn == 0) != narrow_first) {
+      for (int v = wide_first; v < wide_end; ++v) {
+        if (PROGRAMS) {
+          if (record) vn = VnodeView{record[2], record[3], record[1], (int64_t)record[0]};
+          else vn = load_vnode<GATHERED>(a, a.vnode_begin + v);
+        }
+        wide_block<E, D, GATHERED>(a, smem, vn, kvh, chunk, chunks, record);
+        record = nullptr;
+      }
+    } else {
+      // (trailing blocks: one turn for every wave, with or without an item; a wave that shares no vnode and
+      // has none is done)
+      for (bool first = true; item < item_end || (first && share > 1); item += step, first = false) {
+        const bool trailing = narrow_index >= 0;
+        const int vnode = trailing ? item / a.hkv : item;
+        narrow_item<E, D, GATHERED>(a, smem, wave, share, item < item_end, a.narrow_begin + vnode, trailing ? item - vnode * a.hkv : kvh);
+      }
+      if (PROGRAMS && narrow_first) __syncthreads();  // the waves' tiles become the ring of the next wide vnode
+    }
   }
 }
 
@@ -1546,7 +1711,7 @@ __global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 2) deft_stage1_kerne
   const int nchunks = (vn.kv_len + kDeftChunk - 1) / kDeftChunk;
   const int h = lane >> 5;
 
-  for (int row0 = 0; row0 < rows_total; row0 += kWideRows) {
+  for (int row0 = 0; row0 < rows_total; row0 += kDeftRows) {
     const int my_row0 = row0 + 32 * wave;
     const bool active = my_row0 < rows_total;
     const char* q_src = q_row_address32<false>(a, vn, kvh, active ? my_row0 : rows_total);
@@ -1557,7 +1722,7 @@ __global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 2) deft_stage1_kerne
     // the lane's request within the subtree's query set, its mask group and its bit in the group's words
     const int my_req = min(my_row0 + (lane & 31), rows_total - 1) / a.g;
     const int first_group = (row0 / a.g) / d.mask_len;
-    const int groups_here = min((min(row0 + kWideRows, rows_total) - 1) / a.g / d.mask_len - first_group + 1, kDeftMaskGroups);
+    const int groups_here = min((min(row0 + kDeftRows, rows_total) - 1) / a.g / d.mask_len - first_group + 1, kDeftMaskGroups);
     const int my_group = min(my_req / d.mask_len - first_group, kDeftMaskGroups - 1);
     const int my_bit = my_req & (d.mask_len - 1);
     const bool upper = my_bit >= 32;
@@ -1631,6 +1796,8 @@ struct Stage2Args {
   char* o;
   int64_t oo0, oo1;
   int batch, hq;
+  int longest; // no request has more partials than this (the number of vnodes, or more)
+  int splits;  // lane groups that share one (request, head): a power of two, set by the launcher
   int nsplit;  // > 0: gathered mode, request r owns rows [r*nsplit, (r+1)*nsplit)
   // (or null) one record of kReqRecord int32 per request, written by the host: req_lens[r],
   // req_offs[r], then the request's first kReqRecord - 2 entries -- what the block needs before
@@ -1651,18 +1818,26 @@ template <int WIDTH> __device__ __forceinline__ float group_sum(float x) {
   return x;
 }
 
-// A group of D/4 lanes owns one (request, head): lane i fetches the row index and the
-// log-sum-exp of partial i, the group reduces max and weight sum with shuffles, then every
-// lane accumulates its own 4 output dims over the partials, taking weight and row index of
-// partial i from lane i.
+// A group of D/4 lanes serves one (request, head), or every splits-th partial of one: lane i fetches the
+// row index and the log-sum-exp of the group's partial i, the group reduces max and weight sum with
+// shuffles, then every lane accumulates its own 4 output dims over the partials, taking weight and
+// row index of partial i from lane i.  The `splits` groups of a (request, head) sit in one block and
+// are merged through LDS.
+//
+// Bound by the partial rows it reads, and for a batch of few requests by how many of them are in
+// flight: 8 requests x 64 heads with 68 partials each take 64 blocks 11.2 us, one split per group of
+// lanes; with the partials split eight ways 512 blocks.
 template <typename E, int D>
 __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
   constexpr int LPH = D / 4;
   constexpr int HPB = kBlock / LPH;
   const int grp = threadIdx.x / LPH, gl = threadIdx.x % LPH;
   const int req = blockIdx.x;
-  const int head = blockIdx.y * HPB + grp;
-  if (head >= a.hq) return;
+  int S = a.splits;                                         // (a power of two; launch uniform)
+  int split = grp & (S - 1);
+  const int head = blockIdx.y * (HPB / S) + grp / S;
+  const bool exists = head < a.hq;
+  if (S == 1 && !exists) return;
   const int32_t* rec = a.req_table ? a.req_table + (int64_t)req * kReqRecord : nullptr;  // launch uniform
   int off, n, rec_row = -1;
   if (a.nsplit > 0) {
@@ -1676,16 +1851,24 @@ __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
     off = a.req_offs[req];
     n = a.req_lens[req];
   }
+  if (S > 1 && n <= kReqRecEntries) {   // block uniform: a short list is one group's work (merging costs about 1 us)
+    if (split > 0 || !exists) return;
+    S = 1;
+    split = 0;
+  }
+  const int first = split + S * gl;                         // this lane's first entry of the request's list
+  const int mine = exists ? (n - split + S - 1) / S : 0;    // partials of this group (0 or less: none)
 
   float m_run = -INFINITY, l_run = 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int base = 0; base < n; base += LPH) {
-    const int cnt = min(LPH, n - base);
+  for (int base = 0; base < mine; base += LPH) {
+    const int cnt = min(LPH, mine - base);
     int my_row = -1;
     if (gl < cnt) {
-      if (a.nsplit > 0) my_row = off + base + gl;
-      else if (rec && base + gl < kReqRecEntries) my_row = base == 0 ? rec_row : rec[2 + base + gl];
-      else my_row = a.req_entries[off + base + gl];
+      const int entry = first + S * base;
+      if (a.nsplit > 0) my_row = off + entry;
+      else if (rec && entry < kReqRecEntries) my_row = S == 1 && base == 0 ? rec_row : rec[2 + entry];
+      else my_row = a.req_entries[off + entry];
     }
     // Rows in batches of kBatch, all loads of a batch issued before the first is used (the rows
     // are in bounds whatever their weight; a zero weight discards the row's contents).  The
@@ -1717,6 +1900,28 @@ __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[e] += (wi != 0.f) ? part[j][e] * wi : 0.f;
       }
+    }
+  }
+  if (S > 1) {
+    // the groups' states to the first of them
+    __shared__ f32x4 acc_of[kBlock];
+    __shared__ float m_of[HPB], l_of[HPB];
+    acc_of[threadIdx.x] = acc;
+    if (gl == 0) {
+      m_of[grp] = m_run;
+      l_of[grp] = l_run;
+    }
+    __syncthreads();
+    if (split > 0 || !exists) return;
+    float m_all = m_run;
+    for (int i = 1; i < S; ++i) m_all = fmaxf(m_all, m_of[grp + i]);
+    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    l_run = 0.f;
+    for (int i = 0; i < S; ++i) {
+      const float m_i = m_of[grp + i];
+      const float w = (m_i == -INFINITY) ? 0.f : __expf(m_i - m_all);
+      l_run += l_of[grp + i] * w;
+      acc += acc_of[threadIdx.x + i * LPH] * w;
     }
   }
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
@@ -1816,12 +2021,12 @@ inline int narrow_share_for(int64_t items, int head_dim) {
   return share;
 }
 
-template <typename E, int D, bool GATHERED>
+template <typename E, int D, bool GATHERED, bool PROGRAMS>
 int launch_stage1_fused(const Stage1Args& a0, hipStream_t stream) {
   constexpr size_t kWideLds = (size_t)WideGeom<D>::kLds;
   constexpr size_t kNarrowLds = (size_t)kWideWaves * NarrowGeom<D>::kLds;
   constexpr size_t lds = kWideLds > kNarrowLds ? kWideLds : kNarrowLds;
-  auto kern = stage1_fused_kernel<E, D, GATHERED>;
+  auto kern = stage1_fused_kernel<E, D, GATHERED, PROGRAMS>;
   // (raising the dynamic LDS limit is idempotent: two threads that both find the flag clear both raise it)
   static std::atomic<bool> configured_on[kMaxDevices];
   std::atomic<bool>& configured = configured_on[current_device()];
@@ -1837,9 +2042,9 @@ int launch_stage1_fused(const Stage1Args& a0, hipStream_t stream) {
   a.narrow_share = narrow_share_for(narrow_items, D);
   const int per_block = kWideWaves / a.narrow_share;
   const int64_t narrow_blocks = (narrow_items + per_block - 1) / per_block;
-  a.wide_chunks = std::max(1, std::min(8, (a.wide_rows + kWideRows - 1) / kWideRows));
+  a.wide_chunks = std::max(1, std::min(8, (a.wide_rows + WideRows<D>::kBlock - 1) / WideRows<D>::kBlock));
   a.block_slots = (D > 128 ? wave_slots() / 2 : wave_slots()) / kWideWaves;
-  const int64_t wide_blocks = a.prog_table ? (int64_t)a.num_programs * a.hkv : (int64_t)a.vnode_count * a.wide_chunks * a.hkv;
+  const int64_t wide_blocks = PROGRAMS ? (int64_t)a.num_programs * a.hkv : (int64_t)a.vnode_count * a.wide_chunks * a.hkv;
   const int64_t blocks = wide_blocks + narrow_blocks;
   if (blocks == 0) return FT_OK;
   if (blocks > INT32_MAX) return FT_ERR_ARGUMENT;
@@ -1888,7 +2093,10 @@ int launch_stage1_d(const Stage1Args& a, hipStream_t stream) {
     return FT_OK;
   } else {
     if (a.vnode_count == 0 && !a.prog_table) return launch_stage1_narrow<E, D, GATHERED>(a, stream);
-    return launch_stage1_fused<E, D, GATHERED>(a, stream);
+    if constexpr (!GATHERED) {
+      if (a.prog_table) return launch_stage1_fused<E, D, false, true>(a, stream);
+    }
+    return launch_stage1_fused<E, D, GATHERED, false>(a, stream);
   }
 }
 
@@ -1909,10 +2117,17 @@ int launch_stage1(const Stage1Args& a, int d, int dtype, hipStream_t stream) {
   return FT_ERR_DTYPE;
 }
 
+// Lane groups per (request, head): as many as leave the launch at most four blocks per compute unit
+// (wave_slots() / 2): more blocks than that hide each other's round trips anyway.  One group where every
+// list is short.
 template <typename E, int D>
-int launch_stage2_inst(const Stage2Args& a, hipStream_t stream) {
+int launch_stage2_inst(const Stage2Args& a0, hipStream_t stream) {
   constexpr int HPB = kBlock / (D / 4);
-  hipLaunchKernelGGL((stage2_kernel<E, D>), dim3((unsigned)a.batch, (unsigned)((a.hq + HPB - 1) / HPB), 1),
+  Stage2Args a = a0;
+  a.splits = 1;
+  while (a.longest > kReqRecEntries && a.splits < HPB && (int64_t)a.batch * ((a.hq * a.splits * 2 + HPB - 1) / HPB) <= wave_slots() / 2) a.splits *= 2;
+  const int heads = HPB / a.splits;
+  hipLaunchKernelGGL((stage2_kernel<E, D>), dim3((unsigned)a.batch, (unsigned)((a.hq + heads - 1) / heads), 1),
                      dim3(kBlock, 1, 1), 0, stream, a);
   return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
 }
@@ -1935,8 +2150,7 @@ int launch_stage2(const Stage2Args& a, int d, int dtype, hipStream_t stream) {
 
 template <typename E, int D>
 int launch_deft_inst(const DeftArgs& d, hipStream_t stream) {
-  constexpr size_t lds = (size_t)WideGeom<D>::kLds;
-  static_assert(kDeftMaskGroups * kDeftChunk * 8 <= 4 * WideGeom<D>::kIdxCap, "the mask words share the index area");
+  constexpr size_t lds = (size_t)WideGeom<D>::kRing + kDeftMaskGroups * kDeftChunk * 8;   // two super tiles and the mask words
   auto kern = deft_stage1_kernel<E, D>;
   static std::atomic<bool> configured_on[kMaxDevices];
   std::atomic<bool>& configured = configured_on[current_device()];
@@ -2102,7 +2316,7 @@ static int stage2_with_table(const int32_t* req_to_vnode_entries, const int32_t*
                              const int32_t* req_to_vnode_lens, const int32_t* req_table,
                              const float* mid_o, int64_t so0, int64_t so1, const float* mid_lse, int64_t sl0,
                              void* o, int64_t oo0, int64_t oo1,
-                             int batch_size, int num_qo_heads, int head_dim, int dtype, ft_stream_t stream) {
+                             int64_t num_vnodes, int batch_size, int num_qo_heads, int head_dim, int dtype, ft_stream_t stream) {
   if (int rc = check_common(head_dim, 1, dtype)) return rc;
   if (batch_size == 0) return FT_OK;
   if (!req_to_vnode_entries || !req_to_vnode_offs || !req_to_vnode_lens || !mid_o || !mid_lse || !o)
@@ -2114,6 +2328,7 @@ static int stage2_with_table(const int32_t* req_to_vnode_entries, const int32_t*
   a.mid_o = mid_o; a.so0 = so0; a.so1 = so1; a.mid_lse = mid_lse; a.sl0 = sl0;
   a.o = static_cast<char*>(o); a.oo0 = oo0; a.oo1 = oo1;
   a.batch = batch_size; a.hq = num_qo_heads; a.nsplit = 0;
+  a.longest = (int)std::min<int64_t>(num_vnodes, INT32_MAX);
   a.req_table = req_table;
   return launch_stage2(a, head_dim, dtype, stream);
 }
@@ -2124,7 +2339,7 @@ int ft_stage2(const int32_t* req_to_vnode_entries, const int32_t* req_to_vnode_o
               void* o, int64_t oo0, int64_t oo1,
               int batch_size, int num_qo_heads, int head_dim, int dtype, ft_stream_t stream) {
   return stage2_with_table(req_to_vnode_entries, req_to_vnode_offs, req_to_vnode_lens, nullptr, mid_o, so0, so1, mid_lse,
-                           sl0, o, oo0, oo1, batch_size, num_qo_heads, head_dim, dtype, stream);
+                           sl0, o, oo0, oo1, INT32_MAX, batch_size, num_qo_heads, head_dim, dtype, stream);
 }
 
 int ft_stage1_phases(const void* q, const void* k, const void* v,
@@ -2212,7 +2427,7 @@ int ft_stage1_programs(const void* q, const void* k, const void* v,
   if (num_programs > 0) { a.prog_table = prog_table; a.num_programs = num_programs; a.narrow_in_programs = narrow_in_programs; }
   a.narrow_table = narrow_table;
   a.prog_records = num_programs > 0 ? prog_records : nullptr;
-  a.wide_rows = kWideRows;
+  a.wide_rows = 1;   // (a program's block serves all row pieces of its vnodes)
   return launch_stage1<false>(a, head_dim, dtype, stream);
 }
 
@@ -2237,7 +2452,8 @@ int ft_decode_programs(const void* q, const void* k, const void* v, void* o,
                                   sm_scale, dtype, stream))
     return rc;
   return stage2_with_table(req_to_vnode_entries, req_to_vnode_offs, req_to_vnode_lens, req_table, mid_o, so0, so1,
-                           mid_lse, sl0, o, oo0, oo1, batch_size, num_qo_heads, head_dim, dtype, stream);
+                           mid_lse, sl0, o, oo0, oo1, (int64_t)phase_node_nums[0] + phase_node_nums[1], batch_size, num_qo_heads, head_dim, dtype,
+                           stream);
 }
 
 int ft_decode_static(const void* q, const void* k, const void* v, void* o,
@@ -2289,8 +2505,8 @@ int ft_decode(const void* q, const void* k, const void* v, void* o,
                                 mid_lse, sl0, phase_node_nums, phase_node_offsets, phase_q_tile_sizes,
                                 phase_kv_tile_sizes, num_qo_heads, num_kv_heads, head_dim, sm_scale, dtype, stream))
     return rc;
-  return ft_stage2(req_to_vnode_entries, req_to_vnode_offs, req_to_vnode_lens, mid_o, so0, so1, mid_lse, sl0, o, oo0,
-                   oo1, batch_size, num_qo_heads, head_dim, dtype, stream);
+  return stage2_with_table(req_to_vnode_entries, req_to_vnode_offs, req_to_vnode_lens, nullptr, mid_o, so0, so1, mid_lse, sl0, o,
+                           oo0, oo1, (int64_t)phase_node_nums[0] + phase_node_nums[1], batch_size, num_qo_heads, head_dim, dtype, stream);
 }
 
 int ft_deft_stage1(const void* q, const void* k, const void* v,
@@ -2317,7 +2533,7 @@ int ft_deft_stage1(const void* q, const void* k, const void* v,
   // a power of two of at most 64 requests per mask word, and few enough words per token for the
   // 128 query rows a block serves at a time
   if (mask_len < 1 || mask_len > 64 || (mask_len & (mask_len - 1)) != 0) return FT_ERR_ARGUMENT;
-  const int requests_per_pass = (kWideRows + g - 1) / g + 1;
+  const int requests_per_pass = (kDeftRows + g - 1) / g + 1;
   if ((requests_per_pass + mask_len - 1) / mask_len + 1 > kDeftMaskGroups) return FT_ERR_ARGUMENT;
   d.causalmask = causalmask;
   d.causalmask_offset = causalmask_offset;
@@ -2384,7 +2600,7 @@ int ft_gathered_decode(const void* q, const void* k_cache, const void* v_cache,
   Stage2Args b{};
   b.mid_o = mid_o; b.so0 = a.so0; b.so1 = a.so1; b.mid_lse = mid_lse; b.sl0 = a.sl0;
   b.o = static_cast<char*>(o); b.oo0 = oo0; b.oo1 = oo1;
-  b.batch = batch_size; b.hq = num_qo_heads; b.nsplit = nsplit;
+  b.batch = batch_size; b.hq = num_qo_heads; b.nsplit = nsplit; b.longest = nsplit;
   return launch_stage2(b, head_dim, dtype, stream);
 }
 

@@ -1,0 +1,608 @@
+// Launch schedule of the first decode stage: vnode lists re-cut into block programs for a device.
+// Declarations and array layouts: include/fasttree_schedule.h.
+//
+// A launch holds two kinds of work.  *Wide* vnodes (more than 16 query rows) are served by blocks of
+// four waves and are bound by the matrix instructions; *narrow* ones by a wave each, bound by memory.
+// A block program is a list of wide vnodes that one block serves one after the other for one KV
+// head.  Blocks are handed out in index order, two per compute unit, and with 256 of them a round
+// goes once around the machine: block b and block b + (number of units) share a unit.  The schedule
+// therefore places programs on units in pairs, a first row of programs and a second one, and
+// chooses the cut of the runs -- into row chunks and, along the tokens, into pieces -- whose modelled
+// duration is the shortest:
+//
+//  * a unit with programs of TA >= TB (each alone) is done after TA + kPairing * TB: two blocks step
+//    about 1.5 times slower each than one alone (measured: kStep below);
+//  * the narrow vnodes follow in index order and fill the block slots that programs leave or never
+//    had, so short second programs are not idle slots but room for them;
+//  * every piece costs its start-up and wind-down and, per query row, a partial result that the
+//    second stage reads back.
+
+#include "fasttree_schedule.h"
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <new>
+#include <queue>
+#include <unordered_map>
+#include <vector>
+
+namespace {
+
+constexpr int kTile = 32;              // tokens of a step
+constexpr int kCut = 64;               // pieces start at multiples of this many tokens
+constexpr int kMinPiece = 128;         // and are not made shorter than this
+constexpr int kNarrowRows = 16;
+constexpr int kNarrowChunk = 1024;     // tokens one wave walks at most
+constexpr int kBlocksPerCu = 2;
+constexpr int kWavesPerBlock = 4;
+
+// ---- the model (microseconds; measured on the shapes of the kernel's own loop, rows resident in L2)
+
+// One 32-token step of a block that has its compute unit to itself, by 16-row groups of the piece:
+// at head_dim 128 48 rows (one set of waves, tokens split four ways) .51, 64 rows .44, 96 rows .52,
+// 128 rows .69, 192 rows .88 (start of the scale: 16 rows .35).  Other head sizes: measured on full chunks.
+double step_us(int groups, int head_dim) {
+  static const double at128[13] = {0, .35, .42, .51, .44, .53, .53, .69, .69, .86, .87, .88, .88};
+  static const double at256[9] = {0, .91, .91, .92, .92, 1.42, 1.42, 1.42, 1.42};
+  if (head_dim > 128) return at256[std::min(groups, 8)];
+  const double at = at128[std::min(groups, 12)];
+  return head_dim == 128 ? at : head_dim == 64 ? 0.71 * at : 0.6 * at;
+}
+constexpr double kPairing = 0.55;      // see above
+constexpr double kVnode = 5.5;         // start-up and wind-down of a wide vnode
+constexpr double kNarrowStart = 4.5, kNarrowStep = 1.0, kNarrowShare = 0.6;   // a narrow vnode; its waves' merge
+constexpr double kBytesPerUs = 5.6e6;  // rows at random slots, the whole part
+constexpr double kScratchPerUs = 4.0e6;  // partial results, written and read back
+constexpr double kLaunch = 1.5;
+
+struct Run {
+  int64_t start;                 // into the flat slot list
+  std::vector<int32_t> lens;     // the chunks it came in
+  int64_t tokens;
+  const int32_t* reqs;
+  int n;                         // requests
+};
+
+struct Piece {
+  int64_t start;
+  int32_t tokens;
+  const int32_t* reqs;
+  int n;
+  double us;                     // alone on a unit, start-up included
+};
+
+struct Narrow {
+  int64_t start;
+  int32_t tokens;
+  const int32_t* reqs;
+  int n;
+};
+
+struct Machine {
+  int cus, heads, group, head_dim;
+  int units() const { return std::max(1, cus / heads); }   // compute units per KV head
+};
+
+int rows_per_block(int head_dim) { return head_dim <= 128 ? 192 : 128; }
+int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// The (KV run, request list) pairs behind vnode lists: vnodes over one KV slice whose scratch rows
+// adjoin are the query tiles of one chunk; chunks whose slices adjoin and whose requests are equal are
+// the KV splits of one node.
+std::vector<Run> runs_of(int64_t n, const int32_t* ko, const int32_t* kl, const int32_t* qo, const int32_t* ql, const int32_t* q_entries) {
+  std::vector<int64_t> order(n);
+  for (int64_t i = 0; i < n; ++i) order[i] = i;
+  std::sort(order.begin(), order.end(), [&](int64_t a, int64_t b) {
+    if (ko[a] != ko[b]) return ko[a] < ko[b];
+    if (kl[a] != kl[b]) return kl[a] < kl[b];
+    return qo[a] < qo[b];
+  });
+  struct Chunk { int64_t off; int32_t len; const int32_t* reqs; int n; uint64_t key; };
+  std::vector<Chunk> chunks;
+  for (int64_t i = 0; i < n;) {
+    const int64_t v = order[i];
+    int64_t end = (int64_t)qo[v] + ql[v], j = i + 1;
+    for (; j < n; ++j) {
+      const int64_t w = order[j];
+      if (ko[w] != ko[v] || kl[w] != kl[v] || qo[w] != end) break;
+      end += ql[w];
+    }
+    const int32_t* reqs = q_entries + qo[v];
+    const int count = (int)(end - qo[v]);
+    uint64_t key = 1469598103934665603ull;
+    for (int r = 0; r < count; ++r) key = (key ^ (uint32_t)reqs[r]) * 1099511628211ull;
+    chunks.push_back({ko[v], kl[v], reqs, count, key});
+    i = j;
+  }
+  auto same = [](const Chunk& a, const Chunk& b) { return a.n == b.n && a.key == b.key && std::equal(a.reqs, a.reqs + a.n, b.reqs); };
+  std::unordered_multimap<int64_t, int> by_start;
+  by_start.reserve(chunks.size() * 2);
+  for (int i = (int)chunks.size() - 1; i >= 0; --i) by_start.emplace(chunks[i].off, i);
+  std::vector<int> follower(chunks.size(), -1);
+  std::vector<char> led(chunks.size(), 0);
+  for (int i = 0; i < (int)chunks.size(); ++i) {
+    if (chunks[i].len == 0) continue;
+    auto range = by_start.equal_range(chunks[i].off + chunks[i].len);
+    int found = -1;
+    for (auto it = range.first; it != range.second; ++it)
+      if (it->second != i && !led[it->second] && same(chunks[i], chunks[it->second]) && (found < 0 || it->second < found)) found = it->second;
+    if (found >= 0) {
+      follower[i] = found;
+      led[found] = 1;
+    }
+  }
+  std::vector<Run> runs;
+  for (int i = 0; i < (int)chunks.size(); ++i) {
+    if (led[i]) continue;
+    Run r{chunks[i].off, {}, 0, chunks[i].reqs, chunks[i].n};
+    for (int c = i; c >= 0; c = follower[c]) {
+      r.lens.push_back(chunks[c].len);
+      r.tokens += chunks[c].len;
+    }
+    runs.push_back(std::move(r));
+  }
+  return runs;
+}
+
+// The tree's runs.  Top down as the reference's greedy splitter goes (kernel_bench/fasttree.py:64-96),
+// with its padding costs replaced by bytes: a child that stays a vnode of its own adds a partial
+// result (head_dim + 1 floats, written and read) per query head of its requests; one that takes
+// along the run its parent attends reads that run's rows again, unless nobody else is left on it.
+// (A 256-token prompt of 4 samples at one KV head of 16 query heads: the samples stay apart, 33 KB of
+// partials each against 262 KB of rows.)
+struct TreeRuns {
+  std::vector<Run> runs;
+  std::vector<std::vector<int32_t>> served;
+  std::vector<int32_t> kv_entries;
+};
+int tree_runs(int n, const int32_t* parent, const int32_t* seqlen, const int32_t* num_children, const int64_t* req_offs,
+              const int32_t* req_ids, const int64_t* kv_ptrs, const int32_t* slot_map, int64_t slot_map_len, const Machine& m,
+              TreeRuns& t) {
+  auto nreq = [&](int v) { return req_offs[v + 1] - req_offs[v]; };
+  std::vector<int> first(n, -1), next(n, -1), last(n, -1);     // children in ascending id
+  for (int v = 1; v < n; ++v) {
+    const int up = parent[v];
+    if (last[up] < 0) first[up] = v;
+    else next[last[up]] = v;
+    last[up] = v;
+  }
+  const double row_bytes = 2.0 * 4.0 * m.group * m.heads * (m.head_dim + 1), token_bytes = 4.0 * m.head_dim * m.heads;
+  std::vector<int64_t> run(seqlen, seqlen + n);
+  std::vector<char> along(n, 0);          // takes its parent's run along
+  std::vector<int> queue{0};
+  for (size_t at = 0; at < queue.size(); ++at) {
+    const int v = queue[at];
+    int64_t attached = nreq(v);
+    for (int l = first[v]; l >= 0; l = next[l]) {
+      const int64_t rows = nreq(l);
+      const bool rest = rows < attached;
+      if ((rest ? token_bytes * run[v] : 0.0) < row_bytes * rows) {
+        along[l] = 1;
+        attached -= rows;
+        run[l] = seqlen[l] + run[v];
+      }
+      queue.push_back(l);
+    }
+  }
+  // which requests every node's own vnodes serve (kernel_bench/fasttree.py:126-141)
+  t.served.resize(n);
+  std::vector<int> fifo;
+  std::vector<int64_t> waiting(num_children, num_children + n);
+  for (int v = 0; v < n; ++v)
+    if (num_children[v] == 0) {
+      fifo.push_back(v);
+      t.served[v].assign(req_ids + req_offs[v], req_ids + req_offs[v + 1]);
+    }
+  for (size_t at = 0; at < fifo.size(); ++at) {
+    const int v = fifo[at], up = parent[v];
+    if (v == 0 || up < 0) continue;
+    if (!along[v]) t.served[up].insert(t.served[up].end(), req_ids + req_offs[v], req_ids + req_offs[v + 1]);
+    if (--waiting[up] == 0) fifo.push_back(up);
+  }
+  std::vector<int> chain;
+  for (int v = 0; v < n; ++v) {
+    if (t.served[v].empty()) continue;
+    chain.assign(1, v);
+    while (along[chain.back()]) chain.push_back(parent[chain.back()]);
+    const int64_t start = (int64_t)t.kv_entries.size();
+    for (auto it = chain.rbegin(); it != chain.rend(); ++it) {
+      const int64_t lo = kv_ptrs[*it], hi = kv_ptrs[*it + 1];
+      if (lo < 0 || hi < lo || hi > INT32_MAX || (slot_map && hi > slot_map_len) || start + hi - lo > INT32_MAX - 64) return FT_SCHEDULE_ERR_ARGUMENT;
+      for (int64_t p = lo; p < hi; ++p) t.kv_entries.push_back(slot_map ? slot_map[p] : (int32_t)p);
+    }
+    const int64_t tokens = (int64_t)t.kv_entries.size() - start;
+    Run r{start, {}, tokens, t.served[v].data(), (int)t.served[v].size()};
+    // (chunks for the narrow path: a wave should not walk much more than its neighbours)
+    const int64_t parts = std::max<int64_t>(1, ceil_div(tokens, kNarrowChunk)), tiles = ceil_div(tokens, kTile);
+    int64_t done = 0;
+    for (int64_t i = 0; i < parts; ++i) {
+      const int64_t take = std::min((tiles / parts + (i < tiles % parts ? 1 : 0)) * kTile, tokens - done);
+      if (take > 0 || parts == 1) r.lens.push_back((int32_t)take);
+      done += take;
+    }
+    t.runs.push_back(std::move(r));
+  }
+  t.kv_entries.insert(t.kv_entries.end(), 32, -1);
+  return FT_SCHEDULE_OK;
+}
+
+// Narrow vnodes with the longest runs halved while the waves they take fill less than three quarters
+// of the wave slots: a wave walks its run tile by tile, one memory round trip each, so a launch of a
+// few long runs lasts as long as its longest walk.
+std::vector<Narrow> cut_long(std::vector<Narrow> in, int group, int heads, int64_t wave_slots) {
+  auto waves = [&](const Narrow& v) { return ceil_div((int64_t)v.n * group, kNarrowRows) * heads; };
+  int64_t total = 0;
+  for (const Narrow& v : in) total += waves(v);
+  auto shorter = [&](int a, int b) { return in[a].tokens != in[b].tokens ? in[a].tokens < in[b].tokens : a > b; };
+  std::vector<int> order(in.size());
+  for (size_t i = 0; i < in.size(); ++i) order[i] = (int)i;
+  std::priority_queue<int, std::vector<int>, decltype(shorter)> heap(shorter, std::move(order));
+  while (!heap.empty() && 4 * total < 3 * wave_slots && in[heap.top()].tokens >= 2 * kMinPiece) {
+    const int i = heap.top();
+    heap.pop();
+    const int32_t first = (int32_t)(ceil_div(in[i].tokens / 2, kTile) * kTile);
+    if (in[i].tokens - first < kMinPiece) continue;
+    Narrow rest{in[i].start + first, in[i].tokens - first, in[i].reqs, in[i].n};
+    in[i].tokens = first;
+    in.push_back(rest);
+    heap.push(i);
+    heap.push((int)in.size() - 1);
+    total += waves(rest);
+  }
+  return in;
+}
+
+// How a launch's wide runs are cut and placed.
+struct Cut {
+  int rows_cap;      // requests per row chunk
+  double piece_us;   // pieces are made about this long
+  int row_slots;     // program slots per unit: 1 or 2
+};
+
+struct Layout {
+  std::vector<Piece> pieces;
+  std::vector<std::vector<int>> programs;   // pieces of every program, in launch order
+  double wide_us = 0, total_us = 1e30;
+};
+
+struct NarrowLoad {
+  double block_us;    // time the narrow vnodes take of block slots, all heads
+  double longest_us;  // the longest of them
+  double bytes_us;    // at the memory's rate
+};
+
+std::vector<Piece> cut_runs(const std::vector<Run>& wide, const Machine& m, const Cut& cut) {
+  std::vector<Piece> pieces;
+  for (const Run& r : wide) {
+    const int chunks = (int)std::max<int64_t>(1, ceil_div(r.n, cut.rows_cap));
+    const int groups = (int)ceil_div((int64_t)ceil_div(r.n, chunks) * m.group, 16);
+    const double step = step_us(groups, m.head_dim);
+    const int64_t units = ceil_div(r.tokens, kCut);
+    const double run_us = step * ceil_div(r.tokens, kTile);
+    int64_t n = (int64_t)std::ceil(run_us / std::max(1.0, cut.piece_us - kVnode) - 1e-9);
+    n = std::max<int64_t>(1, std::min(n, r.tokens / kMinPiece));
+    for (int c = 0; c < chunks; ++c) {
+      const int base = r.n / chunks, extra = r.n % chunks;
+      const int lo = c * base + std::min(c, extra), size = base + (c < extra ? 1 : 0);
+      int64_t done = 0;
+      for (int64_t i = 0; i < n && done < r.tokens; ++i) {
+        const int64_t share = units / n + (i < units % n ? 1 : 0);
+        const int64_t take = std::min(share * kCut, r.tokens - done);
+        pieces.push_back({r.start + done, (int32_t)take, r.reqs + lo, size, step * ceil_div(take, kTile) + kVnode});
+        done += take;
+      }
+    }
+  }
+  return pieces;
+}
+
+// Longest piece first, each to the unit that is done first with it, into that unit's emptier slot.
+void place(Layout& l, const Machine& m, const Cut& cut, const NarrowLoad& narrow) {
+  const int units = m.units();
+  std::vector<int> order(l.pieces.size());
+  for (size_t i = 0; i < order.size(); ++i) order[i] = (int)i;
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return l.pieces[a].us > l.pieces[b].us; });
+  struct Unit { double t[2] = {0, 0}; std::vector<int> in[2]; };
+  std::vector<Unit> unit(units);
+  auto done = [&](const Unit& u) { return std::max(u.t[0], u.t[1]) + kPairing * std::min(u.t[0], u.t[1]); };
+  typedef std::pair<double, int> Entry;
+  std::priority_queue<Entry, std::vector<Entry>, std::greater<Entry>> next;
+  for (int i = 0; i < units; ++i) next.push({0.0, i});
+  for (int i : order) {
+    const int u = next.top().second;
+    next.pop();
+    const int slot = cut.row_slots == 2 && unit[u].t[1] < unit[u].t[0] ? 1 : 0;
+    unit[u].t[slot] += l.pieces[i].us;
+    unit[u].in[slot].push_back(i);
+    next.push({done(unit[u]), u});
+  }
+  // units with two programs first, so that the second row's programs land beside the first ones
+  std::vector<int> by(units);
+  for (int i = 0; i < units; ++i) by[i] = i;
+  for (Unit& u : unit)
+    if (u.t[1] > u.t[0]) {
+      std::swap(u.t[0], u.t[1]);
+      std::swap(u.in[0], u.in[1]);
+    }
+  std::stable_sort(by.begin(), by.end(), [&](int a, int b) {
+    const bool pa = !unit[a].in[1].empty(), pb = !unit[b].in[1].empty();
+    return pa != pb ? pa : unit[a].t[0] > unit[b].t[0];
+  });
+  l.programs.clear();
+  for (int row = 0; row < 2; ++row)
+    for (int i : by)
+      if (!unit[i].in[row].empty()) l.programs.push_back(std::move(unit[i].in[row]));
+  // ---- duration: the last unit's programs; the narrow vnodes in the slots that are free by then
+  double wide = 0;
+  std::vector<double> free_from;
+  for (const Unit& u : unit) {
+    const double end = done(u);
+    wide = std::max(wide, end);
+    free_from.push_back(end);
+    free_from.push_back(u.t[1] > 0 ? u.t[1] * (1 + kPairing) : 0.0);
+  }
+  l.wide_us = wide;
+  double total = wide;
+  if (narrow.block_us > 0) {
+    std::sort(free_from.begin(), free_from.end());
+    const double per_head = narrow.block_us / m.heads;
+    double have = 0, at = 0;
+    size_t slots = 0;
+    for (; slots < free_from.size(); ++slots) {
+      const double more = (free_from[slots] - at) * slots;
+      if (have + more >= per_head) break;
+      have += more;
+      at = free_from[slots];
+    }
+    const double end = at + (per_head - have) / std::max<size_t>(1, slots);
+    total = std::max({wide, end, narrow.longest_us + free_from[0]});
+  }
+  total = std::max(total, narrow.bytes_us);
+  l.total_us = total;
+}
+
+}  // namespace
+
+struct ft_schedule {
+  std::vector<int32_t> arrays[FT_SCHEDULE_ARRAYS];
+};
+
+namespace {
+
+void build(const Machine& m, int batch, Layout& l, std::vector<Narrow>& narrow, const int32_t* kv_entries, ft_schedule& s) {
+  auto& A = s.arrays;
+  std::vector<int32_t>&ko = A[FT_SCHEDULE_KV_OFFS], &kl = A[FT_SCHEDULE_KV_LENS], &qe = A[FT_SCHEDULE_Q_ENTRIES], &qo = A[FT_SCHEDULE_Q_OFFS],
+                      &ql = A[FT_SCHEDULE_Q_LENS], &table = A[FT_SCHEDULE_PROG_TABLE];
+  auto emit = [&](int64_t start, int32_t tokens, const int32_t* reqs, int n) {
+    ko.push_back((int32_t)start);
+    kl.push_back(tokens);
+    qo.push_back((int32_t)qe.size());
+    ql.push_back(n);
+    qe.insert(qe.end(), reqs, reqs + n);
+  };
+  for (const std::vector<int>& program : l.programs) {
+    table.push_back((int32_t)ko.size());
+    for (int i : program) emit(l.pieces[i].start, l.pieces[i].tokens, l.pieces[i].reqs, l.pieces[i].n);
+    table.push_back((int32_t)ko.size());
+    table.push_back(0);
+    table.push_back(0);
+  }
+  const int32_t wide = (int32_t)ko.size();
+  for (const Narrow& v : narrow) emit(v.start, v.tokens, v.reqs, v.n);
+  // scratch rows of every request, in row order
+  std::vector<int32_t>&re = A[FT_SCHEDULE_REQ_ENTRIES], &ro = A[FT_SCHEDULE_REQ_OFFS], &rl = A[FT_SCHEDULE_REQ_LENS];
+  rl.assign(batch, 0);
+  ro.assign(batch, 0);
+  for (int32_t r : qe) rl[r] += 1;
+  for (int r = 1; r < batch; ++r) ro[r] = ro[r - 1] + rl[r - 1];
+  re.assign(qe.size() + 32, -1);
+  std::vector<int32_t> cursor(ro);
+  for (size_t row = 0; row < qe.size(); ++row) re[cursor[qe[row]]++] = (int32_t)row;
+  const int32_t programs = (int32_t)l.programs.size(), narrows = (int32_t)ko.size() - wide;
+  A[FT_SCHEDULE_COUNTS] = {wide, narrows, programs, 0, 0};
+  // ---- records (layouts: include/fasttree_hip.h)
+  std::vector<int32_t>& req_table = A[FT_SCHEDULE_REQ_TABLE];
+  req_table.assign((size_t)batch * 16, 0);
+  for (int r = 0; r < batch; ++r) {
+    int32_t* rec = &req_table[(size_t)r * 16];
+    rec[0] = rl[r];
+    rec[1] = ro[r];
+    for (int i = 0; i < std::min(rl[r], 14); ++i) rec[2 + i] = re[ro[r] + i];
+  }
+  if (!kv_entries) return;
+  std::vector<int32_t>& nt = A[FT_SCHEDULE_NARROW_TABLE];
+  nt.assign((size_t)narrows * 64, 0);
+  for (int32_t i = 0; i < narrows; ++i) {
+    const int32_t v = wide + i;
+    int32_t* rec = &nt[(size_t)i * 64];
+    rec[0] = ko[v]; rec[1] = kl[v]; rec[2] = qo[v]; rec[3] = ql[v];
+    if (ql[v] > 0)
+      for (int r = 0; r < 16; ++r) rec[4 + r] = qe[qo[v] + std::min(r, ql[v] - 1)];
+    if (kl[v] > 0)
+      for (int t = 0; t < 32; ++t) rec[20 + t] = kv_entries[ko[v] + std::min(t, kl[v] - 1)];
+  }
+  std::vector<int32_t>& pr = A[FT_SCHEDULE_PROG_RECORDS];
+  pr.assign((size_t)programs * 256, 0);
+  for (int32_t p = 0; p < programs; ++p) {
+    const int32_t v = table[4 * p];
+    int32_t* rec = &pr[(size_t)p * 256];
+    rec[0] = ko[v]; rec[1] = kl[v]; rec[2] = qo[v]; rec[3] = ql[v];
+    // (the record holds 128 requests, and what one pass of a block serves)
+    if (ql[v] < 1 || ql[v] > 128 || (int64_t)ql[v] * m.group > rows_per_block(m.head_dim)) continue;
+    rec[4] = 1;
+    for (int r = 0; r < 128; ++r) rec[8 + r] = qe[qo[v] + std::min(r, ql[v] - 1)];
+    if (kl[v] > 0)
+      for (int t = 0; t < 64; ++t) rec[136 + t] = kv_entries[ko[v] + std::min(t, kl[v] - 1)];
+  }
+}
+
+double arrange(const std::vector<Run>& runs, const Machine& m, int batch, const int32_t* kv_entries, ft_schedule& s) {
+  const int block_rows = rows_per_block(m.head_dim);
+  const int slots = (m.head_dim <= 128 ? kBlocksPerCu : 1) * m.cus;      // blocks the device holds at a time
+  const int64_t wave_slots = (int64_t)slots * kWavesPerBlock;
+  std::vector<Run> wide;
+  std::vector<Narrow> narrow;
+  auto go_narrow = [&](const Run& r) {
+    int64_t off = r.start;
+    for (int32_t len : r.lens) {
+      narrow.push_back({off, len, r.reqs, r.n});
+      off += len;
+    }
+  };
+  int64_t wide_blocks = 0;
+  for (const Run& r : runs) {
+    // (a run without tokens has no steps to place: a wave writes its empty partial results)
+    if ((int64_t)r.n * m.group <= kNarrowRows || r.tokens == 0) go_narrow(r);
+    else {
+      wide.push_back(r);
+      wide_blocks += (int64_t)r.lens.size() * ceil_div((int64_t)r.n * m.group, block_rows) * m.heads;
+    }
+  }
+  // Short runs of a few dozen rows are bound by memory latency: where the wide blocks overfill the
+  // machine they go with the narrow vnodes, eight of which a compute unit has in flight.
+  if (wide_blocks > slots) {
+    std::vector<Run> kept;
+    for (Run& r : wide) {
+      const int64_t rows = (int64_t)r.n * m.group;
+      if (rows <= 64 && rows * *std::max_element(r.lens.begin(), r.lens.end()) <= 4096) go_narrow(r);
+      else kept.push_back(std::move(r));
+    }
+    wide.swap(kept);
+  }
+  narrow = cut_long(std::move(narrow), m.group, m.heads, wave_slots);
+  auto passes = [&](const Narrow& v) { return (double)ceil_div((int64_t)v.n * m.group, kNarrowRows); };
+  std::stable_sort(narrow.begin(), narrow.end(), [&](const Narrow& a, const Narrow& b) {
+    return ceil_div(a.tokens, kTile) * passes(a) > ceil_div(b.tokens, kTile) * passes(b);
+  });
+  NarrowLoad load{0, 0, 0};
+  {
+    // the launcher lets 2 or 4 waves share a vnode while that leaves a quarter of the wave slots free
+    int64_t items = 0;
+    for (const Narrow& v : narrow) items += (int64_t)passes(v) * m.heads;
+    int share = 1;
+    while (share < kWavesPerBlock && 4 * items * 2 * share <= 3 * wave_slots) share *= 2;
+    double bytes = 0;
+    for (const Narrow& v : narrow) {
+      const double us = kNarrowStart + kNarrowStep * ceil_div(ceil_div(v.tokens, kTile), share) * passes(v) + (share > 1 ? kNarrowShare : 0.0);
+      load.block_us += us * m.heads * share / kWavesPerBlock;
+      load.longest_us = std::max(load.longest_us, us);
+      bytes += 4.0 * m.head_dim * v.tokens * m.heads;
+    }
+    load.bytes_us = bytes / kBytesPerUs * 256 / m.cus;
+  }
+  Layout best;
+  Cut chosen{1, 0, 1};
+  if (wide.empty()) {
+    best.total_us = std::max({load.bytes_us, load.longest_us, load.block_us / slots});
+  } else {
+    double score = 1e30;
+    for (int rows : {block_rows, 128, 64}) {
+      if (rows > block_rows) continue;
+      Cut cut{std::max(1, rows / m.group), 0, 0};
+      double whole = 0;
+      for (const Run& r : wide) {
+        const int chunks = (int)ceil_div(r.n, cut.rows_cap);
+        whole = std::max(whole, kVnode + step_us((int)ceil_div((int64_t)ceil_div(r.n, chunks) * m.group, 16), m.head_dim) * ceil_div(r.tokens, kTile));
+      }
+      for (cut.row_slots = 1; cut.row_slots <= (m.head_dim <= 128 ? 2 : 1); ++cut.row_slots) {
+        double last = 0;
+        for (double us = whole; us == whole || us > kVnode + 1.0; us = kVnode + (us - kVnode) * 0.82) {
+          cut.piece_us = us;
+          Layout l;
+          l.pieces = cut_runs(wide, m, cut);
+          if ((double)l.pieces.size() == last) continue;
+          last = (double)l.pieces.size();
+          int64_t rows_out = 0;
+          for (const Piece& p : l.pieces) rows_out += p.n;
+          const double scratch = 8.0 * rows_out * m.group * m.heads * (m.head_dim + 1) / kScratchPerUs;
+          if (l.pieces.size() > 4096 || scratch > score) break;
+          place(l, m, cut, load);
+          if (l.total_us + scratch < score) {
+            score = l.total_us + scratch;
+            best = std::move(l);
+            chosen = cut;
+          }
+        }
+      }
+    }
+  }
+  build(m, batch, best, narrow, kv_entries, s);
+  s.arrays[FT_SCHEDULE_COUNTS][3] = wide.empty() ? slots : chosen.row_slots * m.cus;
+  return best.total_us + kLaunch;
+}
+
+}  // namespace
+
+extern "C" {
+
+int ft_schedule_create(int64_t num_vnodes, const int32_t* kv_offs, const int32_t* kv_lens, const int32_t* q_offs, const int32_t* q_lens,
+                       int64_t num_rows, const int32_t* q_entries, int64_t num_kv_entries, const int32_t* kv_entries, int batch_size,
+                       int group, int num_kv_heads, int head_dim, int num_cus, double* modelled_us, ft_schedule** out) {
+  if (!out || (num_vnodes > 0 && (!kv_offs || !kv_lens || !q_offs || !q_lens)) || (num_rows > 0 && !q_entries)) return FT_SCHEDULE_ERR_NULL_POINTER;
+  if (num_vnodes < 0 || num_rows < 0 || batch_size < 0 || group < 1 || num_kv_heads < 1 || head_dim < 1 || num_cus < 1) return FT_SCHEDULE_ERR_ARGUMENT;
+  for (int64_t v = 0; v < num_vnodes; ++v) {
+    if (kv_offs[v] < 0 || kv_lens[v] < 0 || q_offs[v] < 0 || q_lens[v] < 0 || (int64_t)q_offs[v] + q_lens[v] > num_rows) return FT_SCHEDULE_ERR_ARGUMENT;
+    if (kv_entries && (int64_t)kv_offs[v] + kv_lens[v] > num_kv_entries) return FT_SCHEDULE_ERR_ARGUMENT;
+  }
+  for (int64_t i = 0; i < num_rows; ++i)
+    if (q_entries[i] < 0 || q_entries[i] >= batch_size) return FT_SCHEDULE_ERR_ARGUMENT;
+  try {
+    const Machine m{num_cus, num_kv_heads, group, head_dim};
+    ft_schedule* s = new ft_schedule;
+    const double us = arrange(runs_of(num_vnodes, kv_offs, kv_lens, q_offs, q_lens, q_entries), m, batch_size, kv_entries, *s);
+    if (modelled_us) *modelled_us = us;
+    *out = s;
+    return FT_SCHEDULE_OK;
+  } catch (const std::bad_alloc&) {
+    return FT_SCHEDULE_ERR_MEMORY;
+  }
+}
+
+int ft_schedule_tree(int num_nodes, const int32_t* parent, const int32_t* seqlen, const int32_t* num_children, const int64_t* req_offs,
+                     const int32_t* req_ids, const int64_t* kv_ptrs, const int32_t* kv_slot_map, int64_t kv_slot_map_len, int batch_size,
+                     int group, int num_kv_heads, int head_dim, int num_cus, double* modelled_us, ft_schedule** out) {
+  if (!parent || !seqlen || !num_children || !req_offs || !kv_ptrs || !out) return FT_SCHEDULE_ERR_NULL_POINTER;
+  if (num_nodes < 1 || batch_size < 0 || group < 1 || num_kv_heads < 1 || head_dim < 1 || num_cus < 1) return FT_SCHEDULE_ERR_ARGUMENT;
+  for (int v = 0; v < num_nodes; ++v)
+    if ((v > 0 && (parent[v] < 0 || parent[v] >= v)) || seqlen[v] < 0 || req_offs[v + 1] < req_offs[v]) return FT_SCHEDULE_ERR_ARGUMENT;
+  if (req_offs[num_nodes] > 0 && !req_ids) return FT_SCHEDULE_ERR_NULL_POINTER;
+  for (int64_t i = 0; i < req_offs[num_nodes]; ++i)
+    if (req_ids[i] < 0 || req_ids[i] >= batch_size) return FT_SCHEDULE_ERR_ARGUMENT;
+  try {
+    const Machine m{num_cus, num_kv_heads, group, head_dim};
+    TreeRuns t;
+    if (int rc = tree_runs(num_nodes, parent, seqlen, num_children, req_offs, req_ids, kv_ptrs, kv_slot_map, kv_slot_map_len, m, t)) return rc;
+    ft_schedule* s = new ft_schedule;
+    const double us = arrange(t.runs, m, batch_size, t.kv_entries.data(), *s);
+    s->arrays[FT_SCHEDULE_KV_ENTRIES] = std::move(t.kv_entries);
+    if (modelled_us) *modelled_us = us;
+    *out = s;
+    return FT_SCHEDULE_OK;
+  } catch (const std::bad_alloc&) {
+    return FT_SCHEDULE_ERR_MEMORY;
+  }
+}
+
+int64_t ft_schedule_size(const ft_schedule* s, int which) {
+  return s && which >= 0 && which < FT_SCHEDULE_ARRAYS ? (int64_t)s->arrays[which].size() : -1;
+}
+
+int ft_schedule_pack(const ft_schedule* s, int32_t* dst, int64_t capacity, int64_t offsets[FT_SCHEDULE_ARRAYS], int64_t* total) {
+  if (!s || !offsets || !total) return FT_SCHEDULE_ERR_NULL_POINTER;
+  int64_t at = 0;
+  for (int i = 0; i < FT_SCHEDULE_ARRAYS; ++i) {
+    offsets[i] = at;
+    at += ceil_div((int64_t)s->arrays[i].size(), 64) * 64;
+  }
+  *total = at;
+  if (!dst) return FT_SCHEDULE_OK;
+  if (at > capacity) return FT_SCHEDULE_ERR_ARGUMENT;
+  for (int i = 0; i < FT_SCHEDULE_ARRAYS; ++i)
+    if (!s->arrays[i].empty()) std::memcpy(dst + offsets[i], s->arrays[i].data(), s->arrays[i].size() * sizeof(int32_t));
+  return FT_SCHEDULE_OK;
+}
+
+void ft_schedule_destroy(ft_schedule* s) { delete s; }
+
+}  // extern "C"

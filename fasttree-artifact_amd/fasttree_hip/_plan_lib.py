@@ -1,4 +1,5 @@
-"""ctypes binding of libfasttree_plan.so, the native host planner (include/fasttree_plan.h)."""
+"""ctypes binding of libfasttree_plan.so: the native host planner (include/fasttree_plan.h) and the
+launch schedule (include/fasttree_schedule.h)."""
 
 from __future__ import annotations
 
@@ -29,6 +30,19 @@ SIGNATURES = {
     "ft_plan_destroy": (None, [ctypes.c_void_p]),
 }
 
+# order of a schedule's arrays (enum in include/fasttree_schedule.h)
+SCHEDULE_ARRAYS = ("kv_offs", "kv_lens", "q_entries", "q_offs", "q_lens", "req_entries", "req_offs", "req_lens", "prog_table",
+                   "narrow_table", "prog_records", "req_table", "counts", "kv_entries")
+SCHEDULE_SIGNATURES = {
+    "ft_schedule_create": (ctypes.c_int, [ctypes.c_int64, _P32, _P32, _P32, _P32, ctypes.c_int64, _P32, ctypes.c_int64, _P32]
+                           + [ctypes.c_int] * 5 + [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_void_p)]),
+    "ft_schedule_tree": (ctypes.c_int, [ctypes.c_int, _P32, _P32, _P32, _P64, _P32, _P64, _P32, ctypes.c_int64]
+                         + [ctypes.c_int] * 5 + [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_void_p)]),
+    "ft_schedule_size": (ctypes.c_int64, [ctypes.c_void_p, ctypes.c_int]),
+    "ft_schedule_pack": (ctypes.c_int, [ctypes.c_void_p, _P32, ctypes.c_int64, _P64, _P64]),
+    "ft_schedule_destroy": (None, [ctypes.c_void_p]),
+}
+
 _lib = None
 
 
@@ -47,7 +61,7 @@ def load():
             raise FastTreePlannerError(
                 f"{LIB_PATH} is missing: build it with `python -c 'import __graft_entry__ as g; g.build()'`")
         lib = ctypes.CDLL(LIB_PATH)
-        for name, (restype, argtypes) in SIGNATURES.items():
+        for name, (restype, argtypes) in [*SIGNATURES.items(), *SCHEDULE_SIGNATURES.items()]:
             fn = getattr(lib, name)
             fn.restype, fn.argtypes = restype, argtypes
         _lib = lib
@@ -62,22 +76,32 @@ def _ptr32(a):
     return a.ctypes.data_as(_P32)
 
 
+class TreeArrays:
+    """A tree as the arrays the native entry points take."""
+
+    def __init__(self, tree_info, KV_ptrs):
+        self.n = n = len(tree_info)
+        self.parent = _i32([t.parent for t in tree_info])
+        self.seqlen = _i32([t.seqlen for t in tree_info])
+        self.children = _i32([t.num_children for t in tree_info])
+        counts = np.fromiter((len(t.requests) for t in tree_info), dtype=np.int64, count=n)
+        self.req_offs = np.zeros(n + 1, dtype=np.int64)
+        np.cumsum(counts, out=self.req_offs[1:])
+        self.req_ids = _i32([r for t in tree_info for r in t.requests]) if self.req_offs[-1] else np.zeros(1, dtype=np.int32)
+        self.ptrs = np.ascontiguousarray(np.asarray(KV_ptrs, dtype=np.int64))
+        if self.ptrs.shape[0] != n + 1:
+            raise FastTreePlannerError("KV_ptrs must have one entry per node plus one")
+
+
 def plan(tree_info, KV_ptrs, batch_size, num_kv_heads, KV_SPLIT_SIZES, para_threshs1, para_threshs2,
-         alpha, beta, gamma, TSQs, TSKs, kv_group_num, kv_slot_map=None):
+         alpha, beta, gamma, TSQs, TSKs, kv_group_num, kv_slot_map=None, arrays=None):
     """Runs the native planner; returns the list of result arrays (numpy int32), indexed by the
-    constants above."""
+    constants above.  ``tree_info``: the nodes, or a :class:`TreeArrays` made from them; ``arrays``: the
+    constants of the arrays wanted (None: all; the others come back as None)."""
     lib = load()
-    n = len(tree_info)
-    parent = _i32([t.parent for t in tree_info])
-    seqlen = _i32([t.seqlen for t in tree_info])
-    children = _i32([t.num_children for t in tree_info])
-    counts = np.fromiter((len(t.requests) for t in tree_info), dtype=np.int64, count=n)
-    req_offs = np.zeros(n + 1, dtype=np.int64)
-    np.cumsum(counts, out=req_offs[1:])
-    req_ids = _i32([r for t in tree_info for r in t.requests]) if req_offs[-1] else np.zeros(1, dtype=np.int32)
-    ptrs = np.ascontiguousarray(np.asarray(KV_ptrs, dtype=np.int64))
-    if ptrs.shape[0] != n + 1:
-        raise FastTreePlannerError("KV_ptrs must have one entry per node plus one")
+    tree = tree_info if isinstance(tree_info, TreeArrays) else TreeArrays(tree_info, KV_ptrs)
+    n, parent, seqlen, children, req_offs, req_ids, ptrs = (
+        tree.n, tree.parent, tree.seqlen, tree.children, tree.req_offs, tree.req_ids, tree.ptrs)
     splits, th1, th2 = _i32(list(KV_SPLIT_SIZES)[:2]), _i32(list(para_threshs1)[:2]), _i32(list(para_threshs2)[:2])
     tsq, tsk = _i32(list(TSQs)[:2]), _i32(list(TSKs)[:2])
     slot_map = None if kv_slot_map is None else _i32(kv_slot_map)
@@ -93,6 +117,9 @@ def plan(tree_info, KV_ptrs, batch_size, num_kv_heads, KV_SPLIT_SIZES, para_thre
     try:
         out = []
         for which in range(N_ARRAYS):
+            if arrays is not None and which not in arrays:
+                out.append(None)
+                continue
             size = lib.ft_plan_size(handle, which)
             a = np.empty(max(size, 0), dtype=np.int32)
             rc = lib.ft_plan_copy(handle, which, _ptr32(a) if size else None, size)
@@ -102,3 +129,46 @@ def plan(tree_info, KV_ptrs, batch_size, num_kv_heads, KV_SPLIT_SIZES, para_thre
         return out
     finally:
         lib.ft_plan_destroy(handle)
+
+
+def schedule(kv_offs, kv_lens, q_offs, q_lens, q_entries, kv_entries, batch_size, group, num_kv_heads, head_dim, num_cus, allocate):
+    """Runs the native launch schedule on vnode lists (``kv_entries`` may be None: no records then).
+    ``allocate(n)`` gives the int32 numpy array of at least ``n`` entries that the result is packed into.
+    Returns ``(packed, {array name: (first entry, entries)}, modelled microseconds)``."""
+    lib = load()
+    lists = [_i32(x).reshape(-1) for x in (kv_offs, kv_lens, q_offs, q_lens, q_entries)]
+    entries = None if kv_entries is None else _i32(kv_entries).reshape(-1)
+    us, handle = ctypes.c_double(), ctypes.c_void_p()
+    rc = lib.ft_schedule_create(
+        lists[0].shape[0], *(_ptr32(x) for x in lists[:4]), lists[4].shape[0], _ptr32(lists[4]),
+        0 if entries is None else entries.shape[0], None if entries is None else _ptr32(entries),
+        int(batch_size), int(group), int(num_kv_heads), int(head_dim), int(num_cus), ctypes.byref(us), ctypes.byref(handle))
+    return _packed(lib, rc, "ft_schedule_create", handle, us, allocate)
+
+
+def schedule_tree(tree, batch_size, group, num_kv_heads, head_dim, num_cus, kv_slot_map, allocate):
+    """The same from a :class:`TreeArrays` (the array "kv_entries" holds the flat slot list)."""
+    lib = load()
+    slot_map = None if kv_slot_map is None else _i32(kv_slot_map)
+    us, handle = ctypes.c_double(), ctypes.c_void_p()
+    rc = lib.ft_schedule_tree(
+        tree.n, _ptr32(tree.parent), _ptr32(tree.seqlen), _ptr32(tree.children), tree.req_offs.ctypes.data_as(_P64), _ptr32(tree.req_ids),
+        tree.ptrs.ctypes.data_as(_P64), None if slot_map is None else _ptr32(slot_map), 0 if slot_map is None else slot_map.shape[0],
+        int(batch_size), int(group), int(num_kv_heads), int(head_dim), int(num_cus), ctypes.byref(us), ctypes.byref(handle))
+    return _packed(lib, rc, "ft_schedule_tree", handle, us, allocate)
+
+
+def _packed(lib, rc, what, handle, us, allocate):
+    if rc != 0:
+        raise FastTreePlannerError(f"{what} failed: {_ERRORS.get(rc, rc)}")
+    try:
+        offsets, total = (ctypes.c_int64 * len(SCHEDULE_ARRAYS))(), ctypes.c_int64()
+        lib.ft_schedule_pack(handle, None, 0, offsets, ctypes.byref(total))
+        packed = allocate(total.value)
+        rc = lib.ft_schedule_pack(handle, _ptr32(packed), packed.shape[0], offsets, ctypes.byref(total))
+        if rc != 0:
+            raise FastTreePlannerError(f"ft_schedule_pack failed: {_ERRORS.get(rc, rc)}")
+        where = {name: (offsets[i], lib.ft_schedule_size(handle, i)) for i, name in enumerate(SCHEDULE_ARRAYS)}
+        return packed, where, us.value
+    finally:
+        lib.ft_schedule_destroy(handle)

@@ -802,3 +802,94 @@ def _block_programs(runs, batch_size, group, num_kv_heads, *,
         if layout == "resident" or alone[0] <= RESIDENT_MARGIN * packed[0]:
             return alone
     return packed
+
+
+# ---------------------------------------------------------------------------------------
+# What the preparation calls
+# ---------------------------------------------------------------------------------------
+def _tuning():
+    return (block_programs, BLOCKS_PER_CU, MIN_PROGRAM_TILES, MAX_PROGRAM_TILES, MIN_PIECE_TOKENS, RESIDENT_MARGIN, SHORT_PIECE_RATIO,
+            DEALT_MARGIN, LIGHT_WORK, LIGHT_ROWS, NARROW_MIN_PIECE_TOKENS, NARROW_FILL)
+
+
+_TUNING = _tuning()
+
+
+class Arranged:
+    """A launch-order plan on the host: the lists, the program table and the records, by name in
+    ``part`` as views of ``packed`` (one int32 tensor, so that a plan is uploaded with one copy)."""
+
+    def __init__(self, packed, where, modelled_us, num_cus):
+        self.packed, self.where = packed, where
+        self.part = {name: packed[lo: lo + n] for name, (lo, n) in where.items()}
+        self.n_wide, self.n_narrow, self.num_programs, self.block_slots, self.narrow_in_programs = (int(x) for x in self.part["counts"][:5])
+        self.modelled_us, self.num_cus = modelled_us, num_cus
+
+    @property
+    def num_rows(self):
+        return self.where["q_entries"][1]
+
+
+def native_schedule() -> bool:
+    """Whether arranged plans come from the native schedule: unless the constants of this module were
+    changed by hand, which asks for the explicit layouts of :func:`block_programs`."""
+    return _tuning() == _TUNING
+
+
+class _PackedTensor:
+    """Hands the native schedule the memory for its packed result and keeps it as a tensor."""
+
+    def __init__(self, pin):
+        self.pin, self.tensor = pin, None
+
+    def __call__(self, n):
+        import torch
+
+        self.tensor = torch.empty(n, dtype=torch.int32, pin_memory=self.pin)
+        return self.tensor.numpy()
+
+
+def arrange_tree(tree, batch_size, group, num_kv_heads, *, head_dim=128, num_cus=None, kv_slot_map=None, pin=False) -> Arranged:
+    """A tree (:class:`_plan_lib.TreeArrays`) arranged for a device, the sharing of ancestors' tokens
+    decided by what it makes the device move (include/fasttree_schedule.h); otherwise :func:`arrange`."""
+    from . import _plan_lib
+
+    cus = max(1, int(num_cus)) if num_cus else compute_units()
+    memory = _PackedTensor(pin)
+    _, where, us = _plan_lib.schedule_tree(tree, batch_size, group, num_kv_heads, head_dim, cus, kv_slot_map, memory)
+    return Arranged(memory.tensor, where, us, cus)
+
+
+def arrange(kv_offs, kv_lens, q_offs, q_lens, q_entries, batch_size, group, num_kv_heads, *, kv_entries=None, head_dim=128,
+            num_cus=None, pin=False) -> Arranged:
+    """The planner's lists arranged for a device: what ``fasttree_preparation(launch_order=True)`` and
+    the serving plugin upload.  Runs the native schedule (csrc/fasttree_schedule.cpp), whose model
+    places programs on compute units in pairs; with the constants of this module changed by hand the
+    explicit layouts of :func:`block_programs` instead.  With ``kv_entries`` the records the kernels
+    start from are made too.  ``pin``: the packed tensor is in pinned memory."""
+    cus = max(1, int(num_cus)) if num_cus else compute_units()
+    memory = _PackedTensor(pin)
+    if native_schedule():
+        from . import _plan_lib
+        _, where, us = _plan_lib.schedule(kv_offs, kv_lens, q_offs, q_lens, q_entries, kv_entries, batch_size, group, num_kv_heads,
+                                          head_dim, cus, memory)
+        return Arranged(memory.tensor, where, us, cus)
+    sched = block_programs(kv_offs, kv_lens, q_offs, q_lens, q_entries, batch_size, group, num_kv_heads, head_dim=head_dim, num_cus=cus)
+    lists = (sched.kv_offs, sched.kv_lens, sched.q_offs, sched.q_lens)
+    n_wide, n_narrow = sched.phase_node_nums
+    arrays = dict(kv_offs=lists[0], kv_lens=lists[1], q_entries=sched.q_entries, q_offs=lists[2], q_lens=lists[3],
+                  req_entries=sched.req_entries, req_offs=sched.req_offs, req_lens=sched.req_lens, prog_table=sched.prog_table,
+                  req_table=request_records(sched.req_entries, sched.req_offs, sched.req_lens),
+                  counts=[n_wide, n_narrow, sched.num_programs, sched.block_slots, sched.narrow_in_programs])
+    if kv_entries is not None:
+        arrays["narrow_table"] = narrow_records(kv_entries, *lists, sched.q_entries, n_wide, n_narrow)
+        arrays["prog_records"] = program_records(kv_entries, *lists, sched.q_entries, sched.prog_table, 0, group)
+    arrays = {name: np.asarray(a, dtype=np.int32).reshape(-1) for name, a in arrays.items()}
+    where, at = {}, 0
+    for name, a in arrays.items():
+        where[name] = (at, a.size)
+        at += -(-a.size // 64) * 64
+    packed = memory(at)
+    for name, a in arrays.items():
+        packed[where[name][0]: where[name][0] + a.size] = a
+    return Arranged(memory.tensor, where, sched.modelled_us, cus)

@@ -246,27 +246,35 @@ def _fits_native(KV_ptrs, KV_SPLIT_SIZES, para_threshs1, para_threshs2, params) 
             and len(KV_ptrs) > 0 and int(KV_ptrs[-1]) <= limit)
 
 
-def _plan_native(tree_info, KV_ptrs, batch_size, num_kv_heads, KV_SPLIT_SIZES, para_threshs1, para_threshs2,
-                 params: FastTreeParams, kv_slot_map) -> FastTreePlan:
-    """``fasttree_plan`` through libfasttree_plan.so: same result, same printed lines, same
-    replacement of ``params.TSQs`` / ``params.TSKs`` when the second adaptation pass fires."""
+def _native_arrays(tree_info, KV_ptrs, batch_size, num_kv_heads, KV_SPLIT_SIZES, para_threshs1, para_threshs2,
+                   params: FastTreeParams, kv_slot_map, arrays=None):
+    """The arrays of libfasttree_plan.so; prints the planner's lines and replaces ``params.TSQs`` /
+    ``params.TSKs`` when the second adaptation pass fired."""
     L = _plan_lib
     r = L.plan(tree_info, KV_ptrs, batch_size, num_kv_heads, KV_SPLIT_SIZES, para_threshs1, para_threshs2,
                params.alpha, params.beta, params.gamma, params.TSQs, params.TSKs, params.kv_group_num,
-               kv_slot_map=kv_slot_map)
-    history = r[L.PARALLELISMS].reshape(-1, 2).tolist()
-    for para in history:
+               kv_slot_map=kv_slot_map, arrays=arrays)
+    for para in r[L.PARALLELISMS].reshape(-1, 2).tolist():
         _say("parallelisms:", para)
     q_tiles = r[L.Q_TILE_SIZES].tolist()
     if int(r[L.TILES_REPLACED][0]):
         params.set_q_tile_sizes(q_tiles)
         params.set_kv_tile_sizes(r[L.KV_TILE_SIZES].tolist())
-    kv_splits = r[L.KV_SPLIT_SIZES].tolist()
     _say(q_tiles)
-    _say(kv_splits)
+    _say(r[L.KV_SPLIT_SIZES].tolist())
     nums = r[L.PHASE_NODE_NUMS].tolist()
     _say("Above threshold: ", nums[0])
     _say("Below threshold: ", nums[1])
+    return r
+
+
+def _plan_native(tree_info, KV_ptrs, batch_size, num_kv_heads, KV_SPLIT_SIZES, para_threshs1, para_threshs2,
+                 params: FastTreeParams, kv_slot_map) -> FastTreePlan:
+    """``fasttree_plan`` through libfasttree_plan.so: same result, same printed lines, same
+    replacement of ``params.TSQs`` / ``params.TSKs`` when the second adaptation pass fires."""
+    L = _plan_lib
+    r = _native_arrays(tree_info, KV_ptrs, batch_size, num_kv_heads, KV_SPLIT_SIZES, para_threshs1, para_threshs2, params, kv_slot_map)
+    q_tiles, kv_splits, nums = r[L.Q_TILE_SIZES].tolist(), r[L.KV_SPLIT_SIZES].tolist(), r[L.PHASE_NODE_NUMS].tolist()
     return FastTreePlan(
         vnode_to_kv_entries=r[L.KV_ENTRIES],
         vnode_to_kv_offs=r[L.KV_OFFS].tolist(),
@@ -282,8 +290,14 @@ def _plan_native(tree_info, KV_ptrs, batch_size, num_kv_heads, KV_SPLIT_SIZES, p
         node_assignments=r[L.NODE_ASSIGNMENTS].tolist(),
         q_tile_sizes=list(q_tiles),
         kv_split_sizes=kv_splits,
-        parallelisms=history,
+        parallelisms=r[L.PARALLELISMS].reshape(-1, 2).tolist(),
     )
+
+
+def _native_chosen(backend, KV_ptrs, KV_SPLIT_SIZES, para_threshs1, para_threshs2, params) -> bool:
+    choice = backend or BACKEND
+    return choice == "native" or (choice == "auto" and _plan_lib.available() and _fits_native(
+        KV_ptrs, KV_SPLIT_SIZES, para_threshs1, para_threshs2, params))
 
 
 def fasttree_plan(
@@ -307,9 +321,7 @@ def fasttree_plan(
     is node-major and the entries are the logical positions themselves, as in the
     reference's bench.
     """
-    choice = backend or BACKEND
-    if choice == "native" or (choice == "auto" and _plan_lib.available() and _fits_native(
-            KV_ptrs, KV_SPLIT_SIZES, para_threshs1, para_threshs2, params)):
+    if _native_chosen(backend, KV_ptrs, KV_SPLIT_SIZES, para_threshs1, para_threshs2, params):
         return _plan_native(tree_info, KV_ptrs, batch_size, num_kv_heads, KV_SPLIT_SIZES, para_threshs1,
                             para_threshs2, params, kv_slot_map)
 
@@ -457,12 +469,13 @@ class PlanBuffers:
         """Copies ``values`` into the front of buffer ``name`` and returns that part of it."""
         import torch
 
-        host = torch.from_numpy(np.ascontiguousarray(np.asarray(values, dtype=np.int32)))
+        host = values if isinstance(values, torch.Tensor) else torch.from_numpy(np.ascontiguousarray(np.asarray(values, dtype=np.int32)))
         dst = getattr(self, name)
         if host.numel() > dst.numel():
             raise ValueError(f"{name}: {host.numel()} entries do not fit the {dst.numel()} that were allocated")
         part = dst[: host.numel()]
-        part.copy_(host)
+        # (tensors handed in lie in pinned memory: copied in stream order, the allocator keeps the block until then)
+        part.copy_(host, non_blocking=host is values)
         return part
 
 
@@ -479,10 +492,8 @@ def place_plan(kv_entries, vnodes, q_entries, per_request, phase_nums, phase_off
     comes back as a list that also carries the program table and the host-written records."""
     import torch
 
-    from .launch_schedule import LaunchPhases, block_programs
-
-    names = iter(("vnode_to_kv_entries", "vnode_to_kv_offs", "vnode_to_kv_lens", "vnode_to_q_entries", "vnode_to_q_offs",
-                  "vnode_to_q_lens", "req_to_vnode_entries", "req_to_vnode_offs", "req_to_vnode_lens"))
+    names = ("vnode_to_kv_entries", "vnode_to_kv_offs", "vnode_to_kv_lens", "vnode_to_q_entries", "vnode_to_q_offs",
+             "vnode_to_q_lens", "req_to_vnode_entries", "req_to_vnode_offs", "req_to_vnode_lens")
 
     def place(name, values):
         if buffers is not None:
@@ -490,61 +501,75 @@ def place_plan(kv_entries, vnodes, q_entries, per_request, phase_nums, phase_off
         host = torch.from_numpy(np.ascontiguousarray(np.asarray(values, dtype=np.int32)))
         return host.to(device)
 
-    def put(values):
-        return place(next(names), values)  # (the nine arrays are placed in this order below)
-
-    rows = int(len(np.asarray(q_entries).reshape(-1)))
     if launch_order:
-        group = max(1, num_qo_heads // num_kv_heads)
-        if num_cus is None:
-            from .launch_schedule import compute_units
-            num_cus = compute_units(device)
-        sched = block_programs(*vnodes, q_entries, batch_size, group, num_kv_heads, head_dim=head_dim, num_cus=num_cus)
-        vnodes = (sched.kv_offs, sched.kv_lens, sched.q_offs, sched.q_lens)
-        q_entries = sched.q_entries
-        per_request = (sched.req_entries, sched.req_offs, sched.req_lens)
-        rows = sched.num_rows
-        phase_nums, phase_offs = LaunchPhases(sched.phase_node_nums), list(sched.phase_node_offsets)
-        phase_nums.modelled_us, phase_nums.num_cus, phase_nums.block_slots = sched.modelled_us, sched.num_cus, sched.block_slots
-        if sched.num_programs > 0:
-            phase_nums.prog_table = place("prog_table", sched.prog_table.reshape(-1))
-            phase_nums.num_programs = sched.num_programs
-            phase_nums.narrow_in_programs = sched.narrow_in_programs
         from . import launch_schedule
-        if sched.num_programs > 0 and head_dim >= 32 and launch_schedule.USE_PROGRAM_RECORDS:
-            records = launch_schedule.program_records(kv_entries, *vnodes, q_entries, sched.prog_table,
-                                                      phase_offs[0], group)
-            phase_nums.prog_records = place("prog_records", records.reshape(-1))
-        if phase_nums[1] > 0 and head_dim >= 32 and launch_schedule.USE_NARROW_RECORDS:
-            from .launch_schedule import narrow_records
-            records = narrow_records(kv_entries, *vnodes, q_entries, phase_offs[1], phase_nums[1])
-            phase_nums.narrow_table = place("narrow_table", records.reshape(-1))
-        if head_dim >= 32 and launch_schedule.USE_REQUEST_RECORDS:
-            from .launch_schedule import request_records
-            phase_nums.req_table = place("req_table", request_records(*per_request).reshape(-1))
+
+        kv_entries = np.ascontiguousarray(np.asarray(kv_entries, dtype=np.int32))
+        if num_cus is None:
+            num_cus = launch_schedule.compute_units(device)
+        plan = launch_schedule.arrange(*vnodes, q_entries, batch_size, max(1, num_qo_heads // num_kv_heads), num_kv_heads,
+                                       kv_entries=kv_entries, head_dim=head_dim, num_cus=num_cus, pin=_on_gpu(device))
+        return _place_arranged(plan, place("vnode_to_kv_entries", kv_entries), num_qo_heads, head_dim, device, buffers)
+    rows = int(len(np.asarray(q_entries).reshape(-1)))
+    placed = [place(name, values) for name, values in zip(names, (kv_entries, vnodes[0], vnodes[1], q_entries, vnodes[2], vnodes[3],
+                                                                 *per_request))]
+    return (*placed, *_scratch(rows, num_qo_heads, head_dim, device, buffers), phase_nums, phase_offs)
+
+
+def _on_gpu(device):
+    import torch
+
+    return torch.device(device).type == "cuda"
+
+
+def _scratch(rows, num_qo_heads, head_dim, device, buffers):
+    """The two fp32 partial-result buffers of a plan."""
+    import torch
+
     if buffers is not None:
         if rows > buffers.mid_o.shape[0] or buffers.mid_o.shape[1:] != (num_qo_heads, head_dim):
             raise ValueError(f"the scratch of the buffers ({tuple(buffers.mid_o.shape)}) does not hold "
                              f"{rows} rows of {num_qo_heads} x {head_dim}")
-        mid_o, mid_lse = buffers.mid_o[:rows], buffers.mid_lse[:rows]
+        return buffers.mid_o[:rows], buffers.mid_lse[:rows]
+    return (torch.empty((rows, num_qo_heads, head_dim), dtype=torch.float32, device=device),
+            torch.empty((rows, num_qo_heads), dtype=torch.float32, device=device))
+
+
+def _place_arranged(plan, kv_entries, num_qo_heads, head_dim, device, buffers):
+    """The decode call's arguments for a :class:`launch_schedule.Arranged` plan; ``kv_entries``: the flat
+    slot list on the device, or None where it is part of the plan."""
+    from . import launch_schedule
+    from .launch_schedule import LaunchPhases
+
+    if buffers is not None:
+        part = {name: buffers.fill(full, plan.part[name]) for name, full in _BUFFER_OF.items() if name in plan.part}
     else:
-        mid_o = torch.empty((rows, num_qo_heads, head_dim), dtype=torch.float32, device=device)
-        mid_lse = torch.empty((rows, num_qo_heads), dtype=torch.float32, device=device)
-    return (
-        put(kv_entries),
-        put(vnodes[0]),
-        put(vnodes[1]),
-        put(q_entries),
-        put(vnodes[2]),
-        put(vnodes[3]),
-        put(per_request[0]),
-        put(per_request[1]),
-        put(per_request[2]),
-        mid_o,
-        mid_lse,
-        phase_nums,
-        phase_offs,
-    )
+        # one copy for the whole plan; the arrays are views of it
+        whole = plan.packed.to(device, non_blocking=True)
+        part = {name: whole[lo: lo + n] for name, (lo, n) in plan.where.items()}
+    nums = LaunchPhases([plan.n_wide, plan.n_narrow])
+    nums.modelled_us, nums.num_cus, nums.block_slots = plan.modelled_us, plan.num_cus, plan.block_slots
+    if plan.num_programs > 0:
+        nums.prog_table = part["prog_table"]
+        nums.num_programs = plan.num_programs
+        nums.narrow_in_programs = plan.narrow_in_programs
+        if head_dim >= 32 and launch_schedule.USE_PROGRAM_RECORDS:
+            nums.prog_records = part["prog_records"]
+    if plan.n_narrow > 0 and head_dim >= 32 and launch_schedule.USE_NARROW_RECORDS:
+        nums.narrow_table = part["narrow_table"]
+    if head_dim >= 32 and launch_schedule.USE_REQUEST_RECORDS:
+        nums.req_table = part["req_table"]
+    return (part["kv_entries"] if kv_entries is None else kv_entries, part["kv_offs"], part["kv_lens"], part["q_entries"], part["q_offs"],
+            part["q_lens"], part["req_entries"], part["req_offs"], part["req_lens"],
+            *_scratch(plan.num_rows, num_qo_heads, head_dim, device, buffers), nums, [0, plan.n_wide])
+
+
+#: The buffer of :class:`PlanBuffers` each array of an arranged plan goes to.
+_BUFFER_OF = {
+    "kv_entries": "vnode_to_kv_entries", "kv_offs": "vnode_to_kv_offs", "kv_lens": "vnode_to_kv_lens", "q_entries": "vnode_to_q_entries", "q_offs": "vnode_to_q_offs",
+    "q_lens": "vnode_to_q_lens", "req_entries": "req_to_vnode_entries", "req_offs": "req_to_vnode_offs", "req_lens": "req_to_vnode_lens",
+    "prog_table": "prog_table", "narrow_table": "narrow_table", "prog_records": "prog_records", "req_table": "req_table",
+}
 
 
 def fasttree_preparation(
@@ -581,8 +606,27 @@ def fasttree_preparation(
     (:func:`launch_schedule.block_programs`: the same computation as block programs,
     with scratch rows and per-request lists of its own); ``phase_node_nums`` is then a list that
     also carries the program table, which ``fasttree_decode`` picks up; the programs are laid out
-    for ``num_cus`` compute units (None: those ``device`` reports, 256 where it is not a GPU).
+    for ``num_cus`` compute units (None: those ``device`` reports, 256 where it is not a GPU).  Which
+    nodes attend their ancestors' tokens with their own is then decided anew, by what it makes the
+    device move (include/fasttree_schedule.h); the assignments returned are the reference planner's
+    either way.
     """
+    from . import launch_schedule
+
+    # (alpha = beta = 0 takes the padding out of the cost model and leaves gamma to force or forbid every
+    # merge: such a plan keeps the merges it was asked for)
+    if (launch_order and (params.alpha or params.beta) and launch_schedule.native_schedule()
+            and _native_chosen(None, KV_ptrs, KV_SPLIT_SIZES, para_threshs1, para_threshs2, params)):
+        L = _plan_lib
+        tree = L.TreeArrays(tree_info, KV_ptrs)
+        r = _native_arrays(tree, KV_ptrs, batch_size, num_kv_heads, KV_SPLIT_SIZES, para_threshs1, para_threshs2, params, kv_slot_map,
+                           arrays=(L.NODE_ASSIGNMENTS, L.PARALLELISMS, L.PHASE_NODE_NUMS, L.Q_TILE_SIZES, L.KV_SPLIT_SIZES,
+                                   L.KV_TILE_SIZES, L.TILES_REPLACED))
+        arranged = launch_schedule.arrange_tree(
+            tree, batch_size, max(1, num_qo_heads // num_kv_heads), num_kv_heads, head_dim=head_dim,
+            num_cus=launch_schedule.compute_units(device) if num_cus is None else num_cus, kv_slot_map=kv_slot_map, pin=_on_gpu(device))
+        return _place_arranged(arranged, None, num_qo_heads, head_dim, device, buffers), r[L.NODE_ASSIGNMENTS].tolist()
+
     plan = fasttree_plan(
         tree_info, KV_ptrs, batch_size, num_kv_heads,
         KV_SPLIT_SIZES, para_threshs1, para_threshs2, params, kv_slot_map=kv_slot_map,

@@ -324,50 +324,45 @@ def prepare_for_fasttree_meta(batch, fasttree_metadata: FastTreeMetadata):
     meta.phase_node_nums = [len(above), len(below)]
     meta.phase_node_offsets = [0, len(above)]
     lists = [[x[i] for i in perm] for x in (kv_offs, kv_lens, q_offs, q_lens)]
-    meta.prog_table_len = 0
     if getattr(meta, "launch_order", False):
         from . import launch_schedule
-        from .launch_schedule import LaunchPhases, block_programs
+        from .launch_schedule import LaunchPhases, compute_units
 
         # the same computation as block programs: long shared runs (a system prompt
         # under a large batch) cut where the machine is full instead of at the KV split
         tail_ends = [lists[0][v] + lists[1][v] for v in meta.req_last_vnodes]
-        from .launch_schedule import compute_units
-        sched = block_programs(*lists, q_entries, len(batch.reqs), meta.kv_group_num, meta.num_kv_heads,
-                               head_dim=meta.head_dim, num_cus=compute_units(meta.device))
-        lists = [sched.kv_offs, sched.kv_lens, sched.q_offs, sched.q_lens]      # (int32 arrays, uploaded as they are)
-        q_entries = sched.q_entries
-        req_entries = sched.req_entries[: sched.num_rows]
-        req_offs, req_lens = sched.req_offs, sched.req_lens
-        # a request's last vnode is the single-request vnode that ends where its tokens end
-        # (narrow vnodes keep the planner's chunks, so there is exactly one)
-        single = np.flatnonzero(sched.q_lens == 1)
-        ends = (sched.kv_offs[single].astype(np.int64) + sched.kv_lens[single]).tolist()
-        owner = sched.q_entries[sched.q_offs[single]].tolist()
+        plan = launch_schedule.arrange(*lists, q_entries, len(batch.reqs), meta.kv_group_num, meta.num_kv_heads, head_dim=meta.head_dim,
+                                       num_cus=compute_units(meta.device), pin=torch.device(meta.device).type == "cuda")
+        part = plan.part
+        lists = [part["kv_offs"], part["kv_lens"], part["q_offs"], part["q_lens"]]
+        q_entries = part["q_entries"]
+        req_entries, req_offs, req_lens = part["req_entries"][: plan.num_rows], part["req_offs"], part["req_lens"]
+        # a request's last vnode is the single-request vnode that ends where its tokens end: the
+        # last piece of its tail, however the tail was cut
+        new_offs, new_lens, new_q_offs, new_q_lens = (x.numpy() for x in lists)
+        single = np.flatnonzero(new_q_lens == 1)
+        ends = (new_offs[single].astype(np.int64) + new_lens[single]).tolist()
+        owner = q_entries.numpy()[new_q_offs[single]].tolist()
         ends_of = dict(zip(zip(ends, owner), single.tolist()))
         meta.req_last_vnodes = [ends_of[(end, rid)] for rid, end in enumerate(tail_ends)]
-        nums = LaunchPhases(sched.phase_node_nums)
-        if sched.num_programs > 0:
-            table = sched.prog_table.reshape(-1)
-            if table.size > meta.prog_table.numel():
-                raise ValueError(f"{sched.num_programs} block programs do not fit the {meta.prog_table.numel() // 4} "
+        nums = LaunchPhases([plan.n_wide, plan.n_narrow])
+        if plan.num_programs > 0:
+            table = part["prog_table"]
+            if table.numel() > meta.prog_table.numel():
+                raise ValueError(f"{plan.num_programs} block programs do not fit the {meta.prog_table.numel() // 4} "
                                  "that max_vnodes allows")
-            src = torch.from_numpy(np.ascontiguousarray(table))
-            meta.prog_table[: src.numel()].copy_(src, non_blocking=True)
-            nums.prog_table = meta.prog_table[: src.numel()]
-            nums.num_programs = sched.num_programs
-            nums.narrow_in_programs = sched.narrow_in_programs
-        if sched.num_programs > 0 and launch_schedule.USE_REQUEST_RECORDS and len(req_offs) * 16 <= meta.req_table.numel():
-            src = torch.from_numpy(launch_schedule.request_records(req_entries, req_offs, req_lens).reshape(-1))
-            meta.req_table[: src.numel()].copy_(src, non_blocking=True)
-            nums.req_table = meta.req_table[: src.numel()]
-        meta.phase_node_nums, meta.phase_node_offsets = nums, list(sched.phase_node_offsets)
+            meta.prog_table[: table.numel()].copy_(table, non_blocking=True)
+            nums.prog_table = meta.prog_table[: table.numel()]
+            nums.num_programs = plan.num_programs
+            nums.narrow_in_programs = plan.narrow_in_programs
+        if plan.num_programs > 0 and launch_schedule.USE_REQUEST_RECORDS and len(batch.reqs) * 16 <= meta.req_table.numel():
+            table = part["req_table"]
+            meta.req_table[: table.numel()].copy_(table, non_blocking=True)
+            nums.req_table = meta.req_table[: table.numel()]
+        meta.phase_node_nums, meta.phase_node_offsets = nums, [0, plan.n_wide]
 
     def upload(dst, values):
-        if isinstance(values, np.ndarray):
-            src = torch.from_numpy(np.ascontiguousarray(values, dtype=np.int32))
-        else:
-            src = torch.tensor(values, device="cpu", dtype=torch.int32)
+        src = values if isinstance(values, torch.Tensor) else torch.tensor(values, device="cpu", dtype=torch.int32)
         dst[: src.numel()].copy_(src, non_blocking=True)
 
     upload(meta.vnode_to_q_entries, q_entries)

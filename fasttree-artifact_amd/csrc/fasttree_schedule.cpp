@@ -23,6 +23,7 @@
 #include <cmath>
 #include <cstring>
 #include <new>
+#include <numeric>
 #include <queue>
 #include <unordered_map>
 #include <vector>
@@ -32,28 +33,41 @@ namespace {
 constexpr int kTile = 32;              // tokens of a step
 constexpr int kCut = 64;               // pieces start at multiples of this many tokens
 constexpr int kMinPiece = 128;         // and are not made shorter than this
-constexpr int kNarrowRows = 16;
+constexpr int kWaveRows = 32;          // query rows a wave of the narrow path serves per pass
 constexpr int kNarrowChunk = 1024;     // tokens one wave walks at most
 constexpr int kBlocksPerCu = 2;
 constexpr int kWavesPerBlock = 4;
+constexpr int kXcds = 8;
 
 // ---- the model (microseconds; measured on the shapes of the kernel's own loop, rows resident in L2)
 
-// One 32-token step of a block that has its compute unit to itself, by 16-row groups of the piece:
-// at head_dim 128 48 rows (one set of waves, tokens split four ways) .51, 64 rows .44, 96 rows .52,
-// 128 rows .69, 192 rows .88 (start of the scale: 16 rows .35).  Other head sizes: measured on full chunks.
-double step_us(int groups, int head_dim) {
-  static const double at128[13] = {0, .35, .42, .51, .44, .53, .53, .69, .69, .86, .87, .88, .88};
+// One 32-token step of a block that has its compute unit to itself, by 16-row groups of the piece.
+// head_dim 128, rows in L2: 16 rows .35, 48 rows (one set of waves, tokens split four ways) .51, 64 rows
+// .44, 96 rows .52, 128 rows .69, 192 rows .88.  The entries above 128 rows are an eighth longer than that:
+// beside narrow vnodes, in whole launches, pieces of 192 rows fall that much behind those of 128 (a
+// 410-request tree of 32/8 heads: 64.9 us with 192-row pieces, 64.1 with 128-row ones, against 3.6 us
+// the other way without the correction).  Other head sizes: measured on full chunks.
+// The blocks of a run lie on one XCD and share it in its L2 where the KV heads divide evenly over the
+// XCDs; otherwise every XCD reads it, and a step of few rows lasts as long as its loads.
+double step_us(int groups, int head_dim, int heads) {
+  static const double at128[13] = {0, .35, .42, .51, .44, .53, .53, .69, .69, .97, .98, .99, .99};
+  static const double at64[13] = {0, .25, .30, .36, .31, .38, .38, .49, .49, .61, .62, .63, .63};
   static const double at256[9] = {0, .91, .91, .92, .92, 1.42, 1.42, 1.42, 1.42};
   if (head_dim > 128) return at256[std::min(groups, 8)];
-  const double at = at128[std::min(groups, 12)];
-  return head_dim == 128 ? at : head_dim == 64 ? 0.71 * at : 0.6 * at;
+  const int g = std::min(groups, 12);
+  const double at = head_dim == 128 ? at128[g] : head_dim == 64 ? at64[g] : 0.85 * at64[g];
+  return heads % kXcds ? std::max(at, .005 * head_dim) : at;
 }
 constexpr double kPairing = 0.55;      // see above
+constexpr double kYounger = 1.67;      // a second program as long as the first ends this much later than alone: its waves issue second
+constexpr double kNarrowPairing = 0.28;  // the same for narrow vnodes beside a program
+constexpr double kNarrowBeside = 1.4;    // a narrow vnode takes this much longer where programs run
 constexpr double kVnode = 5.5;         // start-up and wind-down of a wide vnode
+constexpr double kChained = 1.0;       // and what one costs more as a later vnode of a program: no other block covers for it
 constexpr double kNarrowStart = 4.5, kNarrowStep = 1.0, kNarrowShare = 0.6;   // a narrow vnode; its waves' merge
 constexpr double kBytesPerUs = 5.6e6;  // rows at random slots, the whole part
 constexpr double kScratchPerUs = 4.0e6;  // partial results, written and read back
+constexpr double kNoOverlap = 0.35;
 constexpr double kLaunch = 1.5;
 
 struct Run {
@@ -201,6 +215,7 @@ int tree_runs(int n, const int32_t* parent, const int32_t* seqlen, const int32_t
     if (--waiting[up] == 0) fifo.push_back(up);
   }
   std::vector<int> chain;
+  t.kv_entries.reserve((size_t)std::min<int64_t>(std::max<int64_t>(kv_ptrs[n], 0), 1 << 26) + 32);
   for (int v = 0; v < n; ++v) {
     if (t.served[v].empty()) continue;
     chain.assign(1, v);
@@ -209,7 +224,12 @@ int tree_runs(int n, const int32_t* parent, const int32_t* seqlen, const int32_t
     for (auto it = chain.rbegin(); it != chain.rend(); ++it) {
       const int64_t lo = kv_ptrs[*it], hi = kv_ptrs[*it + 1];
       if (lo < 0 || hi < lo || hi > INT32_MAX || (slot_map && hi > slot_map_len) || start + hi - lo > INT32_MAX - 64) return FT_SCHEDULE_ERR_ARGUMENT;
-      for (int64_t p = lo; p < hi; ++p) t.kv_entries.push_back(slot_map ? slot_map[p] : (int32_t)p);
+      if (slot_map) {
+        t.kv_entries.insert(t.kv_entries.end(), slot_map + lo, slot_map + hi);
+      } else {
+        t.kv_entries.resize(t.kv_entries.size() + hi - lo);
+        std::iota(t.kv_entries.end() - (hi - lo), t.kv_entries.end(), (int32_t)lo);
+      }
     }
     const int64_t tokens = (int64_t)t.kv_entries.size() - start;
     Run r{start, {}, tokens, t.served[v].data(), (int)t.served[v].size()};
@@ -231,7 +251,7 @@ int tree_runs(int n, const int32_t* parent, const int32_t* seqlen, const int32_t
 // of the wave slots: a wave walks its run tile by tile, one memory round trip each, so a launch of a
 // few long runs lasts as long as its longest walk.
 std::vector<Narrow> cut_long(std::vector<Narrow> in, int group, int heads, int64_t wave_slots) {
-  auto waves = [&](const Narrow& v) { return ceil_div((int64_t)v.n * group, kNarrowRows) * heads; };
+  auto waves = [&](const Narrow& v) { return ceil_div((int64_t)v.n * group, kWaveRows) * heads; };
   int64_t total = 0;
   for (const Narrow& v : in) total += waves(v);
   auto shorter = [&](int a, int b) { return in[a].tokens != in[b].tokens ? in[a].tokens < in[b].tokens : a > b; };
@@ -258,6 +278,7 @@ struct Cut {
   int rows_cap;      // requests per row chunk
   double piece_us;   // pieces are made about this long
   int row_slots;     // program slots per unit: 1 or 2
+  double last;       // the last piece of a run relative to the others (two slots: the second program of a unit is the slower)
 };
 
 struct Layout {
@@ -277,7 +298,7 @@ std::vector<Piece> cut_runs(const std::vector<Run>& wide, const Machine& m, cons
   for (const Run& r : wide) {
     const int chunks = (int)std::max<int64_t>(1, ceil_div(r.n, cut.rows_cap));
     const int groups = (int)ceil_div((int64_t)ceil_div(r.n, chunks) * m.group, 16);
-    const double step = step_us(groups, m.head_dim);
+    const double step = step_us(groups, m.head_dim, m.heads);
     const int64_t units = ceil_div(r.tokens, kCut);
     const double run_us = step * ceil_div(r.tokens, kTile);
     int64_t n = (int64_t)std::ceil(run_us / std::max(1.0, cut.piece_us - kVnode) - 1e-9);
@@ -286,8 +307,10 @@ std::vector<Piece> cut_runs(const std::vector<Run>& wide, const Machine& m, cons
       const int base = r.n / chunks, extra = r.n % chunks;
       const int lo = c * base + std::min(c, extra), size = base + (c < extra ? 1 : 0);
       int64_t done = 0;
+      const int64_t short_units = n > 1 && cut.last < 1.0 ? std::max<int64_t>(kMinPiece / kCut, std::llround(units * cut.last / (n - 1 + cut.last))) : 0;
+      const int64_t evens = short_units ? n - 1 : n, even_units = units - short_units;
       for (int64_t i = 0; i < n && done < r.tokens; ++i) {
-        const int64_t share = units / n + (i < units % n ? 1 : 0);
+        const int64_t share = i == evens ? short_units : even_units / evens + (i < even_units % evens ? 1 : 0);
         const int64_t take = std::min(share * kCut, r.tokens - done);
         pieces.push_back({r.start + done, (int32_t)take, r.reqs + lo, size, step * ceil_div(take, kTile) + kVnode});
         done += take;
@@ -297,6 +320,9 @@ std::vector<Piece> cut_runs(const std::vector<Run>& wide, const Machine& m, cons
   return pieces;
 }
 
+// Reading and computing overlap, but a launch that needs both for long overlaps them only in part.
+double overlapped(double a, double b) { return std::max(a, b) + kNoOverlap * std::min(a, b); }
+
 // Longest piece first, each to the unit that is done first with it, into that unit's emptier slot.
 void place(Layout& l, const Machine& m, const Cut& cut, const NarrowLoad& narrow) {
   const int units = m.units();
@@ -305,7 +331,10 @@ void place(Layout& l, const Machine& m, const Cut& cut, const NarrowLoad& narrow
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return l.pieces[a].us > l.pieces[b].us; });
   struct Unit { double t[2] = {0, 0}; std::vector<int> in[2]; };
   std::vector<Unit> unit(units);
-  auto done = [&](const Unit& u) { return std::max(u.t[0], u.t[1]) + kPairing * std::min(u.t[0], u.t[1]); };
+  auto done = [&](const Unit& u) {
+    const double longer = std::max(u.t[0], u.t[1]), shorter = std::min(u.t[0], u.t[1]);
+    return std::max(longer + kPairing * shorter, kYounger * shorter);
+  };
   typedef std::pair<double, int> Entry;
   std::priority_queue<Entry, std::vector<Entry>, std::greater<Entry>> next;
   for (int i = 0; i < units; ++i) next.push({0.0, i});
@@ -313,7 +342,7 @@ void place(Layout& l, const Machine& m, const Cut& cut, const NarrowLoad& narrow
     const int u = next.top().second;
     next.pop();
     const int slot = cut.row_slots == 2 && unit[u].t[1] < unit[u].t[0] ? 1 : 0;
-    unit[u].t[slot] += l.pieces[i].us;
+    unit[u].t[slot] += l.pieces[i].us + (unit[u].in[slot].empty() ? 0.0 : kChained);
     unit[u].in[slot].push_back(i);
     next.push({done(unit[u]), u});
   }
@@ -333,33 +362,34 @@ void place(Layout& l, const Machine& m, const Cut& cut, const NarrowLoad& narrow
   for (int row = 0; row < 2; ++row)
     for (int i : by)
       if (!unit[i].in[row].empty()) l.programs.push_back(std::move(unit[i].in[row]));
-  // ---- duration: the last unit's programs; the narrow vnodes in the slots that are free by then
-  double wide = 0;
-  std::vector<double> free_from;
-  for (const Unit& u : unit) {
-    const double end = done(u);
-    wide = std::max(wide, end);
-    free_from.push_back(end);
-    free_from.push_back(u.t[1] > 0 ? u.t[1] * (1 + kPairing) : 0.0);
-  }
-  l.wide_us = wide;
-  double total = wide;
+  // ---- duration: the narrow vnodes take the slots as they become free and slow the programs beside them
+  l.wide_us = 0;
+  for (const Unit& u : unit) l.wide_us = std::max(l.wide_us, done(u));
+  double total = l.wide_us;
   if (narrow.block_us > 0) {
-    std::sort(free_from.begin(), free_from.end());
-    const double per_head = narrow.block_us / m.heads;
-    double have = 0, at = 0;
-    size_t slots = 0;
-    for (; slots < free_from.size(); ++slots) {
-      const double more = (free_from[slots] - at) * slots;
-      if (have + more >= per_head) break;
-      have += more;
-      at = free_from[slots];
+    const double work = narrow.block_us / m.heads;
+    double end = 0;
+    auto enough = [&](double t) {   // whether the narrow vnodes fit by time t; `end`: when the programs are done then
+      double have = 0;
+      end = 0;
+      for (const Unit& u : unit) {
+        const double second = u.t[1] > 0 ? u.t[1] * (1 + kPairing) : 0.0;
+        const double beside = std::max(0.0, std::min(t, done(u)) - second);
+        const double last = u.t[0] > 0 ? done(u) + kNarrowPairing * beside : 0.0;
+        have += beside / kNarrowBeside + (kBlocksPerCu == 2 ? std::max(0.0, t - std::max(second, last)) : 0.0) + std::max(0.0, t - last);
+        end = std::max(end, last);
+      }
+      return have >= work;
+    };
+    double lo = 0, hi = l.wide_us + work + 1.0;
+    for (int i = 0; i < 14; ++i) {
+      const double mid = 0.5 * (lo + hi);
+      (enough(mid) ? hi : lo) = mid;
     }
-    const double end = at + (per_head - have) / std::max<size_t>(1, slots);
-    total = std::max({wide, end, narrow.longest_us + free_from[0]});
+    enough(hi);
+    total = std::max({hi, end, narrow.longest_us});
   }
-  total = std::max(total, narrow.bytes_us);
-  l.total_us = total;
+  l.total_us = overlapped(total, narrow.bytes_us);
 }
 
 }  // namespace
@@ -441,19 +471,27 @@ double arrange(const std::vector<Run>& runs, const Machine& m, int batch, const 
   const int block_rows = rows_per_block(m.head_dim);
   const int slots = (m.head_dim <= 128 ? kBlocksPerCu : 1) * m.cus;      // blocks the device holds at a time
   const int64_t wave_slots = (int64_t)slots * kWavesPerBlock;
+  double bytes = 0;
+  for (const Run& r : runs) bytes += 4.0 * m.head_dim * r.tokens * m.heads;
+  const double bytes_us = bytes / kBytesPerUs * 256 / m.cus;
   std::vector<Run> wide;
   std::vector<Narrow> narrow;
   auto go_narrow = [&](const Run& r) {
+    // a wave serves kWaveRows rows per pass; row chunks lie side by side, so that the second one finds the rows in L2
+    const int cap = std::max(1, kWaveRows / m.group), chunks = (int)std::max<int64_t>(1, ceil_div(r.n, cap));
     int64_t off = r.start;
     for (int32_t len : r.lens) {
-      narrow.push_back({off, len, r.reqs, r.n});
+      for (int c = 0; c < chunks; ++c) {
+        const int base = r.n / chunks, extra = r.n % chunks, lo = c * base + std::min(c, extra);
+        narrow.push_back({off, len, r.reqs + lo, base + (c < extra ? 1 : 0)});
+      }
       off += len;
     }
   };
   int64_t wide_blocks = 0;
   for (const Run& r : runs) {
     // (a run without tokens has no steps to place: a wave writes its empty partial results)
-    if ((int64_t)r.n * m.group <= kNarrowRows || r.tokens == 0) go_narrow(r);
+    if ((int64_t)r.n * m.group <= kWaveRows || r.tokens == 0) go_narrow(r);
     else {
       wide.push_back(r);
       wide_blocks += (int64_t)r.lens.size() * ceil_div((int64_t)r.n * m.group, block_rows) * m.heads;
@@ -471,7 +509,7 @@ double arrange(const std::vector<Run>& runs, const Machine& m, int batch, const 
     wide.swap(kept);
   }
   narrow = cut_long(std::move(narrow), m.group, m.heads, wave_slots);
-  auto passes = [&](const Narrow& v) { return (double)ceil_div((int64_t)v.n * m.group, kNarrowRows); };
+  auto passes = [&](const Narrow& v) { return (double)ceil_div((int64_t)v.n * m.group, kWaveRows); };
   std::stable_sort(narrow.begin(), narrow.end(), [&](const Narrow& a, const Narrow& b) {
     return ceil_div(a.tokens, kTile) * passes(a) > ceil_div(b.tokens, kTile) * passes(b);
   });
@@ -482,46 +520,73 @@ double arrange(const std::vector<Run>& runs, const Machine& m, int batch, const 
     for (const Narrow& v : narrow) items += (int64_t)passes(v) * m.heads;
     int share = 1;
     while (share < kWavesPerBlock && 4 * items * 2 * share <= 3 * wave_slots) share *= 2;
-    double bytes = 0;
     for (const Narrow& v : narrow) {
       const double us = kNarrowStart + kNarrowStep * ceil_div(ceil_div(v.tokens, kTile), share) * passes(v) + (share > 1 ? kNarrowShare : 0.0);
       load.block_us += us * m.heads * share / kWavesPerBlock;
       load.longest_us = std::max(load.longest_us, us);
-      bytes += 4.0 * m.head_dim * v.tokens * m.heads;
     }
-    load.bytes_us = bytes / kBytesPerUs * 256 / m.cus;
+    load.bytes_us = bytes_us;
   }
   Layout best;
-  Cut chosen{1, 0, 1};
+  Cut chosen{1, 0, 1, 1.0};
   if (wide.empty()) {
     best.total_us = std::max({load.bytes_us, load.longest_us, load.block_us / slots});
   } else {
     double score = 1e30;
     for (int rows : {block_rows, 128, 64}) {
       if (rows > block_rows) continue;
-      Cut cut{std::max(1, rows / m.group), 0, 0};
+      Cut cut{std::max(1, rows / m.group), 0, 0, 1.0};
       double whole = 0;
       for (const Run& r : wide) {
         const int chunks = (int)ceil_div(r.n, cut.rows_cap);
-        whole = std::max(whole, kVnode + step_us((int)ceil_div((int64_t)ceil_div(r.n, chunks) * m.group, 16), m.head_dim) * ceil_div(r.tokens, kTile));
+        whole = std::max(whole, kVnode + step_us((int)ceil_div((int64_t)ceil_div(r.n, chunks) * m.group, 16), m.head_dim, m.heads) * ceil_div(r.tokens, kTile));
       }
-      for (cut.row_slots = 1; cut.row_slots <= (m.head_dim <= 128 ? 2 : 1); ++cut.row_slots) {
-        double last = 0;
-        for (double us = whole; us == whole || us > kVnode + 1.0; us = kVnode + (us - kVnode) * 0.82) {
+      double wide_sum = 0;
+      for (const Piece& p : cut_runs(wide, m, Cut{cut.rows_cap, whole, 1, 1.0})) wide_sum += p.us;
+      // A launch bound by reading keeps its wide vnodes on one slot per unit and in chunks of 128 rows, so
+      // that every unit streams beside them all along (2048 requests with 1024 tokens each, 32/8 heads:
+      // 1549 us, on both slots 1562, in chunks of 192 rows 1557; a 512-document tree 274 / 282 / 280).
+      // With less than twice as much to read as to compute the second slot pays (1089 requests in 95 groups
+      // of 869 tokens, 24/8 heads: 200 us, on one slot 212).
+      const bool reading = bytes_us > 2 * wide_sum / m.units();
+      if (reading && rows > 128) continue;
+      const int row_slots = m.head_dim > 128 || reading ? 1 : 2;
+      for (cut.row_slots = 1; cut.row_slots <= row_slots; ++cut.row_slots) {
+        size_t last = 0;
+        for (double us = whole; us == whole || us > kVnode + 1.0; us = kVnode + (us - kVnode) * 0.8) {
           cut.piece_us = us;
-          Layout l;
-          l.pieces = cut_runs(wide, m, cut);
-          if ((double)l.pieces.size() == last) continue;
-          last = (double)l.pieces.size();
-          int64_t rows_out = 0;
-          for (const Piece& p : l.pieces) rows_out += p.n;
+          cut.last = 1.0;
+          std::vector<Piece> pieces = cut_runs(wide, m, cut);
+          if (pieces.size() == last) continue;
+          last = pieces.size();
+          double rows_out = 0, sum = 0, longest = 0;
+          for (const Piece& p : pieces) {
+            rows_out += p.n;
+            sum += p.us;
+            longest = std::max(longest, p.us);
+          }
           const double scratch = 8.0 * rows_out * m.group * m.heads * (m.head_dim + 1) / kScratchPerUs;
-          if (l.pieces.size() > 4096 || scratch > score) break;
-          place(l, m, cut, load);
-          if (l.total_us + scratch < score) {
-            score = l.total_us + scratch;
-            best = std::move(l);
-            chosen = cut;
+          if (last > 4096 || scratch > score) break;
+          // (what no placement goes below)
+          const double least = std::max(longest, sum / m.units() * (cut.row_slots == 2 ? 0.5 * (1 + kPairing) : 1.0));
+          if (overlapped(least, load.bytes_us) + scratch >= score) continue;
+          double even_us = 0;
+          for (double ratio : {1.0, 0.87}) {
+            if (ratio < 1.0) {
+              // (a shorter last piece gains a tenth at most)
+              if (cut.row_slots == 1 || even_us > 1.1 * score) break;
+              cut.last = ratio;
+              pieces = cut_runs(wide, m, cut);
+            }
+            Layout l;
+            l.pieces = std::move(pieces);
+            place(l, m, cut, load);
+            even_us = l.total_us + scratch;
+            if (l.total_us + scratch < score) {
+              score = l.total_us + scratch;
+              best = std::move(l);
+              chosen = cut;
+            }
           }
         }
       }

@@ -613,9 +613,9 @@ def fasttree_preparation(
     """
     from . import launch_schedule
 
-    # (alpha = beta = 0 takes the padding out of the cost model and leaves gamma to force or forbid every
-    # merge: such a plan keeps the merges it was asked for)
-    if (launch_order and (params.alpha or params.beta) and launch_schedule.native_schedule()
+    # (alpha = beta = 0 takes the padding out of the cost model, and a gamma far from its defaults outweighs
+    # it: either way every merge is forced or forbidden, and such a plan keeps the merges it was asked for)
+    if (launch_order and (params.alpha or params.beta) and 0 <= params.gamma <= 1 and launch_schedule.native_schedule()
             and _native_chosen(None, KV_ptrs, KV_SPLIT_SIZES, para_threshs1, para_threshs2, params)):
         L = _plan_lib
         tree = L.TreeArrays(tree_info, KV_ptrs)

@@ -474,9 +474,16 @@ class PlanBuffers:
         if host.numel() > dst.numel():
             raise ValueError(f"{name}: {host.numel()} entries do not fit the {dst.numel()} that were allocated")
         part = dst[: host.numel()]
-        # (tensors handed in lie in pinned memory: copied in stream order, the allocator keeps the block until then)
+        # (tensors handed in lie in pinned memory: their copies are queued, and :meth:`finish` waits for all of them)
         part.copy_(host, non_blocking=host is values)
         return part
+
+    def finish(self):
+        """Waits for the copies of a plan's tensors: a plan may be used on any stream once it is returned."""
+        import torch
+
+        if _on_gpu(self.device):
+            torch.cuda.current_stream(self.device).synchronize()
 
 
 def place_plan(kv_entries, vnodes, q_entries, per_request, phase_nums, phase_offs,
@@ -543,9 +550,10 @@ def _place_arranged(plan, kv_entries, num_qo_heads, head_dim, device, buffers):
 
     if buffers is not None:
         part = {name: buffers.fill(full, plan.part[name]) for name, full in _BUFFER_OF.items() if name in plan.part}
+        buffers.finish()
     else:
         # one copy for the whole plan; the arrays are views of it
-        whole = plan.packed.to(device, non_blocking=True)
+        whole = plan.packed.to(device)
         part = {name: whole[lo: lo + n] for name, (lo, n) in plan.where.items()}
     nums = LaunchPhases([plan.n_wide, plan.n_narrow])
     nums.modelled_us, nums.num_cus, nums.block_slots = plan.modelled_us, plan.num_cus, plan.block_slots

@@ -104,6 +104,12 @@ Pair int32_pair(PyObject* o) {
   return p;
 }
 
+// Gives the interpreter up around a launch (a full queue makes it wait).
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
 // What a launch-order plan's phase list carries besides its two counts (null / 0: not there).
 struct PlanTables {
   const int32_t *prog_table = nullptr, *narrow_table = nullptr, *prog_records = nullptr, *req_table = nullptr;
@@ -186,7 +192,9 @@ int decode_call(const at::Tensor& q, const Rows& qr, const at::Tensor& k, const 
   if (scale == -1.0 && PyErr_Occurred()) throw PyFailure{};
   const int d = (int)qr.dim, dtype = dtype_code(q);
   const ft_stream_t stream = stream_of(q);
-  if ((plan.prog_table || plan.narrow_table) && d >= 32)
+  const int heads_kv = (int)k.size(1);
+  if ((plan.prog_table || plan.narrow_table) && d >= 32) {
+    Unlocked unlocked;
     // the launch was arranged as block programs (launch_schedule.block_programs)
     return ft_decode_programs(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), qr.s0, qr.s1, k.stride(0), k.stride(1), v.stride(0),
                               v.stride(1), orow.s0, orow.s1, i32(*index[0]), i32(*index[1]), i32(*index[2]), i32(*index[3]),
@@ -194,13 +202,15 @@ int decode_call(const at::Tensor& q, const Rows& qr, const at::Tensor& k, const 
                               static_cast<float*>(mid_o.data_ptr()), mid_o.stride(0), mid_o.stride(1),
                               static_cast<float*>(mid_lse.data_ptr()), mid_lse.stride(0), nums.v, offs.v, plan.prog_table,
                               plan.num_programs, plan.narrow_in_programs, plan.narrow_table, plan.prog_records, plan.req_table,
-                              (int)qr.n, (int)qr.heads, (int)k.size(1), d, (float)scale, dtype, stream);
+                              (int)qr.n, (int)qr.heads, heads_kv, d, (float)scale, dtype, stream);
+  }
   const Pair q_tiles = int32_pair(phase_q_tiles), kv_tiles = int32_pair(phase_kv_tiles);
+  Unlocked unlocked;
   return ft_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), qr.s0, qr.s1, k.stride(0), k.stride(1), v.stride(0),
                    v.stride(1), orow.s0, orow.s1, i32(*index[0]), i32(*index[1]), i32(*index[2]), i32(*index[3]), i32(*index[4]),
                    i32(*index[5]), i32(*index[6]), i32(*index[7]), i32(*index[8]), static_cast<float*>(mid_o.data_ptr()),
                    mid_o.stride(0), mid_o.stride(1), static_cast<float*>(mid_lse.data_ptr()), mid_lse.stride(0), nums.v, offs.v,
-                   q_tiles.v, kv_tiles.v, (int)qr.n, (int)qr.heads, (int)k.size(1), d, (float)scale, dtype, stream);
+                   q_tiles.v, kv_tiles.v, (int)qr.n, (int)qr.heads, heads_kv, d, (float)scale, dtype, stream);
 }
 
 // decode(q, k_buffer, v_buffer, o, the nine index tensors, mid_o, mid_lse, phase_node_nums,
@@ -234,9 +244,12 @@ int store_call(const at::Tensor& kn, const at::Tensor& vn, const at::Tensor& loc
   if (v.n != k.n || loc.numel() != k.n) refuse("cache_k, cache_v and out_cache_loc must name the same number of tokens");
   if ((loc.scalar_type() != at::kInt && loc.scalar_type() != at::kLong) || !loc.is_contiguous())
     refuse("out_cache_loc must be a contiguous int32 or int64 tensor");
+  const int dtype = dtype_code(kb);
+  const ft_stream_t stream = stream_of(kb);
+  Unlocked unlocked;
   return ft_store_kv(kn.data_ptr(), vn.data_ptr(), k.s0, k.s1, v.s0, v.s1, loc.data_ptr(), loc.scalar_type() == at::kLong, (int)k.n,
                      kb.data_ptr(), vb.data_ptr(), kb.stride(0), kb.stride(1), vb.stride(0), vb.stride(1),
-                     std::min(kb.size(0), vb.size(0)), (int)hkv, (int)d, dtype_code(kb), stream_of(kb));
+                     std::min(kb.size(0), vb.size(0)), (int)hkv, (int)d, dtype, stream);
 }
 
 // store_kv(cache_k, cache_v, out_cache_loc, k_buffer, v_buffer) -> code

@@ -22,7 +22,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
-#include <new>
+#include <memory>
 #include <numeric>
 #include <queue>
 #include <unordered_map>
@@ -614,12 +614,12 @@ int ft_schedule_create(int64_t num_vnodes, const int32_t* kv_offs, const int32_t
     if (q_entries[i] < 0 || q_entries[i] >= batch_size) return FT_SCHEDULE_ERR_ARGUMENT;
   try {
     const Machine m{num_cus, num_kv_heads, group, head_dim};
-    ft_schedule* s = new ft_schedule;
+    auto s = std::make_unique<ft_schedule>();
     const double us = arrange(runs_of(num_vnodes, kv_offs, kv_lens, q_offs, q_lens, q_entries), m, batch_size, kv_entries, *s);
     if (modelled_us) *modelled_us = us;
-    *out = s;
+    *out = s.release();
     return FT_SCHEDULE_OK;
-  } catch (const std::bad_alloc&) {
+  } catch (const std::exception&) {   // bad_alloc, length_error
     return FT_SCHEDULE_ERR_MEMORY;
   }
 }
@@ -638,13 +638,13 @@ int ft_schedule_tree(int num_nodes, const int32_t* parent, const int32_t* seqlen
     const Machine m{num_cus, num_kv_heads, group, head_dim};
     TreeRuns t;
     if (int rc = tree_runs(num_nodes, parent, seqlen, num_children, req_offs, req_ids, kv_ptrs, kv_slot_map, kv_slot_map_len, m, t)) return rc;
-    ft_schedule* s = new ft_schedule;
+    auto s = std::make_unique<ft_schedule>();
     const double us = arrange(t.runs, m, batch_size, t.kv_entries.data(), *s);
     s->arrays[FT_SCHEDULE_KV_ENTRIES] = std::move(t.kv_entries);
     if (modelled_us) *modelled_us = us;
-    *out = s;
+    *out = s.release();
     return FT_SCHEDULE_OK;
-  } catch (const std::bad_alloc&) {
+  } catch (const std::exception&) {   // bad_alloc, length_error
     return FT_SCHEDULE_ERR_MEMORY;
   }
 }

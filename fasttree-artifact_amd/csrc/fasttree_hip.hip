@@ -1119,6 +1119,7 @@ __device__ __forceinline__ void wide_pass(const Stage1Args& a, char* smem, const
   // nothing the compiler itself tracks (the Q fragments) may still be in flight in the loop:
   // a wait for it there would also wait for every direct load
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  wait_direct_loads<0>();              // (no access to LDS moves above it either)
   // (and the compiler must see the fragments as complete, or it keeps a wait for them in the loop)
 #pragma unroll
   for (int qb = 0; qb < NG; ++qb)
@@ -1312,6 +1313,7 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
     // nothing the compiler itself tracks may still be in flight below: a wait for it would
     // also wait for every direct load
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+    wait_direct_loads<0>();              // (no access to LDS moves above it either)
     // (and the compiler must see the fragments as complete, or it keeps a wait for them in the loop)
 #pragma unroll
     for (int qb = 0; qb < NG; ++qb)

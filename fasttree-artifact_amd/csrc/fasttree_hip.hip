@@ -1873,17 +1873,17 @@ template <int WIDTH> __device__ __forceinline__ float group_sum(float x) {
 // Bound by the partial rows it reads, and for a batch of few requests by how many of them are in
 // flight: 8 requests x 64 heads with 68 partials each take 64 blocks 11.2 us, one split per group of
 // lanes; with the partials split eight ways 512 blocks.
-template <typename E, int D>
+template <typename E, int D, bool SPLIT>
 __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
   constexpr int LPH = D / 4;
   constexpr int HPB = kBlock / LPH;
   const int grp = threadIdx.x / LPH, gl = threadIdx.x % LPH;
   const int req = blockIdx.x;
-  int S = a.splits;                                         // (a power of two; launch uniform)
-  int split = grp & (S - 1);
-  const int head = blockIdx.y * (HPB / S) + grp / S;
+  int S = SPLIT ? a.splits : 1;                             // (a power of two; launch uniform)
+  int split = SPLIT ? grp & (S - 1) : 0;
+  const int head = SPLIT ? blockIdx.y * (HPB / S) + grp / S : blockIdx.y * HPB + grp;
   const bool exists = head < a.hq;
-  if (S == 1 && !exists) return;
+  if (!SPLIT && !exists) return;
   const int32_t* rec = a.req_table ? a.req_table + (int64_t)req * kReqRecord : nullptr;  // launch uniform
   int off, n, rec_row = -1;
   if (a.nsplit > 0) {
@@ -1897,13 +1897,13 @@ __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
     off = a.req_offs[req];
     n = a.req_lens[req];
   }
-  if (S > 1 && n <= kReqRecEntries) {   // block uniform: a short list is one group's work (merging costs about 1 us)
+  if (SPLIT && n <= kReqRecEntries) {   // block uniform: a short list is one group's work (merging costs about 1 us)
     if (split > 0 || !exists) return;
     S = 1;
     split = 0;
   }
   const int first = split + S * gl;                         // this lane's first entry of the request's list
-  const int mine = exists ? (n - split + S - 1) / S : 0;    // partials of this group (0 or less: none)
+  const int mine = !SPLIT ? n : exists ? (n - split + S - 1) / S : 0;    // partials of this group (0 or less: none)
 
   float m_run = -INFINITY, l_run = 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
@@ -1948,7 +1948,7 @@ __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
       }
     }
   }
-  if (S > 1) {
+  if (SPLIT && S > 1) {
     // the groups' states to the first of them
     __shared__ f32x4 acc_of[kBlock];
     __shared__ float m_of[HPB], l_of[HPB];
@@ -2169,18 +2169,20 @@ int launch_stage1(const Stage1Args& a, int d, int dtype, hipStream_t stream) {
   return FT_ERR_DTYPE;
 }
 
-// Lane groups per (request, head): as many as leave the launch at most four blocks per compute unit
-// (wave_slots() / 2): more blocks than that hide each other's round trips anyway.  One group where every
-// list is short.
+// Lane groups per (request, head): as many as leave the launch at most two blocks per compute unit
+// (wave_slots() / 4): more blocks than that hide each other's round trips anyway.  One group, and the
+// kernel without the merge, where every list is short or the batch fills the machine by itself (684
+// requests of 32 heads: 8.2 us without the merge's code, 9.6 with it).
 template <typename E, int D>
 int launch_stage2_inst(const Stage2Args& a0, hipStream_t stream) {
   constexpr int HPB = kBlock / (D / 4);
   Stage2Args a = a0;
   a.splits = 1;
-  while (a.longest > kReqRecEntries && a.splits < HPB && (int64_t)a.batch * ((a.hq * a.splits * 2 + HPB - 1) / HPB) <= wave_slots() / 2) a.splits *= 2;
+  while (a.longest > kReqRecEntries && a.splits < HPB && (int64_t)a.batch * ((a.hq * a.splits * 2 + HPB - 1) / HPB) <= wave_slots() / 4) a.splits *= 2;
   const int heads = HPB / a.splits;
-  hipLaunchKernelGGL((stage2_kernel<E, D>), dim3((unsigned)a.batch, (unsigned)((a.hq + heads - 1) / heads), 1),
-                     dim3(kBlock, 1, 1), 0, stream, a);
+  const dim3 grid((unsigned)a.batch, (unsigned)((a.hq + heads - 1) / heads), 1);
+  if (a.splits > 1) hipLaunchKernelGGL((stage2_kernel<E, D, true>), grid, dim3(kBlock, 1, 1), 0, stream, a);
+  else hipLaunchKernelGGL((stage2_kernel<E, D, false>), grid, dim3(kBlock, 1, 1), 0, stream, a);
   return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
 }
 

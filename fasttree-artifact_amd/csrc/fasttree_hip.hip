@@ -998,45 +998,52 @@ struct WidePass {
   const int* record;   // the program's record in LDS, or null
 };
 
+// A wave's state in LDS for another wave to merge: its accumulators as 16-byte words, then m and l.
+// kFloats: per lane.  (16-byte accesses: a quarter of the instructions of 4-byte ones, on a path that every
+// vnode takes once, with cold code.)
+template <int D, int NG> struct SharedState {
+  static constexpr int DB = D / 16;
+  static constexpr int kFloats = NG * (4 * DB + 2);
+  static __device__ __forceinline__ void put(float* at, const WaveState<D, NG>& st) {
+    const int lane = threadIdx.x & 63;
+    f32x4* o = reinterpret_cast<f32x4*>(at) + lane;
+    float* ml = at + NG * DB * 4 * kWave + lane;
+#pragma unroll
+    for (int qb = 0; qb < NG; ++qb) {
+      ml[2 * qb * kWave] = st.m[qb];
+      ml[(2 * qb + 1) * kWave] = st.l[qb];
+#pragma unroll
+      for (int db = 0; db < DB; ++db) o[(qb * DB + db) * kWave] = st.o[qb][db];
+    }
+  }
+  static __device__ __forceinline__ void merge(const float* at, WaveState<D, NG>& st) {
+    const int lane = threadIdx.x & 63;
+    const f32x4* o = reinterpret_cast<const f32x4*>(at) + lane;
+    const float* ml = at + NG * DB * 4 * kWave + lane;
+#pragma unroll
+    for (int qb = 0; qb < NG; ++qb) {
+      const float m2 = ml[2 * qb * kWave], l2 = ml[(2 * qb + 1) * kWave];
+      const float m = fmaxf(st.m[qb], m2);
+      const float a1 = scale_from(st.m[qb], m), a2 = scale_from(m2, m);
+      st.l[qb] = st.l[qb] * a1 + l2 * a2;
+      st.m[qb] = m;
+#pragma unroll
+      for (int db = 0; db < DB; ++db) st.o[qb][db] = st.o[qb][db] * a1 + o[(qb * DB + db) * kWave] * a2;
+    }
+  }
+};
+
 // Merge of the waves that hold the same rows (the token groups of a row set) into token group 0,
 // pairwise through LDS.  Every wave of the block must call this.
 template <int D, int NG>
 __device__ __forceinline__ void merge_token_groups(float* xchg, WaveState<D, NG>& st, const WidePass& p) {
-  constexpr int NV = (D / 16) * 4 + 2;   // floats of state per lane and row group
-  const int lane = threadIdx.x & 63;
+  constexpr int kArea = WideRows<D>::kGroups * SharedState<D, 1>::kFloats * kWave;   // (waves of other sets may hold fewer groups)
+#pragma unroll 1
   for (int half = p.tgroups >> 1; half >= 1; half >>= 1) {
     __syncthreads();
-    if (p.tg >= half && p.tg < 2 * half) {
-      float* dst = xchg + (size_t)(p.set * half + p.tg - half) * WideRows<D>::kGroups * NV * kWave + lane;
-#pragma unroll
-      for (int qb = 0; qb < NG; ++qb) {
-        int n = qb * NV;
-        dst[(n++) * kWave] = st.m[qb];
-        dst[(n++) * kWave] = st.l[qb];
-#pragma unroll
-        for (int db = 0; db < D / 16; ++db)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) dst[(n++) * kWave] = st.o[qb][db][j];
-      }
-    }
+    if (p.tg >= half && p.tg < 2 * half) SharedState<D, NG>::put(xchg + (size_t)(p.set * half + p.tg - half) * kArea, st);
     __syncthreads();
-    if (p.tg < half) {
-      const float* src = xchg + (size_t)(p.set * half + p.tg) * WideRows<D>::kGroups * NV * kWave + lane;
-#pragma unroll
-      for (int qb = 0; qb < NG; ++qb) {
-        int n = qb * NV;
-        const float m2 = src[(n++) * kWave];
-        const float l2 = src[(n++) * kWave];
-        const float m = fmaxf(st.m[qb], m2);
-        const float a1 = scale_from(st.m[qb], m), a2 = scale_from(m2, m);
-        st.l[qb] = st.l[qb] * a1 + l2 * a2;
-        st.m[qb] = m;
-#pragma unroll
-        for (int db = 0; db < D / 16; ++db)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) st.o[qb][db][j] = st.o[qb][db][j] * a1 + src[(n++) * kWave] * a2;
-      }
-    }
+    if (p.tg < half) SharedState<D, NG>::merge(xchg + (size_t)(p.set * half + p.tg) * kArea, st);
   }
 }
 
@@ -1396,43 +1403,15 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
 // them, pairwise through LDS at xchg.  Every wave of the block calls this (block barriers).
 template <int D, int NG>
 __device__ __forceinline__ void merge_shares(float* xchg, WaveState<D, NG>& st, int w, int share) {
-  constexpr int NV = (D / 16) * 4 + 2;  // floats of state per lane and row group
-  static_assert(2 * NG * NV * 4 * kWave <= 4 * NarrowGeom<D>::kLds && NG * NV * 4 * kWave <= 2 * NarrowGeom<D>::kLds,
+  constexpr int kArea = SharedState<D, NG>::kFloats * kWave;
+  static_assert(2 * kArea * 4 <= 4 * NarrowGeom<D>::kLds && kArea * 4 <= 2 * NarrowGeom<D>::kLds,
                 "half of the waves' states fit the LDS areas of all of them");
-  const int lane = threadIdx.x & 63;
+#pragma unroll 1
   for (int half = share >> 1; half >= 1; half >>= 1) {
     __syncthreads();
-    if (w >= half && w < 2 * half) {
-      float* dst = xchg + (size_t)(w - half) * NG * NV * kWave + lane;
-      int n = 0;
-#pragma unroll
-      for (int qb = 0; qb < NG; ++qb) {
-        dst[(n++) * kWave] = st.m[qb];
-        dst[(n++) * kWave] = st.l[qb];
-#pragma unroll
-        for (int db = 0; db < D / 16; ++db)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) dst[(n++) * kWave] = st.o[qb][db][j];
-      }
-    }
+    if (w >= half && w < 2 * half) SharedState<D, NG>::put(xchg + (size_t)(w - half) * kArea, st);
     __syncthreads();
-    if (w < half) {
-      const float* src = xchg + (size_t)w * NG * NV * kWave + lane;
-      int n = 0;
-#pragma unroll
-      for (int qb = 0; qb < NG; ++qb) {
-        const float m2 = src[(n++) * kWave];
-        const float l2 = src[(n++) * kWave];
-        const float m = fmaxf(st.m[qb], m2);
-        const float a1 = scale_from(st.m[qb], m), a2 = scale_from(m2, m);
-        st.l[qb] = st.l[qb] * a1 + l2 * a2;
-        st.m[qb] = m;
-#pragma unroll
-        for (int db = 0; db < D / 16; ++db)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) st.o[qb][db][j] = st.o[qb][db][j] * a1 + src[(n++) * kWave] * a2;
-      }
-    }
+    if (w < half) SharedState<D, NG>::merge(xchg + (size_t)w * kArea, st);
   }
 }
 

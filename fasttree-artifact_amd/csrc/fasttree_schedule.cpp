@@ -69,6 +69,7 @@ constexpr double kBytesPerUs = 5.6e6;  // rows at random slots, the whole part
 constexpr double kScratchPerUs = 4.0e6;  // partial results, written and read back
 constexpr double kNoOverlap = 0.35;
 constexpr double kLaunch = 1.5;
+constexpr double kSmallLaunchBytes = 64e6;   // of K/V rows, for 256 units: about what they read while a wide vnode starts and ends twice
 
 struct Run {
   int64_t start;                 // into the flat slot list
@@ -467,7 +468,17 @@ void build(const Machine& m, int batch, Layout& l, std::vector<Narrow>& narrow, 
   }
 }
 
-double arrange(const std::vector<Run>& runs, const Machine& m, int batch, const int32_t* kv_entries, ft_schedule& s) {
+// A launch: its programs, its narrow vnodes, and what the model expects of both stages.
+struct Launch {
+  Layout layout;
+  std::vector<Narrow> narrow;
+  Cut chosen{1, 0, 1, 1.0};
+  bool programs = false;
+  double score = 1e30;
+};
+
+// The launch with runs of up to narrow_rows query rows served by waves of their own, wave_rows of them each.
+Launch solve(const std::vector<Run>& runs, const Machine& m, int narrow_rows, int wave_rows) {
   const int block_rows = rows_per_block(m.head_dim);
   const int slots = (m.head_dim <= 128 ? kBlocksPerCu : 1) * m.cus;      // blocks the device holds at a time
   const int64_t wave_slots = (int64_t)slots * kWavesPerBlock;
@@ -475,10 +486,11 @@ double arrange(const std::vector<Run>& runs, const Machine& m, int batch, const 
   for (const Run& r : runs) bytes += 4.0 * m.head_dim * r.tokens * m.heads;
   const double bytes_us = bytes / kBytesPerUs * 256 / m.cus;
   std::vector<Run> wide;
-  std::vector<Narrow> narrow;
+  Launch out;
+  std::vector<Narrow>& narrow = out.narrow;
   auto go_narrow = [&](const Run& r) {
-    // a wave serves kWaveRows rows per pass; row chunks lie side by side, so that the second one finds the rows in L2
-    const int cap = std::max(1, kWaveRows / m.group), chunks = (int)std::max<int64_t>(1, ceil_div(r.n, cap));
+    // a wave serves up to kWaveRows rows per pass; row chunks lie side by side, so that the second one finds the rows in L2
+    const int cap = std::max(1, wave_rows / m.group), chunks = (int)std::max<int64_t>(1, ceil_div(r.n, cap));
     int64_t off = r.start;
     for (int32_t len : r.lens) {
       for (int c = 0; c < chunks; ++c) {
@@ -491,7 +503,7 @@ double arrange(const std::vector<Run>& runs, const Machine& m, int batch, const 
   int64_t wide_blocks = 0;
   for (const Run& r : runs) {
     // (a run without tokens has no steps to place: a wave writes its empty partial results)
-    if ((int64_t)r.n * m.group <= kWaveRows || r.tokens == 0) go_narrow(r);
+    if ((int64_t)r.n * m.group <= narrow_rows || r.tokens == 0) go_narrow(r);
     else {
       wide.push_back(r);
       wide_blocks += (int64_t)r.lens.size() * ceil_div((int64_t)r.n * m.group, block_rows) * m.heads;
@@ -509,30 +521,34 @@ double arrange(const std::vector<Run>& runs, const Machine& m, int batch, const 
     wide.swap(kept);
   }
   narrow = cut_long(std::move(narrow), m.group, m.heads, wave_slots);
-  auto passes = [&](const Narrow& v) { return (double)ceil_div((int64_t)v.n * m.group, kWaveRows); };
+  // (a pass of one 16-row group costs less than one of two: at 512-byte rows about half)
+  auto passes = [&](const Narrow& v) {
+    const int64_t rows = (int64_t)v.n * m.group;
+    return rows <= 16 ? (m.head_dim <= 128 ? 0.8 : 0.55) : (double)ceil_div(rows, kWaveRows);
+  };
   std::stable_sort(narrow.begin(), narrow.end(), [&](const Narrow& a, const Narrow& b) {
     return ceil_div(a.tokens, kTile) * passes(a) > ceil_div(b.tokens, kTile) * passes(b);
   });
   NarrowLoad load{0, 0, 0};
   {
     // the launcher lets 2 or 4 waves share a vnode while that leaves a quarter of the wave slots free
-    int64_t items = 0;
-    for (const Narrow& v : narrow) items += (int64_t)passes(v) * m.heads;
+    const int64_t items = (int64_t)narrow.size() * m.heads;
     int share = 1;
     while (share < kWavesPerBlock && 4 * items * 2 * share <= 3 * wave_slots) share *= 2;
     for (const Narrow& v : narrow) {
-      const double us = kNarrowStart + kNarrowStep * ceil_div(ceil_div(v.tokens, kTile), share) * passes(v) + (share > 1 ? kNarrowShare : 0.0);
+      const double us = kNarrowStart + kNarrowStep * std::max(0.6, m.head_dim / 128.0) * ceil_div(ceil_div(v.tokens, kTile), share) * passes(v) + (share > 1 ? kNarrowShare : 0.0);
       load.block_us += us * m.heads * share / kWavesPerBlock;
       load.longest_us = std::max(load.longest_us, us);
     }
     load.bytes_us = bytes_us;
   }
-  Layout best;
-  Cut chosen{1, 0, 1, 1.0};
+  Layout& best = out.layout;
+  Cut& chosen = out.chosen;
+  double& score = out.score;
+  out.programs = !wide.empty();
   if (wide.empty()) {
-    best.total_us = std::max({load.bytes_us, load.longest_us, load.block_us / slots});
+    score = best.total_us = std::max({load.bytes_us, load.longest_us, load.block_us / slots});
   } else {
-    double score = 1e30;
     for (int rows : {block_rows, 128, 64}) {
       if (rows > block_rows) continue;
       Cut cut{std::max(1, rows / m.group), 0, 0, 1.0};
@@ -592,9 +608,34 @@ double arrange(const std::vector<Run>& runs, const Machine& m, int batch, const 
       }
     }
   }
-  build(m, batch, best, narrow, kv_entries, s);
-  s.arrays[FT_SCHEDULE_COUNTS][3] = wide.empty() ? slots : chosen.row_slots * m.cus;
-  return best.total_us + kLaunch;
+  double narrow_out = 0;
+  for (const Narrow& v : narrow) narrow_out += v.n;
+  score += 8.0 * narrow_out * m.group * m.heads * (m.head_dim + 1) / kScratchPerUs;
+  return out;
+}
+
+double arrange(const std::vector<Run>& runs, const Machine& m, int batch, const int32_t* kv_entries, ft_schedule& s) {
+  Launch best = solve(runs, m, kWaveRows, kWaveRows);
+  // In a small launch a wide vnode's start-up is most of it, and runs of a few more rows than a wave's are
+  // sooner done by several waves of one 16-row group each (3 requests of 16/1 heads of 256 on an 881-token run: 18.6 us wide,
+  // 16.9 narrow; a 71-request tree of 16/1 heads 21.6 and 20.1).  A larger one would read their rows twice.
+  double bytes = 0;
+  for (const Run& r : runs) bytes += 4.0 * m.head_dim * r.tokens * m.heads;
+  if (bytes * 256 / m.cus < kSmallLaunchBytes) {
+    int tried = 16;
+    for (int limit : {kWaveRows, 64, 128}) {
+      bool any = false;
+      for (const Run& r : runs) any = any || ((int64_t)r.n * m.group > tried && (int64_t)r.n * m.group <= limit && r.tokens > 0);
+      tried = limit;
+      if (!any) continue;
+      Launch other = solve(runs, m, limit, 16);
+      if (other.score < best.score) best = std::move(other);
+    }
+  }
+  build(m, batch, best.layout, best.narrow, kv_entries, s);
+  const int slots = (m.head_dim <= 128 ? kBlocksPerCu : 1) * m.cus;
+  s.arrays[FT_SCHEDULE_COUNTS][3] = best.programs ? best.chosen.row_slots * m.cus : slots;
+  return best.layout.total_us + kLaunch;
 }
 
 }  // namespace

@@ -617,8 +617,10 @@ Launch solve(const std::vector<Run>& runs, const Machine& m, int narrow_rows, in
 double arrange(const std::vector<Run>& runs, const Machine& m, int batch, const int32_t* kv_entries, ft_schedule& s) {
   Launch best = solve(runs, m, kWaveRows, kWaveRows);
   // In a small launch a wide vnode's start-up is most of it, and runs of a few more rows than a wave's are
-  // sooner done by several waves of one 16-row group each (3 requests of 16/1 heads of 256 on an 881-token run: 18.6 us wide,
-  // 16.9 narrow; a 71-request tree of 16/1 heads 21.6 and 20.1).  A larger one would read their rows twice.
+  // sooner done by several waves of one 16-row group each (whole calls: 3 requests of 16/1 heads of 256 on an
+  // 881-token run 18.6 us wide, 14.8 narrow; 50 requests of 32/8 heads of 256 in six groups of 611 tokens
+  // 30.9 and 24.9; 25 requests of 32/8 heads in two groups of 352 tokens 17.9 and 12.3).  A larger one would
+  // read their rows twice.
   double bytes = 0;
   for (const Run& r : runs) bytes += 4.0 * m.head_dim * r.tokens * m.heads;
   if (bytes * 256 / m.cus < kSmallLaunchBytes) {

@@ -114,6 +114,8 @@ __device__ __forceinline__ int lane_here() {
   asm volatile("" : "+v"(lane));
   return lane;
 }
+// The four low bits of x reversed (each on its own, so that constant parts fold).
+__device__ __forceinline__ constexpr int reversed4(int x) { return ((x & 1) << 3) | ((x & 2) << 1) | ((x >> 1) & 2) | ((x >> 3) & 1); }
 // Orders this wave's LDS traffic around a point where lanes read what other lanes of the
 // same wave wrote.  LDS executes one wave's instructions in order, so no wait is needed;
 // the fences only stop the compiler from moving accesses across.
@@ -556,13 +558,22 @@ template <int D> struct WideRows {
 };
 constexpr int kDeftRows = 32 * kWideWaves;        // (the comparison engine's kernel: 32 rows per wave)
 
+// The XOR that places the 16-byte chunks of a row in LDS.  Operands are read 16 rows at a time (K, one
+// chunk) and 4 rows x 2 chunks at a time (V, transposed), and either has to hit all 64 banks.  Rows of 256
+// bytes and more start at the same bank: their four low bits, the two pairs swapped, give every row its own
+// chunk.  Shorter rows fill the banks between them: what the row number leaves to the chunk are its
+// higher bits, so the bits are reversed before they are cut off (64-dim heads: 2-way conflicts in both
+// reads with the pairs swapped, none so; 380 requests of 64/8 heads 22.5 -> 21.8 us, a 94-request tree of 16/1
+// heads 23.1 -> 21.5).
+template <int D> __device__ __forceinline__ constexpr int chunk_swizzle(int row) {
+  return (D < 128 ? reversed4(row) : ((row & 3) << 2) | ((row >> 2) & 3)) & (D / 8 - 1);
+}
+
 // LDS layout of the wide kernel: rows of 2*D bytes back to back (no padding), 64-token super
 // tiles of two 32-token tiles, a ring of kBufs buffers, then the rings of slot indices and a
 // program's record.  A row's 16-byte chunks are stored XOR-permuted: chunk c of row r sits in slot
-// c ^ swz(r).  swz swaps the two low bit pairs of r, which makes both read patterns conflict free
-// for 256-byte rows: the K operand read (16 different rows, same chunk) and the transposed V
-// read (4 consecutive rows x 4 consecutive chunks).  Loads go global -> LDS directly; one wave
-// instruction fills a 1 KB group of consecutive rows.
+// c ^ swz(r) (chunk_swizzle above).  Loads go global -> LDS directly; one wave instruction fills a 1 KB
+// group of consecutive rows.
 template <int D> struct WideGeom {
   static constexpr int kRowBytes = 2 * D;
   static constexpr int kChunks = D / 8;                  // 16-byte chunks per row
@@ -580,7 +591,7 @@ template <int D> struct WideGeom {
   static constexpr int kIdxBytes = kWideWaves * 4 * 4 * kTokens;                   // per wave: the slot indices of four super tiles
   static constexpr int kRecord = kRing + kIdxBytes;      // byte offset of the program's record (kProgRecord ints)
   static constexpr int kLds = kRecord + 1024;
-  static __device__ __forceinline__ int swz(int row) { return (((row & 3) << 2) | ((row >> 2) & 3)) & (kChunks - 1); }
+  static __device__ __forceinline__ int swz(int row) { return chunk_swizzle<D>(row); }
 };
 
 // State of one wave for 32 query rows (32x32x16 tiles).  o[db][j] = O[row lane%32][dim 32*db + 8*(j/4) +
@@ -1231,7 +1242,7 @@ template <int D> struct NarrowGeom {
   static constexpr int kIdxSlot = 4 * kWave;                    // bytes of one tile's indices (32, and the 32 after them)
   static constexpr int kLds = kBytes + 4 * kIdxSlot;            // per wave; a multiple of the row size
   static constexpr int kGroups = 2;                             // 16-row groups per pass (three spill beside the wide path's code)
-  static __device__ __forceinline__ int swz(int row) { return (((row & 3) << 2) | ((row >> 2) & 3)) & (kChunks - 1); }
+  static __device__ __forceinline__ int swz(int row) { return chunk_swizzle<D>(row); }
 };
 
 // Layout of a narrow vnode's record in Stage1Args::narrow_table (ints): kv_off, kv_len, q_off,

@@ -128,6 +128,21 @@ __device__ __forceinline__ float scale_from(float m_part, float m_all) {
   return (m_part == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_part - m_all);
 }
 
+// x / d for 0 <= x < 2^31 by a multiplication: mul = ceil(2^(31 + shift) / d) with shift = ceil(log2 d), whose
+// excess over the exact factor is less than 2^-31 of it.  (The compiler's division by a value it does not know is
+// some 25 instructions, and what runs once per block is fetched cold.)
+struct Divisor {
+  unsigned mul, shift;
+  __host__ __device__ constexpr int operator()(int x) const { return (int)((unsigned)(((uint64_t)(2u * (unsigned)x) * mul) >> 32) >> shift); }
+};
+__host__ __device__ constexpr Divisor divisor(int d) {
+  unsigned shift = 0;
+  while ((int64_t(1) << shift) < d) ++shift;
+  return Divisor{(unsigned)(((uint64_t(1) << (31 + shift)) + d - 1) / d), shift};
+}
+static_assert(divisor(1)(INT32_MAX) == INT32_MAX && divisor(64)(INT32_MAX) == INT32_MAX / 64 && divisor(7)(INT32_MAX) == INT32_MAX / 7 &&
+              divisor(3)(INT32_MAX - 1) == (INT32_MAX - 1) / 3 && divisor(65535)(65534) == 0 && divisor(65535)(65535) == 1);
+
 struct Stage1Args {
   const char* q;
   const char* k;
@@ -163,6 +178,7 @@ struct Stage1Args {
                                    // which the per-wave staging kernels compute as a zero-padded 32-dim contraction
   int g;
   int hkv;
+  Divisor by_g, by_hkv;
   float scale_log2;  // sm_scale * log2(e)
   float* mid_o;
   int64_t so0, so1;
@@ -210,21 +226,26 @@ __device__ __forceinline__ const Stage1Args& args_again() {
   return *(const Stage1Args*)p;
 }
 
+// The plan's lists and tables, which no kernel writes, as the constant address space: reads at an address that
+// is the same for the whole wave are scalar loads wherever they stand.
+typedef const int32_t __attribute__((address_space(4)))* PlanInts;
+__device__ __forceinline__ PlanInts plan_ints(const int32_t* p) { return (PlanInts)(uintptr_t)p; }
+
 template <bool GATHERED>
 __device__ __forceinline__ VnodeView load_vnode(const Stage1Args& a, int vnode) {
   VnodeView w;
   if constexpr (GATHERED) {
     int req = vnode / a.nsplit, split = vnode - req * a.nsplit;
-    int len = a.cache_seqlens[req] - split * a.kv_split;
+    int len = plan_ints(a.cache_seqlens)[req] - split * a.kv_split;
     w.kv_len = len < 0 ? 0 : (len > a.kv_split ? a.kv_split : len);
     w.kv_base = (int64_t)req * a.max_seqlen + (int64_t)split * a.kv_split;
     w.q_off = vnode;
     w.q_len = 1;
   } else {
-    w.q_off = a.q_offs[vnode];
-    w.q_len = a.q_lens[vnode];
-    w.kv_len = a.kv_lens[vnode];
-    w.kv_base = a.kv_offs[vnode];
+    w.q_off = plan_ints(a.q_offs)[vnode];
+    w.q_len = plan_ints(a.q_lens)[vnode];
+    w.kv_len = plan_ints(a.kv_lens)[vnode];
+    w.kv_base = plan_ints(a.kv_offs)[vnode];
   }
   return w;
 }
@@ -450,7 +471,8 @@ __device__ __forceinline__ void wave_attend(const Stage1Args& a, const VnodeView
   finish_state<D, NQB>(st);
 }
 
-template <int D, int NQB>
+// (PADDED: the kernel's D may be more than the tensors' head dimension)
+template <int D, int NQB, bool PADDED = false>
 __device__ __forceinline__ void write_partials(const Stage1Args& a, const VnodeView& vn, int kvh, int row0,
                                                const WaveState<D, NQB>& st, int ngroups = NQB) {
   constexpr int DB = D / 16;
@@ -461,7 +483,7 @@ __device__ __forceinline__ void write_partials(const Stage1Args& a, const VnodeV
   for (int qb = 0; qb < NQB; ++qb) {
     const int r = row0 + 16 * qb + p;
     if (qb >= ngroups || r >= rows_total) continue;
-    const int ri = r / a.g, rj = r - ri * a.g;
+    const int ri = a.by_g(r), rj = r - ri * a.g;
     const int64_t row = vn.q_off + ri;
     const int head = kvh * a.g + rj;
     const float l = st.l[qb];
@@ -469,7 +491,7 @@ __device__ __forceinline__ void write_partials(const Stage1Args& a, const VnodeV
     float* dst = a.mid_o + row * a.so0 + (int64_t)head * a.so1 + 4 * c;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
-      if (16 * db < a.real_dim) *reinterpret_cast<f32x4*>(dst + 16 * db) = st.o[qb][db] * inv;
+      if (!PADDED || 16 * db < a.real_dim) *reinterpret_cast<f32x4*>(dst + 16 * db) = st.o[qb][db] * inv;
     if (c == 0) a.mid_lse[row * a.sl0 + head] = l > 0.f ? (__builtin_amdgcn_logf(l) + st.m[qb]) * kLn2 : -INFINITY;
   }
 }
@@ -536,7 +558,7 @@ __global__ void __launch_bounds__(kBlock) stage1_kernel(Stage1Args a) {
     for (int row0 = 0; row0 < rows_total; row0 += 16 * NQB) {
       WaveState<D, NQB> st;
       wave_attend<E, D, NQB, GATHERED>(a, vn, kvh, row0, 0, 1, my_lds, st);
-      write_partials<D, NQB>(a, vn, kvh, row0, st);
+      write_partials<D, NQB, true>(a, vn, kvh, row0, st);
     }
   } else {
     const VnodeView vn = load_vnode<GATHERED>(a, a.vnode_begin + blockIdx.x);
@@ -545,7 +567,7 @@ __global__ void __launch_bounds__(kBlock) stage1_kernel(Stage1Args a) {
       WaveState<D, NQB> st;
       wave_attend<E, D, NQB, GATHERED>(a, vn, kvh, row0, wave, kWavesPerBlock, my_lds, st);
       merge_waves<D, NQB>(reinterpret_cast<float*>(smem), st);
-      if (wave == 0) write_partials<D, NQB>(a, vn, kvh, row0, st);
+      if (wave == 0) write_partials<D, NQB, true>(a, vn, kvh, row0, st);
       __syncthreads();  // staging LDS is reused by the next row chunk
     }
   }
@@ -586,8 +608,7 @@ template <int D> __device__ __forceinline__ constexpr int chunk_swizzle(int row)
 }
 
 // LDS layout of the wide kernel: rows of 2*D bytes back to back (no padding), 64-token super
-// tiles of two 32-token tiles, a ring of kBufs buffers, then the rings of slot indices and a
-// program's record.  A row's 16-byte chunks are stored XOR-permuted: chunk c of row r sits in slot
+// tiles of two 32-token tiles, a ring of kBufs buffers, then the rings of slot indices.  A row's 16-byte chunks are stored XOR-permuted: chunk c of row r sits in slot
 // c ^ swz(r) (chunk_swizzle above).  Loads go global -> LDS directly; one wave instruction fills a 1 KB
 // group of consecutive rows.
 template <int D> struct WideGeom {
@@ -605,8 +626,7 @@ template <int D> struct WideGeom {
   static constexpr int kUnits = 2 * kGroups / kWideWaves;                       // loads per wave and super tile
   static constexpr int kSlots = kGroups >= kWideWaves ? kGroups / kWideWaves : 1;  // distinct rows among them
   static constexpr int kIdxBytes = kWideWaves * 4 * 4 * kTokens;                   // per wave: the slot indices of four super tiles
-  static constexpr int kRecord = kRing + kIdxBytes;      // byte offset of the program's record (kProgRecord ints)
-  static constexpr int kLds = kRecord + 1024;
+  static constexpr int kLds = kRing + kIdxBytes;
   static __device__ __forceinline__ int swz(int row) { return chunk_swizzle<D>(row); }
 };
 
@@ -629,47 +649,28 @@ __device__ __forceinline__ void reset_state(WideState<D>& st) {
     for (int j = 0; j < 16; ++j) st.o[db][j] = 0.f;
 }
 
-// Query fragments of a wave's 32 rows, loaded in two steps so that other loads can be put
-// between the two dependent ones: the address of a lane's row (needs the request id of the row,
-// one load), then the fragments.  qf[ks]: row row0 + lane%32, dims 16*ks + 8*(lane/32) .. +7;
-// zero past the vnode (src == nullptr).
-// The record of a block program (kProgRecord ints, one thread of the block each): entries 0..3 are
-// kv_off, kv_len, q_off and q_len of the program's first wide vnode, entry 4 says whether the rest is
-// there (the vnode exists, fits one pass of a block and has at most 128 requests), entries kProgRecRequests.. the
-// requests of its scratch rows, entries kProgRecSlots.. the pool slots of its first 64 tokens (the
-// last token repeated past the end of a shorter run).  With it a block knows after one memory round
-// trip what it otherwise learns in three (its table entry, the vnode's list entries, the request
-// and slot lists) before it can ask for query and K/V rows.
+// The record of a block program (kProgRecord ints): entries 0..3 are kv_off, kv_len, q_off and q_len of the
+// program's first wide vnode, entry 4 says whether the rest is there (the vnode exists, fits one pass of a block
+// and has at most 128 requests), entries kProgRecRequests.. the requests of its scratch rows, entries
+// kProgRecSlots.. the pool slots of its first 64 tokens (the last token repeated past the end of a shorter run).
+// With it a block knows after one memory round trip what it otherwise learns in three (its table entry, the
+// vnode's list entries, the request and slot lists) before it can ask for query and K/V rows.
 constexpr int kProgRecord = 256;
 constexpr int kProgRecRequests = 8;
 constexpr int kProgRecSlots = kProgRecRequests + 128;
-static_assert(kProgRecSlots + 64 <= kProgRecord && kProgRecord == 4 * 64, "one entry per thread of a block");
+static_assert(kProgRecSlots + 64 <= kProgRecord);
 
-// (requests: the record's request entries in LDS, or null: the request of a row is read from the list)
-template <bool GATHERED>
-__device__ __forceinline__ const char* q_row_address32(const Stage1Args& a, const VnodeView& vn, int kvh, int row0,
-                                                       const int* requests = nullptr) {
+// Query fragments of a wave's 32 rows, loaded in two steps so that other loads can be put between the two
+// dependent ones: the address of a lane's row (needs the request id of the row, one load), then the
+// fragments.  qf[ks]: row row0 + lane%32, dims 16*ks + 8*(lane/32) .. +7; zero past the vnode (src == nullptr).
+__device__ __forceinline__ const char* q_row_address32(const Stage1Args& a, const VnodeView& vn, int kvh, int row0) {
   const int lane = threadIdx.x & 63;
   const int r = row0 + (lane & 31), h = lane >> 5;
   if (r >= vn.q_len * a.g) return nullptr;
-  const int ri = r / a.g;
+  const int ri = a.by_g(r);
   const int rj = r - ri * a.g;
-  const int64_t entry = GATHERED ? (int64_t)(vn.q_off / a.nsplit)
-                                 : (int64_t)(requests ? requests[ri] : a.q_entries[vn.q_off + ri]);
+  const int64_t entry = (int64_t)a.q_entries[vn.q_off + ri];
   return a.q + 2 * (entry * a.sq0 + (int64_t)(kvh * a.g + rj) * a.sq1 + 8 * h);
-}
-// The same for 16-row groups: row row0 + lane%16, fragment ks: dims 32*ks + 8*(lane/16) .. +7.
-template <bool GATHERED>
-__device__ __forceinline__ const char* q_row_address16(const Stage1Args& a, const VnodeView& vn, int kvh, int row0,
-                                                       const int* requests = nullptr) {
-  const int lane = lane_here();
-  const int r = row0 + (lane & 15), c = lane >> 4;
-  if (r >= vn.q_len * a.g) return nullptr;
-  const int ri = r / a.g;
-  const int rj = r - ri * a.g;
-  const int64_t entry = GATHERED ? (int64_t)(vn.q_off / a.nsplit)
-                                 : (int64_t)(requests ? requests[ri] : a.q_entries[vn.q_off + ri]);
-  return a.q + 2 * (entry * a.sq0 + (int64_t)(kvh * a.g + rj) * a.sq1 + 8 * c);
 }
 template <int D>
 __device__ __forceinline__ void load_q_frags32(const char* src, u32x4 (&qf)[D / 16]) {
@@ -722,8 +723,10 @@ __device__ __forceinline__ void load_direct16(const char* src, unsigned lds_base
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "{m0}"(lds_base) : "memory");
 }
 // The same for 4 bytes per lane at base + offset (base wave uniform), landing at lds_base + 4 * lane.
+// A vector memory instruction may read a scalar register five wait states after a vector instruction wrote it (a
+// spilled base comes back by v_readlane), and inside assembly the compiler does not see to that.
 __device__ __forceinline__ void load_direct4(const void* base, unsigned offset, unsigned lds_base) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(offset), "s"(base), "{m0}"(lds_base) : "memory");
+  asm volatile("s_nop 4\n\tglobal_load_lds_dword %0, %1" ::"v"(offset), "s"(base), "{m0}"(lds_base) : "memory");
 }
 // Wait until at most N of this wave's vector-memory operations are still in flight (they finish
 // in order).
@@ -1022,7 +1025,6 @@ struct WidePass {
   int row0;            // the wave's first query row
   int groups;          // its 16-row groups (0: it only loads)
   int set, tg, tgroups;  // its row set, its token group, token groups of the pass
-  const int* record;   // the program's record in LDS, or null
 };
 
 // A wave's state in LDS for another wave to merge: its accumulators as 16-byte words, then m and l.
@@ -1074,92 +1076,122 @@ __device__ __forceinline__ void merge_token_groups(float* xchg, WaveState<D, NG>
   }
 }
 
-// One wave's pass over a vnode's KV run for NG row groups (p.groups <= NG of them exist).  The block
-// streams the run through a ring of two 64-token LDS buffers with direct global->LDS loads, one
-// super tile ahead of the one being consumed.  The slot indices travel the same way, two super
-// tiles further ahead, into a ring of the wave's own (it reads the indices of the 16 rows it
-// loads): nothing the compiler tracks is in flight in the loop, no register holds an index longer
-// than one super tile, and runs of any length need no staging step.
-template <typename E, int D, int NG, bool GATHERED>
-__device__ __forceinline__ void wide_pass(const Stage1Args& a, char* smem, const VnodeView& vn, const WidePass& p) {
+// What a wave does to stream a KV run into the block's ring: it requests slot indices (into a ring of its own, so
+// that nothing the compiler tracks is in flight in the loop and no register holds an index longer than one super
+// tile), reads back those of the rows it loads, and requests the rows.  Tokens past the run repeat its last
+// token: the scores of such rows are masked and their V rows are finite.
+template <int D, bool GATHERED> struct RowStream {
   using W = WideGeom<D>;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = lane_here();
-  const int nsuper = (vn.kv_len + W::kTokens - 1) / W::kTokens;
-  const unsigned ring = lds_offset(smem);
-  const unsigned idx_ring = ring + W::kRing + wave * (4 * 4 * W::kTokens);   // four super tiles of indices
-  const int32_t* entries = GATHERED ? nullptr : a.kv_entries + vn.kv_base;
-
-  // loader role of this lane: 16-byte slot `pos` of row `grp_row` in each 1 KB group it fills
-  const int grp_row = lane / W::kChunks, pos = lane % W::kChunks;
-  const char* kbase = a.k + 2 * ((int64_t)p.kvh * a.sk1);
-  const char* vbase = a.v + 2 * ((int64_t)p.kvh * a.sv1);
-  const unsigned k_stride = (unsigned)(2 * a.sk0), v_stride = (unsigned)(2 * a.sv0);  // bytes, < 2^32 (checked by the host)
-  auto group_of = [&](int u) { return W::kGroups >= kWideWaves ? u * kWideWaves + wave : wave % W::kGroups; };
-
-  // indices of super tile j, requested into the wave's ring; those of the rows this wave loads, read back.
-  // Tokens past the run repeat its last token: the scores of such rows are masked and their V rows are finite.
-  auto issue_indices = [&](int j) {
-    if constexpr (!GATHERED) {
-      if (j < nsuper) load_direct4(entries, 4u * (unsigned)min(j * W::kTokens + lane, vn.kv_len - 1), idx_ring + (j & 3) * (4 * W::kTokens));
-    }
-  };
+  const char *kbase, *vbase;
+  unsigned k_stride, v_stride;   // bytes, < 2^32 (checked by the host)
+  const int32_t* entries;
+  int64_t kv_base;
+  int kv_len, nsuper;
+  unsigned ring, idx_ring;       // idx_ring: four super tiles of indices
+  int wave, lane;
   unsigned srow[W::kSlots];
-  auto read_rows = [&](int j) {
+
+  // (loader role of a lane: 16-byte slot `pos` of row `row(u)` in each 1 KB group it fills)
+  __device__ __forceinline__ int group(int u) const { return W::kGroups >= kWideWaves ? u * kWideWaves + wave : wave % W::kGroups; }
+  __device__ __forceinline__ int row(int u) const { return group(u) * W::kGroupRows + lane / W::kChunks; }
+
+  __device__ __forceinline__ RowStream(const Stage1Args& a, char* smem, int kvh) {
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    lane = lane_here();
+    kbase = a.k + 2 * ((int64_t)kvh * a.sk1);
+    vbase = a.v + 2 * ((int64_t)kvh * a.sv1);
+    k_stride = (unsigned)(2 * a.sk0);
+    v_stride = (unsigned)(2 * a.sv0);
+    ring = lds_offset(smem);
+    idx_ring = ring + W::kRing + wave * (4 * 4 * W::kTokens);
+  }
+  __device__ __forceinline__ void open(const Stage1Args& a, const VnodeView& vn) {
+    kv_len = vn.kv_len;
+    kv_base = vn.kv_base;
+    nsuper = (kv_len + W::kTokens - 1) / W::kTokens;
+    entries = GATHERED ? nullptr : a.kv_entries + vn.kv_base;
+  }
+  __device__ __forceinline__ void issue_indices(int j) const {
+    if constexpr (!GATHERED) {
+      if (j < nsuper) load_direct4(entries, 4u * (unsigned)min(j * W::kTokens + lane, kv_len - 1), idx_ring + (j & 3) * (4 * W::kTokens));
+    }
+  }
+  __device__ __forceinline__ void read_rows(int j) {
     if (j >= nsuper) return;
 #pragma unroll
     for (int u = 0; u < W::kSlots; ++u) {
-      const int row = group_of(u) * W::kGroupRows + grp_row;
-      if constexpr (GATHERED) srow[u] = (unsigned)(vn.kv_base + min(j * W::kTokens + row, vn.kv_len - 1));
-      else srow[u] = lds_read4(idx_ring + (j & 3) * (4 * W::kTokens) + 4 * row);
+      if constexpr (GATHERED) srow[u] = (unsigned)(kv_base + min(j * W::kTokens + row(u), kv_len - 1));
+      else srow[u] = lds_read4(idx_ring + (j & 3) * (4 * W::kTokens) + 4 * row(u));
     }
-  };
+  }
   // rows of super tile j -> ring buffer j % 2
-  auto issue_rows = [&](int j) {
+  __device__ __forceinline__ void issue_rows(int j) const {
     if (j >= nsuper) return;
     const unsigned buf = ring + (unsigned)(j & 1) * W::kBytes;
+    const int pos = lane % W::kChunks;
 #pragma unroll
     for (int u = 0; u < W::kUnits; ++u) {
       // unit u of this wave: K groups first, then V groups
       const bool is_v = W::kGroups >= kWideWaves ? u >= W::kSlots : wave >= W::kGroups;
-      const int sl = u % W::kSlots, grp = group_of(sl);
-      const int row = grp * W::kGroupRows + grp_row;
+      const int sl = u % W::kSlots;
       const char* src = (is_v ? vbase : kbase) + (uint64_t)srow[sl] * (is_v ? v_stride : k_stride);
-      load_direct16(src + 16 * (pos ^ W::swz(row)), buf + (is_v ? W::kBytesK : 0) + grp * 1024);
+      load_direct16(src + 16 * (pos ^ W::swz(row(sl))), buf + (is_v ? W::kBytesK : 0) + group(sl) * 1024);
     }
-  };
-
-  // start-up chain: [request ids of the rows, slot indices] -> [Q fragments, first K/V rows]; with the
-  // program's record the first super tile's rows are requested at once
-  if (nsuper > 0) {
-    if (!GATHERED && p.record) {
-#pragma unroll
-      for (int u = 0; u < W::kSlots; ++u) srow[u] = (unsigned)p.record[kProgRecSlots + group_of(u) * W::kGroupRows + grp_row];
-      issue_rows(0);
-    } else {
-      issue_indices(0);
-    }
-    issue_indices(1);
-    issue_indices(2);
   }
+};
+
+// What a wave reads of a program's record, all of it in one memory round trip: the slots of the rows it loads
+// first (straight into RowStream::srow), and the requests of the scratch rows, two per lane.
+struct RecordRequests {
+  int even, odd;
+  __device__ __forceinline__ RecordRequests() : even(0), odd(0) {}
+  __device__ __forceinline__ void load(const int32_t* record) {
+    const int lane = lane_here();
+    even = record[kProgRecRequests + 2 * lane];
+    odd = record[kProgRecRequests + 2 * lane + 1];
+  }
+  // (i differs from lane to lane; every lane of the wave takes part)
+  __device__ __forceinline__ int of(int i) const {
+    const int e = __shfl(even, i >> 1), o = __shfl(odd, i >> 1);
+    return i & 1 ? o : e;
+  }
+};
+
+// One wave's pass over a vnode's KV run for NG row groups (p.groups <= NG of them exist).  The block
+// streams the run through a ring of two 64-token LDS buffers with direct global->LDS loads, one
+// super tile ahead of the one being consumed; the slot indices travel the same way, two super tiles further
+// ahead.  The caller has opened the run and requested the indices of its first super tiles, and its first rows
+// too if `started`; `requests`: those of the vnode's scratch rows, if `listed`.
+template <typename E, int D, int NG, bool GATHERED>
+__device__ __forceinline__ void wide_pass(const Stage1Args& a, char* smem, const VnodeView& vn, const WidePass& p, RowStream<D, GATHERED>& rows,
+                                          bool started, const RecordRequests& requests) {
+  using W = WideGeom<D>;
+  // Rows past the vnode (and those of a wave that only loads) compute its last row again: nothing of theirs
+  // is written, and no lane waits on a branch.
   const char* src[NG];
+  {
+    const int p16 = rows.lane & 15, c = rows.lane >> 4;
 #pragma unroll
-  for (int qb = 0; qb < NG; ++qb)
-    src[qb] = q_row_address16<GATHERED>(a, vn, p.kvh, qb < p.groups ? p.row0 + 16 * qb : vn.q_len * a.g,
-                                        p.record ? p.record + kProgRecRequests : nullptr);
-  if (!p.record && nsuper > 0) {
+    for (int qb = 0; qb < NG; ++qb) {
+      const int r = min(p.row0 + 16 * qb + p16, vn.q_len * a.g - 1), ri = a.by_g(r), rj = r - ri * a.g;
+      int64_t entry;
+      if constexpr (GATHERED) entry = vn.q_off / a.nsplit;
+      else if (started) entry = requests.of(ri);
+      else entry = a.q_entries[vn.q_off + ri];
+      src[qb] = a.q + 2 * (entry * a.sq0 + (int64_t)(p.kvh * a.g + rj) * a.sq1 + 8 * c);
+    }
+  }
+  if (!started && rows.nsuper > 0) {
     wait_direct_loads<0>();
-    read_rows(0);
-    issue_rows(0);
+    rows.read_rows(0);
+    rows.issue_rows(0);
   }
   // (the fragments after the rows: ahead of them they would be a round trip of their own)
   u32x4 qf[NG][D / 32];
 #pragma unroll
   for (int qb = 0; qb < NG; ++qb)
 #pragma unroll
-    for (int ks = 0; ks < D / 32; ++ks) {
-      u32x4 z = {0u, 0u, 0u, 0u};
-      qf[qb][ks] = src[qb] ? *reinterpret_cast<const u32x4*>(src[qb] + 64 * ks) : z;
-    }
+    for (int ks = 0; ks < D / 32; ++ks) qf[qb][ks] = *reinterpret_cast<const u32x4*>(src[qb] + 64 * ks);
   // nothing the compiler itself tracks (the Q fragments) may still be in flight in the loop:
   // a wait for it there would also wait for every direct load
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
@@ -1171,15 +1203,15 @@ __device__ __forceinline__ void wide_pass(const Stage1Args& a, char* smem, const
     for (int ks = 0; ks < D / 32; ++ks) asm volatile("" : "+v"(qf[qb][ks]));
   WaveState<D, NG> st;
   reset_state<D, NG>(st);
-  const WideLane16 la = init_lane16<D>(ring, ring + W::kBytesK);
-  read_rows(1);
+  const WideLane16 la = init_lane16<D>(rows.ring, rows.ring + W::kBytesK);
+  rows.read_rows(1);
 
-  for (int super = 0; super < nsuper; ++super) {
+  for (int super = 0; super < rows.nsuper; ++super) {
     wait_direct_loads<0>();
     __syncthreads();   // publishes super tile `super` to the block; the buffer consumed before it is free
-    issue_rows(super + 1);
-    issue_indices(super + 3);
-    read_rows(super + 2);
+    rows.issue_rows(super + 1);
+    rows.issue_indices(super + 3);
+    rows.read_rows(super + 2);
 #pragma unroll 1
     for (int sub = 0; sub < W::kSub; ++sub) {
       const int tile = super * W::kSub + sub;
@@ -1206,15 +1238,24 @@ __device__ __forceinline__ void wide_pass(const Stage1Args& a, char* smem, const
 // One block (kWideWaves waves) serves the row pieces chunk, chunk + chunks, ... (WideRows<D>::kBlock
 // query rows each) of a vnode for one kv head.  Per pass over the run the waves form row sets x
 // token groups: a wave consumes the 32-token tiles t with t % tgroups == tg for its row set's 16-row
-// groups, and the states of the token groups of a row set are merged at the end.
+// groups, and the states of the token groups of a row set are merged at the end.  `listed`: `rows` holds the slots
+// of the run's first super tile and `requests` the vnode's requests (a program's record).
 template <typename E, int D, bool GATHERED>
-__device__ __forceinline__ void wide_block(const Stage1Args& a, char* smem, const VnodeView& view, int kvh, int chunk,
-                                           int chunks, const int* record) {
-  const VnodeView vn = uniform(view);
+__device__ __forceinline__ void wide_block(const Stage1Args& a, char* smem, const VnodeView& vn, int kvh, int chunk, int chunks,
+                                           RowStream<D, GATHERED>& rows, bool listed, const RecordRequests& requests) {
   constexpr int NQ = WideRows<D>::kGroups, kRows = WideRows<D>::kBlock;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int rows_total = vn.q_len * a.g;
   for (int piece = chunk; piece * kRows < rows_total; piece += chunks) {
+    // (one copy of this for every number of row groups, ahead of what differs between them: the first rows are on
+    // their way before the code that consumes them is fetched)
+    const bool started = listed && piece == 0;      // (the record covers the vnode's first kRows rows)
+    rows.open(a, vn);
+    if (rows.nsuper > 0) {
+      if (started) rows.issue_rows(0);
+      else rows.issue_indices(0);
+      rows.issue_indices(1);
+      rows.issue_indices(2);
+    }
     const int row0 = piece * kRows;
     const int groups = (min(row0 + kRows, rows_total) - row0 + 15) >> 4;
     // as many token groups as leave every wave at most NQ row groups: fewer waves then read the same K/V
@@ -1225,22 +1266,22 @@ __device__ __forceinline__ void wide_block(const Stage1Args& a, char* smem, cons
     // requests of 16/1 heads of 256: 23.0 -> 20.0 us; a step takes the same with two groups or four).
     constexpr int kGroupsWanted = D <= 128 ? NQ * kWideWaves : kWideWaves;
     constexpr int kMostTokenGroups = D <= 128 ? WideGeom<D>::kSub : kWideWaves;
-    int tgroups = 1;
-    while (tgroups < kMostTokenGroups && groups * 2 * tgroups <= kGroupsWanted) tgroups <<= 1;
-    const int sets = kWideWaves / tgroups;
+    int log_tgroups = 0;
+    while ((1 << log_tgroups) < kMostTokenGroups && groups * (2 << log_tgroups) <= kGroupsWanted) ++log_tgroups;
+    static_assert(kWideWaves == 4, "row sets are 4 >> log_tgroups");
+    const int log_sets = 2 - log_tgroups;
     WidePass p;
     p.kvh = kvh;
-    p.set = wave / tgroups;
-    p.tg = wave % tgroups;
-    p.tgroups = tgroups;
-    const int share = groups / sets, extra = groups - share * sets;     // row groups per set: share, one more in the first `extra`
+    p.set = rows.wave >> log_tgroups;
+    p.tgroups = 1 << log_tgroups;
+    p.tg = rows.wave & (p.tgroups - 1);
+    const int share = groups >> log_sets, extra = groups - (share << log_sets);     // row groups per set: share, one more in the first `extra`
     p.groups = share + (p.set < extra ? 1 : 0);
     p.row0 = row0 + 16 * (p.set * share + min(p.set, extra));
-    p.record = !GATHERED && piece == 0 ? record : nullptr;               // (the record covers the vnode's first kRows rows)
-    // (wave uniform; every path has the same block barriers)
-    if (NQ >= 3 && p.groups == 3) wide_pass<E, D, NQ, GATHERED>(a, smem, vn, p);
-    else if (p.groups == 2) wide_pass<E, D, 2, GATHERED>(a, smem, vn, p);
-    else wide_pass<E, D, 1, GATHERED>(a, smem, vn, p);
+    // (wave uniform; every path has the same block barriers.  One request's rows, at most 64, leave a wave two groups.)
+    if (NQ >= 3 && !GATHERED && p.groups == 3) wide_pass<E, D, NQ, GATHERED>(a, smem, vn, p, rows, started, requests);
+    else if (p.groups == 2) wide_pass<E, D, 2, GATHERED>(a, smem, vn, p, rows, started, requests);
+    else wide_pass<E, D, 1, GATHERED>(a, smem, vn, p, rows, started, requests);
   }
 }
 
@@ -1345,19 +1386,18 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
       issue_indices(0, tile0);
     }
     if (!pairs) issue_indices(1, tile0 + tstride);
-    // Fragment ks of a lane: row row0 + 16*qb + p, dims 32*ks + 8*c .. +7; zero past the vnode.
+    // Fragment ks of a lane: row row0 + 16*qb + p, dims 32*ks + 8*c .. +7.  (Rows past the vnode compute its last
+    // row again: nothing of theirs is written, and no lane waits on a branch.)
     const char* src[NG];
-    const bool listed_in_record = inlined && vn.q_len <= kNarrowRecRequests;
+    const bool listed_in_record = inlined && vn.q_len <= kNarrowRecRequests;   // wave uniform
 #pragma unroll
     for (int qb = 0; qb < NG; ++qb) {
-      const int r = row0 + 16 * qb + p, rc = min(r, max(vn.q_len * a.g - 1, 0)), ri = rc / a.g, rj = rc - ri * a.g;
-      const int listed = listed_in_record ? __shfl(rec, 4 + ri) : 0;   // (every lane takes part in the exchange)
-      src[qb] = nullptr;
-      if (r < vn.q_len * a.g) {
-        const int64_t entry = GATHERED ? (int64_t)(vn.q_off / a.nsplit)
-                                       : (listed_in_record ? (int64_t)listed : (int64_t)a.q_entries[vn.q_off + ri]);
-        src[qb] = a.q + 2 * (entry * a.sq0 + (int64_t)(kvh * a.g + rj) * a.sq1 + 8 * c);
-      }
+      const int r = min(row0 + 16 * qb + p, vn.q_len * a.g - 1), ri = a.by_g(r), rj = r - ri * a.g;
+      int64_t entry;
+      if constexpr (GATHERED) entry = vn.q_off / a.nsplit;
+      else if (listed_in_record) entry = __shfl(rec, 4 + ri);
+      else entry = a.q_entries[vn.q_off + ri];
+      src[qb] = a.q + 2 * (entry * a.sq0 + (int64_t)(kvh * a.g + rj) * a.sq1 + 8 * c);
     }
     if (!from_record) {
       wait_direct_loads<0>();
@@ -1370,10 +1410,7 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
 #pragma unroll
     for (int qb = 0; qb < NG; ++qb)
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        u32x4 z = {0u, 0u, 0u, 0u};
-        qf[qb][ks] = src[qb] ? *reinterpret_cast<const u32x4*>(src[qb] + 64 * ks) : z;
-      }
+      for (int ks = 0; ks < KS; ++ks) qf[qb][ks] = *reinterpret_cast<const u32x4*>(src[qb] + 64 * ks);
     // nothing the compiler itself tracks may still be in flight below: a wait for it would
     // also wait for every direct load
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
@@ -1495,10 +1532,10 @@ __device__ __forceinline__ void narrow_item(const Stage1Args& a, char* smem, int
     vn = uniform(load_vnode<GATHERED>(a, vnode));
   }
   int groups = (vn.q_len * a.g + 15) >> 4;
-  if (share > 1) {
+  const int nwaves = blockDim.x >> 6;
+  if (share > 1 && share < nwaves) {
     // every wave of the block makes the same passes (block barriers inside): the most row groups any of
     // its vnodes has, agreed on through one word of each wave's LDS area
-    const int nwaves = blockDim.x >> 6;
     *reinterpret_cast<volatile int*>(smem + p.lds0) = groups;
     __syncthreads();
     for (int i = 0; i < nwaves; ++i) groups = max(groups, *reinterpret_cast<volatile int*>(smem + (size_t)i * N::kLds));
@@ -1523,7 +1560,7 @@ template <typename E, int D, bool GATHERED>
 __global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 2) stage1_narrow_kernel(Stage1Args a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int local_vnode = uniform(blockIdx.x / a.hkv);
+  const int local_vnode = a.by_hkv(blockIdx.x);
   narrow_item<E, D, GATHERED>(a, smem, wave, a.narrow_share, true, a.narrow_begin + local_vnode,
                               blockIdx.x - local_vnode * a.hkv);
 }
@@ -1632,6 +1669,34 @@ __device__ __forceinline__ int wide_vnode_of_rank(const Stage1Args& a, char* sme
   return v;
 }
 
+// The wide vnodes of one block program for one kv head (kv head fastest among the blocks: the eight blocks of a program
+// land on the eight XCDs, and a head's K/V only ever enters one XCD's L2), one after the other.
+template <typename E, int D, bool AGAIN>
+__device__ __forceinline__ void program_block(const Stage1Args& a, char* smem, int program, int kvh) {
+  const PlanInts table = plan_ints(a.prog_table) + 4 * (int64_t)program;
+  const int first = table[0], end = table[1];
+  RowStream<D, false> rows(a, smem, kvh);
+  RecordRequests requests;
+  VnodeView vn{0, 0, 0, 0};
+  bool listed = false;
+  const bool record = a.prog_records != nullptr;   // launch uniform
+  if (record) {
+    // table entry and record in one round trip
+    const int32_t* at = a.prog_records + (int64_t)program * kProgRecord;
+#pragma unroll
+    for (int u = 0; u < WideGeom<D>::kSlots; ++u) rows.srow[u] = (unsigned)at[kProgRecSlots + rows.row(u)];
+    requests.load(at);
+    const PlanInts head = plan_ints(at);
+    vn = VnodeView{head[2], head[3], head[1], (int64_t)head[0]};
+    listed = head[4] != 0;
+  }
+  for (int v = first; v < end; ++v) {
+    if (v > first || !record) vn = load_vnode<false>(a, a.vnode_begin + v);
+    wide_block<E, D, false>(AGAIN ? args_again() : a, smem, vn, kvh, 0, 1, rows, listed, requests);
+    listed = false;
+  }
+}
+
 // The item of a wave of the fused kernel's trailing blocks: `index` counts them behind the `in_programs`
 // items of the programs.  The waves of the last block that have none get `end`: up to three lie past it,
 // which is past 2^31 for a launch of the most items the host allows, hence the sum without sign.
@@ -1641,95 +1706,82 @@ __host__ __device__ constexpr int trailing_item(int index, int in_programs, int 
 static_assert(trailing_item(5, 7, 20) == 12 && trailing_item(12, 7, 20) == 19 && trailing_item(13, 7, 20) == 20);
 static_assert(trailing_item(INT32_MAX - 10, 9, INT32_MAX) == INT32_MAX - 1 && trailing_item(INT32_MAX - 10, 13, INT32_MAX) == INT32_MAX);
 
-// Launch order of the fused kernel.  Wide blocks come rank-major, then row chunk, kv head fastest
-// (blocks that stream the same KV run are launched together and share it in L2); the narrow
-// blocks follow and fill the machine while the wide blocks drain.
-// PROGRAMS: the wide vnodes come as block programs (Stage1Args::prog_table), else as the planner's list.
+// How the fused kernel gets its wide vnodes: as the planner's list; as block programs (Stage1Args::prog_table); as
+// block programs that also serve narrow vnodes (Stage1Args::narrow_in_programs).
+constexpr int kLists = 0, kPrograms = 1, kEmbedding = 2;
+
+// What bounds the start of a block is the fetch of its instructions, which every launch begins with an empty
+// cache for: with one loop over both kinds of work, compiler-made divisions and the program's record handed round
+// through LDS, 232 blocks of a 33 thousand token run asked for their first rows 3.9 us after they had their record, and
+// 1.6 us when the same code ran a second time.  So each kind of work is a straight line from here, each wave reads
+// what it needs of a record straight into registers, and the rows are on their way before the code that consumes
+// them is fetched (whole calls: 6 waves' worth of leaves 10.4 -> 9.7 us, 111 ragged requests 14.5 -> 13.6, the
+// 400-request tree in the planner's lists 66.3 -> 64.0).
+// Launch order of the fused kernel.  Wide blocks come first: programs in index order, kv head fastest, or
+// rank-major, then row chunk, kv head fastest (blocks that stream the same KV run are launched together and share it
+// in L2); the narrow blocks follow and fill the machine while the wide blocks drain.
 // Waves per SIMD that the registers must leave room for: as many blocks per compute unit as its LDS holds of
 // 512-byte rows (one) and 256-byte rows (two).  Below that three fit the 168 registers that the kernel takes by
 // itself, or a few more: for the planner's lists they are kept to (534 requests of 32/8 heads of 64: 102.6 us with
 // 168, 110.4 with 171); under that limit programs come out slower.
-constexpr int fused_waves(int D, bool programs) { return D > 128 ? 1 : D == 128 || programs ? 2 : 3; }
-template <typename E, int D, bool GATHERED, bool PROGRAMS>
-__global__ void __launch_bounds__(kWideBlock, fused_waves(D, PROGRAMS)) stage1_fused_kernel(Stage1Args a) {
+constexpr int fused_waves(int D, int mode) { return D > 128 ? 1 : D == 128 || mode != kLists ? 2 : 3; }
+template <typename E, int D, bool GATHERED, int MODE>
+__global__ void __launch_bounds__(kWideBlock, fused_waves(D, MODE)) stage1_fused_kernel(Stage1Args a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  const int wide_blocks = PROGRAMS ? a.num_programs * a.hkv : a.vnode_count * a.wide_chunks * a.hkv;
+  const int wide_blocks = MODE != kLists ? a.num_programs * a.hkv : a.vnode_count * a.wide_chunks * a.hkv;
   const int narrow_index = (int)blockIdx.x - wide_blocks;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // this block's wide vnodes [wide_first, wide_end) and, per wave, its narrow vnodes: item, item + step, .. below
-  // item_end, numbered vnode-major with hkv items each
-  int wide_first = 0, wide_end = 0, kvh = 0, chunk = 0, chunks = 1;
-  int share = 1, item = 0, item_end = 0, step = kWideWaves;
-  bool narrow_first = false;
-  int* record = nullptr;
-  VnodeView vn{0, 0, 0, 0};
-  if (narrow_index < 0 && PROGRAMS) {
-    // A block program written by the host, for one kv head (kv head fastest: the eight blocks of
-    // a program land on the eight XCDs, and a head's K/V only ever enters one XCD's L2): its wide
-    // vnodes one after the other, and its narrow vnodes, one wave each, before or after them.
-    // Of the two blocks that share a compute unit one starts with its narrow vnodes and the
-    // other ends with them, so that the memory-bound narrow vnodes of one run under the
-    // arithmetic-bound wide vnodes of the other.
-    const int program = uniform((int)blockIdx.x / a.hkv);
-    kvh = (int)blockIdx.x - program * a.hkv;
-    wide_first = a.prog_table[4 * program];
-    wide_end = a.prog_table[4 * program + 1];
-    const int first = a.prog_table[4 * program + 2], count = a.prog_table[4 * program + 3];
-    narrow_first = count < 0;
-    item = first + wave;
-    item_end = first + (count < 0 ? -count : count);
-    // the program's record, requested together with its table entry
-    if (!GATHERED && a.prog_records != nullptr) {   // launch uniform
-      record = reinterpret_cast<int*>(smem + WideGeom<D>::kRecord);
-      record[threadIdx.x] = a.prog_records[(int64_t)program * kProgRecord + threadIdx.x];
-      __syncthreads();
-      if (narrow_first || __builtin_amdgcn_readfirstlane(record[4]) == 0) record = nullptr;   // block uniform
-    }
-  } else if (narrow_index < 0) {
-    const int per_rank = a.wide_chunks * a.hkv;
-    const int rank = uniform((int)blockIdx.x / per_rank);
-    const int rest = (int)blockIdx.x - rank * per_rank;
-    // Launch slot `rest / hkv` of a rank serves chunk (slot + rank / 2) % chunks.  Consecutive
-    // blocks of one kv head go round robin to the four shader engines of an XCD, strictly in
-    // order (a block waits for its engine even when others have room); without the rotation an
-    // engine would only ever get first chunks, which run longer than last ones.
-    const int slot = uniform(rest / a.hkv);
-    kvh = rest - slot * a.hkv;
-    chunks = a.wide_chunks;
-    chunk = uniform((slot + (rank >> 1)) % chunks);
-    (void)wide_vnode_of_rank<GATHERED>(a, smem, rank, vn);
-    wide_end = 1;
-  } else {
-    share = a.narrow_share;
-    item_end = a.narrow_count * a.hkv;
-    item = trailing_item(uniform(narrow_index * (kWideWaves / share) + wave / share), a.narrow_in_programs * a.hkv, item_end);
-    step = item_end - item;   // one item
-  }
   // (128-byte rows in programs: fewer lanes are spilled, and the reads cost more than they save: 36.9 -> 37.7 us
   // for 608 requests of 24/8 heads of 64.  512-byte rows: most trees gain 1 to 3 %, but 32 requests of 64/8 heads of
   // 256 on 15 thousand tokens lose, 121.1 -> 123.3 us.)
-  constexpr bool kAgain = D == 128 || (D < 128 && !PROGRAMS);
-  // (one call each, in either order, so that the kernel holds one copy of the code)
-#pragma unroll 1
-  for (int turn = 0; turn < 2; ++turn) {
-    if ((turn == 0) != narrow_first) {
-      for (int v = wide_first; v < wide_end; ++v) {
-        if (PROGRAMS) {
-          if (record) vn = VnodeView{record[2], record[3], record[1], (int64_t)record[0]};
-          else vn = load_vnode<GATHERED>(a, a.vnode_begin + v);
-        }
-        wide_block<E, D, GATHERED>(kAgain ? args_again() : a, smem, vn, kvh, chunk, chunks, record);
-        record = nullptr;
-      }
+  constexpr bool kAgain = D == 128 || (D < 128 && MODE == kLists);
+  if (narrow_index < 0) {
+    if constexpr (MODE == kLists) {
+      const int per_rank = a.wide_chunks * a.hkv;
+      const int rank = uniform((int)blockIdx.x / per_rank);
+      const int rest = (int)blockIdx.x - rank * per_rank;
+      // Launch slot `rest / hkv` of a rank serves chunk (slot + rank / 2) % chunks.  Consecutive
+      // blocks of one kv head go round robin to the four shader engines of an XCD, strictly in
+      // order (a block waits for its engine even when others have room); without the rotation an
+      // engine would only ever get first chunks, which run longer than last ones.
+      const int slot = a.by_hkv(rest), kvh = rest - slot * a.hkv;
+      const int chunks = a.wide_chunks, chunk = uniform((slot + (rank >> 1)) % chunks);
+      VnodeView vn{0, 0, 0, 0};
+      (void)wide_vnode_of_rank<GATHERED>(a, smem, rank, vn);
+      vn = uniform(vn);
+      const Stage1Args& b = kAgain ? args_again() : a;
+      RowStream<D, GATHERED> rows(b, smem, kvh);
+      wide_block<E, D, GATHERED>(b, smem, vn, kvh, chunk, chunks, rows, false, RecordRequests());
+    } else if constexpr (MODE == kPrograms) {
+      const int program = a.by_hkv(blockIdx.x);
+      program_block<E, D, kAgain>(a, smem, program, (int)blockIdx.x - program * a.hkv);
     } else {
-      // (trailing blocks: one turn for every wave, with or without an item; a wave that shares no vnode and
-      // has none is done)
-      for (bool first = true; item < item_end || (first && share > 1); item += step, first = false) {
-        const bool trailing = narrow_index >= 0;
-        const int vnode = trailing ? uniform(item / a.hkv) : item;
-        narrow_item<E, D, GATHERED>(kAgain ? args_again() : a, smem, wave, share, item < item_end, a.narrow_begin + vnode, trailing ? item - vnode * a.hkv : kvh);
+      // A program's narrow vnodes, one wave each, before its wide ones (a negative count) or after them: of the
+      // two blocks that share a compute unit one starts with its narrow vnodes and the other ends with them, so that
+      // the memory-bound narrow vnodes of one run under the arithmetic-bound wide vnodes of the other.
+      const int program = a.by_hkv(blockIdx.x), kvh = (int)blockIdx.x - program * a.hkv;
+      const PlanInts table = plan_ints(a.prog_table) + 4 * (int64_t)program;
+      const int first = table[2], count = table[3];
+      // (one call each, in either order, so that the kernel holds one copy of the code)
+#pragma unroll 1
+      for (int turn = 0; turn < 2; ++turn) {
+        if ((turn == 0) == (count < 0)) {
+          for (int v = first + wave; v < first + abs(count); v += kWideWaves)
+            narrow_item<E, D, GATHERED>(kAgain ? args_again() : a, smem, wave, 1, true, a.narrow_begin + v, kvh);
+          __syncthreads();  // the waves' tiles become the ring of the next wide vnode
+        } else {
+          program_block<E, D, kAgain>(a, smem, program, kvh);
+        }
       }
-      if (PROGRAMS && narrow_first) __syncthreads();  // the waves' tiles become the ring of the next wide vnode
+    }
+  } else {
+    // trailing blocks: an item per wave, or per `share` waves; a wave that shares no vnode and has none is done
+    const int share = a.narrow_share, log_share = share >> 1;   // 1, 2, 4 -> 0, 1, 2
+    const int end = a.narrow_count * a.hkv;
+    const int item = trailing_item((narrow_index * kWideWaves + wave) >> log_share, MODE == kEmbedding ? a.narrow_in_programs * a.hkv : 0, end);
+    if (item < end || share > 1) {
+      const int vnode = a.by_hkv(item);
+      narrow_item<E, D, GATHERED>(kAgain ? args_again() : a, smem, wave, share, item < end, a.narrow_begin + vnode, item - vnode * a.hkv);
     }
   }
 }
@@ -1790,7 +1842,7 @@ __global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 2) deft_stage1_kerne
   for (int row0 = 0; row0 < rows_total; row0 += kDeftRows) {
     const int my_row0 = row0 + 32 * wave;
     const bool active = my_row0 < rows_total;
-    const char* q_src = q_row_address32<false>(a, vn, kvh, active ? my_row0 : rows_total);
+    const char* q_src = q_row_address32(a, vn, kvh, active ? my_row0 : rows_total);
     u32x4 qf[D / 16];
     load_q_frags32<D>(q_src, qf);
     WideState<D> st;
@@ -2097,12 +2149,12 @@ inline int narrow_share_for(int64_t items, int head_dim) {
   return share;
 }
 
-template <typename E, int D, bool GATHERED, bool PROGRAMS>
+template <typename E, int D, bool GATHERED, int MODE>
 int launch_stage1_fused(const Stage1Args& a0, hipStream_t stream) {
   constexpr size_t kWideLds = (size_t)WideGeom<D>::kLds;
   constexpr size_t kNarrowLds = (size_t)kWideWaves * NarrowGeom<D>::kLds;
   constexpr size_t lds = kWideLds > kNarrowLds ? kWideLds : kNarrowLds;
-  auto kern = stage1_fused_kernel<E, D, GATHERED, PROGRAMS>;
+  auto kern = stage1_fused_kernel<E, D, GATHERED, MODE>;
   // (raising the dynamic LDS limit is idempotent: two threads that both find the flag clear both raise it)
   static std::atomic<bool> configured_on[kMaxDevices];
   std::atomic<bool>& configured = configured_on[current_device()];
@@ -2126,7 +2178,7 @@ int launch_stage1_fused(const Stage1Args& a0, hipStream_t stream) {
   a.join_rows = WideRows<D>::kBlock;
   if (a.wide_chunks == 1 && (int64_t)a.vnode_count * a.hkv * a.wide_rows < (int64_t)a.join_rows * (wave_slots() / kWaveSlotsPerCu))
     a.join_rows = std::min(a.join_rows, 128);
-  const int64_t wide_blocks = PROGRAMS ? (int64_t)a.num_programs * a.hkv : (int64_t)a.vnode_count * a.wide_chunks * a.hkv;
+  const int64_t wide_blocks = MODE != kLists ? (int64_t)a.num_programs * a.hkv : (int64_t)a.vnode_count * a.wide_chunks * a.hkv;
   const int64_t blocks = wide_blocks + narrow_blocks;
   if (blocks == 0) return FT_OK;
   if (blocks > INT32_MAX) return FT_ERR_ARGUMENT;
@@ -2176,9 +2228,10 @@ int launch_stage1_d(const Stage1Args& a, hipStream_t stream) {
   } else {
     if (a.vnode_count == 0 && !a.prog_table) return launch_stage1_narrow<E, D, GATHERED>(a, stream);
     if constexpr (!GATHERED) {
-      if (a.prog_table) return launch_stage1_fused<E, D, false, true>(a, stream);
+      if (a.prog_table && a.narrow_in_programs > 0) return launch_stage1_fused<E, D, false, kEmbedding>(a, stream);
+      if (a.prog_table) return launch_stage1_fused<E, D, false, kPrograms>(a, stream);
     }
-    return launch_stage1_fused<E, D, GATHERED, false>(a, stream);
+    return launch_stage1_fused<E, D, GATHERED, kLists>(a, stream);
   }
 }
 
@@ -2356,6 +2409,8 @@ static int stage1_setup(Stage1Args& a, const void* q, const void* k, const void*
   a.q_entries = vnode_to_q_entries; a.q_offs = vnode_to_q_offs; a.q_lens = vnode_to_q_lens;
   a.g = kv_group_num;
   a.hkv = num_kv_heads;
+  a.by_g = divisor(a.g);
+  a.by_hkv = divisor(a.hkv);
   a.real_dim = head_dim;
   a.scale_log2 = sm_scale * kLog2e;
   a.mid_o = mid_o; a.so0 = so0; a.so1 = so1; a.mid_lse = mid_lse; a.sl0 = sl0;
@@ -2675,6 +2730,8 @@ int ft_gathered_decode(const void* q, const void* k_cache, const void* v_cache,
   else { a.vnode_begin = 0; a.vnode_count = batch_size * nsplit; a.wide_rows = g; }
   a.g = g;
   a.hkv = num_kv_heads;
+  a.by_g = divisor(a.g);
+  a.by_hkv = divisor(a.hkv);
   a.real_dim = head_dim;
   a.scale_log2 = sm_scale * kLog2e;
   a.mid_o = mid_o; a.so0 = (int64_t)num_qo_heads * head_dim; a.so1 = head_dim;

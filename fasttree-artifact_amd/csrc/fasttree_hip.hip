@@ -112,10 +112,9 @@ __device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(
 __device__ __forceinline__ int lane_here() {
   int lane = threadIdx.x & 63;
   asm volatile("" : "+v"(lane));
+  __builtin_assume(lane >= 0 && lane < 64);
   return lane;
 }
-// The four low bits of x reversed (each on its own, so that constant parts fold).
-__device__ __forceinline__ constexpr int reversed4(int x) { return ((x & 1) << 3) | ((x & 2) << 1) | ((x >> 1) & 2) | ((x >> 3) & 1); }
 // Orders this wave's LDS traffic around a point where lanes read what other lanes of the
 // same wave wrote.  LDS executes one wave's instructions in order, so no wait is needed;
 // the fences only stop the compiler from moving accesses across.
@@ -596,15 +595,15 @@ template <int D> struct WideRows {
 };
 constexpr int kDeftRows = 32 * kWideWaves;        // (the comparison engine's kernel: 32 rows per wave)
 
-// The XOR that places the 16-byte chunks of a row in LDS.  Operands are read 16 rows at a time (K, one
-// chunk) and 4 rows x 2 chunks at a time (V, transposed), and either has to hit all 64 banks.  Rows of 256
-// bytes and more start at the same bank: their four low bits, the two pairs swapped, give every row its own
-// chunk.  Shorter rows fill the banks between them: what the row number leaves to the chunk are its
-// higher bits, so the bits are reversed before they are cut off (64-dim heads: 2-way conflicts in both
-// reads with the pairs swapped, none so; 380 requests of 64/8 heads 22.5 -> 21.8 us, a 94-request tree of 16/1
-// heads 23.1 -> 21.5).
+// The XOR that places the 16-byte chunks of a row in LDS.  A K operand is read by 16 rows x 4 chunks in 16-byte
+// words, of which rows 0-3 and 12-15 of one chunk go together with rows 4-11 of the next; a V operand, transposed, by
+// 16 rows x 2 chunks in 8-byte words, 8 rows at a time: either has to hit all 64 banks.  Rows of 256 bytes and more
+// start at the same bank, and their two low bits move a row by 4 chunks; shorter ones fill the banks between them.
+// The next two bits, negated, set the quarters apart in both.  (The 400-request tree at head_dim 128: no conflicts
+// counted in 4.5 million cycles of LDS access; with the two pairs of bits swapped, which suits the 32-row operands of
+// 32x32x16 instructions, 4.0 million of 8.5: 62.4 -> 61.5 us.  Either serves those too.)
 template <int D> __device__ __forceinline__ constexpr int chunk_swizzle(int row) {
-  return (D < 128 ? reversed4(row) : ((row & 3) << 2) | ((row >> 2) & 3)) & (D / 8 - 1);
+  return (D >= 128 ? (row & 3) << 2 : D == 64 ? (row & 2) << 1 : 0) | (-(row >> 2) & 3);
 }
 
 // LDS layout of the wide kernel: rows of 2*D bytes back to back (no padding), 64-token super

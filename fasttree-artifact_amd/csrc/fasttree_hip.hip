@@ -962,7 +962,7 @@ template <typename E, int D, int NQ>
 __device__ __forceinline__ void tile_softmax(f32x4 (&s)[2][NQ], int valid, float sc, WaveState<D, NQ>& st, u32x4 (&pf)[NQ]) {
   if (valid < kTileTokens) {  // wave uniform
     asm volatile("" ::: "memory");  // keeps this a branch: as selects it would run on every tile
-    const int c = (threadIdx.x & 63) >> 4;
+    const int c = lane_here() >> 4;
 #pragma unroll
     for (int tb = 0; tb < 2; ++tb)
 #pragma unroll
@@ -1033,7 +1033,7 @@ template <int D, int NG> struct SharedState {
   static constexpr int DB = D / 16;
   static constexpr int kFloats = NG * (4 * DB + 2);
   static __device__ __forceinline__ void put(float* at, const WaveState<D, NG>& st) {
-    const int lane = threadIdx.x & 63;
+    const int lane = lane_here();
     f32x4* o = reinterpret_cast<f32x4*>(at) + lane;
     float* ml = at + NG * DB * 4 * kWave + lane;
 #pragma unroll
@@ -1045,7 +1045,7 @@ template <int D, int NG> struct SharedState {
     }
   }
   static __device__ __forceinline__ void merge(const float* at, WaveState<D, NG>& st) {
-    const int lane = threadIdx.x & 63;
+    const int lane = lane_here();
     const f32x4* o = reinterpret_cast<const f32x4*>(at) + lane;
     const float* ml = at + NG * DB * 4 * kWave + lane;
 #pragma unroll
@@ -1167,24 +1167,37 @@ __device__ __forceinline__ void wide_pass(const Stage1Args& a, char* smem, const
   using W = WideGeom<D>;
   // Rows past the vnode (and those of a wave that only loads) compute its last row again: nothing of theirs
   // is written, and no lane waits on a branch.
-  const char* src[NG];
-  {
-    const int p16 = rows.lane & 15, c = rows.lane >> 4;
+  int req[NG], head[NG];
 #pragma unroll
-    for (int qb = 0; qb < NG; ++qb) {
-      const int r = min(p.row0 + 16 * qb + p16, vn.q_len * a.g - 1), ri = a.by_g(r), rj = r - ri * a.g;
-      int64_t entry;
-      if constexpr (GATHERED) entry = vn.q_off / a.nsplit;
-      else if (started) entry = requests.of(ri);
-      else entry = a.q_entries[vn.q_off + ri];
-      src[qb] = a.q + 2 * (entry * a.sq0 + (int64_t)(p.kvh * a.g + rj) * a.sq1 + 8 * c);
+  for (int qb = 0; qb < NG; ++qb) {
+    const int r = min(p.row0 + 16 * qb + (rows.lane & 15), vn.q_len * a.g - 1);
+    req[qb] = a.by_g(r);
+    head[qb] = p.kvh * a.g + r - req[qb] * a.g;
+  }
+  if (started) {
+#pragma unroll
+    for (int qb = 0; qb < NG; ++qb) req[qb] = requests.of(req[qb]);
+  } else {
+    if constexpr (GATHERED) {
+#pragma unroll
+      for (int qb = 0; qb < NG; ++qb) req[qb] = vn.q_off / a.nsplit;
+    } else {
+#pragma unroll
+      for (int qb = 0; qb < NG; ++qb) req[qb] = a.q_entries[vn.q_off + req[qb]];
+      // (awaited here: a wait for them where the two branches meet would be a wait for all direct loads in both)
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+#pragma unroll
+      for (int qb = 0; qb < NG; ++qb) asm volatile("" : "+v"(req[qb]));
+    }
+    if (rows.nsuper > 0) {
+      wait_direct_loads<0>();
+      rows.read_rows(0);
+      rows.issue_rows(0);
     }
   }
-  if (!started && rows.nsuper > 0) {
-    wait_direct_loads<0>();
-    rows.read_rows(0);
-    rows.issue_rows(0);
-  }
+  const char* src[NG];
+#pragma unroll
+  for (int qb = 0; qb < NG; ++qb) src[qb] = a.q + 2 * ((int64_t)req[qb] * a.sq0 + (int64_t)head[qb] * a.sq1 + 8 * (rows.lane >> 4));
   // (the fragments after the rows: ahead of them they would be a round trip of their own)
   u32x4 qf[NG][D / 32];
 #pragma unroll
@@ -1293,6 +1306,11 @@ __device__ __forceinline__ void wide_block(const Stage1Args& a, char* smem, cons
 // and no barrier holds one wave's loads back for another's arithmetic.  A leaf vnode of a few dozen
 // tokens costs little more than its two memory round trips (record, rows).  Slot indices travel the
 // same way, two tiles ahead.
+//
+// What bounds a leaf is that chain of round trips, so nothing the compiler tracks may be awaited between the first
+// rows' requests and the query fragments': the request ids and the record were, and a vnode's queries were asked for
+// when its rows had landed (1423 leaves of 135 tokens and 64-dim heads: 112.4 us so, 99.9 now; 380 of 86 tokens
+// 22.9 and 21.3; 6 waves' worth of leaves 9.7 and 9.2).
 // ---------------------------------------------------------------------------------------
 template <int D> struct NarrowGeom {
   static constexpr int kRowBytes = 2 * D;
@@ -1314,95 +1332,118 @@ constexpr int kNarrowRecord = 64;
 constexpr int kNarrowRecRequests = 16;
 constexpr int kNarrowRecSlots = 4 + kNarrowRecRequests;
 
-// One wave's share of a narrow vnode for the NG 16-row groups from row0: the tiles tile0,
-// tile0 + tstride, ... of the run, staged in the wave's own LDS area at lds0.  `rec` is the lane's
-// int of the vnode's record when `inlined` (else unused).
-template <typename E, int D, int NG, bool GATHERED>
-__device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeView& vn, char* smem, unsigned lds0,
-                                              int kvh, int row0, int tile0, int tstride, WaveState<D, NG>& st,
-                                              int rec, bool inlined) {
+// What a wave does to stream its tiles of a narrow vnode's run into its own LDS area.  It asks for slot indices (into a
+// ring in LDS), reads back those of the rows it loads, and asks for the rows.  A wave that walks every tile asks for
+// two tiles' indices at a time, one that shares its run for one tile's.  Tokens past the run repeat its last token
+// (their scores are masked, their V rows are finite).
+template <int D, bool GATHERED> struct NarrowStream {
   using N = NarrowGeom<D>;
-  constexpr int KS = D / 32;
-  const int lane = lane_here();
-  const int p = lane & 15, c = lane >> 4;
-  const int ntiles = (vn.kv_len + kTileTokens - 1) / kTileTokens;
-  const unsigned tile_addr = lds_offset(smem) + lds0;  // the wave's K tile; its V tile follows, then the index ring
-  const unsigned idx_ring = tile_addr + N::kBytes;
-  const int32_t* entries = GATHERED ? nullptr : a.kv_entries + vn.kv_base;
-
-  const char* kbase = a.k + 2 * ((int64_t)kvh * a.sk1);
-  const char* vbase = a.v + 2 * ((int64_t)kvh * a.sv1);
-  const unsigned k_stride = (unsigned)(2 * a.sk0), v_stride = (unsigned)(2 * a.sv0);  // bytes, < 2^32 (checked by the host)
-
-  // The slot indices of 64 tokens from the wave's i-th tile on -> the index ring.  A wave that walks every
-  // tile asks for two tiles' indices at a time (even i), one that shares its run for one tile's.
-  const bool pairs = tstride == 1;   // wave uniform
-  auto issue_indices = [&](int i, int tile) {
-    if constexpr (!GATHERED)
-      load_direct4(entries, 4u * (unsigned)min(tile * kTileTokens + lane, vn.kv_len - 1),
-                   idx_ring + ((pairs ? i >> 1 : i) & 3) * N::kIdxSlot);
-  };
-  // The cache rows this lane loads of the wave's i-th tile.  Tokens past the run repeat its last token
-  // (their scores are masked, their V rows are finite).
+  const char *kbase, *vbase;
+  unsigned k_stride, v_stride;   // bytes, < 2^32 (checked by the host)
+  unsigned tile_addr, idx_ring;  // the wave's K tile (its V tile follows), its index ring
+  const int32_t* entries;
+  int64_t kv_base;
+  int kv_len, ntiles, tile0, stride;   // the wave serves the tiles tile0, tile0 + stride, ...
+  int lane;
   unsigned srow[N::kLoads];
-  auto read_rows = [&](int i, int tile) {
-    const int grp_row = lane / N::kChunks;
-    const unsigned at = idx_ring + (pairs ? (i & 7) * (N::kIdxSlot / 2) : (i & 3) * N::kIdxSlot);
+
+  __device__ __forceinline__ NarrowStream(const Stage1Args& a, char* smem, unsigned lds0, int kvh, int w, int share) {
+    kbase = a.k + 2 * ((int64_t)kvh * a.sk1);
+    vbase = a.v + 2 * ((int64_t)kvh * a.sv1);
+    k_stride = (unsigned)(2 * a.sk0);
+    v_stride = (unsigned)(2 * a.sv0);
+    tile_addr = lds_offset(smem) + lds0;
+    tile0 = w;
+    stride = share;
+  }
+  // (lane and tile_addr made opaque: the addresses made from them stay in the pass, or the compiler computes some
+  // 100 of them ahead of the loop over passes, which nearly always makes one)
+  __device__ __forceinline__ void open(const Stage1Args& a, const VnodeView& vn) {
+    lane = lane_here();
+    asm volatile("" : "+s"(tile_addr));
+    idx_ring = tile_addr + N::kBytes;
+    kv_len = vn.kv_len;
+    kv_base = vn.kv_base;
+    ntiles = (kv_len + kTileTokens - 1) / kTileTokens;
+    entries = GATHERED ? nullptr : a.kv_entries + vn.kv_base;
+  }
+  __device__ __forceinline__ bool pairs() const { return stride == 1; }   // wave uniform
+  // (loader role of a lane: 16-byte slot `pos` of row `row(g)` in each 1 KB group)
+  __device__ __forceinline__ int row(int g) const { return g * N::kGroupRows + lane / N::kChunks; }
+  // the slot indices of 64 tokens from the wave's i-th tile on
+  __device__ __forceinline__ void issue_indices(int i, int tile) const {
+    if constexpr (!GATHERED)
+      load_direct4(entries, 4u * (unsigned)min(tile * kTileTokens + lane, kv_len - 1), idx_ring + ((pairs() ? i >> 1 : i) & 3) * N::kIdxSlot);
+  }
+  // the cache rows this lane loads of the wave's i-th tile
+  __device__ __forceinline__ void read_rows(int i, int tile) {
+    const unsigned at = idx_ring + (pairs() ? (i & 7) * (N::kIdxSlot / 2) : (i & 3) * N::kIdxSlot);
 #pragma unroll
     for (int g = 0; g < N::kLoads; ++g) {
-      const int row = g * N::kGroupRows + grp_row;
-      if constexpr (GATHERED) srow[g] = (unsigned)(vn.kv_base + min(tile * kTileTokens + row, vn.kv_len - 1));
-      else srow[g] = lds_read4(at + 4 * row);
+      if constexpr (GATHERED) srow[g] = (unsigned)(kv_base + min(tile * kTileTokens + row(g), kv_len - 1));
+      else srow[g] = lds_read4(at + 4 * row(g));
     }
-  };
+  }
+  // the same of the run's first tile, from the vnode's record (a lane's int of it)
+  __device__ __forceinline__ void rows_of_record(int rec) {
+#pragma unroll
+    for (int g = 0; g < N::kLoads; ++g) srow[g] = (unsigned)__shfl(rec, kNarrowRecSlots + row(g));
+  }
   // those rows of K (or V) -> the wave's K (V) tile
-  auto issue = [&](bool is_v) {
-    // loader role: 16-byte slot `pos` of row `grp_row` in each 1 KB group
-    const int grp_row = lane / N::kChunks, pos = lane % N::kChunks;
+  __device__ __forceinline__ void issue(bool is_v) const {
+    const int pos = lane % N::kChunks;
 #pragma unroll
     for (int g = 0; g < N::kLoads; ++g) {
-      const int row = g * N::kGroupRows + grp_row;
-      const char* src = (is_v ? vbase : kbase) + (uint64_t)srow[g] * (is_v ? v_stride : k_stride) + 16 * (pos ^ N::swz(row));
+      const char* src = (is_v ? vbase : kbase) + (uint64_t)srow[g] * (is_v ? v_stride : k_stride) + 16 * (pos ^ N::swz(row(g)));
       load_direct16(src, tile_addr + (is_v ? N::kBytesK : 0) + g * 1024);
     }
-  };
+  }
+};
 
-  reset_state<D, NG>(st);
+// One wave's share of a narrow vnode for the NG 16-row groups from row0.  The caller has opened the run and asked for
+// the wave's first indices, and for its first rows too if `started`.  `rec` is the lane's int of the vnode's record when
+// `inlined` (else unused).
+template <typename E, int D, int NG, bool GATHERED>
+__device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeView& vn, NarrowStream<D, GATHERED>& rows, bool started,
+                                              int kvh, int row0, WaveState<D, NG>& st, int rec, bool inlined) {
+  using N = NarrowGeom<D>;
+  constexpr int KS = D / 32;
+  const int p = rows.lane & 15, c = rows.lane >> 4;
+  const int ntiles = rows.ntiles, tile0 = rows.tile0, tstride = rows.stride;
+  const bool pairs = rows.pairs();
+
   if (tile0 < ntiles) {
-    // start-up chain: [requests of the rows, slot indices] -> [Q fragments, first K/V rows].  With the
-    // vnode's record at hand and the run's first tile to serve, the first 32 slot indices are already
-    // here: the rows are requested at once.
-    const bool from_record = !GATHERED && inlined && tile0 == 0;
-    if (from_record) {
-      if (lane >= kNarrowRecSlots && lane < kNarrowRecSlots + kTileTokens)
-        *reinterpret_cast<int*>(smem + lds0 + N::kBytes + 4 * (lane - kNarrowRecSlots)) = rec;
-      wave_lds_fence();
-      read_rows(0, 0);
-      issue(false);
-      issue(true);
-      if (pairs) issue_indices(0, 0);   // (the second tile's indices, and the first one's over themselves)
-    } else {
-      issue_indices(0, tile0);
-    }
-    if (!pairs) issue_indices(1, tile0 + tstride);
     // Fragment ks of a lane: row row0 + 16*qb + p, dims 32*ks + 8*c .. +7.  (Rows past the vnode compute its last
     // row again: nothing of theirs is written, and no lane waits on a branch.)
-    const char* src[NG];
-    const bool listed_in_record = inlined && vn.q_len <= kNarrowRecRequests;   // wave uniform
+    int req[NG], head[NG];
 #pragma unroll
     for (int qb = 0; qb < NG; ++qb) {
-      const int r = min(row0 + 16 * qb + p, vn.q_len * a.g - 1), ri = a.by_g(r), rj = r - ri * a.g;
-      int64_t entry;
-      if constexpr (GATHERED) entry = vn.q_off / a.nsplit;
-      else if (listed_in_record) entry = __shfl(rec, 4 + ri);
-      else entry = a.q_entries[vn.q_off + ri];
-      src[qb] = a.q + 2 * (entry * a.sq0 + (int64_t)(kvh * a.g + rj) * a.sq1 + 8 * c);
+      const int r = min(row0 + 16 * qb + p, vn.q_len * a.g - 1);
+      req[qb] = a.by_g(r);
+      head[qb] = kvh * a.g + r - req[qb] * a.g;
     }
-    if (!from_record) {
+    if constexpr (GATHERED) {
+#pragma unroll
+      for (int qb = 0; qb < NG; ++qb) req[qb] = vn.q_off / a.nsplit;
+    } else if (inlined && vn.q_len <= kNarrowRecRequests) {   // wave uniform: they are in the record
+#pragma unroll
+      for (int qb = 0; qb < NG; ++qb) req[qb] = __shfl(rec, 4 + req[qb]);
+    } else {
+#pragma unroll
+      for (int qb = 0; qb < NG; ++qb) req[qb] = a.q_entries[vn.q_off + req[qb]];
+      // (awaited here: a wait for them where the two branches meet would be a wait for all direct loads in both)
+      __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+#pragma unroll
+      for (int qb = 0; qb < NG; ++qb) asm volatile("" : "+v"(req[qb]));
+    }
+    const char* src[NG];
+#pragma unroll
+    for (int qb = 0; qb < NG; ++qb) src[qb] = a.q + 2 * ((int64_t)req[qb] * a.sq0 + (int64_t)head[qb] * a.sq1 + 8 * c);
+    if (!started) {
       wait_direct_loads<0>();
-      read_rows(0, tile0);
-      issue(false);
-      issue(true);
+      rows.read_rows(0, tile0);
+      rows.issue(false);
+      rows.issue(true);
     }
     // (the fragments after the rows: ahead of them they would be a round trip of their own)
     u32x4 qf[NG][KS];
@@ -1410,6 +1451,8 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
     for (int qb = 0; qb < NG; ++qb)
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) qf[qb][ks] = *reinterpret_cast<const u32x4*>(src[qb] + 64 * ks);
+    reset_state<D, NG>(st);
+    const WideLane16 la = init_lane16<D>(rows.tile_addr, rows.tile_addr + N::kBytesK);
     // nothing the compiler itself tracks may still be in flight below: a wait for it would
     // also wait for every direct load
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
@@ -1419,7 +1462,6 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
     for (int qb = 0; qb < NG; ++qb)
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) asm volatile("" : "+v"(qf[qb][ks]));
-    const WideLane16 la = init_lane16<D>(tile_addr, tile_addr + N::kBytesK);
     // The next rows are asked for as soon as a tile's operands are in registers, ahead of the arithmetic on
     // them; at 512-byte rows there are no registers for that, and they follow it.
     constexpr bool kEarly = D <= 128;
@@ -1431,19 +1473,19 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
       VOperands<D> v;
       const bool indices = !GATHERED && more && (!pairs || (i & 1) == 0);   // wave uniform
       wait_direct_loads<N::kLoads>();  // K (and the next tile's indices) landed; V may still be in flight
-      if (kEarly && more) read_rows(i + 1, next);
+      if (kEarly && more) rows.read_rows(i + 1, next);
       auto next_k = [&] {
         if (!more) return;
-        if constexpr (!kEarly) read_rows(i + 1, next);
+        if constexpr (!kEarly) rows.read_rows(i + 1, next);
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the K tile has been read
-        issue(false);
-        if (indices) issue_indices(i + 2, next + tstride);
+        rows.issue(false);
+        if (indices) rows.issue_indices(i + 2, next + tstride);
       };
       auto next_v = [&] {
         if (!more) return;
-        if constexpr (!kEarly) read_rows(i + 1, next);
+        if constexpr (!kEarly) rows.read_rows(i + 1, next);
         __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the V tile has been read
-        issue(true);
+        rows.issue(true);
       };
       if constexpr (kEarly) {
         tile_scores<E, D, NG>(la.k, qf, sc, next_k);
@@ -1464,6 +1506,8 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
         next_v();
       }
     }
+  } else {
+    reset_state<D, NG>(st);
   }
   finish_state<D, NG>(st);
 }
@@ -1488,15 +1532,14 @@ __device__ __forceinline__ void merge_shares(float* xchg, WaveState<D, NG>& st, 
 // its rows, and then the wave only keeps the block's barriers company).
 struct NarrowPass {
   int kvh, row0, w, share, rec;
-  bool inlined;
-  unsigned lds0;      // byte offset of the wave's area in the block's LDS segment
-  unsigned xchg;      // and of the areas of the waves that share the vnode
+  bool inlined, started;
+  unsigned xchg;      // byte offset of the areas of the waves that share the vnode in the block's LDS segment
 };
 template <typename E, int D, int NG, bool GATHERED>
-__device__ __forceinline__ void narrow_pass(const Stage1Args& a, char* smem, const VnodeView& vn, const NarrowPass& p) {
+__device__ __forceinline__ void narrow_pass(const Stage1Args& a, char* smem, const VnodeView& vn, NarrowStream<D, GATHERED>& stream, const NarrowPass& p) {
   WaveState<D, NG> st;
   const bool rows = p.row0 < vn.q_len * a.g;
-  if (rows) narrow_attend<E, D, NG, GATHERED>(a, vn, smem, p.lds0, p.kvh, p.row0, p.w, p.share, st, p.rec, p.inlined);
+  if (rows) narrow_attend<E, D, NG, GATHERED>(a, vn, stream, p.started, p.kvh, p.row0, st, p.rec, p.inlined);
   else reset_state<D, NG>(st);
   if (p.share > 1) merge_shares<D, NG>(reinterpret_cast<float*>(smem + p.xchg), st, p.w, p.share);
   if (rows && p.w == 0) write_partials<D, NG>(a, vn, p.kvh, p.row0, st);
@@ -1506,23 +1549,26 @@ __device__ __forceinline__ void narrow_pass(const Stage1Args& a, char* smem, con
 // for the whole launch; the host picks more than one when there are fewer vnodes than wave
 // slots): wave w of the vnode takes the tiles w, w + share, ..., and the shares are merged
 // through LDS.  `slot` is the wave's index in the block; a wave without a vnode (exists ==
-// false) only keeps the block's barriers company.  More rows than a pass holds take several passes, as
-// even as possible.
-template <typename E, int D, bool GATHERED>
+// false) only keeps the block's barriers company.  More rows than a pass holds take several passes.
+// ALONE: the block serves no other vnode.
+template <typename E, int D, bool GATHERED, bool ALONE>
 __device__ __forceinline__ void narrow_item(const Stage1Args& a, char* smem, int slot, int share, bool exists,
                                             int vnode, int kvh) {
   using N = NarrowGeom<D>;
+  static_assert(N::kGroups == 2, "passes of two row groups, then of one");
   VnodeView vn{0, 0, 0, 0};
   NarrowPass p;
   p.kvh = kvh;
   p.share = share;
   p.w = slot & (share - 1);
-  p.lds0 = (unsigned)slot * N::kLds;
   p.xchg = (unsigned)(slot - p.w) * N::kLds;
   p.rec = 0;
   p.inlined = !GATHERED && a.narrow_table != nullptr;   // launch uniform
+  if (p.inlined && exists) p.rec = a.narrow_table[(int64_t)(vnode - a.narrow_begin) * kNarrowRecord + lane_here()];
+  // (what does not depend on the record, while it is on its way)
+  NarrowStream<D, GATHERED> rows(a, smem, (unsigned)slot * N::kLds, kvh, p.w, share);
+  asm volatile("" : "+s"(rows.kbase), "+s"(rows.vbase), "+s"(rows.k_stride), "+s"(rows.v_stride));
   if (p.inlined) {
-    if (exists) p.rec = a.narrow_table[(int64_t)(vnode - a.narrow_begin) * kNarrowRecord + lane_here()];
     vn.kv_base = __builtin_amdgcn_readlane(p.rec, 0);
     vn.kv_len = __builtin_amdgcn_readlane(p.rec, 1);
     vn.q_off = __builtin_amdgcn_readlane(p.rec, 2);
@@ -1530,24 +1576,36 @@ __device__ __forceinline__ void narrow_item(const Stage1Args& a, char* smem, int
   } else if (exists) {
     vn = uniform(load_vnode<GATHERED>(a, vnode));
   }
+  // (complete for the compiler on every path: a wait for it behind the first direct loads would be a wait for those)
+  asm volatile("" : "+v"(p.rec));
   int groups = (vn.q_len * a.g + 15) >> 4;
-  const int nwaves = blockDim.x >> 6;
-  if (share > 1 && share < nwaves) {
+  if (!ALONE && share > 1 && share < kWideWaves) {
     // every wave of the block makes the same passes (block barriers inside): the most row groups any of
     // its vnodes has, agreed on through one word of each wave's LDS area
-    *reinterpret_cast<volatile int*>(smem + p.lds0) = groups;
+    const unsigned word = lds_offset(smem);
+    *reinterpret_cast<__attribute__((address_space(3))) int*>((uintptr_t)(word + (unsigned)slot * N::kLds)) = groups;
     __syncthreads();
-    for (int i = 0; i < nwaves; ++i) groups = max(groups, *reinterpret_cast<volatile int*>(smem + (size_t)i * N::kLds));
+    for (int i = 0; i < kWideWaves; ++i) groups = max(groups, (int)lds_read4(word + (unsigned)i * N::kLds));
     groups = __builtin_amdgcn_readfirstlane(groups);
     __syncthreads();
   }
-  const int passes = (groups + N::kGroups - 1) / N::kGroups;
-  for (int pass = 0, done = 0; pass < passes; ++pass) {
-    const int ng = (groups - done + passes - pass - 1) / (passes - pass);
+  for (int done = 0; done < groups; done += N::kGroups) {
     p.row0 = 16 * done;
-    done += ng;
-    if (ng == 2) narrow_pass<E, D, 2, GATHERED>(a, smem, vn, p);
-    else narrow_pass<E, D, 1, GATHERED>(a, smem, vn, p);
+    // With the vnode's record at hand and the run's first tile to serve, the first 32 slot indices are already
+    // here: the rows are requested at once, ahead of the code that differs between the numbers of row groups.
+    rows.open(a, vn);
+    p.started = !GATHERED && p.inlined && rows.tile0 == 0;
+    if (p.row0 < vn.q_len * a.g && rows.tile0 < rows.ntiles) {
+      if (p.started) {
+        rows.rows_of_record(p.rec);
+        rows.issue(false);
+        rows.issue(true);
+      }
+      if (!p.started || rows.pairs()) rows.issue_indices(0, rows.tile0);   // (the second tile's indices too)
+      if (!rows.pairs()) rows.issue_indices(1, rows.tile0 + rows.stride);
+    }
+    if (groups - done >= 2) narrow_pass<E, D, 2, GATHERED>(a, smem, vn, rows, p);
+    else narrow_pass<E, D, 1, GATHERED>(a, smem, vn, rows, p);
     if (share > 1) __syncthreads();  // the exchange area is the staging area of the next pass
   }
 }
@@ -1560,7 +1618,7 @@ __global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 2) stage1_narrow_ker
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int local_vnode = a.by_hkv(blockIdx.x);
-  narrow_item<E, D, GATHERED>(a, smem, wave, a.narrow_share, true, a.narrow_begin + local_vnode,
+  narrow_item<E, D, GATHERED, true>(a, smem, wave, a.narrow_share, true, a.narrow_begin + local_vnode,
                               blockIdx.x - local_vnode * a.hkv);
 }
 
@@ -1685,6 +1743,10 @@ __device__ __forceinline__ void program_block(const Stage1Args& a, char* smem, i
 #pragma unroll
     for (int u = 0; u < WideGeom<D>::kSlots; ++u) rows.srow[u] = (unsigned)at[kProgRecSlots + rows.row(u)];
     requests.load(at);
+    // (awaited together: a wait for the last of them behind the first direct loads would be a wait for those too)
+    asm volatile("" : "+v"(requests.even), "+v"(requests.odd));
+#pragma unroll
+    for (int u = 0; u < WideGeom<D>::kSlots; ++u) asm volatile("" : "+v"(rows.srow[u]));
     const PlanInts head = plan_ints(at);
     vn = VnodeView{head[2], head[3], head[1], (int64_t)head[0]};
     listed = head[4] != 0;
@@ -1766,7 +1828,7 @@ __global__ void __launch_bounds__(kWideBlock, fused_waves(D, MODE)) stage1_fused
       for (int turn = 0; turn < 2; ++turn) {
         if ((turn == 0) == (count < 0)) {
           for (int v = first + wave; v < first + abs(count); v += kWideWaves)
-            narrow_item<E, D, GATHERED>(kAgain ? args_again() : a, smem, wave, 1, true, a.narrow_begin + v, kvh);
+            narrow_item<E, D, GATHERED, false>(kAgain ? args_again() : a, smem, wave, 1, true, a.narrow_begin + v, kvh);
           __syncthreads();  // the waves' tiles become the ring of the next wide vnode
         } else {
           program_block<E, D, kAgain>(a, smem, program, kvh);
@@ -1780,7 +1842,7 @@ __global__ void __launch_bounds__(kWideBlock, fused_waves(D, MODE)) stage1_fused
     const int item = trailing_item((narrow_index * kWideWaves + wave) >> log_share, MODE == kEmbedding ? a.narrow_in_programs * a.hkv : 0, end);
     if (item < end || share > 1) {
       const int vnode = a.by_hkv(item);
-      narrow_item<E, D, GATHERED>(kAgain ? args_again() : a, smem, wave, share, item < end, a.narrow_begin + vnode, item - vnode * a.hkv);
+      narrow_item<E, D, GATHERED, false>(kAgain ? args_again() : a, smem, wave, share, item < end, a.narrow_begin + vnode, item - vnode * a.hkv);
     }
   }
 }

@@ -1740,16 +1740,18 @@ __device__ __forceinline__ void program_block(const Stage1Args& a, char* smem, i
   if (record) {
     // table entry and record in one round trip
     const int32_t* at = a.prog_records + (int64_t)program * kProgRecord;
+    const PlanInts head = plan_ints(at);
+    vn = VnodeView{head[2], head[3], head[1], (int64_t)head[0]};
+    listed = head[4] != 0;
 #pragma unroll
     for (int u = 0; u < WideGeom<D>::kSlots; ++u) rows.srow[u] = (unsigned)at[kProgRecSlots + rows.row(u)];
     requests.load(at);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" : "+s"(vn.q_off), "+s"(vn.q_len), "+s"(vn.kv_len), "+s"(vn.kv_base));
     // (awaited together: a wait for the last of them behind the first direct loads would be a wait for those too)
     asm volatile("" : "+v"(requests.even), "+v"(requests.odd));
 #pragma unroll
     for (int u = 0; u < WideGeom<D>::kSlots; ++u) asm volatile("" : "+v"(rows.srow[u]));
-    const PlanInts head = plan_ints(at);
-    vn = VnodeView{head[2], head[3], head[1], (int64_t)head[0]};
-    listed = head[4] != 0;
   }
   for (int v = first; v < end; ++v) {
     if (v > first || !record) vn = load_vnode<false>(a, a.vnode_begin + v);
@@ -1792,10 +1794,9 @@ __global__ void __launch_bounds__(kWideBlock, fused_waves(D, MODE)) stage1_fused
   const int wide_blocks = MODE != kLists ? a.num_programs * a.hkv : a.vnode_count * a.wide_chunks * a.hkv;
   const int narrow_index = (int)blockIdx.x - wide_blocks;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // (128-byte rows in programs: fewer lanes are spilled, and the reads cost more than they save: 36.9 -> 37.7 us
-  // for 608 requests of 24/8 heads of 64.  512-byte rows: most trees gain 1 to 3 %, but 32 requests of 64/8 heads of
-  // 256 on 15 thousand tokens lose, 121.1 -> 123.3 us.)
-  constexpr bool kAgain = D == 128 || (D < 128 && MODE == kLists);
+  // (512-byte rows: most trees gain 1 to 3 % by it, but 32 requests of 64/8 heads of 256 on 15 thousand tokens lose,
+  // 121.1 -> 123.3 us.)
+  constexpr bool kAgain = D <= 128;
   if (narrow_index < 0) {
     if constexpr (MODE == kLists) {
       const int per_rank = a.wide_chunks * a.hkv;

@@ -1987,7 +1987,7 @@ struct Stage2Args {
   int64_t oo0, oo1;
   int batch, hq;
   int longest; // no request has more partials than this (the number of vnodes, or more)
-  int splits;  // lane groups that share one (request, head): a power of two, set by the launcher
+  int log_splits;  // 1 << this many waves share a request's list, set by the launcher
   int nsplit;  // > 0: gathered mode, request r owns rows [r*nsplit, (r+1)*nsplit)
   // (or null) one record of kReqRecord int32 per request, written by the host: req_lens[r],
   // req_offs[r], then the request's first kReqRecord - 2 entries -- what the block needs before
@@ -1997,127 +1997,123 @@ struct Stage2Args {
 constexpr int kReqRecord = 16;
 constexpr int kReqRecEntries = kReqRecord - 2;
 
-template <int WIDTH> __device__ __forceinline__ float group_max(float x) {
-#pragma unroll
-  for (int d = WIDTH / 2; d >= 1; d >>= 1) x = fmaxf(x, __shfl_xor(x, d, WIDTH));
-  return x;
-}
-template <int WIDTH> __device__ __forceinline__ float group_sum(float x) {
-#pragma unroll
-  for (int d = WIDTH / 2; d >= 1; d >>= 1) x += __shfl_xor(x, d, WIDTH);
-  return x;
-}
-
-// A group of D/4 lanes serves one (request, head), or every splits-th partial of one: lane i fetches the
-// row index and the log-sum-exp of the group's partial i, the group reduces max and weight sum with
-// shuffles, then every lane accumulates its own 4 output dims over the partials, taking weight and
-// row index of partial i from lane i.  The `splits` groups of a (request, head) sit in one block and
-// are merged through LDS.
+// D/4 lanes serve one (request, head), a wave several heads of one request; `splits` waves of a block (1, 2 or 4) take
+// parts of the request's list and are merged through LDS.  A wave reads the list of its request as scalars (from the
+// request's record with its length and offset, else from the list), so a lane asks for its four output dims of eight
+// partial rows, and for their log-sum-exps, with nothing but its own address and a scalar.
 //
-// Bound by the partial rows it reads, and for a batch of few requests by how many of them are in
-// flight: 8 requests x 64 heads with 68 partials each take 64 blocks 11.2 us, one split per group of
-// lanes; with the partials split eight ways 512 blocks.
+// Bound by the partial rows it reads, and for a batch of few requests by how many of them are in flight (8 requests x
+// 64 heads with 68 partials each: 64 blocks of whole lists 11.2 us) and by the fetch of its instructions, 2.7 KB where a
+// list spread over lanes and handed round by shuffles took 4.0 (whole calls: 4 requests of a short prompt 9.1 -> 8.4 us,
+// 111 ragged requests of 64-dim heads 13.6 -> 12.7, 16/1 heads of 256 18.2 -> 17.4, the 400-request tree 61.9 -> 61.0).
 template <typename E, int D, bool SPLIT>
 __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
   constexpr int LPH = D / 4;
-  constexpr int HPB = kBlock / LPH;
-  const int grp = threadIdx.x / LPH, gl = threadIdx.x % LPH;
+  constexpr int HPW = kWave / LPH;                          // heads of a wave
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int gl = lane % LPH;
   const int req = blockIdx.x;
-  int S = SPLIT ? a.splits : 1;                             // (a power of two; launch uniform)
-  int split = SPLIT ? grp & (S - 1) : 0;
-  const int head = SPLIT ? blockIdx.y * (HPB / S) + grp / S : blockIdx.y * HPB + grp;
+  const int log_splits = SPLIT ? a.log_splits : 0;          // launch uniform
+  const int head = ((((int)blockIdx.y * kWavesPerBlock) + wave) >> log_splits) * HPW + lane / LPH;
   const bool exists = head < a.hq;
-  if (!SPLIT && !exists) return;
-  const int32_t* rec = a.req_table ? a.req_table + (int64_t)req * kReqRecord : nullptr;  // launch uniform
-  int off, n, rec_row = -1;
+  const int head_in = exists ? head : a.hq - 1;             // (lanes past the last head read that one's rows and store nothing)
+  // this wave's part [first, first + n) of the request's list, from `list` on
+  int n, first = 0, row0 = 0;
+  PlanInts list = nullptr;
+  constexpr int kBatch = 8;
+  int row[kBatch];
   if (a.nsplit > 0) {
-    off = req * a.nsplit;
     n = a.nsplit;
-  } else if (rec) {
+    row0 = req * a.nsplit;
+  } else if (a.req_table) {                                 // launch uniform
+    const PlanInts rec = plan_ints(a.req_table) + (int64_t)req * kReqRecord;
     n = rec[0];
-    off = rec[1];
-    rec_row = rec[2 + min(gl, kReqRecEntries - 1)];  // (requested together with the two words above)
+    const int off = rec[1];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) row[j] = rec[2 + j];
+    list = n <= kReqRecEntries ? rec + 2 : plan_ints(a.req_entries) + off;
   } else {
-    off = a.req_offs[req];
-    n = a.req_lens[req];
+    n = plan_ints(a.req_lens)[req];
+    list = plan_ints(a.req_entries) + plan_ints(a.req_offs)[req];
   }
-  if (SPLIT && n <= kReqRecEntries) {   // block uniform: a short list is one group's work (merging costs about 1 us)
-    if (split > 0 || !exists) return;
-    S = 1;
-    split = 0;
+  int split = 0, splits = 1;
+  if constexpr (SPLIT) {
+    // (a short list is one wave's work: merging costs about 1 us)
+    split = wave & ((1 << log_splits) - 1);
+    if (n <= kReqRecEntries) {
+      if (split > 0) return;
+    } else {
+      splits = 1 << log_splits;
+      const int part = (n + splits - 1) >> log_splits;
+      first = split * part;
+      n = max(0, min(n - first, part));
+    }
   }
-  const int first = split + S * gl;                         // this lane's first entry of the request's list
-  const int mine = !SPLIT ? n : exists ? (n - split + S - 1) / S : 0;    // partials of this group (0 or less: none)
+  const bool in_record = a.nsplit == 0 && a.req_table != nullptr && first == 0;   // the first batch's rows are in `row`
 
+  const char* o_lane = reinterpret_cast<const char*>(a.mid_o + (int64_t)head_in * a.so1 + 4 * gl);
+  const char* lse_lane = reinterpret_cast<const char*>(a.mid_lse + head_in);
   float m_run = -INFINITY, l_run = 0.f;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int base = 0; base < mine; base += LPH) {
-    const int cnt = min(LPH, mine - base);
-    int my_row = -1;
-    if (gl < cnt) {
-      const int entry = first + S * base;
-      if (a.nsplit > 0) my_row = off + entry;
-      else if (rec && entry < kReqRecEntries) my_row = S == 1 && base == 0 ? rec_row : rec[2 + entry];
-      else my_row = a.req_entries[off + entry];
-    }
-    // Rows in batches of kBatch, all loads of a batch issued before the first is used (the rows
-    // are in bounds whatever their weight; a zero weight discards the row's contents).  The
-    // first batch is requested together with the log-sum-exp values, not after them: both
-    // depend on the row indices only.
-    constexpr int kBatch = 8;
-    f32x4 part[kBatch];
-    auto request = [&](int i0) {
+  for (int i0 = 0; i0 < n; i0 += kBatch) {
+    // rows of this batch; past the end the first one again (a zero weight discards what is read of it)
+    if (a.nsplit > 0) {
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        const int ri = __shfl(my_row, min(i0 + j, cnt - 1), LPH);
-        part[j] = *reinterpret_cast<const f32x4*>(a.mid_o + (int64_t)ri * a.so0 + (int64_t)head * a.so1 + 4 * gl);
-      }
-    };
-    float my_lse = -INFINITY;
-    if (gl < cnt) my_lse = a.mid_lse[(int64_t)my_row * a.sl0 + head];
-    request(0);
-    const float m_new = fmaxf(m_run, group_max<LPH>(my_lse));
-    const float w = (my_lse == -INFINITY) ? 0.f : __expf(my_lse - m_new);
+      for (int j = 0; j < kBatch; ++j) row[j] = row0 + first + i0 + j;
+    } else if (i0 > 0 || !in_record) {
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) row[j] = list[first + min(i0 + j, n - 1)];
+    }
+    float lse[kBatch];
+    f32x4 part[kBatch];
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      const int64_t r = i0 + j < n ? row[j] : row[0];
+      lse[j] = *reinterpret_cast<const float*>(lse_lane + 4 * r * a.sl0);
+      part[j] = *reinterpret_cast<const f32x4*>(o_lane + 4 * r * a.so0);
+    }
+    float m_new = m_run;
+#pragma unroll
+    for (int j = 0; j < kBatch; ++j) {
+      lse[j] = i0 + j < n ? lse[j] : -INFINITY;
+      m_new = fmaxf(m_new, lse[j]);
+    }
     const float keep = (m_run == -INFINITY) ? 0.f : __expf(m_run - m_new);
-    l_run = l_run * keep + group_sum<LPH>(w);
+    l_run *= keep;
     acc *= keep;
     m_run = m_new;
-    for (int i0 = 0; i0 < cnt; i0 += kBatch) {
-      if (i0 > 0) request(i0);
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        const float wi = (i0 + j < cnt) ? __shfl(w, min(i0 + j, cnt - 1), LPH) : 0.f;
+    for (int j = 0; j < kBatch; ++j) {
+      const float w = (lse[j] == -INFINITY) ? 0.f : __expf(lse[j] - m_new);
+      l_run += w;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] += (wi != 0.f) ? part[j][e] * wi : 0.f;
-      }
+      for (int e = 0; e < 4; ++e) acc[e] += (w != 0.f) ? part[j][e] * w : 0.f;
     }
   }
-  if (SPLIT && S > 1) {
-    // the groups' states to the first of them
+  if (SPLIT && splits > 1) {
+    // the waves' states to the first of them
     __shared__ f32x4 acc_of[kBlock];
-    __shared__ float m_of[HPB], l_of[HPB];
+    __shared__ float m_of[kBlock], l_of[kBlock];
     acc_of[threadIdx.x] = acc;
-    if (gl == 0) {
-      m_of[grp] = m_run;
-      l_of[grp] = l_run;
-    }
+    m_of[threadIdx.x] = m_run;
+    l_of[threadIdx.x] = l_run;
     __syncthreads();
-    if (split > 0 || !exists) return;
+    if (split > 0) return;
     float m_all = m_run;
-    for (int i = 1; i < S; ++i) m_all = fmaxf(m_all, m_of[grp + i]);
+    for (int i = 1; i < splits; ++i) m_all = fmaxf(m_all, m_of[threadIdx.x + i * kWave]);
     acc = f32x4{0.f, 0.f, 0.f, 0.f};
     l_run = 0.f;
-    for (int i = 0; i < S; ++i) {
-      const float m_i = m_of[grp + i];
+    for (int i = 0; i < splits; ++i) {
+      const float m_i = m_of[threadIdx.x + i * kWave];
       const float w = (m_i == -INFINITY) ? 0.f : __expf(m_i - m_all);
-      l_run += l_of[grp + i] * w;
-      acc += acc_of[threadIdx.x + i * LPH] * w;
+      l_run += l_of[threadIdx.x + i * kWave] * w;
+      acc += acc_of[threadIdx.x + i * kWave] * w;
     }
   }
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
   acc *= inv;
   u32x2 out = {E::pack2(acc[0], acc[1]), E::pack2(acc[2], acc[3])};
-  *reinterpret_cast<u32x2*>(a.o + 2 * ((int64_t)req * a.oo0 + (int64_t)head * a.oo1 + 4 * gl)) = out;
+  if (exists) *reinterpret_cast<u32x2*>(a.o + 2 * ((int64_t)req * a.oo0 + (int64_t)head * a.oo1 + 4 * gl)) = out;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2314,19 +2310,18 @@ int launch_stage1(const Stage1Args& a, int d, int dtype, hipStream_t stream) {
   return FT_ERR_DTYPE;
 }
 
-// Lane groups per (request, head): as many as leave the launch at most two blocks per compute unit
-// (wave_slots() / 4): more blocks than that hide each other's round trips anyway.  One group, and the
-// kernel without the merge, where every list is short or the batch fills the machine by itself (684
-// requests of 32 heads: 8.2 us without the merge's code, 9.6 with it).
+// Waves per list: as many as leave the launch at most two blocks per compute unit (wave_slots() / 4): more blocks than
+// that hide each other's round trips anyway.  One wave, and the kernel without the merge, where every list is short or
+// the batch fills the machine by itself (684 requests of 32 heads: 8.2 us without the merge's code, 9.6 with it).
 template <typename E, int D>
 int launch_stage2_inst(const Stage2Args& a0, hipStream_t stream) {
-  constexpr int HPB = kBlock / (D / 4);
+  constexpr int kHeads = kWavesPerBlock * kWave / (D / 4);   // of a block whose waves share no list
   Stage2Args a = a0;
-  a.splits = 1;
-  while (a.longest > kReqRecEntries && a.splits < HPB && (int64_t)a.batch * ((a.hq * a.splits * 2 + HPB - 1) / HPB) <= wave_slots() / 4) a.splits *= 2;
-  const int heads = HPB / a.splits;
-  const dim3 grid((unsigned)a.batch, (unsigned)((a.hq + heads - 1) / heads), 1);
-  if (a.splits > 1) hipLaunchKernelGGL((stage2_kernel<E, D, true>), grid, dim3(kBlock, 1, 1), 0, stream, a);
+  a.log_splits = 0;
+  auto blocks_per_request = [&](int log_splits) { return ((int64_t)(a.hq << log_splits) + kHeads - 1) / kHeads; };
+  while (a.longest > kReqRecEntries && (1 << a.log_splits) < kWavesPerBlock && a.batch * blocks_per_request(a.log_splits + 1) <= wave_slots() / 4) ++a.log_splits;
+  const dim3 grid((unsigned)a.batch, (unsigned)blocks_per_request(a.log_splits), 1);
+  if (a.log_splits > 0) hipLaunchKernelGGL((stage2_kernel<E, D, true>), grid, dim3(kBlock, 1, 1), 0, stream, a);
   else hipLaunchKernelGGL((stage2_kernel<E, D, false>), grid, dim3(kBlock, 1, 1), 0, stream, a);
   return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
 }

@@ -1,0 +1,44 @@
+"""The merge launch on its own: list lengths around its batches of eight rows and around the fourteen a record
+holds, with few requests (a list's parts merged over the waves of a block) and with many."""
+
+import pytest
+import torch
+
+from fasttree_hip.decode import fasttree_decode_stage2
+
+LENGTHS = [0, 1, 7, 8, 9, 14, 15, 16, 17, 33, 70]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("head_dim,heads", [(16, 6), (32, 5), (64, 24), (128, 9), (256, 3)])
+@pytest.mark.parametrize("copies", [1, 40])
+def test_merge_of_lists_of_every_length(head_dim, heads, copies, dtype, device):
+    print(f"\n[gpu case] merge {head_dim} x {heads}, {copies} copies, {dtype}", flush=True)
+    gen = torch.Generator().manual_seed(head_dim + copies)
+    lens = torch.tensor(LENGTHS * copies, dtype=torch.int32)
+    rows = int(lens.sum())
+    entries = torch.randperm(rows, generator=gen).to(torch.int32)
+    offs = (torch.cumsum(lens, 0) - lens).to(torch.int32)
+    mid_o = torch.randn(rows, heads, head_dim, generator=gen)
+    mid_lse = 6 * torch.randn(rows, heads, generator=gen)
+    # rows that attended nothing: output 0, log-sum-exp -inf; for one request all of them
+    mid_lse[torch.rand(rows, heads, generator=gen) < 0.1] = float("-inf")
+    nothing = len(LENGTHS) - 2
+    mid_lse[entries[offs[nothing]: offs[nothing] + lens[nothing]].long()] = float("-inf")
+    mid_o[mid_lse == float("-inf")] = 0
+    o = torch.full((len(lens), heads, head_dim), float("nan"), dtype=dtype, device=device)
+    fasttree_decode_stage2(entries.to(device), offs.to(device), lens.to(device), mid_o.to(device), mid_lse.to(device), o)
+    o = o.cpu().double()
+    # rounding to a significand of 11 (fp16) or 8 (bf16) bits is off by at most 2^-11 or 2^-8 of the value; the weights
+    # are good to 1e-5; fp16's smallest step is 2^-24
+    rounding = 2.0 ** (-11 if dtype is torch.float16 else -8)
+    for r, (off, n) in enumerate(zip(offs.tolist(), lens.tolist())):
+        at = entries[off: off + n].long()
+        lse, x = mid_lse[at].double(), mid_o[at].double()
+        top = lse.max(0).values if n else torch.full((heads,), float("-inf"), dtype=torch.float64)
+        w = torch.where(lse == float("-inf"), 0.0, torch.exp(lse - top))
+        total = w.sum(0)
+        want = torch.where(total > 0, 1 / total, 0.0)[:, None] * (w[:, :, None] * x).sum(0)
+        bound = rounding * want.abs() + 1e-5 * (x.abs().amax() if n else 0.0) + 2.0 ** -25
+        assert bool(((o[r] - want).abs() <= bound).all()), (r, n, float(((o[r] - want).abs() - bound).max()))

@@ -177,7 +177,7 @@ struct Stage1Args {
                                    // which the per-wave staging kernels compute as a zero-padded 32-dim contraction
   int g;
   int hkv;
-  Divisor by_g, by_hkv;
+  Divisor by_g, by_hkv, by_chunks;
   float scale_log2;  // sm_scale * log2(e)
   float* mid_o;
   int64_t so0, so1;
@@ -1635,38 +1635,46 @@ __global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 2) stage1_narrow_ker
 // most `cap` query rows (what the blocks of one vnode serve in a single pass): a tile of 16
 // requests x 4 heads fills only half of a block's rows, and two such tiles would stage the same
 // run twice.  The first vnode of a group carries the group; the others become empty items.
+//
+// Every block does this before its first load, with cold code: 3.4 us of a block's start with 64-bit divisions, five
+// barriers and the vnodes' entries through LDS; the 400-request tree 60.6 -> 59.9 us with the form below.
 constexpr int kMaxRanked = kWideBlock;
+// a / b for whole 0 <= a < 2048 and 1 <= b < 2^24: (a + 1/2) / b is at least 1 / 2b from a whole number, which the error
+// of the reciprocal, less than 2^-20 of the quotient, does not reach.
+__device__ __forceinline__ int small_quotient(int a, int b) { return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b)); }
 template <bool GATHERED>
-__device__ __forceinline__ int wide_vnode_of_rank(const Stage1Args& a, char* smem, int target, VnodeView& view) {
+__device__ __forceinline__ void wide_vnode_of_rank(const Stage1Args& a, char* smem, int target, VnodeView& view) {
   const int n = a.vnode_count;
   if (n < 2 || n > kMaxRanked) {
     view = load_vnode<GATHERED>(a, a.vnode_begin + target);
-    return target;
+    return;
   }
   // keys[u]: work of vnode u in 23 bits (a float's exponent and leading mantissa bits), then
   // 256 - u: larger key = earlier, no two equal; 0 for a vnode that is not the head of a group
   unsigned* keys = reinterpret_cast<unsigned*>(smem);
-  VnodeView* views = reinterpret_cast<VnodeView*>(keys + kMaxRanked);
-  int* group_q_len = reinterpret_cast<int*>(views + kMaxRanked);
-  unsigned long long* joined = reinterpret_cast<unsigned long long*>(group_q_len + kMaxRanked);  // one bit per vnode
-  int* found = reinterpret_cast<int*>(joined + kMaxRanked / 64);
+  int* q_len_of = reinterpret_cast<int*>(keys + kMaxRanked);
+  int* q_end_of = q_len_of + kMaxRanked;                               // scratch rows end, per vnode
+  unsigned long long* joined = reinterpret_cast<unsigned long long*>(q_end_of + kMaxRanked);  // one bit per vnode
+  VnodeView* found = reinterpret_cast<VnodeView*>(joined + kMaxRanked / 64);
   const int tid = threadIdx.x;
-  if (tid < n) views[tid] = load_vnode<GATHERED>(a, a.vnode_begin + tid);  // the block's own vnode is among them
-  if (tid == 0) *found = -1;
-  __syncthreads();
-  // bit u: vnode u continues vnode u - 1 (same run, adjoining scratch rows).  Nothing is joined
-  // while there are no more blocks than compute units: two half-filled blocks side by side
+  VnodeView mine{0, 0, 0, 0};
+  // bit u: vnode u continues vnode u - 1 (same run, adjoining scratch rows; both read here, in one round trip).
+  // Nothing is joined while there are no more blocks than compute units: two half-filled blocks side by side
   // finish sooner than one full block.
   bool joins = false;
-  if (tid > 0 && tid < n && 2LL * n * a.hkv * a.wide_chunks > a.block_slots) {
-    const VnodeView& p = views[tid - 1];
-    const VnodeView& c = views[tid];
-    joins = p.kv_base == c.kv_base && p.kv_len == c.kv_len && p.q_off + p.q_len == c.q_off;
+  if (tid < n) {
+    mine = load_vnode<GATHERED>(a, a.vnode_begin + tid);  // the block's own vnode is among them
+    const VnodeView p = load_vnode<GATHERED>(a, a.vnode_begin + max(tid - 1, 0));
+    joins = tid > 0 && 2LL * n * a.hkv * a.wide_chunks > a.block_slots && p.kv_base == mine.kv_base && p.kv_len == mine.kv_len &&
+            p.q_off + p.q_len == mine.q_off;
+    q_len_of[tid] = mine.q_len;
+    q_end_of[tid] = mine.q_off + mine.q_len;
   }
   const unsigned long long wave_bits = __ballot(joins);
   if ((tid & 63) == 0) joined[tid >> 6] = wave_bits;
+  if (tid == 0) *found = VnodeView{0, 0, 0, 0};    // (stays where there are more ranks than groups: an empty item)
   __syncthreads();
-  unsigned mine = 0;
+  unsigned key = 0;
   if (tid < n) {
     // first and last vnode of the chain of joined vnodes that holds this one
     int first = tid;
@@ -1685,25 +1693,21 @@ __device__ __forceinline__ int wide_vnode_of_rank(const Stage1Args& a, char* sme
         break;
       }
     }
-    // groups of m vnodes from the start of the chain; the chain's first vnode is a full query tile
-    const long long cap = (long long)a.join_rows * a.wide_chunks;
-    const long long tile_rows = max(1LL, (long long)views[first].q_len * a.g);
-    const int m = (int)max(1LL, cap / tile_rows);
-    const int head = first + (tid - first) / m * m;
-    int q_len = 0;
+    // groups of m vnodes from the start of the chain; the chain's first vnode is a full query tile (a cap of at most
+    // 8 chunks of 192 rows; g at most 64)
+    const int m = max(1, small_quotient(a.join_rows * a.wide_chunks, max(1, min(q_len_of[first], 4096) * a.g)));
+    const int head = first + small_quotient(tid - first, m) * m;
     if (head == tid) {
-      const VnodeView& tail = views[min(last, head + m - 1)];
-      q_len = tail.q_off + tail.q_len - views[tid].q_off;
-      const float work = (float)q_len * (float)a.g * (float)views[tid].kv_len;
+      mine.q_len = q_end_of[min(last, head + m - 1)] - mine.q_off;
+      const float work = (float)mine.q_len * (float)a.g * (float)mine.kv_len;
       // (256 - tid is never 0: the key of a vnode without work must not be the 0 of "no group")
       static_assert(kMaxRanked <= 256, "the low nine bits of a key hold 256 - tid");
-      mine = ((__builtin_bit_cast(unsigned, work) >> 8) << 9) | (unsigned)(256 - tid);
+      key = ((__builtin_bit_cast(unsigned, work) >> 8) << 9) | (unsigned)(256 - tid);
     }
-    group_q_len[tid] = q_len;
   }
-  keys[tid] = mine;  // all kMaxRanked entries: the vector reads below run over the padding
+  keys[tid] = key;  // all kMaxRanked entries: the vector reads below run over the padding
   __syncthreads();
-  if (mine != 0) {
+  if (key != 0) {
     int rank = 0;
     for (int j0 = 0; j0 < n; j0 += 16) {  // (keys past n are 0 and count for nothing)
       u32x4 k[4];
@@ -1712,21 +1716,13 @@ __device__ __forceinline__ int wide_vnode_of_rank(const Stage1Args& a, char* sme
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) rank += k[i][e] > mine ? 1 : 0;
+        for (int e = 0; e < 4; ++e) rank += k[i][e] > key ? 1 : 0;
     }
-    if (rank == target) *found = tid;
+    if (rank == target) *found = mine;
   }
   __syncthreads();
-  const int v = *found;
-  if (v < 0) {  // more ranks than groups: an empty item
-    view = VnodeView{0, 0, 0, 0};
-    __syncthreads();
-    return 0;
-  }
-  view = views[v];
-  view.q_len = group_q_len[v];
+  view = *found;
   __syncthreads();  // the ranking area is reused as the staging ring
-  return v;
 }
 
 // The wide vnodes of one block program for one kv head (kv head fastest among the blocks: the eight blocks of a program
@@ -1802,17 +1798,15 @@ __global__ void __launch_bounds__(kWideBlock, fused_waves(D, MODE)) stage1_fused
   constexpr bool kAgain = D <= 128;
   if (narrow_index < 0) {
     if constexpr (MODE == kLists) {
-      const int per_rank = a.wide_chunks * a.hkv;
-      const int rank = uniform((int)blockIdx.x / per_rank);
-      const int rest = (int)blockIdx.x - rank * per_rank;
-      // Launch slot `rest / hkv` of a rank serves chunk (slot + rank / 2) % chunks.  Consecutive
+      const int slot_of_all = a.by_hkv(blockIdx.x), kvh = (int)blockIdx.x - slot_of_all * a.hkv;
+      const int rank = a.by_chunks(slot_of_all);
+      // Launch slot s of a rank serves chunk (s + rank / 2) % chunks.  Consecutive
       // blocks of one kv head go round robin to the four shader engines of an XCD, strictly in
       // order (a block waits for its engine even when others have room); without the rotation an
       // engine would only ever get first chunks, which run longer than last ones.
-      const int slot = a.by_hkv(rest), kvh = rest - slot * a.hkv;
-      const int chunks = a.wide_chunks, chunk = uniform((slot + (rank >> 1)) % chunks);
+      const int chunks = a.wide_chunks, turned = slot_of_all - rank * chunks + (rank >> 1), chunk = turned - a.by_chunks(turned) * chunks;
       VnodeView vn{0, 0, 0, 0};
-      (void)wide_vnode_of_rank<GATHERED>(a, smem, rank, vn);
+      wide_vnode_of_rank<GATHERED>(a, smem, rank, vn);
       vn = uniform(vn);
       const Stage1Args& b = kAgain ? args_again() : a;
       RowStream<D, GATHERED> rows(b, smem, kvh);
@@ -2232,6 +2226,7 @@ int launch_stage1_fused(const Stage1Args& a0, hipStream_t stream) {
   const int per_block = kWideWaves / a.narrow_share;
   const int64_t narrow_blocks = (narrow_items + per_block - 1) / per_block;
   a.wide_chunks = std::max(1, std::min(8, (a.wide_rows + WideRows<D>::kBlock - 1) / WideRows<D>::kBlock));
+  a.by_chunks = divisor(a.wide_chunks);
   a.block_slots = (D > 128 ? wave_slots() / 2 : wave_slots()) / kWideWaves;
   // Vnodes of one run are joined to full blocks only where that leaves a block per compute unit: 11 query
   // tiles of 64 rows over three 1024-token splits and 8 KV heads take 46.7 us as 96 blocks of 192 rows and

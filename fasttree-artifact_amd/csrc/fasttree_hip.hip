@@ -105,6 +105,8 @@ __device__ __forceinline__ float xor32_max(float x) { LanePair h = halves32(x); 
 __device__ __forceinline__ float xor16_sum(float x) { LanePair h = halves16(x); return h.lo + h.hi; }
 __device__ __forceinline__ float xor32_sum(float x) { LanePair h = halves32(x); return h.lo + h.hi; }
 __device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
+// x of the lane numbered `from` (0..63, may differ from lane to lane; every lane of the wave takes part).
+__device__ __forceinline__ int lane_value(int x, int from) { return __builtin_amdgcn_ds_bpermute(4 * from, x); }
 // The lane's number, opaque to the compiler: what is derived from it stays where it is used.  (In a
 // kernel whose loops hold several kinds of work the compiler would otherwise compute every kind's
 // lane addresses ahead of all of them and spill them: scratch reloads inside a stream of direct
@@ -1151,7 +1153,7 @@ struct RecordRequests {
   }
   // (i differs from lane to lane; every lane of the wave takes part)
   __device__ __forceinline__ int of(int i) const {
-    const int e = __shfl(even, i >> 1), o = __shfl(odd, i >> 1);
+    const int e = lane_value(even, i >> 1), o = lane_value(odd, i >> 1);
     return i & 1 ? o : e;
   }
 };
@@ -1390,7 +1392,7 @@ template <int D, bool GATHERED> struct NarrowStream {
   // the same of the run's first tile, from the vnode's record (a lane's int of it)
   __device__ __forceinline__ void rows_of_record(int rec) {
 #pragma unroll
-    for (int g = 0; g < N::kLoads; ++g) srow[g] = (unsigned)__shfl(rec, kNarrowRecSlots + row(g));
+    for (int g = 0; g < N::kLoads; ++g) srow[g] = (unsigned)lane_value(rec, kNarrowRecSlots + row(g));
   }
   // those rows of K (or V) -> the wave's K (V) tile
   __device__ __forceinline__ void issue(bool is_v) const {
@@ -1430,7 +1432,7 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
       for (int qb = 0; qb < NG; ++qb) req[qb] = vn.q_off / a.nsplit;
     } else if (inlined && vn.q_len <= kNarrowRecRequests) {   // wave uniform: they are in the record
 #pragma unroll
-      for (int qb = 0; qb < NG; ++qb) req[qb] = __shfl(rec, 4 + req[qb]);
+      for (int qb = 0; qb < NG; ++qb) req[qb] = lane_value(rec, 4 + req[qb]);
     } else {
 #pragma unroll
       for (int qb = 0; qb < NG; ++qb) req[qb] = a.q_entries[vn.q_off + req[qb]];
@@ -1531,6 +1533,69 @@ __device__ __forceinline__ void merge_shares(float* xchg, WaveState<D, NG>& st, 
   }
 }
 
+// The merged rows of a narrow vnode from the states of the SHARE waves that served it, in LDS at xchg: this wave, the
+// w-th, merges and writes its part of the dims of every row.
+template <int D, int NG, int SHARE>
+__device__ __forceinline__ void write_merged_shares(const Stage1Args& a, const float* xchg, const VnodeView& vn, int kvh, int row0, int w) {
+  constexpr int DB = D / 16, kML = NG * DB * 4 * kWave;
+  constexpr int kStep = NarrowGeom<D>::kLds / 4;           // floats from one wave's area to the next one's
+  constexpr int kParts = DB / SHARE;                       // dim blocks of a wave
+  const int lane = lane_here(), p = lane & 15, c = lane >> 4;
+#pragma unroll 1
+  for (int qb = 0; qb < NG; ++qb) {
+    const float* ml = xchg + kML + 2 * qb * kWave + lane;
+    const f32x4* o = reinterpret_cast<const f32x4*>(xchg) + (qb * DB + w * kParts) * kWave + lane;
+    float m_of[SHARE], l_of[SHARE];
+    f32x4 o_of[SHARE][kParts];
+#pragma unroll
+    for (int i = 0; i < SHARE; ++i) {
+      m_of[i] = ml[i * kStep];
+      l_of[i] = ml[i * kStep + kWave];
+#pragma unroll
+      for (int db = 0; db < kParts; ++db) o_of[i][db] = o[i * (kStep / 4) + db * kWave];
+    }
+    float m = m_of[0], l = 0.f;
+#pragma unroll
+    for (int i = 1; i < SHARE; ++i) m = fmaxf(m, m_of[i]);
+    f32x4 sum[kParts];
+#pragma unroll
+    for (int db = 0; db < kParts; ++db) sum[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < SHARE; ++i) {
+      const float weight = scale_from(m_of[i], m);
+      l += l_of[i] * weight;
+#pragma unroll
+      for (int db = 0; db < kParts; ++db) sum[db] += o_of[i][db] * weight;
+    }
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    const int r = row0 + 16 * qb + p;
+    if (r < vn.q_len * a.g) {
+      const int ri = a.by_g(r), head = kvh * a.g + r - ri * a.g;
+      const int64_t row = vn.q_off + ri;
+      float* dst = a.mid_o + row * a.so0 + (int64_t)head * a.so1 + 4 * c + 16 * w * kParts;
+#pragma unroll
+      for (int db = 0; db < kParts; ++db) *reinterpret_cast<f32x4*>(dst + 16 * db) = sum[db] * inv;
+      if (w == 0 && c == 0) a.mid_lse[row * a.sl0 + head] = l > 0.f ? (__builtin_amdgcn_logf(l) + m) * kLn2 : -INFINITY;
+    }
+  }
+}
+// Merge of the states of the `share` waves (2 or 4) of one narrow vnode through LDS at xchg, and the write of the merged
+// rows, in one exchange in which every wave merges its part: pairwise, into one wave that then writes them, a launch of
+// few vnodes spends 1.4 us here, in code it fetches cold (4 requests of a short prompt 8.45 us, 8.0 so; 30 of 16/1 heads
+// 9.35 and 8.85; serving 1.2 % shorter).  Every wave of the block calls this (a block barrier); `rows`: whether the vnode
+// has rows in this pass.
+template <int D, int NG>
+__device__ __forceinline__ void merge_and_write_shares(const Stage1Args& a, float* xchg, const VnodeView& vn, int kvh, int row0, bool rows,
+                                                       const WaveState<D, NG>& st, int w, int share) {
+  static_assert(SharedState<D, NG>::kFloats * kWave * 4 <= NarrowGeom<D>::kLds, "a wave's state fits its LDS area");
+  asm volatile("" : "+s"(w), "+s"(share), "+s"(kvh));      // (what is made from them stays here)
+  if (rows) SharedState<D, NG>::put(xchg + w * (NarrowGeom<D>::kLds / 4), st);
+  __syncthreads();
+  if (!rows) return;
+  if (share == 2) write_merged_shares<D, NG, 2>(a, xchg, vn, kvh, row0, w);
+  else write_merged_shares<D, NG, 4>(a, xchg, vn, kvh, row0, w);
+}
+
 // What one wave does for a narrow vnode in one pass (NG row groups from row0; none if row0 is past
 // its rows, and then the wave only keeps the block's barriers company).
 struct NarrowPass {
@@ -1544,7 +1609,17 @@ __device__ __forceinline__ void narrow_pass(const Stage1Args& a, char* smem, con
   const bool rows = p.row0 < vn.q_len * a.g;
   if (rows) narrow_attend<E, D, NG, GATHERED>(a, vn, stream, p.started, p.kvh, p.row0, st, p.rec, p.inlined);
   else reset_state<D, NG>(st);
-  if (p.share > 1) merge_shares<D, NG>(reinterpret_cast<float*>(smem + p.xchg), st, p.w, p.share);
+  float* xchg = reinterpret_cast<float*>(smem + p.xchg);
+  // (rows of less than 256 bytes keep the pairwise merge: with the other one the kernel for narrow vnodes alone takes 131
+  // registers instead of 126, three waves per SIMD instead of four, and 269 requests of 64/8 heads of 64 83.1 us instead
+  // of 81.9)
+  if constexpr (D >= 128) {
+    if (p.share > 1) {
+      merge_and_write_shares<D, NG>(a, xchg, vn, p.kvh, p.row0, rows, st, p.w, p.share);
+      return;
+    }
+  }
+  if (p.share > 1) merge_shares<D, NG>(xchg, st, p.w, p.share);
   if (rows && p.w == 0) write_partials<D, NG>(a, vn, p.kvh, p.row0, st);
 }
 

@@ -9,8 +9,8 @@
 // O^T = V^T P^T, so the probabilities go from the first contraction's accumulators
 // straight into the second contraction's B operand without leaving registers.
 //
-// Stage 2 merges each request's partials with their log-sum-exp weights using shuffles
-// inside a group of D/4 lanes.
+// Stage 2 merges each request's partials with their log-sum-exp weights: D/4 lanes per (request,
+// head), and several waves per list where whole lists would leave the machine idle.
 //
 // Reference for the arithmetic: kernel_bench/fasttree.py:299-413 (stage 1), :482-546
 // (stage 2), :582-642 (the call that chains them).
@@ -1280,7 +1280,10 @@ __device__ __forceinline__ void wide_block(const Stage1Args& a, char* smem, cons
     // LDS for fewer waves, but then the groups' states are merged, in code that every launch fetches cold, and a wave
     // has one tile between two barriers (12 requests of 32/8 heads on 8192 tokens, 48 rows: 15.3 us with two groups, 14.7
     // with one; 64 rows on a 4096-token prefix 25.4 and 24.5, 16 requests each in 20 groups of 96 rows 47.4 and 46.7, of 80
-    // rows 34.9 and 35.5).  At 512-byte rows a block has its unit to itself (64 requests of 16/1 heads of 256: 23.0 us
+    // rows 34.9 and 35.5).  Each group's first maximum has the probability 1, which the storage type holds exactly, so one
+    // group rounds a little more of P than two (shared prefixes of fp16 against 64 bits, relative RMS over ten inputs 2.88e-4
+    // with two groups and 2.90e-4 with one; the largest error does not differ), as one piece of a run does beside two.
+    // At 512-byte rows a block has its unit to itself (64 requests of 16/1 heads of 256: 23.0 us
     // with two groups of two row groups, 20.0 with four of one).
     constexpr int kMostTokenGroups = D <= 128 ? WideGeom<D>::kSub : kWideWaves;
     int log_tgroups = 0;
@@ -1843,8 +1846,9 @@ __host__ __device__ constexpr int trailing_item(int index, int in_programs, int 
 static_assert(trailing_item(5, 7, 20) == 12 && trailing_item(12, 7, 20) == 19 && trailing_item(13, 7, 20) == 20);
 static_assert(trailing_item(INT32_MAX - 10, 9, INT32_MAX) == INT32_MAX - 1 && trailing_item(INT32_MAX - 10, 13, INT32_MAX) == INT32_MAX);
 
-// How the fused kernel gets its wide vnodes: as the planner's list; as block programs (Stage1Args::prog_table); as
-// block programs that also serve narrow vnodes (Stage1Args::narrow_in_programs).
+// How a fused launch gets its wide vnodes: as the planner's list; as block programs (Stage1Args::prog_table); as
+// block programs that also serve narrow vnodes (Stage1Args::narrow_in_programs).  A kernel for each: one holds no code
+// that its launches do not run.
 constexpr int kLists = 0, kPrograms = 1, kEmbedding = 2;
 
 // What bounds the start of a block is the fetch of its instructions, which every launch begins with an empty
@@ -1863,8 +1867,7 @@ constexpr int kLists = 0, kPrograms = 1, kEmbedding = 2;
 // 168, 110.4 with 171); under that limit programs come out slower.
 constexpr int fused_waves(int D, int mode) { return D > 128 ? 1 : D == 128 || mode != kLists ? 2 : 3; }
 template <typename E, int D, bool GATHERED, int MODE>
-__global__ void __launch_bounds__(kWideBlock, fused_waves(D, MODE)) stage1_fused_kernel(Stage1Args a) {
-  extern __shared__ __attribute__((aligned(1024))) char smem[];
+__device__ __forceinline__ void fused_block(const Stage1Args& a, char* smem) {
   const int wide_blocks = MODE != kLists ? a.num_programs * a.hkv : a.vnode_count * a.wide_chunks * a.hkv;
   const int narrow_index = (int)blockIdx.x - wide_blocks;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1918,6 +1921,18 @@ __global__ void __launch_bounds__(kWideBlock, fused_waves(D, MODE)) stage1_fused
       narrow_item<E, D, GATHERED, false>(kAgain ? args_again() : a, smem, wave, share, item < end, a.narrow_begin + vnode, item - vnode * a.hkv);
     }
   }
+}
+
+template <typename E, int D, bool GATHERED, bool PROGRAMS>
+__global__ void __launch_bounds__(kWideBlock, fused_waves(D, PROGRAMS ? kPrograms : kLists)) stage1_fused_kernel(Stage1Args a) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  fused_block<E, D, GATHERED, PROGRAMS ? kPrograms : kLists>(a, smem);
+}
+
+template <typename E, int D>
+__global__ void __launch_bounds__(kWideBlock, fused_waves(D, kEmbedding)) stage1_embedding_kernel(Stage1Args a) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  fused_block<E, D, false, kEmbedding>(a, smem);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2284,7 +2299,9 @@ int launch_stage1_fused(const Stage1Args& a0, hipStream_t stream) {
   constexpr size_t kWideLds = (size_t)WideGeom<D>::kLds;
   constexpr size_t kNarrowLds = (size_t)kWideWaves * NarrowGeom<D>::kLds;
   constexpr size_t lds = kWideLds > kNarrowLds ? kWideLds : kNarrowLds;
-  auto kern = stage1_fused_kernel<E, D, GATHERED, MODE>;
+  void (*kern)(Stage1Args) = nullptr;
+  if constexpr (MODE == kEmbedding) kern = stage1_embedding_kernel<E, D>;
+  else kern = stage1_fused_kernel<E, D, GATHERED, MODE == kPrograms>;
   // (raising the dynamic LDS limit is idempotent: two threads that both find the flag clear both raise it)
   static std::atomic<bool> configured_on[kMaxDevices];
   std::atomic<bool>& configured = configured_on[current_device()];

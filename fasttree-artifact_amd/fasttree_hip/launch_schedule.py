@@ -77,8 +77,9 @@ VNODE_STARTUP_TILES = 5.0
 #: A narrow vnode on one wave, in the same unit: its start-up and one 32-token step.
 NARROW_STARTUP_TILES = 3.8
 NARROW_STEP_TILES = 0.85
-#: What the merge of the waves that share one narrow vnode costs each of them (two block barriers
-#: and an exchange of the state through LDS per halving), in the same unit.
+#: What the merge of the waves that share one narrow vnode costs each of them, in the same unit (measured
+#: with two block barriers and an exchange of the state through LDS per halving, as below 128 dims; one
+#: exchange serves all of them from there on, and other values of the schedule's constants gain nothing).
 NARROW_SHARE_TILES = 0.5
 #: Microseconds per tile step of a block that shares its compute unit with another wide block,
 #: and of one that does not (measured on the 3-level tree of the headline benchmark).

@@ -1025,7 +1025,7 @@ struct WidePass {
   int kvh;
   int row0;            // the wave's first query row
   int groups;          // its 16-row groups (0: it only loads)
-  int set, tg, tgroups;  // its row set, its token group, token groups of the pass (several: a wave has one row group at most)
+  int set, tg, tgroups;  // its row set, its token group, token groups of the pass
 };
 
 // A wave's state in LDS for another wave to merge: its accumulators as 16-byte words, then m and l.
@@ -1063,17 +1063,17 @@ template <int D, int NG> struct SharedState {
   }
 };
 
-// Merge of the waves that hold the same 16 rows (the token groups of a row set) into token group 0,
+// Merge of the waves that hold the same rows (the token groups of a row set) into token group 0,
 // pairwise through LDS.  Every wave of the block must call this.
-template <int D>
-__device__ __forceinline__ void merge_token_groups(float* xchg, WaveState<D, 1>& st, const WidePass& p) {
-  constexpr int kArea = SharedState<D, 1>::kFloats * kWave;
+template <int D, int NG>
+__device__ __forceinline__ void merge_token_groups(float* xchg, WaveState<D, NG>& st, const WidePass& p) {
+  constexpr int kArea = WideRows<D>::kGroups * SharedState<D, 1>::kFloats * kWave;   // (waves of other sets may hold fewer groups)
 #pragma unroll 1
   for (int half = p.tgroups >> 1; half >= 1; half >>= 1) {
     __syncthreads();
-    if (p.tg >= half && p.tg < 2 * half) SharedState<D, 1>::put(xchg + (size_t)(p.set * half + p.tg - half) * kArea, st);
+    if (p.tg >= half && p.tg < 2 * half) SharedState<D, NG>::put(xchg + (size_t)(p.set * half + p.tg - half) * kArea, st);
     __syncthreads();
-    if (p.tg < half) SharedState<D, 1>::merge(xchg + (size_t)(p.set * half + p.tg) * kArea, st);
+    if (p.tg < half) SharedState<D, NG>::merge(xchg + (size_t)(p.set * half + p.tg) * kArea, st);
   }
 }
 
@@ -1230,7 +1230,7 @@ __device__ __forceinline__ void wide_pass(const Stage1Args& a, char* smem, const
     for (int sub = 0; sub < W::kSub; ++sub) {
       const int tile = super * W::kSub + sub;
       const int valid = vn.kv_len - tile * kTileTokens;
-      if ((NG == 1 && (tile & (p.tgroups - 1)) != p.tg) || valid <= 0 || p.groups == 0) continue;
+      if ((tile & (p.tgroups - 1)) != p.tg || valid <= 0 || p.groups == 0) continue;
       const unsigned off = (super & 1) * W::kBytes + sub * W::kTileBytes;
       f32x4 sc[2][NG];
       u32x4 pf[NG];
@@ -1244,9 +1244,7 @@ __device__ __forceinline__ void wide_pass(const Stage1Args& a, char* smem, const
     }
   }
   finish_state<D, NG>(st);
-  if constexpr (NG == 1) {
-    if (p.tgroups > 1) merge_token_groups<D>(reinterpret_cast<float*>(smem), st, p);
-  }
+  if (p.tgroups > 1) merge_token_groups<D, NG>(reinterpret_cast<float*>(smem), st, p);
   if (p.tg == 0) write_partials<D, NG>(a, vn, p.kvh, p.row0, st, p.groups);
   __syncthreads();  // the ring is reused by the next pass
 }
@@ -1274,20 +1272,19 @@ __device__ __forceinline__ void wide_block(const Stage1Args& a, char* smem, cons
     }
     const int row0 = piece * kRows;
     const int groups = (min(row0 + kRows, rows_total) - row0 + 15) >> 4;
-    // As many token groups as leave a wave one row group, and no more than a super tile has tiles: between two barriers
-    // a wave of a third group would have none (one vnode of 48 rows and 1024 tokens per block, a step of 32 tokens: four
-    // groups .52 us, two .43).  More rows per wave, and token groups for 64 and 96 rows, would read a K/V operand from
-    // LDS for fewer waves, but then the groups' states are merged, in code that every launch fetches cold, and a wave
-    // has one tile between two barriers (12 requests of 32/8 heads on 8192 tokens, 48 rows: 15.3 us with two groups, 14.7
-    // with one; 64 rows on a 4096-token prefix 25.4 and 24.5, 16 requests each in 20 groups of 96 rows 47.4 and 46.7, of 80
-    // rows 34.9 and 35.5).  Each group's first maximum has the probability 1, which the storage type holds exactly, so one
-    // group rounds a little more of P than two (shared prefixes of fp16 against 64 bits, relative RMS over ten inputs 2.88e-4
-    // with two groups and 2.90e-4 with one; the largest error does not differ), as one piece of a run does beside two.
-    // At 512-byte rows a block has its unit to itself (64 requests of 16/1 heads of 256: 23.0 us
-    // with two groups of two row groups, 20.0 with four of one).
+    // As many token groups as leave every wave at most NQ row groups: fewer waves then read the same K/V
+    // operands from LDS.  No more than a super tile has tiles: between two barriers a wave of a third group
+    // would have none (one vnode of 48 rows and 1024 tokens per block, a step of 32 tokens: four groups .52 us, two
+    // .43; of 32 rows .43 and .37; a 111-request tree of 16/1 heads with four such vnodes 32.9 -> 27.9 us).  At 512-byte
+    // rows, where a block has its unit to itself and merging a row group moves 16 KB, as leave every wave one (64
+    // requests of 16/1 heads of 256: 23.0 -> 20.0 us; a step takes the same with two groups or four).
+    // One token group from 33 rows on spares most passes the merge, but each group's first maximum has the probability
+    // 1, which the storage type holds exactly, and one group so rounds more of P than two: it costs precision (shared
+    // prefixes of fp16 against 64 bits, relative RMS over ten inputs 2.88e-4 with two groups, 2.90e-4 with one).
+    constexpr int kGroupsWanted = D <= 128 ? NQ * kWideWaves : kWideWaves;
     constexpr int kMostTokenGroups = D <= 128 ? WideGeom<D>::kSub : kWideWaves;
     int log_tgroups = 0;
-    while ((1 << log_tgroups) < kMostTokenGroups && groups * (2 << log_tgroups) <= kWideWaves) ++log_tgroups;
+    while ((1 << log_tgroups) < kMostTokenGroups && groups * (2 << log_tgroups) <= kGroupsWanted) ++log_tgroups;
     static_assert(kWideWaves == 4, "row sets are 4 >> log_tgroups");
     const int log_sets = 2 - log_tgroups;
     WidePass p;

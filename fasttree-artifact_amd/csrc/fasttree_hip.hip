@@ -2072,6 +2072,7 @@ struct Stage2Args {
   int batch, hq;
   int longest; // no request has more partials than this (the number of vnodes, or more)
   int log_splits;  // 1 << this many waves share a request's list, set by the launcher
+  int log_groups;  // and in kLongLists at most 1 << this many groups of D/4 lanes one of more than kLongList entries
   int nsplit;  // > 0: gathered mode, request r owns rows [r*nsplit, (r+1)*nsplit)
   // (or null) one record of kReqRecord int32 per request, written by the host: req_lens[r],
   // req_offs[r], then the request's first kReqRecord - 2 entries -- what the block needs before
@@ -2080,6 +2081,93 @@ struct Stage2Args {
 };
 constexpr int kReqRecord = 16;
 constexpr int kReqRecEntries = kReqRecord - 2;
+// How a launch reads its lists: each by one wave; each of more than kReqRecEntries entries by several waves; as that,
+// but those of more than kLongList entries by groups of lanes.
+constexpr int kWholeLists = 0, kSplitLists = 1, kLongLists = 2;
+constexpr int kLongList = 64;
+
+// The merge of a list of more than kLongList entries, n of them, from `list` on (or the rows from row0 on).  Four waves
+// would read it in many batches, one round trip after the other, so it is cut finer: a group of D/4 lanes takes a part for
+// one head.  Its lanes hold an entry each, with the entry's weight, fetch the next ones ahead and hand them round.
+template <typename E, int D>
+__device__ __forceinline__ void merge_long_list(const Stage2Args& a, int req, int n, int row0, PlanInts list) {
+  constexpr int LPH = D / 4, kGroups = kBlock / LPH, kBatch = LPH < 8 ? LPH : 8;
+  const int group = threadIdx.x / LPH, gl = threadIdx.x % LPH;
+  const int log_parts = min(a.log_groups, 31 - __builtin_clz((unsigned)n / kBatch));   // (parts of kBatch entries and more)
+  if (((int)blockIdx.y * kGroups) >> log_parts >= a.hq) return;     // block uniform
+  const int parts = 1 << log_parts, part_of_group = group & (parts - 1);
+  const int head = ((int)blockIdx.y * kGroups + group) >> log_parts;
+  const bool exists = head < a.hq;
+  const int head_in = exists ? head : a.hq - 1;             // (lanes past the last head read that one's rows and store nothing)
+  const int size = (n + parts - 1) >> log_parts, first = part_of_group * size, mine = min(n - first, size);
+
+  const char* o_lane = reinterpret_cast<const char*>(a.mid_o + (int64_t)head_in * a.so1 + 4 * gl);
+  auto entry = [&](int i0) {                                // (past the part its last entry again, or the list's: not counted)
+    const int i = min(first + i0 + gl, min(first + size, n) - 1);
+    return a.nsplit > 0 ? row0 + i : list[i];
+  };
+  // x of the group's lane j (a constant after unrolling)
+  auto of_lane = [](int x, int j) { return LPH == kWave ? __builtin_amdgcn_readlane(x, j) : __shfl(x, j, LPH); };
+  float m_run = -INFINITY, l_run = 0.f;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  int row = entry(0);
+  for (int base = 0; base < mine; base += LPH) {
+    const int held = min(LPH, mine - base);
+    float lse = a.mid_lse[(int64_t)row * a.sl0 + head_in];
+    const int row_here = row;
+    if (base + LPH < mine) row = entry(base + LPH);
+    lse = gl < held ? lse : -INFINITY;
+    f32x4 part[kBatch];
+    auto request = [&](int i0) {
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j)
+        part[j] = *reinterpret_cast<const f32x4*>(o_lane + 4 * (int64_t)of_lane(row_here, i0 + j) * a.so0);
+    };
+    request(0);
+    float m_new = lse;
+#pragma unroll
+    for (int d = LPH / 2; d >= 1; d >>= 1) m_new = fmaxf(m_new, __shfl_xor(m_new, d, LPH));
+    m_new = fmaxf(m_run, m_new);
+    const float keep = (m_run == -INFINITY) ? 0.f : __expf(m_run - m_new);
+    const float w = (lse == -INFINITY) ? 0.f : __expf(lse - m_new);
+    l_run *= keep;
+    acc *= keep;
+    m_run = m_new;
+    for (int i0 = 0; i0 < held; i0 += kBatch) {
+      if (i0 > 0) request(i0);
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) {
+        const float w_j = __builtin_bit_cast(float, of_lane(__builtin_bit_cast(int, w), i0 + j));
+        l_run += w_j;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] += (w_j != 0.f) ? part[j][e] * w_j : 0.f;
+      }
+    }
+  }
+  // the groups' states to the first of them
+  __shared__ f32x4 acc_of[kBlock];
+  __shared__ float m_of[kGroups], l_of[kGroups];
+  acc_of[threadIdx.x] = acc;
+  if (gl == 0) {
+    m_of[group] = m_run;
+    l_of[group] = l_run;
+  }
+  __syncthreads();
+  if (part_of_group > 0 || !exists) return;
+  float m_all = m_run;
+  for (int i = 1; i < parts; ++i) m_all = fmaxf(m_all, m_of[group + i]);
+  acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  l_run = 0.f;
+  for (int i = 0; i < parts; ++i) {
+    const float m_i = m_of[group + i];
+    const float w = (m_i == -INFINITY) ? 0.f : __expf(m_i - m_all);
+    l_run += l_of[group + i] * w;
+    acc += acc_of[threadIdx.x + i * LPH] * w;
+  }
+  acc *= l_run > 0.f ? 1.f / l_run : 0.f;
+  const u32x2 out = {E::pack2(acc[0], acc[1]), E::pack2(acc[2], acc[3])};
+  *reinterpret_cast<u32x2*>(a.o + 2 * ((int64_t)req * a.oo0 + (int64_t)head * a.oo1 + 4 * gl)) = out;
+}
 
 // D/4 lanes serve one (request, head), a wave several heads of one request; `splits` waves of a block (1, 2 or 4) take
 // parts of the request's list and are merged through LDS.  A wave reads the list of its request as scalars (from the
@@ -2087,11 +2175,12 @@ constexpr int kReqRecEntries = kReqRecord - 2;
 // partial rows, and for their log-sum-exps, with nothing but its own address and a scalar.
 //
 // Bound by the partial rows it reads, and for a batch of few requests by how many of them are in flight (8 requests x
-// 64 heads with 68 partials each: 64 blocks of whole lists 11.2 us) and by the fetch of its instructions, 2.7 KB where a
+// 64 heads with 68 partials each: 64 blocks of whole lists 11.5 us, in eight parts each 6.7) and by the fetch of its instructions, 2.7 KB where a
 // list spread over lanes and handed round by shuffles took 4.0 (whole calls: 4 requests of a short prompt 9.1 -> 8.4 us,
 // 111 ragged requests of 64-dim heads 13.6 -> 12.7, 16/1 heads of 256 18.2 -> 17.4, the 400-request tree 61.9 -> 61.0).
-template <typename E, int D, bool SPLIT>
+template <typename E, int D, int LISTS>
 __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
+  constexpr bool SPLIT = LISTS != kWholeLists;
   constexpr int LPH = D / 4;
   constexpr int HPW = kWave / LPH;                          // heads of a wave
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -2119,6 +2208,11 @@ __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
   } else {
     n = plan_ints(a.req_lens)[req];
     list = plan_ints(a.req_entries) + plan_ints(a.req_offs)[req];
+  }
+  if constexpr (LISTS == kLongLists) {
+    if (n > kLongList) return merge_long_list<E, D>(a, req, n, row0, list);
+    // (the grid has the blocks that the one way or the other needs)
+    if ((((int)blockIdx.y * kWavesPerBlock) >> log_splits) * HPW >= a.hq) return;
   }
   int split = 0, splits = 1;
   if constexpr (SPLIT) {
@@ -2399,7 +2493,12 @@ int launch_stage1(const Stage1Args& a, int d, int dtype, hipStream_t stream) {
 
 // Waves per list: as many as leave the launch at most two blocks per compute unit (wave_slots() / 4): more blocks than
 // that hide each other's round trips anyway.  One wave, and the kernel without the merge, where every list is short or
-// the batch fills the machine by itself (684 requests of 32 heads: 8.2 us without the merge's code, 9.6 with it).
+// the batch fills the machine by itself.
+// Lane groups per list of more than kLongList entries by the same rule, where that makes more parts than four waves do (warm, the
+// merge alone, four waves and lane groups; 512 entries: one request of 32 heads of 128 16.5 and 7.3 us, of 64 heads of 64 16.6 and
+// 6.8, of 16 heads of 256 18.6 and 10.9; 128 entries 5.8 and 4.1, 5.8 and 4.1, 6.2 and 4.7; 65 entries 4.9 and 4.2, 4.9 and 4.7,
+// 5.2 and 4.2).  In four parts, or eight of 32 dims, waves read more of a row at once (64 requests of 24 heads of 64 with 512
+// entries: 38.6 and 41.5; of 32 heads of 32: 28.4 and 30.2); 512-byte rows are a wave's in either case.
 template <typename E, int D>
 int launch_stage2_inst(const Stage2Args& a0, hipStream_t stream) {
   constexpr int kHeads = kWavesPerBlock * kWave / (D / 4);   // of a block whose waves share no list
@@ -2407,9 +2506,14 @@ int launch_stage2_inst(const Stage2Args& a0, hipStream_t stream) {
   a.log_splits = 0;
   auto blocks_per_request = [&](int log_splits) { return ((int64_t)(a.hq << log_splits) + kHeads - 1) / kHeads; };
   while (a.longest > kReqRecEntries && (1 << a.log_splits) < kWavesPerBlock && a.batch * blocks_per_request(a.log_splits + 1) <= wave_slots() / 4) ++a.log_splits;
-  const dim3 grid((unsigned)a.batch, (unsigned)blocks_per_request(a.log_splits), 1);
-  if (a.log_splits > 0) hipLaunchKernelGGL((stage2_kernel<E, D, true>), grid, dim3(kBlock, 1, 1), 0, stream, a);
-  else hipLaunchKernelGGL((stage2_kernel<E, D, false>), grid, dim3(kBlock, 1, 1), 0, stream, a);
+  a.log_groups = 0;
+  while (a.longest > kLongList && (1 << a.log_groups) < kHeads && a.batch * blocks_per_request(a.log_groups + 1) <= wave_slots() / 4) ++a.log_groups;
+  constexpr int kLeast = D <= 32 ? 16 : D <= 128 ? 8 : 4;
+  if ((1 << a.log_groups) < kLeast) a.log_groups = 0;
+  const dim3 grid((unsigned)a.batch, (unsigned)blocks_per_request(std::max(a.log_splits, a.log_groups)), 1);
+  if (a.log_groups > 0) hipLaunchKernelGGL((stage2_kernel<E, D, kLongLists>), grid, dim3(kBlock, 1, 1), 0, stream, a);
+  else if (a.log_splits > 0) hipLaunchKernelGGL((stage2_kernel<E, D, kSplitLists>), grid, dim3(kBlock, 1, 1), 0, stream, a);
+  else hipLaunchKernelGGL((stage2_kernel<E, D, kWholeLists>), grid, dim3(kBlock, 1, 1), 0, stream, a);
   return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
 }
 

@@ -1,5 +1,5 @@
 """The merge launch on its own: list lengths around its batches of eight rows and around the fourteen a record
-holds, with few requests (a list's parts merged over the waves of a block) and with many."""
+holds, with few requests (a list's parts merged over the waves of a block) and with many; lists over 64 entries."""
 
 import pytest
 import torch
@@ -15,8 +15,22 @@ LENGTHS = [0, 1, 7, 8, 9, 14, 15, 16, 17, 33, 70]
 @pytest.mark.parametrize("copies", [1, 40])
 def test_merge_of_lists_of_every_length(head_dim, heads, copies, dtype, device):
     print(f"\n[gpu case] merge {head_dim} x {heads}, {copies} copies, {dtype}", flush=True)
+    _check_merge(LENGTHS, copies, head_dim, heads, dtype, device)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("head_dim,heads", [(16, 6), (32, 5), (64, 24), (128, 9), (256, 3)])
+@pytest.mark.parametrize("lengths", [[65], [64, 63], [513, 0, 3], [66, 127, 128, 129, 15, 100], [1000, 20, 64] * 9], ids=len)
+def test_merge_of_long_lists(head_dim, heads, lengths, dtype, device):
+    """Lists of more than 64 entries, of which few requests' are cut for groups of lanes, beside shorter ones."""
+    print(f"\n[gpu case] merge {head_dim} x {heads}, {lengths[:6]}, {dtype}", flush=True)
+    _check_merge(lengths, 1, head_dim, heads, dtype, device)
+
+
+def _check_merge(lengths, copies, head_dim, heads, dtype, device):
     gen = torch.Generator().manual_seed(head_dim + copies)
-    lens = torch.tensor(LENGTHS * copies, dtype=torch.int32)
+    lens = torch.tensor(lengths * copies, dtype=torch.int32)
     rows = int(lens.sum())
     entries = torch.randperm(rows, generator=gen).to(torch.int32)
     offs = (torch.cumsum(lens, 0) - lens).to(torch.int32)
@@ -24,7 +38,7 @@ def test_merge_of_lists_of_every_length(head_dim, heads, copies, dtype, device):
     mid_lse = 6 * torch.randn(rows, heads, generator=gen)
     # rows that attended nothing: output 0, log-sum-exp -inf; for one request all of them
     mid_lse[torch.rand(rows, heads, generator=gen) < 0.1] = float("-inf")
-    nothing = len(LENGTHS) - 2
+    nothing = max(len(lengths) - 2, 0)
     mid_lse[entries[offs[nothing]: offs[nothing] + lens[nothing]].long()] = float("-inf")
     mid_o[mid_lse == float("-inf")] = 0
     o = torch.full((len(lens), heads, head_dim), float("nan"), dtype=dtype, device=device)

@@ -651,8 +651,8 @@ __device__ __forceinline__ void reset_state(WideState<D>& st) {
 }
 
 // The record of a block program (kProgRecord ints): entries 0..3 are kv_off, kv_len, q_off and q_len of the
-// program's first wide vnode, entry 4 says whether the rest is there (the vnode exists, fits one pass of a block
-// and has at most 128 requests), entries kProgRecRequests.. the requests of its scratch rows, entries
+// program's first wide vnode (if it has one, with or without the rest), entry 4 says whether the rest is there (the
+// vnode exists and has at most 128 requests), entries kProgRecRequests.. the requests of its scratch rows, entries
 // kProgRecSlots.. the pool slots of its first 64 tokens (the last token repeated past the end of a shorter run).
 // With it a block knows after one memory round trip what it otherwise learns in three (its table entry, the
 // vnode's list entries, the request and slot lists) before it can ask for query and K/V rows.
@@ -1162,7 +1162,7 @@ struct RecordRequests {
 // streams the run through a ring of two 64-token LDS buffers with direct global->LDS loads, one
 // super tile ahead of the one being consumed; the slot indices travel the same way, two super tiles further
 // ahead.  The caller has opened the run and requested the indices of its first super tiles, and its first rows
-// too if `started`; `requests`: those of the vnode's scratch rows, if `listed`.
+// too if `started`; `requests`: those of the vnode's scratch rows, if `started`.
 template <typename E, int D, int NG, bool GATHERED>
 __device__ __forceinline__ void wide_pass(const Stage1Args& a, char* smem, const VnodeView& vn, const WidePass& p, RowStream<D, GATHERED>& rows,
                                           bool started, const RecordRequests& requests) {

@@ -242,8 +242,8 @@ def program_records(kv_entries, kv_offs, kv_lens, q_offs, q_lens, q_entries, pro
     vnode, in one place, so that it can ask for query and K/V rows after one memory round trip
     (the record, fetched together with the table entry) instead of three (table entry, the
     vnode's list entries, its request and slot lists).  Entries: ``kv_off, kv_len, q_off, q_len`` of
-    vnode ``first + prog_table[p][0]``; a flag (1: the program has a wide vnode of at most 128 query
-    rows and the rest is filled in); from entry 8 the requests of its scratch rows; from entry 136
+    vnode ``first + prog_table[p][0]``, whatever the flag says; a flag (1: the program has a wide vnode of at
+    most 128 query rows and the rest is filled in); from entry 8 the requests of its scratch rows; from entry 136
     the pool slots of its first 64 tokens (the last token repeated past the end of a shorter run).
     Returns an int32 array ``[num_programs, 256]``."""
     prog_table = np.asarray(prog_table, dtype=np.int64).reshape(-1, 4)

@@ -143,8 +143,9 @@ int ft_decode(const void* q, const void* k, const void* v, void* o,
  * agree with the lists; they are trusted like them.
  *
  * prog_records (or NULL) holds one record of 256 int32 per program: entries 0..3 the kv_off, kv_len,
- * q_off and q_len of the program's first vnode of the first range; entry 4 is 1 when the rest is filled
- * in (the program has such a vnode and it has at most 128 query rows = q_len * group), else 0; entries
+ * q_off and q_len of the program's first vnode of the first range, whenever it has one and whatever
+ * entry 4 says; entry 4 is 1 when the rest is filled in, which takes such a vnode with at most 128 requests
+ * (q_len), else 0, and the rest is not used then; entries
  * 8..135 the requests of its scratch rows (vnode_to_q_entries[q_off ...]); entries 136..199 the pool slots
  * of its first 64 tokens (vnode_to_kv_entries[kv_off + min(t, kv_len - 1)]); the rest is padding.  A block
  * then asks for the query and K/V rows of its first vnode after one memory round trip (record and table

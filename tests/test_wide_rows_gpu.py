@@ -1,6 +1,7 @@
 """Row groups, token groups and tile remainders of the wide and narrow passes: the numbers of query rows
 and tokens at which a block changes how its waves share them (16-row groups, three or two of them per
-wave, one, two or four token groups, 64-token super tiles with a ring of two), in both list orders."""
+wave, one, two or four token groups, 64-token super tiles with a ring of two), in both list orders and from
+lists made by hand."""
 import math
 
 import pytest
@@ -103,3 +104,32 @@ def test_token_groups_round_their_own_probabilities(rows, d, dtype, device):
     # w and the sums are good to a few 2^-24 each; w rounded to 16 bits would be off by more than 2^-13, the result by
     # 2 / (1 + w)^2, at least half, of that
     assert float((got - (1 - w) / (1 + w)).abs().max()) < 2.0 ** -18
+
+
+@pytest.mark.parametrize("d,dtype", [(128, torch.float16), (64, torch.bfloat16), (256, torch.float16)])
+@pytest.mark.parametrize("rows", [5, 16, 17, 32, 48, 80])
+def test_partials_of_one_wide_vnode(rows, d, dtype, device):
+    """A wide phase of one vnode, from lists made by hand (the planner gives runs this short or narrow to other
+    phases): two token groups, at head_dim 256 four up to 16 rows, two up to 32, then one; at these lengths some of
+    them get no tile."""
+    print("\n[gpu case] one wide vnode", rows, d, dtype, flush=True)
+    heads = 2
+    gen = torch.Generator().manual_seed(rows)
+    i32 = lambda x: torch.as_tensor(x, dtype=torch.int32, device=device)  # noqa: E731
+    scale = 1.0 / math.sqrt(d)
+    for tokens in TOKENS:
+        q = torch.randn(rows, heads, d, generator=gen).to(dtype)
+        k, v = (torch.randn(400, heads, d, generator=gen).to(dtype) for _ in range(2))
+        slots = torch.randperm(400, generator=gen)[:tokens]
+        mid_o = torch.full((rows, heads, d), float("nan"), device=device)
+        mid_lse = torch.full((rows, heads), float("nan"), device=device)
+        fasttree_decode_stage1(q.to(device), k.to(device), v.to(device), i32(slots), i32([0]), i32([tokens]), i32(range(rows)), i32([0]),
+                               i32([rows]), scale, mid_o, mid_lse, [1, 0], [0, 1], [512, 16], [32, 32])
+        s = torch.einsum("rhd,thd->rht", q.double(), k[slots].double()) * scale
+        p = torch.softmax(s, -1)
+        want = torch.einsum("rht,thd->rhd", p, v[slots].double())
+        # a probability is rounded to 16 bits once: off by 2^-11 (2^-8) of itself, fp16's small ones by 2^-25 of the largest
+        spread = torch.einsum("rht,thd->rhd", p, v[slots].double().abs())
+        bound = 2.0 ** (-11 if dtype is torch.float16 else -8) * spread + 2.0 ** -25 * tokens * float(v.abs().max()) + 1e-5
+        assert bool(((mid_o.cpu().double() - want).abs() <= bound).all()), tokens
+        assert float((mid_lse.cpu().double() - torch.logsumexp(s, -1)).abs().max()) < 1e-4, tokens

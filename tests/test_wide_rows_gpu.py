@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from cases import build_tree
-from fasttree_hip.decode import fasttree_decode, fasttree_decode_stage1
+from fasttree_hip.decode import fasttree_decode, fasttree_decode_stage1, gathered_decode
 from fasttree_hip.inputs import make_decode_inputs
 from fasttree_hip.planner import FastTreeParams, fasttree_preparation
 from test_decode_gpu import _dense_check
@@ -133,3 +133,30 @@ def test_partials_of_one_wide_vnode(rows, d, dtype, device):
         bound = 2.0 ** (-11 if dtype is torch.float16 else -8) * spread + 2.0 ** -25 * tokens * float(v.abs().max()) + 1e-5
         assert bool(((mid_o.cpu().double() - want).abs() <= bound).all()), tokens
         assert float((mid_lse.cpu().double() - torch.logsumexp(s, -1)).abs().max()) < 1e-4, tokens
+
+
+@pytest.mark.parametrize("d,dtype", [(128, torch.float16), (64, torch.bfloat16), (256, torch.float16)])
+@pytest.mark.parametrize("group", [17, 32, 33, 48, 64])
+def test_gathered_decode_of_large_groups(group, d, dtype, device):
+    """Gathered caches with more than 16 query heads per KV head, which are wide vnodes there: two token groups with a row
+    group per wave and with two, whole runs and splits of 8 tokens, most of them empty, whose lists of 88 entries the
+    merge cuts for groups of lanes."""
+    print("\n[gpu case] gathered, large groups", group, d, dtype, flush=True)
+    heads, lens = 2, [700, 1, 131]
+    gen = torch.Generator().manual_seed(group)
+    scale = 1.0 / math.sqrt(d)
+    q = torch.randn(len(lens), group * heads, d, generator=gen).to(dtype)
+    k, v = (torch.randn(len(lens), max(lens), heads, d, generator=gen).to(dtype) for _ in range(2))
+    for kv_split in (8, 700):
+        o = torch.full_like(q, float("nan"), device=device)
+        gathered_decode(q.to(device), k.to(device), v.to(device), torch.tensor(lens, dtype=torch.int32, device=device), o, scale,
+                        kv_split=kv_split)
+        got = o.cpu().double()
+        for r, n in enumerate(lens):
+            kr, vr = (x[r, :n].double().repeat_interleave(group, dim=1) for x in (k, v))
+            p = torch.softmax(torch.einsum("hd,thd->ht", q[r].double(), kr) * scale, -1)
+            want = torch.einsum("ht,thd->hd", p, vr)
+            # a probability is rounded to 16 bits once, as in the test above, and so is the result
+            eps = 2.0 ** (-11 if dtype is torch.float16 else -8)
+            bound = eps * (torch.einsum("ht,thd->hd", p, vr.abs()) + want.abs()) + 2.0 ** -25 * n * float(vr.abs().max()) + 1e-5
+            assert bool(((got[r] - want).abs() <= bound).all()), (kv_split, r)

@@ -405,7 +405,7 @@ __device__ __forceinline__ void tile_step(const char* ldsK, const char* ldsV, in
 
 // One wave attends NQB*16 query rows to tokens [tile0*32, ...) in steps of tile_step_n tiles,
 // staging each tile in its own LDS area.  Rows travel global -> registers -> LDS; the next tile
-// is in flight while a tile is consumed.  (Used for head_dim 256 only.)
+// is in flight while a tile is consumed.  (Used for head_dim 16 only, as a zero-padded 32.)
 template <typename E, int D, int NQB, bool GATHERED>
 __device__ __forceinline__ void wave_attend(const Stage1Args& a, const VnodeView& vn, int kvh, int row0,
                                             int tile0, int tile_step_n, char* lds, WaveState<D, NQB>& st) {
@@ -579,12 +579,12 @@ __global__ void __launch_bounds__(kBlock) stage1_kernel(Stage1Args a) {
 // SIMD and one wave's waits are filled by the other's instructions.
 //
 // What bounds a launch is the start, the waits and the end of its blocks, with the matrix pipes far
-// from full: 1.10 PFLOP/s where two blocks of 192 rows on each unit read one run of 8192 tokens (the
-// pipes busy 49 % of the cycles at 2133 MHz; a large library matrix product reaches 1.21), and .55
-// in a decode step of 128 requests, whose blocks run for some 30 steps (22 %, 2575 MHz).  48 query
+// from full: 1.07 PFLOP/s where two blocks of 192 rows on each unit read one run of 8192 tokens (the
+// pipes busy 49 % of the cycles at 2090 MHz; a large library matrix product reaches 1.21), and .60
+// in a decode step of 400 requests, whose blocks run for some 30 steps (24 %, 2633 MHz).  48 query
 // rows per wave read a K or V operand from LDS once for three row groups and spread a tile's loads
-// and barrier over 1.5 times the rows: a step of 96 rows takes .53 us against .69 with 32x32x16
-// instructions and 32 rows per wave, 192 rows .87 (head_dim 128, 8 runs of 8 heads).
+// and barrier over 1.5 times the rows: a step of 96 rows takes .52 us against .69 with 32x32x16
+// instructions and 32 rows per wave, 192 rows .86 (head_dim 128, 8 runs of 8 heads).
 // 48 rows take 96 accumulator and 48 query registers of the 256 a wave has.
 // ---------------------------------------------------------------------------------------
 constexpr int kWideWaves = 4;
@@ -1859,9 +1859,9 @@ constexpr int kLists = 0, kPrograms = 1, kEmbedding = 2;
 // rank-major, then row chunk, kv head fastest (blocks that stream the same KV run are launched together and share it
 // in L2); the narrow blocks follow and fill the machine while the wide blocks drain.
 // Waves per SIMD that the registers must leave room for: as many blocks per compute unit as its LDS holds of
-// 512-byte rows (one) and 256-byte rows (two).  Below that three fit the 168 registers that the kernel takes by
-// itself, or a few more: for the planner's lists they are kept to (534 requests of 32/8 heads of 64: 102.6 us with
-// 168, 110.4 with 171); under that limit programs come out slower.
+// 512-byte rows (one) and 256-byte rows (two).  Below that three have 168 registers each, and the
+// kernels take 155 to 160: for the planner's lists they are kept to that (534 requests of 32/8 heads of 64: 102.6 us with
+// 168, 110.4 with the 171 that an earlier form took by itself); programs came out slower under the limit.
 constexpr int fused_waves(int D, int mode) { return D > 128 ? 1 : D == 128 || mode != kLists ? 2 : 3; }
 template <typename E, int D, bool GATHERED, int MODE>
 __device__ __forceinline__ void fused_block(const Stage1Args& a, char* smem) {
@@ -2454,7 +2454,7 @@ int launch_stage1_narrow(const Stage1Args& a0, hipStream_t stream) {
 template <typename E, int D, bool GATHERED, bool STAGED = false>
 int launch_stage1_d(const Stage1Args& a, hipStream_t stream) {
   if constexpr (STAGED) {
-    // 128-token double buffers of 512-byte rows do not fit in LDS: per-wave staging kernels
+    // head_dim 16: rows half as long as a 32-dim contraction's, padded with zeros on their way through registers
     if (a.vnode_count > 0)
       if (int rc = launch_stage1_inst<E, D, 2, true, GATHERED>(a, a.hkv, stream)) return rc;
     if (a.narrow_count > 0) {

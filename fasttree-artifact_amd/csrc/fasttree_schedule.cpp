@@ -42,13 +42,15 @@ constexpr int kXcds = 8;
 // ---- the model (microseconds; measured on the shapes of the kernel's own loop, rows resident in L2)
 
 // One 32-token step of a block that has its compute unit to itself, by 16-row groups of the piece.
-// head_dim 128, rows in L2: 16 and 32 rows .37, 48 and 64 rows .43, 96 rows .53, 128 rows .68, 192 rows .87.  The
+// head_dim 128, rows in L2: 20 and 32 rows .35, 48 and 64 rows .42, 80 and 96 rows .52, 128 rows .67, 192 rows .86
+// (.36, .43, .53, .69 and .88 on the kernel that the table was set with).  The
 // entries for 32 and 48 rows are those of a kernel that split their tokens four ways (.42 and .51): with the
-// present figures in their place trees of 64/8 heads are cut finer and take 3 to 4 % longer (26.3 -> 27.5, 35.2 ->
+// figures measured since in their place trees of 64/8 heads are cut finer and took 3 to 4 % longer (26.3 -> 27.5, 35.2 ->
 // 36.2 and 132 -> 136 us), so short pieces of few rows cost more than their steps.  The entries above 128 rows are
-// an eighth longer than a block alone takes, since it is beside another one that pieces of 192 rows fall behind:
-// two such blocks on a unit take 1.71 times one's time a step, two of 128 rows 1.51 (1.39 and .96 us; .81 and .64
-// alone), 1.44 times as long as 128 rows as in this table.  Other head sizes: measured on full chunks.
+// an eighth longer than a block alone takes: beside another block pieces of 192 rows fall behind.  In calls one at a
+// time two such blocks on a unit took 1.71 times one's time a step, two of 128 rows 1.51 (1.39 and .96 us; .81 and .64
+// alone), 1.44 times as long as 128 rows as in this table; in a queue of calls, on the present kernel, 1.54 and 1.44
+// (1.34 and 1.03 us; .87 and .72 alone).  Other head sizes: measured on full chunks.
 // The blocks of a run lie on one XCD and share it in its L2 where the KV heads divide evenly over the
 // XCDs; otherwise every XCD reads it, and a step of few rows lasts as long as its loads.
 double step_us(int groups, int head_dim, int heads) {

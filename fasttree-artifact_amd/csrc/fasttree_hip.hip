@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <atomic>
 #include <stdint.h>
+#include <type_traits>
 
 #include "../../include/fasttree_hip.h"
 
@@ -2085,6 +2086,10 @@ constexpr int kReqRecEntries = kReqRecord - 2;
 // but those of more than kLongList entries by groups of lanes.
 constexpr int kWholeLists = 0, kSplitLists = 1, kLongLists = 2;
 constexpr int kLongList = 64;
+// Rows a wave asks for at once.  A list of more is cut where the machine has room for the waves: the second batch is a memory
+// round trip, the merge through LDS less (16 requests of 32/32 heads with 9 rows each, whole calls: 14.2 us in two batches, 13.8
+// by four waves).
+constexpr int kOneWave = 8;
 
 // The merge of a list of more than kLongList entries, n of them, from `list` on (or the rows from row0 on).  Four waves
 // would read it in many batches, one round trip after the other, so it is cut finer: a group of D/4 lanes takes a part for
@@ -2169,56 +2174,127 @@ __device__ __forceinline__ void merge_long_list(const Stage2Args& a, int req, in
   *reinterpret_cast<u32x2*>(a.o + 2 * ((int64_t)req * a.oo0 + (int64_t)head * a.oo1 + 4 * gl)) = out;
 }
 
-// D/4 lanes serve one (request, head), a wave several heads of one request; `splits` waves of a block (1, 2 or 4) take
-// parts of the request's list and are merged through LDS.  A wave reads the list of its request as scalars (from the
-// request's record with its length and offset, else from the list), so a lane asks for its four output dims of eight
-// partial rows, and for their log-sum-exps, with nothing but its own address and a scalar.
+// How the merge kernel spreads a request's heads: a lane holds kVec output dims of one head, and a head has whole rows of
+// 16 lanes, so that what such a row's lanes hold of a list can be handed round inside it.
+template <int D> struct MergeGeom {
+  static constexpr int kVec = D >= 64 ? 4 : D / 16;
+  static constexpr int kLanes = D / kVec;                   // lanes of a head: 16, 32 or 64
+  static constexpr int kHeads = kWave / kLanes;             // heads of a wave
+  typedef float Vec __attribute__((ext_vector_type(kVec)));
+};
+constexpr int kListRow = 16;                                // entries of a list that a row of lanes holds at a time
+
+// x of lane J of this lane's row of 16 lanes.
+template <int J> __device__ __forceinline__ int row_lane(int x) { return __builtin_amdgcn_mov_dpp(x, 0x150 + J, 0xf, 0xf, true); }
+// x of the lane N places on in this lane's row of 16, around its end.
+template <int N> __device__ __forceinline__ float row_turned(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x120 + N, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row_max(float x) {
+  x = fmaxf(x, row_turned<8>(x));
+  x = fmaxf(x, row_turned<4>(x));
+  x = fmaxf(x, row_turned<2>(x));
+  return fmaxf(x, row_turned<1>(x));
+}
+__device__ __forceinline__ float row_sum(float x) {
+  x += row_turned<8>(x);
+  x += row_turned<4>(x);
+  x += row_turned<2>(x);
+  return x + row_turned<1>(x);
+}
+
+// The N entries from J0 on of the 16 that the rows of lanes hold: their partial rows are asked for, all of them before
+// the first is used, and added with their weights.
+template <int D, int J0, int N> struct MergeBatch {
+  using G = MergeGeom<D>;
+  typedef typename G::Vec Vec;
+  Vec part[N];
+
+  // (`off`: of the row of the lane's entry, in bytes)
+  template <int J = 0> __device__ __forceinline__ void request(const char* o_lane, uint64_t off) {
+    const uint64_t base = (uint64_t)(uintptr_t)o_lane;
+    unsigned carry, none;
+    const unsigned lo = __builtin_addc((unsigned)base, (unsigned)row_lane<J0 + J>((int)(unsigned)off), 0u, &carry);
+    const unsigned hi = __builtin_addc((unsigned)(base >> 32), (unsigned)row_lane<J0 + J>((int)(unsigned)(off >> 32)), carry, &none);
+    part[J] = *reinterpret_cast<const __attribute__((address_space(1))) Vec*>((uintptr_t)(((uint64_t)hi << 32) | lo));
+    if constexpr (J + 1 < N) request<J + 1>(o_lane, off);
+  }
+  // What the row of an entry of no weight holds is not looked at: it may have attended no token.
+  template <int J = 0> __device__ __forceinline__ void forget_weightless(float w) {
+    const bool none = __builtin_bit_cast(float, row_lane<J0 + J>(__builtin_bit_cast(int, w))) == 0.f;
+#pragma unroll
+    for (int e = 0; e < G::kVec; ++e) part[J][e] = none ? 0.f : part[J][e];
+    if constexpr (J + 1 < N) forget_weightless<J + 1>(w);
+  }
+  template <int J = 0> __device__ __forceinline__ void add(float w, Vec& acc) const {
+    const float w_j = __builtin_bit_cast(float, row_lane<J0 + J>(__builtin_bit_cast(int, w)));
+#pragma unroll
+    for (int e = 0; e < G::kVec; ++e) acc[e] = __builtin_fmaf(w_j, part[J][e], acc[e]);
+    if constexpr (J + 1 < N) add<J + 1>(w, acc);
+  }
+};
+
+// f with n, 1 to 8, as a constant.  (Code for each: a branch per entry and row takes as many instructions as the entry.)
+template <typename F> __device__ __forceinline__ void with_count(int n, F f) {
+#define FT_COUNT(k) f(std::integral_constant<int, k>())
+  if (n <= 4) {
+    if (n <= 2) { if (n == 1) FT_COUNT(1); else FT_COUNT(2); }
+    else { if (n == 3) FT_COUNT(3); else FT_COUNT(4); }
+  } else {
+    if (n <= 6) { if (n == 5) FT_COUNT(5); else FT_COUNT(6); }
+    else { if (n == 7) FT_COUNT(7); else FT_COUNT(8); }
+  }
+#undef FT_COUNT
+}
+
+// `splits` waves of a block (1, 2 or 4) take parts of the request's list and are merged through LDS.  Lane i of every row
+// of 16 lanes holds entry i of (16 entries of) the wave's part: its row's offset, its log-sum-exp for the row's head, its
+// weight.  A lane then asks for its output dims of every entry's row with the offset of the lane that holds it.
 //
-// Bound by the partial rows it reads, and for a batch of few requests by how many of them are in flight (8 requests x
-// 64 heads with 68 partials each: 64 blocks of whole lists 11.5 us, in eight parts each 6.7) and by the fetch of its instructions, 2.7 KB where a
-// list spread over lanes and handed round by shuffles took 4.0 (whole calls: 4 requests of a short prompt 9.1 -> 8.4 us,
-// 111 ragged requests of 64-dim heads 13.6 -> 12.7, 16/1 heads of 256 18.2 -> 17.4, the 400-request tree 61.9 -> 61.0).
+// Bound by the partial rows it reads in large launches (33 MB of the 400-request tree in 6.9 us), and in small ones by
+// the instructions a wave issues one after the other, some 4.6 cycles each, and by how many rows are in flight.  With a
+// list's entries as scalars, each with its own 64-bit address arithmetic, exponential and weight for the whole wave, and
+// batches of eight rows whatever the list's length, a wave took 453 instructions for lists of three; 230 so (whole calls: 4 requests
+// of a short prompt 7.96 -> 7.62 us, 16 of 32/32 heads 14.17 -> 13.54, 64 on a shared prefix 25.4 -> 24.6, 111 ragged requests
+// of 64-dim heads 12.55 -> 12.4, 64 of 16/1 heads of 256 17.44 -> 17.18).
 template <typename E, int D, int LISTS>
 __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
+  using G = MergeGeom<D>;
+  typedef typename G::Vec Vec;
   constexpr bool SPLIT = LISTS != kWholeLists;
-  constexpr int LPH = D / 4;
-  constexpr int HPW = kWave / LPH;                          // heads of a wave
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int gl = lane % LPH;
+  const int gl = lane % G::kLanes, c = lane % kListRow;
   const int req = blockIdx.x;
   const int log_splits = SPLIT ? a.log_splits : 0;          // launch uniform
-  const int head = ((((int)blockIdx.y * kWavesPerBlock) + wave) >> log_splits) * HPW + lane / LPH;
+  const int head = ((((int)blockIdx.y * kWavesPerBlock) + wave) >> log_splits) * G::kHeads + lane / G::kLanes;
   const bool exists = head < a.hq;
   const int head_in = exists ? head : a.hq - 1;             // (lanes past the last head read that one's rows and store nothing)
   // this wave's part [first, first + n) of the request's list, from `list` on
-  int n, first = 0, row0 = 0;
-  PlanInts list = nullptr;
-  constexpr int kBatch = 8;
-  int row[kBatch];
+  int n, first = 0, row0 = 0, recorded = 0;
+  bool in_record = false;                                   // block uniform: the list is in the request's record
+  const int32_t* list = nullptr;
   if (a.nsplit > 0) {
     n = a.nsplit;
     row0 = req * a.nsplit;
   } else if (a.req_table) {                                 // launch uniform
-    const PlanInts rec = plan_ints(a.req_table) + (int64_t)req * kReqRecord;
-    n = rec[0];
-    const int off = rec[1];
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) row[j] = rec[2 + j];
-    list = n <= kReqRecEntries ? rec + 2 : plan_ints(a.req_entries) + off;
+    const int32_t* rec = a.req_table + (int64_t)req * kReqRecord;
+    recorded = rec[2 + min(c, kReqRecEntries - 1)];         // (in one round trip with the length)
+    n = plan_ints(rec)[0];
+    list = a.req_entries + plan_ints(rec)[1];
+    in_record = n <= kReqRecEntries;
   } else {
     n = plan_ints(a.req_lens)[req];
-    list = plan_ints(a.req_entries) + plan_ints(a.req_offs)[req];
+    list = a.req_entries + plan_ints(a.req_offs)[req];
   }
   if constexpr (LISTS == kLongLists) {
-    if (n > kLongList) return merge_long_list<E, D>(a, req, n, row0, list);
+    if (n > kLongList) return merge_long_list<E, D>(a, req, n, row0, plan_ints(list));
     // (the grid has the blocks that the one way or the other needs)
-    if ((((int)blockIdx.y * kWavesPerBlock) >> log_splits) * HPW >= a.hq) return;
+    if ((((int)blockIdx.y * kWavesPerBlock) >> log_splits) * G::kHeads >= a.hq) return;
   }
   int split = 0, splits = 1;
   if constexpr (SPLIT) {
-    // (a short list is one wave's work: merging costs about 1 us)
     split = wave & ((1 << log_splits) - 1);
-    if (n <= kReqRecEntries) {
+    if (n <= kOneWave) {
       if (split > 0) return;
     } else {
       splits = 1 << log_splits;
@@ -2227,50 +2303,57 @@ __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
       n = max(0, min(n - first, part));
     }
   }
-  const bool in_record = a.nsplit == 0 && a.req_table != nullptr && first == 0;   // the first batch's rows are in `row`
 
-  const char* o_lane = reinterpret_cast<const char*>(a.mid_o + (int64_t)head_in * a.so1 + 4 * gl);
+  // (rows and heads as numbers without sign: a product with a 64-bit stride is two instructions)
+  const char* o_lane = reinterpret_cast<const char*>(a.mid_o) + ((uint64_t)(unsigned)head_in * (uint64_t)(4 * a.so1) + 4 * G::kVec * gl);
   const char* lse_lane = reinterpret_cast<const char*>(a.mid_lse + head_in);
   float m_run = -INFINITY, l_run = 0.f;
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int i0 = 0; i0 < n; i0 += kBatch) {
-    // rows of this batch; past the end the first one again (a zero weight discards what is read of it)
-    if (a.nsplit > 0) {
-#pragma unroll
-      for (int j = 0; j < kBatch; ++j) row[j] = row0 + first + i0 + j;
-    } else if (i0 > 0 || !in_record) {
-#pragma unroll
-      for (int j = 0; j < kBatch; ++j) row[j] = list[first + min(i0 + j, n - 1)];
+  Vec acc = {};
+  for (int i0 = 0; i0 < n; i0 += kListRow) {
+    int held = n - i0;
+    asm volatile("" : "+s"(held));     // (or what every count below makes of it is computed ahead of the loop)
+    // (lanes past the part hold an entry of it that has no weight there)
+    int row;
+    if (in_record) {
+      row = SPLIT && first > 0 ? lane_value(recorded, lane - c + ((first + c) & (kListRow - 1))) : recorded;
+      row = c < held ? row : row_lane<0>(row);
+    } else {
+      const int i = first + i0 + min(c, held - 1);
+      row = a.nsplit > 0 ? row0 + i : list[i];
     }
-    float lse[kBatch];
-    f32x4 part[kBatch];
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const int64_t r = i0 + j < n ? row[j] : row[0];
-      lse[j] = *reinterpret_cast<const float*>(lse_lane + 4 * r * a.sl0);
-      part[j] = *reinterpret_cast<const f32x4*>(o_lane + 4 * r * a.so0);
-    }
-    float m_new = m_run;
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      lse[j] = i0 + j < n ? lse[j] : -INFINITY;
-      m_new = fmaxf(m_new, lse[j]);
-    }
-    const float keep = (m_run == -INFINITY) ? 0.f : __expf(m_run - m_new);
-    l_run *= keep;
-    acc *= keep;
-    m_run = m_new;
-#pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const float w = (lse[j] == -INFINITY) ? 0.f : __expf(lse[j] - m_new);
-      l_run += w;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] += (w != 0.f) ? part[j][e] * w : 0.f;
-    }
+    float lse = *reinterpret_cast<const float*>(lse_lane + (uint64_t)(unsigned)row * (uint64_t)(4 * a.sl0));
+    const uint64_t off = (uint64_t)(unsigned)row * (uint64_t)(4 * a.so0);
+    float w;
+    bool zeros;
+    with_count(min(held, 8), [&](auto count) {
+      MergeBatch<D, 0, count()> rows;
+      rows.request(o_lane, off);
+      lse = c < held ? lse : -INFINITY;
+      const float m_new = fmaxf(m_run, row_max(lse));
+      const float m_from = m_new == -INFINITY ? 0.f : m_new;  // (every log-sum-exp so far is -inf: every weight is 0)
+      w = __expf(lse - m_from);
+      zeros = __builtin_amdgcn_ballot_w64(c < held && w == 0.f) != 0;
+      if (i0 > 0) {
+        const float keep = __expf(m_run - m_from);
+        l_run *= keep;
+        acc = keep == 0.f ? Vec{} : acc * keep;
+      }
+      l_run += row_sum(w);
+      m_run = m_new;
+      if (zeros) rows.forget_weightless(w);
+      rows.add(w, acc);
+    });
+    if (held > 8)
+      with_count(min(held - 8, 8), [&](auto count) {
+        MergeBatch<D, 8, count()> rows;
+        rows.request(o_lane, off);
+        if (zeros) rows.forget_weightless(w);
+        rows.add(w, acc);
+      });
   }
   if (SPLIT && splits > 1) {
     // the waves' states to the first of them
-    __shared__ f32x4 acc_of[kBlock];
+    __shared__ Vec acc_of[kBlock];
     __shared__ float m_of[kBlock], l_of[kBlock];
     acc_of[threadIdx.x] = acc;
     m_of[threadIdx.x] = m_run;
@@ -2279,19 +2362,22 @@ __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
     if (split > 0) return;
     float m_all = m_run;
     for (int i = 1; i < splits; ++i) m_all = fmaxf(m_all, m_of[threadIdx.x + i * kWave]);
-    acc = f32x4{0.f, 0.f, 0.f, 0.f};
+    acc = Vec{};
     l_run = 0.f;
     for (int i = 0; i < splits; ++i) {
       const float m_i = m_of[threadIdx.x + i * kWave];
       const float w = (m_i == -INFINITY) ? 0.f : __expf(m_i - m_all);
       l_run += l_of[threadIdx.x + i * kWave] * w;
-      acc += acc_of[threadIdx.x + i * kWave] * w;
+      acc = w == 0.f ? acc : acc + acc_of[threadIdx.x + i * kWave] * w;
     }
   }
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
   acc *= inv;
-  u32x2 out = {E::pack2(acc[0], acc[1]), E::pack2(acc[2], acc[3])};
-  if (exists) *reinterpret_cast<u32x2*>(a.o + 2 * ((int64_t)req * a.oo0 + (int64_t)head * a.oo1 + 4 * gl)) = out;
+  if (!exists) return;
+  char* out = a.o + 2 * ((int64_t)req * a.oo0 + (int64_t)head * a.oo1 + G::kVec * gl);
+  if constexpr (G::kVec == 4) *reinterpret_cast<u32x2*>(out) = u32x2{E::pack2(acc[0], acc[1]), E::pack2(acc[2], acc[3])};
+  else if constexpr (G::kVec == 2) *reinterpret_cast<unsigned*>(out) = E::pack2(acc[0], acc[1]);
+  else *reinterpret_cast<unsigned short*>(out) = (unsigned short)E::pack2(acc[0], 0.f);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2501,16 +2587,18 @@ int launch_stage1(const Stage1Args& a, int d, int dtype, hipStream_t stream) {
 // entries: 38.6 and 41.5; of 32 heads of 32: 28.4 and 30.2); 512-byte rows are a wave's in either case.
 template <typename E, int D>
 int launch_stage2_inst(const Stage2Args& a0, hipStream_t stream) {
-  constexpr int kHeads = kWavesPerBlock * kWave / (D / 4);   // of a block whose waves share no list
+  constexpr int kHeads = kWavesPerBlock * MergeGeom<D>::kHeads;   // of a block whose waves share no list
+  constexpr int kLaneGroups = kBlock / (D / 4);                   // of a block, for long lists
   Stage2Args a = a0;
+  auto blocks_per_request = [&](int per_block, int log_parts) { return ((int64_t)(a.hq << log_parts) + per_block - 1) / per_block; };
+  auto room = [&](int per_block, int log_parts) { return a.batch * blocks_per_request(per_block, log_parts) <= wave_slots() / 4; };
   a.log_splits = 0;
-  auto blocks_per_request = [&](int log_splits) { return ((int64_t)(a.hq << log_splits) + kHeads - 1) / kHeads; };
-  while (a.longest > kReqRecEntries && (1 << a.log_splits) < kWavesPerBlock && a.batch * blocks_per_request(a.log_splits + 1) <= wave_slots() / 4) ++a.log_splits;
+  while (a.longest > kOneWave && (1 << a.log_splits) < kWavesPerBlock && room(kHeads, a.log_splits + 1)) ++a.log_splits;
   a.log_groups = 0;
-  while (a.longest > kLongList && (1 << a.log_groups) < kHeads && a.batch * blocks_per_request(a.log_groups + 1) <= wave_slots() / 4) ++a.log_groups;
+  while (a.longest > kLongList && (1 << a.log_groups) < kLaneGroups && room(kLaneGroups, a.log_groups + 1)) ++a.log_groups;
   constexpr int kLeast = D <= 32 ? 16 : D <= 128 ? 8 : 4;
   if ((1 << a.log_groups) < kLeast) a.log_groups = 0;
-  const dim3 grid((unsigned)a.batch, (unsigned)blocks_per_request(std::max(a.log_splits, a.log_groups)), 1);
+  const dim3 grid((unsigned)a.batch, (unsigned)std::max(blocks_per_request(kHeads, a.log_splits), a.log_groups ? blocks_per_request(kLaneGroups, a.log_groups) : 0), 1);
   if (a.log_groups > 0) hipLaunchKernelGGL((stage2_kernel<E, D, kLongLists>), grid, dim3(kBlock, 1, 1), 0, stream, a);
   else if (a.log_splits > 0) hipLaunchKernelGGL((stage2_kernel<E, D, kSplitLists>), grid, dim3(kBlock, 1, 1), 0, stream, a);
   else hipLaunchKernelGGL((stage2_kernel<E, D, kWholeLists>), grid, dim3(kBlock, 1, 1), 0, stream, a);

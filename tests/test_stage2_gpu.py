@@ -28,7 +28,17 @@ def test_merge_of_long_lists(head_dim, heads, lengths, dtype, device):
     _check_merge(lengths, 1, head_dim, heads, dtype, device)
 
 
-def _check_merge(lengths, copies, head_dim, heads, dtype, device):
+@pytest.mark.gpu
+@pytest.mark.parametrize("head_dim,heads", [(16, 6), (32, 5), (64, 24), (128, 9), (256, 3)])
+@pytest.mark.parametrize("copies", [1, 40])
+def test_rows_without_weight_are_not_looked_at(head_dim, heads, copies, device):
+    """Every count of rows up to one past the sixteen that a row of lanes holds, the rows of log-sum-exp -inf (and those
+    so far below the rest that their weight is 0) holding NaN and infinities."""
+    print(f"\n[gpu case] merge without weight {head_dim} x {heads}, {copies} copies", flush=True)
+    _check_merge(list(range(1, 18)), copies, head_dim, heads, torch.float16, device, unseen=True)
+
+
+def _check_merge(lengths, copies, head_dim, heads, dtype, device, unseen=False):
     gen = torch.Generator().manual_seed(head_dim + copies)
     lens = torch.tensor(lengths * copies, dtype=torch.int32)
     rows = int(lens.sum())
@@ -41,8 +51,21 @@ def _check_merge(lengths, copies, head_dim, heads, dtype, device):
     nothing = max(len(lengths) - 2, 0)
     mid_lse[entries[offs[nothing]: offs[nothing] + lens[nothing]].long()] = float("-inf")
     mid_o[mid_lse == float("-inf")] = 0
+    given_o, given_lse = mid_o, mid_lse
+    if unseen:
+        # (exp of less than -104 is 0 in fp32, subnormal numbers included)
+        given_lse, given_o = mid_lse.clone(), mid_o.clone()
+        given_lse[(mid_lse == float("-inf")) & (torch.rand(rows, heads, generator=gen) < 0.3)] = -1e4
+        odd = torch.tensor([float("nan"), float("inf"), float("-inf")])
+        given_o[mid_lse == float("-inf")] = odd[torch.randint(3, given_o.shape, generator=gen)][mid_lse == float("-inf")]
+        alone = given_lse.clone()
+        for off, n in zip(offs.tolist(), lens.tolist()):        # where no row of a list has weight they would be the maximum
+            at = entries[off: off + n].long()
+            none = (mid_lse[at] == float("-inf")).all(0)
+            alone[at] = torch.where(none, float("-inf"), given_lse[at])
+        given_lse = alone
     o = torch.full((len(lens), heads, head_dim), float("nan"), dtype=dtype, device=device)
-    fasttree_decode_stage2(entries.to(device), offs.to(device), lens.to(device), mid_o.to(device), mid_lse.to(device), o)
+    fasttree_decode_stage2(entries.to(device), offs.to(device), lens.to(device), given_o.to(device), given_lse.to(device), o)
     o = o.cpu().double()
     # rounding to a significand of 11 (fp16) or 8 (bf16) bits is off by at most 2^-11 or 2^-8 of the value; the weights
     # are good to 1e-5; fp16's smallest step is 2^-24

@@ -2393,23 +2393,24 @@ struct StoreArgs {
   char* v_pool;
   int64_t sk0, sk1, sv0, sv1;
   int64_t num_slots;
-  int tokens, hkv, chunks;     // chunks = 16-byte pieces per (token, head) row
+  int hkv, chunks;             // chunks = 16-byte pieces per (token, head) row
+  Divisor by_chunks;
 };
 
-// One thread moves 16 bytes of a K row and the same 16 bytes of the V row.  A token whose slot
-// lies outside the pool is skipped.
-__global__ void __launch_bounds__(256) store_kv_kernel(StoreArgs a) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int per_token = a.hkv * a.chunks;
-  const int64_t token = i / per_token;
-  if (token >= a.tokens) return;
-  const int rest = (int)(i - token * per_token);
-  const int head = rest / a.chunks, chunk = rest - head * a.chunks;
-  const int64_t slot = a.loc_is_int64 ? static_cast<const int64_t*>(a.loc)[token]
-                                      : (int64_t) static_cast<const int32_t*>(a.loc)[token];
-  if (slot < 0 || slot >= a.num_slots) return;
+// A block serves one token (or, of many heads, a part of it), a thread 16 bytes of its K row and the same 16 bytes of
+// its V row.  A token whose slot lies outside the pool is skipped.  Bound by memory round trips and by the translation of
+// addresses in pools that nothing has touched since the last forward: the rows are asked for beside the slot.
+constexpr int kStoreBlock = 256;
+__global__ void __launch_bounds__(kStoreBlock) store_kv_kernel(StoreArgs a) {
+  const int token = blockIdx.x, i = blockIdx.y * blockDim.x + threadIdx.x;
+  if (i >= a.hkv * a.chunks) return;
+  const int head = a.by_chunks(i), chunk = i - head * a.chunks;
   const u32x4 kx = *reinterpret_cast<const u32x4*>(a.k_new + 2 * (token * a.kn0 + head * a.kn1) + 16 * chunk);
   const u32x4 vx = *reinterpret_cast<const u32x4*>(a.v_new + 2 * (token * a.vn0 + head * a.vn1) + 16 * chunk);
+  const PlanInts loc = plan_ints(static_cast<const int32_t*>(a.loc));
+  const int64_t slot = a.loc_is_int64 ? (int64_t)(((uint64_t)(unsigned)loc[2 * (int64_t)token + 1] << 32) | (unsigned)loc[2 * (int64_t)token])
+                                      : (int64_t)loc[token];
+  if (slot < 0 || slot >= a.num_slots) return;
   *reinterpret_cast<u32x4*>(a.k_pool + 2 * (slot * a.sk0 + head * a.sk1) + 16 * chunk) = kx;
   *reinterpret_cast<u32x4*>(a.v_pool + 2 * (slot * a.sv0 + head * a.sv1) + 16 * chunk) = vx;
 }
@@ -3100,11 +3101,11 @@ int ft_store_kv(const void* k_new, const void* v_new, int64_t kn0, int64_t kn1, 
   a.loc = out_cache_loc; a.loc_is_int64 = loc_is_int64 ? 1 : 0;
   a.k_pool = static_cast<char*>(k_pool); a.v_pool = static_cast<char*>(v_pool);
   a.sk0 = sk0; a.sk1 = sk1; a.sv0 = sv0; a.sv1 = sv1;
-  a.num_slots = num_slots; a.tokens = num_tokens; a.hkv = num_kv_heads; a.chunks = head_dim / 8;
-  const int64_t threads = (int64_t)num_tokens * num_kv_heads * a.chunks;
-  const int64_t blocks = (threads + 255) / 256;
-  if (blocks > INT32_MAX) return FT_ERR_ARGUMENT;
-  hipLaunchKernelGGL(store_kv_kernel, dim3((unsigned)blocks, 1, 1), dim3(256, 1, 1), 0, stream, a);
+  a.num_slots = num_slots; a.hkv = num_kv_heads; a.chunks = head_dim / 8;
+  a.by_chunks = divisor(a.chunks);
+  const int pieces = num_kv_heads * a.chunks, threads = std::min(kStoreBlock, (pieces + kWave - 1) / kWave * kWave);
+  hipLaunchKernelGGL(store_kv_kernel, dim3((unsigned)num_tokens, (unsigned)((pieces + threads - 1) / threads), 1), dim3((unsigned)threads, 1, 1), 0,
+                     stream, a);
   return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
 }
 

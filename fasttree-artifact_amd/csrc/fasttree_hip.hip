@@ -56,6 +56,12 @@ struct F16 {
     h2 v = {(_Float16)lo, (_Float16)hi};
     return __builtin_bit_cast(unsigned, v);
   }
+  // what packing lo and hi rounded off, packed
+  static __device__ __forceinline__ unsigned pack2_rest(float lo, float hi, unsigned packed) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const h2 v = __builtin_bit_cast(h2, packed);
+    return pack2(__builtin_fmaf((float)v[0], -1.f, lo), __builtin_fmaf((float)v[1], -1.f, hi));   // (one mixed instruction each)
+  }
   // acc + lo + hi of a packed pair, in fp32
   static __device__ __forceinline__ float add_pair(unsigned packed, float acc) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -74,6 +80,10 @@ struct BF16 {
     typedef __bf16 b2 __attribute__((ext_vector_type(2)));
     b2 v = {(__bf16)lo, (__bf16)hi};
     return __builtin_bit_cast(unsigned, v);
+  }
+  // what packing lo and hi rounded off, packed
+  static __device__ __forceinline__ unsigned pack2_rest(float lo, float hi, unsigned packed) {
+    return pack2(lo - __builtin_bit_cast(float, packed << 16), hi - __builtin_bit_cast(float, packed & 0xffff0000u));
   }
   static __device__ __forceinline__ float add_pair(unsigned packed, float acc) {
     typedef __bf16 b2 __attribute__((ext_vector_type(2)));
@@ -960,9 +970,10 @@ template <int D> struct VOperands {
 // Scores to probabilities, online.  valid < 32 only on a run's last, partial tile.  The check whether a
 // row's soft-max reference has to move (see kSlack) needs no exchange between the four lanes that
 // share the row: each compares its own eight scores, and only when some lane of the wave finds one
-// too large are the maxima exchanged and the accumulators rescaled.
-template <typename E, int D, int NQ>
-__device__ __forceinline__ void tile_softmax(f32x4 (&s)[2][NQ], int valid, float sc, WaveState<D, NQ>& st, u32x4 (&pf)[NQ]) {
+// too large are the maxima exchanged and the accumulators rescaled.  REST: what rounding the probabilities to the
+// storage type leaves over goes to `rest`.
+template <typename E, int D, int NQ, bool REST = false>
+__device__ __forceinline__ void tile_softmax(f32x4 (&s)[2][NQ], int valid, float sc, WaveState<D, NQ>& st, u32x4 (&pf)[NQ], u32x4* rest = nullptr) {
   if (valid < kTileTokens) {  // wave uniform
     asm volatile("" ::: "memory");  // keeps this a branch: as selects it would run on every tile
     const int c = lane_here() >> 4;
@@ -1003,12 +1014,15 @@ __device__ __forceinline__ void tile_softmax(f32x4 (&s)[2][NQ], int valid, float
     for (int j = 0; j < 8; ++j) x[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j >> 2][qb][j & 3], sc, neg_m));
     st.l[qb] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
     pf[qb] = u32x4{E::pack2(x[0], x[1]), E::pack2(x[2], x[3]), E::pack2(x[4], x[5]), E::pack2(x[6], x[7])};
+    if constexpr (REST)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) rest[qb][j] = E::pack2_rest(x[2 * j], x[2 * j + 1], pf[qb][j]);
   }
 }
 
-// O^T += V^T P^T; `v` holds the operands of the first dim blocks.  read_all(): as in tile_scores.
-template <typename E, int D, int NQ, typename F = Nothing>
-__device__ __forceinline__ void tile_pv(unsigned vb, VOperands<D>& v, const u32x4 (&pf)[NQ], WaveState<D, NQ>& st, F read_all = F()) {
+// O^T += V^T P^T; `v` holds the operands of the first dim blocks.  read_all(): as in tile_scores; rest: as in tile_softmax.
+template <typename E, int D, int NQ, bool REST = false, typename F = Nothing>
+__device__ __forceinline__ void tile_pv(unsigned vb, VOperands<D>& v, const u32x4 (&pf)[NQ], WaveState<D, NQ>& st, F read_all = F(), const u32x4* rest = nullptr) {
   constexpr int DB = D / 16, VB = VOperands<D>::kBatch;
 #pragma unroll
   for (int d0 = 0; d0 < DB; d0 += VB) {
@@ -1018,6 +1032,11 @@ __device__ __forceinline__ void tile_pv(unsigned vb, VOperands<D>& v, const u32x
     for (int db = 0; db < VB; ++db)
 #pragma unroll
       for (int qb = 0; qb < NQ; ++qb) st.o[qb][d0 + db] = E::mfma(v.f[db], pf[qb], st.o[qb][d0 + db]);
+    if constexpr (REST)
+#pragma unroll
+      for (int db = 0; db < VB; ++db)
+#pragma unroll
+        for (int qb = 0; qb < NQ; ++qb) st.o[qb][d0 + db] = E::mfma(v.f[db], rest[qb], st.o[qb][d0 + db]);
   }
 }
 
@@ -1409,7 +1428,7 @@ template <int D, bool GATHERED> struct NarrowStream {
 // One wave's share of a narrow vnode for the NG 16-row groups from row0.  The caller has opened the run and asked for
 // the wave's first indices, and for its first rows too if `started`.  `rec` is the lane's int of the vnode's record when
 // `inlined` (else unused).
-template <typename E, int D, int NG, bool GATHERED>
+template <typename E, int D, int NG, bool GATHERED, bool REST = false>
 __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeView& vn, NarrowStream<D, GATHERED>& rows, bool started,
                                               int kvh, int row0, WaveState<D, NG>& st, int rec, bool inlined) {
   using N = NarrowGeom<D>;
@@ -1499,16 +1518,17 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
         tile_scores<E, D, NG>(la.k, qf, sc);
         next_k();
       }
-      tile_softmax<E, D, NG>(sc, vn.kv_len - tile * kTileTokens, a.scale_log2, st, pf);
+      u32x4 rest[NG];
+      tile_softmax<E, D, NG, REST>(sc, vn.kv_len - tile * kTileTokens, a.scale_log2, st, pf, rest);
       // V landed; the next K and indices may be in flight
       if (indices) wait_direct_loads<N::kLoads + 1>();
       else if (more) wait_direct_loads<N::kLoads>();
       else wait_direct_loads<0>();
       v.request(la.v, 0);
       if constexpr (kEarly) {
-        tile_pv<E, D, NG>(la.v, v, pf, st, next_v);
+        tile_pv<E, D, NG, REST>(la.v, v, pf, st, next_v, rest);
       } else {
-        tile_pv<E, D, NG>(la.v, v, pf, st);
+        tile_pv<E, D, NG, REST>(la.v, v, pf, st, Nothing(), rest);
         next_v();
       }
     }
@@ -1535,12 +1555,19 @@ __device__ __forceinline__ void merge_shares(float* xchg, WaveState<D, NG>& st, 
 }
 
 // The merged rows of a narrow vnode from the states of the SHARE waves that served it, in LDS at xchg: this wave, the
-// w-th, merges and writes its part of the dims of every row.
-template <int D, int NG, int SHARE>
-__device__ __forceinline__ void write_merged_shares(const Stage1Args& a, const float* xchg, const VnodeView& vn, int kvh, int row0, int w) {
+// w-th, merges and writes its part of the dims of every row.  `more` is given the rows
+// too: request(ri), called by every lane of the wave, names the vnode's ri-th request; write(req, head, dim, x) has in x the
+// dims dim .. dim + 3 of that request's row.
+struct WriteNoMore {
+  __device__ __forceinline__ int request(int) const { return 0; }
+  __device__ __forceinline__ void write(int, int, int, const f32x4&) const {}
+};
+template <int D, int NG, int SHARE, typename F = WriteNoMore>
+__device__ __forceinline__ void write_merged_shares(const Stage1Args& a, const float* xchg, const VnodeView& vn, int kvh, int row0, int w, const F& more = F()) {
   constexpr int DB = D / 16, kML = NG * DB * 4 * kWave;
   constexpr int kStep = NarrowGeom<D>::kLds / 4;           // floats from one wave's area to the next one's
-  constexpr int kParts = DB / SHARE;                       // dim blocks of a wave
+  constexpr int kParts = DB >= SHARE ? DB / SHARE : 1;     // dim blocks of a wave
+  if (DB < SHARE && w >= DB) return;
   const int lane = lane_here(), p = lane & 15, c = lane >> 4;
 #pragma unroll 1
   for (int qb = 0; qb < NG; ++qb) {
@@ -1569,13 +1596,16 @@ __device__ __forceinline__ void write_merged_shares(const Stage1Args& a, const f
       for (int db = 0; db < kParts; ++db) sum[db] += o_of[i][db] * weight;
     }
     const float inv = l > 0.f ? 1.f / l : 0.f;
-    const int r = row0 + 16 * qb + p;
-    if (r < vn.q_len * a.g) {
-      const int ri = a.by_g(r), head = kvh * a.g + r - ri * a.g;
+    const int r = min(row0 + 16 * qb + p, vn.q_len * a.g - 1), ri = a.by_g(r), head = kvh * a.g + r - ri * a.g;
+    const int req = more.request(ri);
+    if (row0 + 16 * qb + p <= r) {
       const int64_t row = vn.q_off + ri;
       float* dst = a.mid_o + row * a.so0 + (int64_t)head * a.so1 + 4 * c + 16 * w * kParts;
 #pragma unroll
-      for (int db = 0; db < kParts; ++db) *reinterpret_cast<f32x4*>(dst + 16 * db) = sum[db] * inv;
+      for (int db = 0; db < kParts; ++db) {
+        *reinterpret_cast<f32x4*>(dst + 16 * db) = sum[db] * inv;
+        more.write(req, head, 4 * c + 16 * (w * kParts + db), sum[db] * inv);
+      }
       if (w == 0 && c == 0) a.mid_lse[row * a.sl0 + head] = l > 0.f ? (__builtin_amdgcn_logf(l) + m) * kLn2 : -INFINITY;
     }
   }
@@ -1699,6 +1729,80 @@ __global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 2) stage1_narrow_ker
   const int local_vnode = a.by_hkv(blockIdx.x);
   narrow_item<E, D, GATHERED, true>(a, smem, wave, a.narrow_share, true, a.narrow_begin + local_vnode,
                               blockIdx.x - local_vnode * a.hkv);
+}
+
+// Whole paths (small launches; see ft_decode_programs): every request is in one vnode, whose run is the request's whole path,
+// so a vnode's merged rows are the requests' outputs and there is no second launch.  One block per (vnode, kv head), whose
+// waves take every kPathWaves-th tile of the run; each starts from a record of its own, with the slots of its first tile.
+//
+// Bound by the chain of a launch's start, two memory round trips (record, rows) and one more per tile of the same wave, and the
+// merge, in few blocks: as many waves as the unit's LDS holds tiles for, 8 of 17 KB or 4 of 33 KB.  (4 requests of a short
+// prompt, whole calls: 7.5 us in two launches, 6.4 so, and a launch less for the host: 8.3 and 6.2 back to back.)
+//
+// A path in so few parts has fewer soft-max references than one in pieces, each the maximum of its part, whose probability is
+// 1 and not rounded: the parts of a path would round more of P (408 tokens, against 64 bits 2.67e-4 and 2.71e-4, fp16).  So what
+// the rounding leaves over is contracted too, a third of a microsecond, and only the output's rounding is left (2.08e-4).
+template <int D> constexpr int kPathWaves = FT_PATH_WAVES(D);
+struct PathArgs {
+  Stage1Args s;                  // (first: args_again() reads it at the start of the arguments)
+  const int32_t* wave_records;   // kPathWaves records of kNarrowRecord ints per vnode
+  char* o;
+  int64_t oo0, oo1;
+};
+template <typename E> struct WriteOutput {
+  const PathArgs& d;
+  int q_off, rec;
+  bool recorded;                 // wave uniform: the vnode's requests are in the record
+  __device__ __forceinline__ int request(int ri) const {
+    int req = lane_value(rec, 4 + (ri & (kNarrowRecRequests - 1)));
+    if (!recorded) req = d.s.q_entries[q_off + ri];
+    return req;
+  }
+  __device__ __forceinline__ void write(int req, int head, int dim, const f32x4& x) const {
+    *reinterpret_cast<u32x2*>(d.o + 2 * ((int64_t)req * d.oo0 + (int64_t)head * d.oo1 + dim)) = u32x2{E::pack2(x[0], x[1]), E::pack2(x[2], x[3])};
+  }
+};
+template <typename E, int D, int NG>
+__device__ __forceinline__ void path_pass(const PathArgs& d, char* smem, const VnodeView& vn, NarrowStream<D, false>& rows, int kvh, int row0, int rec) {
+  const Stage1Args& a = d.s;
+  static_assert(SharedState<D, NG>::kFloats * kWave * 4 <= NarrowGeom<D>::kLds, "a wave's state fits its LDS area");
+  WaveState<D, NG> st;
+  narrow_attend<E, D, NG, false, true>(a, vn, rows, true, kvh, row0, st, rec, true);
+  float* xchg = reinterpret_cast<float*>(smem);
+  SharedState<D, NG>::put(xchg + rows.tile0 * (NarrowGeom<D>::kLds / 4), st);
+  __syncthreads();
+  const WriteOutput<E> out{d, vn.q_off, rec, vn.q_len <= kNarrowRecRequests};
+  write_merged_shares<D, NG, kPathWaves<D>>(a, xchg, vn, kvh, row0, rows.tile0, out);
+}
+template <typename E, int D>
+__global__ void __launch_bounds__(kWave * kPathWaves<D>, D <= 128 ? 2 : 1) stage1_paths_kernel(PathArgs d) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  const Stage1Args& a = d.s;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int vnode = a.by_hkv(blockIdx.x), kvh = (int)blockIdx.x - vnode * a.hkv;
+  int rec = d.wave_records[((int64_t)vnode * kPathWaves<D> + wave) * kNarrowRecord + lane_here()];
+  NarrowStream<D, false> rows(a, smem, (unsigned)wave * NarrowGeom<D>::kLds, kvh, wave, kPathWaves<D>);
+  asm volatile("" : "+s"(rows.kbase), "+s"(rows.vbase), "+s"(rows.k_stride), "+s"(rows.v_stride));
+  VnodeView vn;
+  vn.kv_base = __builtin_amdgcn_readlane(rec, 0);
+  vn.kv_len = __builtin_amdgcn_readlane(rec, 1);
+  vn.q_off = __builtin_amdgcn_readlane(rec, 2);
+  vn.q_len = __builtin_amdgcn_readlane(rec, 3);
+  // (complete for the compiler: a wait for it behind the first direct loads would be a wait for those)
+  asm volatile("" : "+v"(rec));
+  const int groups = (vn.q_len * a.g + 15) >> 4;
+  for (int done = 0; done < groups; done += NarrowGeom<D>::kGroups) {
+    rows.open(a, vn);
+    if (rows.tile0 < rows.ntiles) {
+      rows.rows_of_record(rec);
+      rows.issue(false);
+      rows.issue(true);
+      rows.issue_indices(1, rows.tile0 + rows.stride);
+    }
+    if (groups - done >= 2) path_pass<E, D, 2>(d, smem, vn, rows, kvh, 16 * done, rec);
+    else path_pass<E, D, 1>(d, smem, vn, rows, kvh, 16 * done, rec);
+    __syncthreads();  // the exchange area is the staging area of the next pass
+  }
 }
 
 // Blocks are handed to compute units in index order as units become free, so serving the wide
@@ -2536,6 +2640,41 @@ int launch_stage1_narrow(const Stage1Args& a0, hipStream_t stream) {
   return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
 }
 
+template <typename E, int D>
+int launch_stage1_paths_d(const PathArgs& d, hipStream_t stream) {
+  const int64_t blocks = (int64_t)d.s.narrow_count * d.s.hkv;
+  if (blocks == 0) return FT_OK;
+  if (blocks > INT32_MAX) return FT_ERR_ARGUMENT;
+  auto kern = stage1_paths_kernel<E, D>;
+  constexpr size_t lds = (size_t)kPathWaves<D> * NarrowGeom<D>::kLds;
+  // (raising the dynamic LDS limit is idempotent: two threads that both find the flag clear both raise it)
+  static std::atomic<bool> configured_on[kMaxDevices];
+  std::atomic<bool>& configured = configured_on[current_device()];
+  if (!configured.load(std::memory_order_acquire)) {
+    if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+      (void)hipGetLastError();
+      return FT_ERR_LAUNCH;
+    }
+    configured.store(true, std::memory_order_release);
+  }
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, 1, 1), dim3(kWave * kPathWaves<D>, 1, 1), lds, stream, d);
+  return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
+}
+int launch_stage1_paths(const PathArgs& a, int head_dim, int dtype, hipStream_t stream) {
+#define FT_DISPATCH_D(E)                                         \
+  switch (head_dim) {                                            \
+    case 32: return launch_stage1_paths_d<E, 32>(a, stream);     \
+    case 64: return launch_stage1_paths_d<E, 64>(a, stream);     \
+    case 128: return launch_stage1_paths_d<E, 128>(a, stream);   \
+    case 256: return launch_stage1_paths_d<E, 256>(a, stream);   \
+    default: return FT_ERR_HEAD_DIM;                             \
+  }
+  if (dtype == FT_DTYPE_F16) { FT_DISPATCH_D(F16) }
+  if (dtype == FT_DTYPE_BF16) { FT_DISPATCH_D(BF16) }
+#undef FT_DISPATCH_D
+  return FT_ERR_DTYPE;
+}
+
 // `a` names two vnode ranges: [vnode_begin, +vnode_count) of wide vnodes (more than 16 query
 // rows) and [narrow_begin, +narrow_count) of narrow ones.
 template <typename E, int D, bool GATHERED, bool STAGED = false>
@@ -2921,6 +3060,28 @@ int ft_decode_programs(const void* q, const void* k, const void* v, void* o,
                        const int32_t* narrow_table, const int32_t* prog_records, const int32_t* req_table,
                        int batch_size, int num_qo_heads, int num_kv_heads, int head_dim,
                        float sm_scale, int dtype, ft_stream_t stream) {
+  if (narrow_in_programs == FT_WHOLE_PATHS) {
+    // (checked as the two launches would be)
+    if (!phase_node_nums || !phase_node_offsets) return FT_ERR_NULL_POINTER;
+    if (num_kv_heads < 1 || num_qo_heads % num_kv_heads != 0) return FT_ERR_GROUP;
+    const int g = num_qo_heads / num_kv_heads;
+    if (int rc = check_common(head_dim, g, dtype)) return rc;
+    if (head_dim < 32) return FT_ERR_HEAD_DIM;
+    if (phase_node_nums[0] != 0 || num_programs != 0 || batch_size < 0 || num_qo_heads < 1) return FT_ERR_ARGUMENT;
+    if (phase_node_nums[1] == 0 || batch_size == 0) return FT_OK;
+    PathArgs d{};
+    if (int rc = stage1_setup(d.s, q, k, v, sq0, sq1, sk0, sk1, sv0, sv1, vnode_to_kv_entries, vnode_to_kv_offs,
+                              vnode_to_kv_lens, vnode_to_q_entries, vnode_to_q_offs, vnode_to_q_lens, num_kv_heads, g,
+                              head_dim, sm_scale, mid_o, so0, so1, mid_lse, sl0, dtype))
+      return rc;
+    if (!prog_records || !req_to_vnode_entries || !req_to_vnode_offs || !req_to_vnode_lens || !o) return FT_ERR_NULL_POINTER;
+    if (!range_ok(phase_node_offsets[1], phase_node_nums[1], num_kv_heads)) return FT_ERR_ARGUMENT;
+    if (!aligned16(o) || (oo0 | oo1) % 4 != 0) return FT_ERR_ALIGNMENT;
+    d.s.narrow_begin = phase_node_offsets[1]; d.s.narrow_count = phase_node_nums[1];
+    d.wave_records = prog_records;
+    d.o = static_cast<char*>(o); d.oo0 = oo0; d.oo1 = oo1;
+    return launch_stage1_paths(d, head_dim, dtype, stream);
+  }
   if (int rc = ft_stage1_programs(q, k, v, sq0, sq1, sk0, sk1, sv0, sv1, vnode_to_kv_entries, vnode_to_kv_offs,
                                   vnode_to_kv_lens, vnode_to_q_entries, vnode_to_q_offs, vnode_to_q_lens, mid_o, so0,
                                   so1, mid_lse, sl0, phase_node_nums, phase_node_offsets, prog_table, num_programs,

@@ -18,6 +18,7 @@
 //    second stage reads back.
 
 #include "fasttree_schedule.h"
+#include "fasttree_hip.h"
 
 #include <algorithm>
 #include <cmath>
@@ -81,6 +82,13 @@ constexpr double kSmallLaunchBytes = 64e6;
 // Of two decisions on what attends what, a launch is clearly better that is modelled shorter by a twentieth and by this
 // many microseconds: below that the model chose wrongly as often as not (12.0 us instead of 10.5, 12.6 instead of 11.9).
 constexpr double kClearlyBetter = 0.95, kClearlyUs = 1.5;
+
+// A launch of whole paths, both launches of any other plan in one: its start and end, and a round of tiles (as many as a
+// block has waves, 128 KB at 256-byte rows, which a unit takes in at 64 bytes a cycle), longer by kPathShared of it where every
+// unit has a block.  Whole calls of head_dim 128, whole paths and otherwise, us: 4 requests of 32/8 heads with 80 tokens each
+// 4.3 and 6.5, 408 tokens 6.4 and 7.5, 924 tokens 8.4 and 7.7 (not taken), 1524 tokens 10.5 and 8.4; 31 with 300 tokens 6.5 and
+// 9.6, with 1100 11.4 and 11.2; 240 of 16/1 heads with 288 tokens 7.0 and 9.4, with 1100 12.1 and 17.3.
+constexpr double kPathStart = 3.8, kPathRound = 1.1, kPathShared = 0.43;
 
 struct Run {
   int64_t start;                 // into the flat slot list
@@ -496,6 +504,19 @@ void build(const Machine& m, int batch, Layout& l, std::vector<Narrow>& narrow, 
   }
 }
 
+// A record per wave of every narrow vnode, of a plan of whole paths.
+void wave_records(const Machine& m, const int32_t* kv_entries, ft_schedule& s) {
+  const std::vector<int32_t>& nt = s.arrays[FT_SCHEDULE_NARROW_TABLE];
+  std::vector<int32_t>& wr = s.arrays[FT_SCHEDULE_WAVE_RECORDS];
+  const int waves = FT_PATH_WAVES(m.head_dim);
+  wr.reserve(nt.size() * waves);
+  for (size_t at = 0; at < nt.size(); at += 64)
+    for (int w = 0; w < waves; ++w) {
+      int32_t* rec = &*wr.insert(wr.end(), nt.begin() + at, nt.begin() + at + 64);
+      for (int i = 0; i < kTile; ++i) rec[20 + i] = kv_entries[rec[0] + std::min(w * kTile + i, rec[1] - 1)];
+    }
+}
+
 // A launch: its programs, its narrow vnodes, and what the model expects of both stages.
 struct Launch {
   Layout layout;
@@ -678,6 +699,43 @@ Launch best_launch(const std::vector<Run>& runs, const Machine& m, double bound 
   return best;
 }
 
+// What a launch of whole paths is modelled to take: `paths` vnodes, the longest of `longest` tokens.
+double whole_paths_us(int64_t paths, int64_t longest, const Machine& m) {
+  const int64_t rounds = ceil_div(ceil_div(longest, kTile), FT_PATH_WAVES(m.head_dim));
+  return kPathStart + kPathRound * (1 + kPathShared * paths * m.heads / m.cus) * std::min(1.5, m.head_dim / 128.0) * rounds;
+}
+
+// A tree's whole paths, one vnode per leaf, where they are a launch of less than a block per unit that takes less than
+// `bound` (`taken`).
+int whole_paths(const Tree& tree, const Machine& m, int batch, double bound, TreeRuns& t, double& us, bool& taken) {
+  taken = false;
+  std::vector<int64_t> path(tree.n);
+  int64_t leaves = 0, longest = 0;
+  for (int v = 0; v < tree.n; ++v) {
+    path[v] = tree.seqlen[v] + (v > 0 ? path[tree.parent[v]] : 0);
+    if (tree.num_children[v] > 0) continue;
+    longest = std::max(longest, path[v]);
+    ++leaves;
+    if (path[v] < 1 || tree.requests(v) * m.group > kWaveRows) return FT_SCHEDULE_OK;
+  }
+  us = whole_paths_us(leaves, longest, m);
+  if (m.head_dim < 32 || leaves * m.heads >= m.cus || us >= bound) return FT_SCHEDULE_OK;
+  std::vector<int32_t> all(tree.n, 1);
+  all[0] = 0;
+  if (int rc = tree_runs(tree, std::move(all), t)) return rc;
+  int64_t requests = 0;
+  for (const Run& r : t.runs) requests += r.n;
+  // (every request in one vnode, whatever the arguments say of inner nodes)
+  std::vector<char> seen(batch, 0);
+  for (const Run& r : t.runs)
+    for (int i = 0; i < r.n; ++i) {
+      if (seen[r.reqs[i]]) return FT_SCHEDULE_OK;
+      seen[r.reqs[i]] = 1;
+    }
+  taken = requests == batch && (int64_t)t.runs.size() == leaves;
+  return FT_SCHEDULE_OK;
+}
+
 // (request, token) pairs of a list of runs, pieces or narrow vnodes.
 template <typename List, typename Tokens>
 double pairs(const List& list, Tokens tokens) {
@@ -772,7 +830,19 @@ int ft_schedule_tree_weighed(int num_nodes, const int32_t* parent, const int32_t
       }
     }
     auto s = std::make_unique<ft_schedule>();
+    TreeRuns u;
+    double us = 0;
+    bool whole;
+    if (int rc = whole_paths(tree, m, batch_size, kClearlyBetter * (launch.score + kLaunch), u, us, whole)) return rc;
+    if (whole) {
+      launch = Launch{};
+      for (const Run& r : u.runs) launch.narrow.push_back({r.start, (int32_t)r.tokens, r.reqs, r.n});
+      std::stable_sort(launch.narrow.begin(), launch.narrow.end(), [](const Narrow& a, const Narrow& b) { return a.tokens > b.tokens; });
+      launch.layout.total_us = us - kLaunch;
+      t = std::move(u);
+    }
     if (int rc = finish(launch, t.runs, m, batch_size, t.kv_entries.data(), *s, modelled_us)) return rc;
+    if (whole) wave_records(m, t.kv_entries.data(), *s);
     s->arrays[FT_SCHEDULE_KV_ENTRIES] = std::move(t.kv_entries);
     s->arrays[FT_SCHEDULE_NODE_ASSIGNMENTS] = std::move(t.along);
     *out = s.release();

@@ -22,7 +22,7 @@ namespace {
 
 PyObject* g_library_error = nullptr;   // fasttree_hip._lib.FastTreeLibraryError
 // attribute names of a launch-order plan's phase list, interned once
-PyObject *g_prog_table, *g_narrow_table, *g_prog_records, *g_req_table, *g_num_programs, *g_narrow_in_programs;
+PyObject *g_prog_table, *g_narrow_table, *g_prog_records, *g_req_table, *g_num_programs, *g_narrow_in_programs, *g_wave_records;
 
 // what decode_layer reads from a FastTreeMetadata, in the order of the decode call's arguments
 constexpr int kMetaAttributes = 14;
@@ -152,6 +152,9 @@ PlanTables plan_tables(PyObject* phases) {
     t.prog_records = table_address(phases, g_prog_records);
     t.num_programs = count_of(phases, g_num_programs);
     t.narrow_in_programs = count_of(phases, g_narrow_in_programs);
+  } else if (const int32_t* records = table_address(phases, g_wave_records)) {   // a plan of whole paths
+    t.prog_records = records;
+    t.narrow_in_programs = FT_WHOLE_PATHS;
   }
   return t;
 }
@@ -317,7 +320,8 @@ PyMODINIT_FUNC PyInit__torch_binding(void) {
   if (!g_library_error) return nullptr;
   struct { PyObject** at; const char* name; } names[] = {
       {&g_prog_table, "prog_table"}, {&g_narrow_table, "narrow_table"}, {&g_prog_records, "prog_records"},
-      {&g_req_table, "req_table"}, {&g_num_programs, "num_programs"}, {&g_narrow_in_programs, "narrow_in_programs"}};
+      {&g_req_table, "req_table"}, {&g_num_programs, "num_programs"}, {&g_narrow_in_programs, "narrow_in_programs"},
+      {&g_wave_records, "wave_records"}};
   for (auto& n : names)
     if (!(*n.at = PyUnicode_InternFromString(n.name))) return nullptr;
   for (int i = 0; i < kMetaAttributes; ++i)

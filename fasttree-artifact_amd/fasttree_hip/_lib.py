@@ -14,6 +14,7 @@ LIB_NAME = "libfasttree_hip.so"
 LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
 
 FT_DTYPE_F16 = 0
+FT_WHOLE_PATHS = -1
 FT_DTYPE_BF16 = 1
 
 FT_ERR_HEAD_DIM = -3

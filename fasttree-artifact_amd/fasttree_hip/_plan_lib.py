@@ -32,7 +32,7 @@ SIGNATURES = {
 
 # order of a schedule's arrays (enum in include/fasttree_schedule.h)
 SCHEDULE_ARRAYS = ("kv_offs", "kv_lens", "q_entries", "q_offs", "q_lens", "req_entries", "req_offs", "req_lens", "prog_table",
-                   "narrow_table", "prog_records", "req_table", "counts", "kv_entries", "node_assignments")
+                   "narrow_table", "prog_records", "req_table", "counts", "kv_entries", "node_assignments", "wave_records")
 SCHEDULE_SIGNATURES = {
     "ft_schedule_create": (ctypes.c_int, [ctypes.c_int64, _P32, _P32, _P32, _P32, ctypes.c_int64, _P32, ctypes.c_int64, _P32]
                            + [ctypes.c_int] * 5 + [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_void_p)]),

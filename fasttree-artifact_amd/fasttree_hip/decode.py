@@ -34,8 +34,18 @@ def _narrow_table_ptr(phase_node_nums):
     return table.data_ptr() if table is not None else None
 
 
-def _prog_records_ptr(phase_node_nums):
-    """Device pointer of the records of the block programs a launch-order plan carries, or None."""
+def _narrow_in_programs(phase_node_nums):
+    """The decode call's argument of that name: FT_WHOLE_PATHS for a plan of whole paths."""
+    if getattr(phase_node_nums, "prog_table", None) is not None:
+        return int(getattr(phase_node_nums, "narrow_in_programs", 0))
+    return _lib.FT_WHOLE_PATHS if getattr(phase_node_nums, "wave_records", None) is not None else 0
+
+
+def _prog_records_ptr(phase_node_nums, paths=False):
+    """Device pointer of the records of the block programs a launch-order plan carries (with ``paths``, or of the waves
+    of a plan of whole paths), or None."""
+    if paths and _narrow_in_programs(phase_node_nums) == _lib.FT_WHOLE_PATHS:
+        return phase_node_nums.wave_records.data_ptr()
     table = getattr(phase_node_nums, "prog_records", None)
     return table.data_ptr() if table is not None and getattr(phase_node_nums, "prog_table", None) is not None else None
 
@@ -117,8 +127,8 @@ def fasttree_decode_static(q, k_buffer, v_buffer, o, vnode_to_kv_entries, vnode_
         _lib.int32_pair(phase_node_nums), _lib.int32_pair(phase_node_offsets),
         programs.data_ptr() if programs is not None else None,
         int(getattr(phase_node_nums, "num_programs", 0)) if programs is not None else 0,
-        int(getattr(phase_node_nums, "narrow_in_programs", 0)) if programs is not None else 0,
-        _narrow_table_ptr(phase_node_nums), _prog_records_ptr(phase_node_nums), _req_table_ptr(phase_node_nums),
+        _narrow_in_programs(phase_node_nums), _narrow_table_ptr(phase_node_nums), _prog_records_ptr(phase_node_nums, paths=True),
+        _req_table_ptr(phase_node_nums),
         q.shape[0], q.shape[1], k_buffer.shape[1], q.shape[-1],
         float(sm_scale), _dtype_code(q), _stream_handle(q),
     )

@@ -156,6 +156,9 @@ class LaunchPhases(list):
     req_table = None
     #: int32 device tensor of :func:`program_records` (256 entries per program), or None
     prog_records = None
+    #: int32 device tensor, 64 entries per wave of every vnode, of a plan of whole paths (include/fasttree_hip.h,
+    #: FT_WHOLE_PATHS), whose decode call is one launch; None for every other plan
+    wave_records = None
     #: what the schedule's model expects the first-stage launch to take, and the machine it was laid out for
     modelled_us = None
     num_cus = None
@@ -834,10 +837,11 @@ class Arranged:
     def num_rows(self):
         return self.where["q_entries"][1]
 
-    def fits(self, rows, vnodes, kv_entries=None):
+    def fits(self, rows, vnodes, kv_entries=None, wave_records=0):
         """Whether buffers of these sizes hold the plan."""
         return (self.num_rows <= rows and max(self.n_wide + self.n_narrow, self.num_programs) <= vnodes
-                and (kv_entries is None or self.where["kv_entries"][1] <= kv_entries))
+                and (kv_entries is None or self.where["kv_entries"][1] <= kv_entries)
+                and self.where.get("wave_records", (0, 0))[1] <= wave_records)
 
 
 class _PackedTensor:

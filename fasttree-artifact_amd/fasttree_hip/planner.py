@@ -474,6 +474,7 @@ class PlanBuffers:
         self.narrow_table = ints(64 * max_vnodes)     # (launch_schedule.NARROW_RECORD entries per narrow vnode)
         self.req_table = ints(16 * max_batch_size)    # (launch_schedule.REQUEST_RECORD entries per request)
         self.prog_records = ints(256 * max_vnodes)    # (launch_schedule.PROGRAM_RECORD entries per program)
+        self.wave_records = ints(64 * 8 * min(int(max_vnodes), 512))   # (of plans of whole paths: a vnode per unit at most)
         self.mid_o = torch.empty((int(max_rows), num_qo_heads, head_dim), dtype=torch.float32, device=device)
         self.mid_lse = torch.empty((int(max_rows), num_qo_heads), dtype=torch.float32, device=device)
 
@@ -565,7 +566,8 @@ def _place_arranged(plan, kv_entries, num_qo_heads, head_dim, device, buffers):
     from .launch_schedule import LaunchPhases
 
     if buffers is not None:
-        part = {name: buffers.fill(full, plan.part[name]) for name, full in _BUFFER_OF.items() if name in plan.part}
+        part = {name: buffers.fill(full, plan.part[name]) for name, full in _BUFFER_OF.items()
+                if name in plan.part and (name != "wave_records" or plan.where[name][1] > 0)}
         wait_for_copies(buffers.device)
     else:
         # one copy for the whole plan; the arrays are views of it
@@ -583,6 +585,8 @@ def _place_arranged(plan, kv_entries, num_qo_heads, head_dim, device, buffers):
         nums.narrow_table = part["narrow_table"]
     if head_dim >= 32 and launch_schedule.USE_REQUEST_RECORDS:
         nums.req_table = part["req_table"]
+    if plan.where.get("wave_records", (0, 0))[1] > 0:
+        nums.wave_records = part["wave_records"]
     return (part["kv_entries"] if kv_entries is None else kv_entries, part["kv_offs"], part["kv_lens"], part["q_entries"], part["q_offs"],
             part["q_lens"], part["req_entries"], part["req_offs"], part["req_lens"],
             *_scratch(plan.num_rows, num_qo_heads, head_dim, device, buffers), nums, [0, plan.n_wide])
@@ -593,6 +597,7 @@ _BUFFER_OF = {
     "kv_entries": "vnode_to_kv_entries", "kv_offs": "vnode_to_kv_offs", "kv_lens": "vnode_to_kv_lens", "q_entries": "vnode_to_q_entries", "q_offs": "vnode_to_q_offs",
     "q_lens": "vnode_to_q_lens", "req_entries": "req_to_vnode_entries", "req_offs": "req_to_vnode_offs", "req_lens": "req_to_vnode_lens",
     "prog_table": "prog_table", "narrow_table": "narrow_table", "prog_records": "prog_records", "req_table": "req_table",
+    "wave_records": "wave_records",
 }
 
 
@@ -654,7 +659,8 @@ def fasttree_preparation(
             num_cus=launch_schedule.compute_units(device) if num_cus is None else num_cus, kv_slot_map=kv_slot_map, pin=_on_gpu(device),
             decided=r[L.NODE_ASSIGNMENTS])
         # (buffers sized for the planner's own lists may not hold this plan: they get one made from those lists)
-        if buffers is None or arranged.fits(buffers.mid_o.shape[0], buffers.vnode_to_kv_offs.numel(), buffers.vnode_to_kv_entries.numel()):
+        if buffers is None or arranged.fits(
+                buffers.mid_o.shape[0], buffers.vnode_to_kv_offs.numel(), buffers.vnode_to_kv_entries.numel(), buffers.wave_records.numel()):
             _report(r, params)
             assignments = arranged.part["node_assignments"].tolist()
             return _place_arranged(arranged, None, num_qo_heads, head_dim, device, buffers), assignments

@@ -158,7 +158,17 @@ int ft_decode(const void* q, const void* k, const void* v, void* o,
  * second launch then knows which partial rows to ask for after one memory round trip instead of two
  * (length and offset, then the entries); entries beyond the fourteenth are read from the list.
  * Trusted like the lists.
+ *
+ * ft_decode_programs and ft_decode_static with narrow_in_programs == FT_WHOLE_PATHS: no programs and no
+ * vnodes of the first range, and every request is in exactly one vnode of the second, whose run is the request's whole
+ * path.  The call is one launch then: it writes o beside the partial results (mid_o, mid_lse as ever), and every
+ * (vnode, KV head) is a block of FT_PATH_WAVES(head_dim) waves, which take every FT_PATH_WAVES-th 32-token tile of the
+ * run.  prog_records holds FT_PATH_WAVES records per vnode of the second range, laid out as narrow_table's, the w-th
+ * with the slots of the run's w-th tile (vnode_to_kv_entries[kv_off + min(32 w + t, kv_len - 1)]).  The lists are otherwise
+ * those of a complete plan.
  */
+#define FT_WHOLE_PATHS (-1)
+#define FT_PATH_WAVES(head_dim) ((head_dim) <= 128 ? 8 : 4)
 int ft_stage1_programs(const void* q, const void* k, const void* v,
                        int64_t sq0, int64_t sq1, int64_t sk0, int64_t sk1, int64_t sv0, int64_t sv1,
                        const int32_t* vnode_to_kv_entries, const int32_t* vnode_to_kv_offs,

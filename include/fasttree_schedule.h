@@ -25,12 +25,14 @@ enum {
  * per-request entries end with 32 x -1); then the program table (4 per program), a record of 64 per
  * narrow vnode, 256 per program and 16 per request (layouts: include/fasttree_hip.h; the first two
  * kinds only where kv_entries were given); FT_SCHEDULE_COUNTS: wide vnodes, narrow vnodes, programs,
- * block slots the programs were laid out on, narrow vnodes that belong to programs (none). */
+ * block slots the programs were laid out on, narrow vnodes that belong to programs (none).
+ * FT_SCHEDULE_WAVE_RECORDS is filled where the plan is one of whole paths (include/fasttree_hip.h,
+ * FT_WHOLE_PATHS), which ft_schedule_tree makes of small trees, else empty. */
 enum {
   FT_SCHEDULE_KV_OFFS = 0, FT_SCHEDULE_KV_LENS, FT_SCHEDULE_Q_ENTRIES, FT_SCHEDULE_Q_OFFS, FT_SCHEDULE_Q_LENS,
   FT_SCHEDULE_REQ_ENTRIES, FT_SCHEDULE_REQ_OFFS, FT_SCHEDULE_REQ_LENS, FT_SCHEDULE_PROG_TABLE,
   FT_SCHEDULE_NARROW_TABLE, FT_SCHEDULE_PROG_RECORDS, FT_SCHEDULE_REQ_TABLE, FT_SCHEDULE_COUNTS,
-  FT_SCHEDULE_KV_ENTRIES, FT_SCHEDULE_NODE_ASSIGNMENTS, FT_SCHEDULE_ARRAYS
+  FT_SCHEDULE_KV_ENTRIES, FT_SCHEDULE_NODE_ASSIGNMENTS, FT_SCHEDULE_WAVE_RECORDS, FT_SCHEDULE_ARRAYS
 };
 
 /* Arranges vnode lists.  kv_offs / kv_lens / q_offs / q_lens: one entry per vnode (any order);

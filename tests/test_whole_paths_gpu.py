@@ -1,0 +1,117 @@
+"""Plans of whole paths (a request's path is one vnode, the call one launch): path lengths at the edges of tiles and of
+the rounds of tiles that a block's waves take, every head size, one and two groups of 16 query rows."""
+import math
+
+import pytest
+import torch
+
+from fasttree_hip.decode import fasttree_decode, fasttree_decode_stage1, fasttree_decode_stage2, fasttree_decode_static
+from fasttree_hip.inputs import make_decode_inputs
+from fasttree_hip.kv_tree import generate_tree, nodes_from_rows
+from fasttree_hip.planner import FastTreeParams, PlanBuffers, fasttree_preparation
+from test_decode_gpu import _dense_check
+
+
+def _plan(sizes, lens, group, heads, d, dtype, device, buffers=None, num_cus=None, seed=0):
+    tree = nodes_from_rows(generate_tree(sizes, lens))
+    inp = make_decode_inputs(tree, group * heads, heads, d, device=device, dtype=dtype, seed=seed, shuffle_slots=True)
+    params = FastTreeParams()
+    params.set_q_tile_sizes([max(1, 64 // group), max(1, 16 // group)])
+    params.set_kv_tile_sizes([32, 32])
+    params.set_kv_group_num(group)
+    aux, _ = fasttree_preparation(tree, inp.KV_ptrs, inp.batch_size, group * heads, heads, d, [1024, 256], [256, 1024], [256, 256], params,
+                                  device=device, kv_slot_map=inp.slot_map, launch_order=True, buffers=buffers, num_cus=num_cus)
+    return tree, inp, aux, (list(params.TSQs), list(params.TSKs), 1.0 / math.sqrt(d))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,group,heads,dtype", [(128, 4, 8, torch.float16), (128, 16, 1, torch.bfloat16), (128, 32, 2, torch.float16),
+                                                 (64, 3, 8, torch.bfloat16), (64, 20, 2, torch.float16), (32, 1, 4, torch.float16),
+                                                 (256, 16, 1, torch.bfloat16), (256, 24, 2, torch.float16)])
+@pytest.mark.parametrize("lens", [[1, 1], [20, 11], [20, 12], [20, 13], [120, 8], [121, 8], [250, 6], [250, 7], [400, 9], [507, 6]],
+                         ids=lambda x: str(sum(x)))
+def test_path_lengths(lens, d, group, heads, dtype, device):
+    if dtype is torch.bfloat16 and sum(lens) == 2:
+        # (outputs of two tokens are 0.7 in the mean and the output's rounding, up to 2^-9 of a value, takes half of the bar
+        # of 1e-3 by itself, that of the two probabilities as much)
+        lens = [5, 4]
+    print(f"\n[gpu case] whole paths of {sum(lens)} tokens, {group * heads}/{heads} heads of {d}, {dtype}", flush=True)
+    tree, inp, aux, rest = _plan([1, 3], lens, group, heads, d, dtype, device, seed=sum(lens))
+    if aux[11].wave_records is None:
+        assert d == 256 and sum(lens) > 128, "a launch of paths this short is one of whole paths"
+        pytest.skip("long paths of wide rows are laid out in pieces")
+    assert list(aux[11]) == [0, 3] and aux[3].numel() == 3
+    o = torch.full_like(inp.Q, float("nan"))
+    fasttree_decode(inp.Q, inp.K_pool, inp.V_pool, o, *aux, *rest)
+    _dense_check(tree, inp, o, f"whole paths of {sum(lens)} tokens", dtype=dtype)
+    # the partial results are those of a plan as any other, and so is the plan in two launches
+    mid_o, mid_lse, two = aux[9].clone(), aux[10].clone(), torch.empty_like(o)
+    fasttree_decode_stage1(inp.Q, inp.K_pool, inp.V_pool, *aux[:6], rest[2], aux[9], aux[10], aux[11], aux[12], *rest[:2])
+    assert torch.allclose(mid_lse, aux[10], rtol=0, atol=1e-3) and torch.allclose(mid_o, aux[9], rtol=0, atol=4e-3 if dtype is torch.float16 else 3e-2)
+    fasttree_decode_stage2(*aux[6:9], mid_o, mid_lse, two)
+    assert torch.equal(two, o), "the merge of one partial result is the rounded result"
+
+
+@pytest.mark.gpu
+def test_paths_of_unequal_length_in_other_entry_points(device):
+    """A plan in buffers made beforehand, with o in rows of another pitch; the entry point that keeps its scratch to
+    itself; a captured call, replayed between others."""
+    print("\n[gpu case] whole paths in buffers, static, captured", flush=True)
+    buffers = PlanBuffers(32, 128, 8192, 256, 256, 64)
+    tree, inp, aux, rest = _plan([1, 2, 9], [190, 70, 33], 4, 8, 128, torch.float16, device, buffers=buffers, seed=5)
+    assert aux[11].wave_records is not None and aux[11].wave_records.data_ptr() == buffers.wave_records.data_ptr()
+    want = torch.full_like(inp.Q, float("nan"))
+    fasttree_decode(inp.Q, inp.K_pool, inp.V_pool, want, *aux, *rest)
+    _dense_check(tree, inp, want, "whole paths in buffers")
+    pitched = torch.full((inp.batch_size, 40, 160), float("nan"), dtype=torch.float16, device=device)
+    fasttree_decode(inp.Q, inp.K_pool, inp.V_pool, pitched[:, 4:36, 16:144], *aux, *rest)
+    assert torch.equal(pitched[:, 4:36, 16:144], want) and bool(torch.isnan(pitched[:, :4]).all()) and bool(torch.isnan(pitched[..., 144:]).all())
+    o = torch.full_like(want, float("nan"))
+    fasttree_decode_static(inp.Q, inp.K_pool, inp.V_pool, o, *aux[:9], aux[11], aux[12], rest[2])
+    assert torch.equal(o, want)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    q = inp.Q.clone()
+    with torch.cuda.stream(side):
+        fasttree_decode(q, inp.K_pool, inp.V_pool, o, *aux, *rest)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        fasttree_decode(q, inp.K_pool, inp.V_pool, o, *aux, *rest)
+    for turn in range(3):
+        q.copy_(inp.Q * (turn + 1))
+        fasttree_decode(q, inp.K_pool, inp.V_pool, want, *aux, *rest)
+        o.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(o, want), turn
+
+
+def test_which_trees_are_laid_out_as_whole_paths():
+    """Short paths with less than a block per unit; not long ones, not more of them."""
+    def whole(sizes, lens, group, heads, d=128, cus=256):
+        tree = nodes_from_rows(generate_tree(sizes, lens))
+        from fasttree_hip.kv_tree import assign_requests, kv_prefix_sums
+        batch, ptrs = assign_requests(tree), kv_prefix_sums(tree)
+        params = FastTreeParams()
+        params.set_q_tile_sizes([max(1, 64 // group), max(1, 16 // group)])
+        params.set_kv_tile_sizes([32, 32])
+        params.set_kv_group_num(group)
+        aux, assigned = fasttree_preparation(tree, ptrs, batch, group * heads, heads, d, [1024, 256], [256, 1024], [256, 256], params, device="cpu",
+                                             launch_order=True, num_cus=cus)
+        if aux[11].wave_records is None:
+            return False
+        assert assigned == [0] + [1] * (len(tree) - 1) and list(aux[11]) == [0, batch] and aux[11].num_programs == 0
+        waves = 8 if d <= 128 else 4
+        rec = aux[11].wave_records.view(batch, waves, 64)
+        for v in range(batch):
+            off, n = int(aux[1][v]), int(aux[2][v])
+            for w in range(waves):
+                assert rec[v, w, :4].tolist() == [off, n, int(aux[4][v]), 1] and int(rec[v, w, 4]) == int(aux[3][aux[4][v]])
+                at = [min(32 * w + t, n - 1) for t in range(32)]
+                assert rec[v, w, 20:52].tolist() == aux[0][[off + t for t in at]].tolist()
+        return True
+
+    assert whole([1, 4], [384, 24], 4, 8) and whole([1, 31], [200, 100], 4, 8) and whole([1, 4], [384, 24], 4, 8, d=64)
+    assert whole([1, 200], [300, 30], 16, 1, d=256)
+    assert not whole([1, 4], [3000, 24], 4, 8) and not whole([1, 32], [200, 100], 4, 8) and not whole([1, 31], [200, 100], 4, 8, cus=128)

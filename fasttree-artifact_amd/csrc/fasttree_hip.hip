@@ -1040,6 +1040,9 @@ __device__ __forceinline__ void tile_pv(unsigned vb, VOperands<D>& v, const u32x
   }
 }
 
+// Token groups of a pass at most (see wide_block).
+template <int D> struct WideGroups { static constexpr int kMost = D <= 128 ? WideGeom<D>::kSub : kWideWaves; };
+
 // What the waves of a block share in one pass over a KV run, and what a wave does in it.
 struct WidePass {
   int kvh;
@@ -1094,6 +1097,89 @@ __device__ __forceinline__ void merge_token_groups(float* xchg, WaveState<D, NG>
     if (p.tg >= half && p.tg < 2 * half) SharedState<D, NG>::put(xchg + (size_t)(p.set * half + p.tg - half) * kArea, st);
     __syncthreads();
     if (p.tg < half) SharedState<D, NG>::merge(xchg + (size_t)(p.set * half + p.tg) * kArea, st);
+  }
+}
+
+// The rows of a wave that holds all of its tokens, written through its area `at` of LDS (16 rows of 4 * D bytes), whole rows
+// at a time: straight from the accumulators an instruction writes 64 bytes to each of 16 rows, and four waves' 128 rows of
+// 512 bytes leave a unit in 1.7 us, in whole rows in 1.3 (.7 where other units don't write; the 400-request tree, whole
+// calls, 60.4 -> 59.8 us; at 512-byte K/V rows, where a block is alone on its unit, nothing is gained).
+template <int D, int NG>
+__device__ __forceinline__ void write_rows(const Stage1Args& a, unsigned at, const VnodeView& vn, const WidePass& p, const WaveState<D, NG>& st) {
+  constexpr int kChunks = D / 4;                             // 16-byte pieces of a row
+  constexpr int kRows = kWave / kChunks;                     // rows an instruction writes
+  static_assert(16 * 16 * kChunks <= WideGeom<D>::kBytes / kWideWaves, "the rows fit a wave's part of a buffer");
+  const int lane = lane_here(), r16 = lane & 15, c = lane >> 4;
+  const int rows_total = vn.q_len * a.g;
+  // piece k of row r lies in place k ^ swz(r) of the row, so that neither way 8 lanes meet in a bank
+  auto place = [&](int r, int k) { return at + (unsigned)(r * (16 * kChunks) + 16 * (k ^ ((r & 7) << 2 & (kChunks - 1)))); };
+#pragma unroll
+  for (int qb = 0; qb < NG; ++qb) {
+    if (qb >= p.groups) break;                               // (a wave without rows writes none)
+    const int r = min(p.row0 + 16 * qb + r16, rows_total - 1), there = rows_total - (p.row0 + 16 * qb);
+    const int ri = a.by_g(r), head = p.kvh * a.g + r - ri * a.g;
+    const int64_t row = vn.q_off + ri;
+    const float l = st.l[qb], inv = l > 0.f ? 1.f / l : 0.f;
+    const uint64_t dst = (uint64_t)(uintptr_t)(a.mid_o + row * a.so0 + (int64_t)head * a.so1);
+    wave_lds_fence();
+#pragma unroll
+    for (int db = 0; db < D / 16; ++db)
+      *reinterpret_cast<__attribute__((address_space(3))) f32x4*>((uintptr_t)place(r16, 4 * db + c)) = st.o[qb][db] * inv;
+    if (c == 0 && r16 < there) a.mid_lse[row * a.sl0 + head] = l > 0.f ? (__builtin_amdgcn_logf(l) + st.m[qb]) * kLn2 : -INFINITY;
+    wave_lds_fence();
+    const int k = lane % kChunks, first = lane / kChunks;
+#pragma unroll
+    for (int i = 0; i < 16; i += kRows) {
+      const f32x4 x = *reinterpret_cast<const __attribute__((address_space(3))) f32x4*>((uintptr_t)place(i + first, k));
+      const unsigned lo = (unsigned)lane_value((int)(unsigned)dst, i + first), hi = (unsigned)lane_value((int)(unsigned)(dst >> 32), i + first);
+      if (i + first < there)
+        *reinterpret_cast<__attribute__((address_space(1))) f32x4*>((uintptr_t)(((uint64_t)hi << 32) | lo) + 16 * k) = x;
+    }
+  }
+}
+
+// The two token groups of a row set merged, and the merged rows written, in one exchange through LDS at xchg: this wave,
+// of token group HALF, hands the other wave of its set the other half of the dims and merges and writes its own half.  Merged
+// into one wave that then writes, a vnode of 64 rows spent 2.1 us here (64 requests on a shared prefix, whole calls, 24.9 ->
+// 24.35 us; 111 ragged requests of 64-dim heads 12.45 -> 12.25; not at head_dim 256, where there are no registers for it: 17.2
+// -> 20.4).  Every wave of the block must call this, one half or the other.
+template <int D, int NG, int HALF>
+__device__ __forceinline__ void merge_and_write_half(const Stage1Args& a, float* xchg, const VnodeView& vn, const WidePass& p, const WaveState<D, NG>& st) {
+  constexpr int HB = D / 32;                                 // dim blocks of a half
+  constexpr int kArea = WideRows<D>::kGroups * (4 * HB + 2) * kWave;   // floats (the other set's waves may hold fewer groups)
+  static_assert(WideGroups<D>::kMost == 2 && kWideWaves * kArea * 4 <= WideGeom<D>::kLds, "the waves' halves fit the block's LDS");
+  const int lane = lane_here(), r16 = lane & 15, c = lane >> 4;
+  float* mine = xchg + (size_t)(2 * p.set + HALF) * kArea;
+  const float* other = xchg + (size_t)(2 * p.set + 1 - HALF) * kArea;
+  __syncthreads();
+#pragma unroll
+  for (int qb = 0; qb < NG; ++qb) {
+    mine[(4 * HB * NG + 2 * qb) * kWave + lane] = st.m[qb];
+    mine[(4 * HB * NG + 2 * qb + 1) * kWave + lane] = st.l[qb];
+#pragma unroll
+    for (int db = 0; db < HB; ++db) reinterpret_cast<f32x4*>(mine)[(qb * HB + db) * kWave + lane] = st.o[qb][(1 - HALF) * HB + db];
+  }
+  __syncthreads();
+  const int rows_total = vn.q_len * a.g;
+#pragma unroll
+  for (int qb = 0; qb < NG; ++qb) {
+    const float m2 = other[(4 * HB * NG + 2 * qb) * kWave + lane], l2 = other[(4 * HB * NG + 2 * qb + 1) * kWave + lane];
+    const float m = fmaxf(st.m[qb], m2);
+    const float a1 = scale_from(st.m[qb], m), a2 = scale_from(m2, m);
+    const float l = st.l[qb] * a1 + l2 * a2;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    f32x4 o[HB];
+#pragma unroll
+    for (int db = 0; db < HB; ++db)
+      o[db] = (st.o[qb][HALF * HB + db] * a1 + reinterpret_cast<const f32x4*>(other)[(qb * HB + db) * kWave + lane] * a2) * inv;
+    const int r = p.row0 + 16 * qb + r16;
+    if (qb >= p.groups || r >= rows_total) continue;
+    const int ri = a.by_g(r), head = p.kvh * a.g + r - ri * a.g;
+    const int64_t row = vn.q_off + ri;
+    float* dst = a.mid_o + row * a.so0 + (int64_t)head * a.so1 + 4 * c + 16 * HALF * HB;
+#pragma unroll
+    for (int db = 0; db < HB; ++db) *reinterpret_cast<f32x4*>(dst + 16 * db) = o[db];
+    if (HALF == 0 && c == 0) a.mid_lse[row * a.sl0 + head] = l > 0.f ? (__builtin_amdgcn_logf(l) + m) * kLn2 : -INFINITY;
   }
 }
 
@@ -1264,8 +1350,15 @@ __device__ __forceinline__ void wide_pass(const Stage1Args& a, char* smem, const
     }
   }
   finish_state<D, NG>(st);
-  if (p.tgroups > 1) merge_token_groups<D, NG>(reinterpret_cast<float*>(smem), st, p);
-  if (p.tg == 0) write_partials<D, NG>(a, vn, p.kvh, p.row0, st, p.groups);
+  if constexpr (D <= 128) {
+    // (the buffer that the run's last super tile does not lie in: read out before the barrier of that super tile)
+    if (p.tgroups == 1) write_rows<D, NG>(a, rows.ring + (unsigned)(rows.nsuper & 1) * W::kBytes + (unsigned)rows.wave * (W::kBytes / kWideWaves), vn, p, st);
+    else if (p.tg == 0) merge_and_write_half<D, NG, 0>(a, reinterpret_cast<float*>(smem), vn, p, st);
+    else merge_and_write_half<D, NG, 1>(a, reinterpret_cast<float*>(smem), vn, p, st);
+  } else {
+    if (p.tgroups > 1) merge_token_groups<D, NG>(reinterpret_cast<float*>(smem), st, p);
+    if (p.tg == 0) write_partials<D, NG>(a, vn, p.kvh, p.row0, st, p.groups);
+  }
   __syncthreads();  // the ring is reused by the next pass
 }
 
@@ -1302,9 +1395,8 @@ __device__ __forceinline__ void wide_block(const Stage1Args& a, char* smem, cons
     // 1, which the storage type holds exactly, and one group so rounds more of P than two: it costs precision (shared
     // prefixes of fp16 against 64 bits, relative RMS over ten inputs 2.88e-4 with two groups, 2.90e-4 with one).
     constexpr int kGroupsWanted = D <= 128 ? NQ * kWideWaves : kWideWaves;
-    constexpr int kMostTokenGroups = D <= 128 ? WideGeom<D>::kSub : kWideWaves;
     int log_tgroups = 0;
-    while ((1 << log_tgroups) < kMostTokenGroups && groups * (2 << log_tgroups) <= kGroupsWanted) ++log_tgroups;
+    while ((1 << log_tgroups) < WideGroups<D>::kMost && groups * (2 << log_tgroups) <= kGroupsWanted) ++log_tgroups;
     static_assert(kWideWaves == 4, "row sets are 4 >> log_tgroups");
     const int log_sets = 2 - log_tgroups;
     WidePass p;

@@ -798,6 +798,14 @@ int ft_schedule_tree_weighed(int num_nodes, const int32_t* parent, const int32_t
                              const int32_t* req_ids, const int64_t* kv_ptrs, const int32_t* kv_slot_map, int64_t kv_slot_map_len,
                              const int32_t* decided, int batch_size, int group, int num_kv_heads, int head_dim, int num_cus,
                              double* modelled_us, ft_schedule** out) {
+  return ft_schedule_tree_within(num_nodes, parent, seqlen, num_children, req_offs, req_ids, kv_ptrs, kv_slot_map, kv_slot_map_len, decided, -1,
+                                 batch_size, group, num_kv_heads, head_dim, num_cus, modelled_us, out);
+}
+
+int ft_schedule_tree_within(int num_nodes, const int32_t* parent, const int32_t* seqlen, const int32_t* num_children, const int64_t* req_offs,
+                            const int32_t* req_ids, const int64_t* kv_ptrs, const int32_t* kv_slot_map, int64_t kv_slot_map_len,
+                            const int32_t* decided, int64_t most_kv_entries, int batch_size, int group, int num_kv_heads, int head_dim,
+                            int num_cus, double* modelled_us, ft_schedule** out) {
   if (!parent || !seqlen || !num_children || !req_offs || !kv_ptrs || !out) return FT_SCHEDULE_ERR_NULL_POINTER;
   if (num_nodes < 1 || batch_size < 0 || group < 1 || num_kv_heads < 1 || head_dim < 1 || num_cus < 1) return FT_SCHEDULE_ERR_ARGUMENT;
   for (int v = 0; v < num_nodes; ++v) {
@@ -834,6 +842,8 @@ int ft_schedule_tree_weighed(int num_nodes, const int32_t* parent, const int32_t
     double us = 0;
     bool whole;
     if (int rc = whole_paths(tree, m, batch_size, kClearlyBetter * (launch.score + kLaunch), u, us, whole)) return rc;
+    // (a path's tokens stand in the slot list once per leaf)
+    if (most_kv_entries >= 0 && (int64_t)u.kv_entries.size() > most_kv_entries) whole = false;
     if (whole) {
       launch = Launch{};
       for (const Run& r : u.runs) launch.narrow.push_back({r.start, (int32_t)r.tokens, r.reqs, r.n});

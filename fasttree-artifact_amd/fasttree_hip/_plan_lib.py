@@ -40,6 +40,8 @@ SCHEDULE_SIGNATURES = {
                          + [ctypes.c_int] * 5 + [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_void_p)]),
     "ft_schedule_tree_weighed": (ctypes.c_int, [ctypes.c_int, _P32, _P32, _P32, _P64, _P32, _P64, _P32, ctypes.c_int64, _P32]
                                  + [ctypes.c_int] * 5 + [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_void_p)]),
+    "ft_schedule_tree_within": (ctypes.c_int, [ctypes.c_int, _P32, _P32, _P32, _P64, _P32, _P64, _P32, ctypes.c_int64, _P32, ctypes.c_int64]
+                                + [ctypes.c_int] * 5 + [ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_void_p)]),
     "ft_schedule_size": (ctypes.c_int64, [ctypes.c_void_p, ctypes.c_int]),
     "ft_schedule_pack": (ctypes.c_int, [ctypes.c_void_p, _P32, ctypes.c_int64, _P64, _P64]),
     "ft_schedule_destroy": (None, [ctypes.c_void_p]),
@@ -148,20 +150,21 @@ def schedule(kv_offs, kv_lens, q_offs, q_lens, q_entries, kv_entries, batch_size
     return _packed(lib, rc, "ft_schedule_create", handle, us, allocate)
 
 
-def schedule_tree(tree, batch_size, group, num_kv_heads, head_dim, num_cus, kv_slot_map, allocate, decided=None):
+def schedule_tree(tree, batch_size, group, num_kv_heads, head_dim, num_cus, kv_slot_map, allocate, decided=None, most_kv_entries=None):
     """The same from a :class:`TreeArrays` (the array "kv_entries" holds the flat slot list, "node_assignments"
-    which nodes attend their parents' runs with their own); ``decided``: a second decision on that to weigh."""
+    which nodes attend their parents' runs with their own); ``decided``: a second decision on that to weigh; ``most_kv_entries``: entries that the
+    caller's slot list has room for (None: any number)."""
     lib = load()
     slot_map = None if kv_slot_map is None else _i32(kv_slot_map)
     us, handle = ctypes.c_double(), ctypes.c_void_p()
     other = None if decided is None else _i32(decided)
     if other is not None and other.shape[0] != tree.n:
         raise FastTreePlannerError("one decision per node")
-    rc = lib.ft_schedule_tree_weighed(
+    rc = lib.ft_schedule_tree_within(
         tree.n, _ptr32(tree.parent), _ptr32(tree.seqlen), _ptr32(tree.children), tree.req_offs.ctypes.data_as(_P64), _ptr32(tree.req_ids),
         tree.ptrs.ctypes.data_as(_P64), None if slot_map is None else _ptr32(slot_map), 0 if slot_map is None else slot_map.shape[0],
-        None if other is None else _ptr32(other), int(batch_size), int(group), int(num_kv_heads), int(head_dim), int(num_cus),
-        ctypes.byref(us), ctypes.byref(handle))
+        None if other is None else _ptr32(other), -1 if most_kv_entries is None else int(most_kv_entries),
+        int(batch_size), int(group), int(num_kv_heads), int(head_dim), int(num_cus), ctypes.byref(us), ctypes.byref(handle))
     return _packed(lib, rc, "ft_schedule_tree", handle, us, allocate)
 
 

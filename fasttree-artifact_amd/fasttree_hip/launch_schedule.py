@@ -865,15 +865,17 @@ def arrange_within(rows, vnodes, *lists, **kw) -> Arranged:
     return plan if not native_schedule() or plan.fits(rows, vnodes) else arrange(*lists, native=False, **kw)
 
 
-def arrange_tree(tree, batch_size, group, num_kv_heads, *, head_dim=128, num_cus=None, kv_slot_map=None, pin=False, decided=None) -> Arranged:
+def arrange_tree(tree, batch_size, group, num_kv_heads, *, head_dim=128, num_cus=None, kv_slot_map=None, pin=False, decided=None,
+                 most_kv_entries=None) -> Arranged:
     """A tree (:class:`_plan_lib.TreeArrays`) arranged for a device, the sharing of ancestors' tokens
     decided by what it makes the device move, or as ``decided`` says where that launch is modelled clearly
-    shorter (include/fasttree_schedule.h); otherwise :func:`arrange`."""
+    shorter (include/fasttree_schedule.h); ``most_kv_entries``: entries that the caller's slot list has room for, where that
+    bounds it; otherwise :func:`arrange`."""
     from . import _plan_lib
 
     cus = max(1, int(num_cus)) if num_cus else compute_units()
     memory = _PackedTensor(pin)
-    _, where, us = _plan_lib.schedule_tree(tree, batch_size, group, num_kv_heads, head_dim, cus, kv_slot_map, memory, decided)
+    _, where, us = _plan_lib.schedule_tree(tree, batch_size, group, num_kv_heads, head_dim, cus, kv_slot_map, memory, decided, most_kv_entries)
     return Arranged(memory.tensor, where, us, cus)
 
 

@@ -657,7 +657,7 @@ def fasttree_preparation(
         arranged = launch_schedule.arrange_tree(
             tree, batch_size, max(1, num_qo_heads // num_kv_heads), num_kv_heads, head_dim=head_dim,
             num_cus=launch_schedule.compute_units(device) if num_cus is None else num_cus, kv_slot_map=kv_slot_map, pin=_on_gpu(device),
-            decided=r[L.NODE_ASSIGNMENTS])
+            decided=r[L.NODE_ASSIGNMENTS], most_kv_entries=None if buffers is None else buffers.vnode_to_kv_entries.numel())
         # (buffers sized for the planner's own lists may not hold this plan: they get one made from those lists)
         if buffers is None or arranged.fits(
                 buffers.mid_o.shape[0], buffers.vnode_to_kv_offs.numel(), buffers.vnode_to_kv_entries.numel(), buffers.wave_records.numel()):

@@ -62,6 +62,15 @@ int ft_schedule_tree_weighed(int num_nodes, const int32_t* parent, const int32_t
                              const int32_t* kv_slot_map, int64_t kv_slot_map_len, const int32_t* decided, int batch_size,
                              int group, int num_kv_heads, int head_dim, int num_cus, double* modelled_us, ft_schedule** out);
 
+/* As ft_schedule_tree_weighed, for a caller whose room for FT_SCHEDULE_KV_ENTRIES is most_kv_entries entries (-1: any number):
+ * no plan of whole paths is made that needs more, as such a plan lists a token once for every leaf below it.  (A plan that
+ * lists every token once is made all the same.) */
+int ft_schedule_tree_within(int num_nodes, const int32_t* parent, const int32_t* seqlen, const int32_t* num_children,
+                            const int64_t* req_offs, const int32_t* req_ids, const int64_t* kv_ptrs,
+                            const int32_t* kv_slot_map, int64_t kv_slot_map_len, const int32_t* decided,
+                            int64_t most_kv_entries, int batch_size, int group, int num_kv_heads, int head_dim, int num_cus,
+                            double* modelled_us, ft_schedule** out);
+
 /* Entries of one array, or -1. */
 int64_t ft_schedule_size(const ft_schedule* schedule, int which);
 

@@ -115,3 +115,20 @@ def test_which_trees_are_laid_out_as_whole_paths():
     assert whole([1, 4], [384, 24], 4, 8) and whole([1, 31], [200, 100], 4, 8) and whole([1, 4], [384, 24], 4, 8, d=64)
     assert whole([1, 200], [300, 30], 16, 1, d=256)
     assert not whole([1, 4], [3000, 24], 4, 8) and not whole([1, 32], [200, 100], 4, 8) and not whole([1, 31], [200, 100], 4, 8, cus=128)
+
+
+@pytest.mark.parametrize("short_by", [0, 1])
+def test_whole_paths_need_room_in_the_slot_list(short_by):
+    """A plan of whole paths lists a token once per leaf; buffers that have no room for that hold the plan that lists it once."""
+    paths = 4 * (384 + 24) + 32
+    buffers = PlanBuffers(32, 128, paths - short_by, 256, 256, 64, device="cpu")
+    tree = nodes_from_rows(generate_tree([1, 4], [384, 24]))
+    from fasttree_hip.kv_tree import assign_requests, kv_prefix_sums
+    params = FastTreeParams()
+    params.set_q_tile_sizes([16, 4])
+    params.set_kv_tile_sizes([32, 32])
+    params.set_kv_group_num(4)
+    aux, assigned = fasttree_preparation(tree, kv_prefix_sums(tree), assign_requests(tree), 32, 8, 128, [1024, 256], [256, 1024], [256, 256], params,
+                                         device="cpu", launch_order=True, num_cus=256, buffers=buffers)
+    assert (aux[11].wave_records is None) == bool(short_by)
+    assert aux[0].numel() == (384 + 4 * 24 + 32 if short_by else paths) and aux[11].modelled_us is not None

@@ -223,6 +223,25 @@ __device__ __forceinline__ VnodeView uniform(const VnodeView& w) {
   return u;
 }
 
+// What a block of the fused kernel needs before it can ask for its record.  These are arguments of their own ahead of
+// Stage1Args: built with -amdgpu-kernarg-preload-count, leading scalar arguments are in registers when a wave starts, and
+// the record is asked for at once and not after a memory round trip for the arguments, which nothing has read before.  So are
+// those of the kernels of narrow vnodes alone, of whole paths and of the merge; .2 us a launch (whole calls: 4 requests of a
+// short prompt 6.44 -> 6.23 us, 16 of 32/32 heads 15.98 -> 15.60, 64 of 16/1 heads of 256 17.10 -> 16.56, 64 on a shared prefix
+// 29.0 -> 28.6, a long document 42.8 -> 42.4).
+#define FT_FIRST_PARAMETERS                                                                                        \
+  const int32_t *first_table, const int32_t *first_records, const int32_t *first_narrow, int first_wide_blocks, int first_hkv, \
+      unsigned first_mul, unsigned first_shift, int first_share, int first_items
+#define FT_FIRST First{first_table, first_records, first_narrow, first_wide_blocks, first_hkv, Divisor{first_mul, first_shift}, first_share, first_items}
+struct First {
+  const int32_t *prog_table, *prog_records, *narrow_table;
+  int wide_blocks, hkv;
+  Divisor by_hkv;
+  int narrow_share, narrow_items;
+};
+constexpr int kFirstBytes = sizeof(First);
+static_assert(kFirstBytes == 3 * 8 + 6 * 4 && kFirstBytes % 8 == 0, "the parameters lie as the struct does");
+
 // The kernel's arguments, read anew from where the launch put them, by code that one path of a kernel runs:
 // what a path has read as a reference to the kernel's own parameter is held in scalar registers from its start
 // on, beside what the other paths hold, and spilled into lanes of vector registers: 688 reads of such lanes in
@@ -231,7 +250,7 @@ __device__ __forceinline__ VnodeView uniform(const VnodeView& w) {
 // 28-token leaves, 32/32 heads: 65.4 -> 61.2 us; 240 of 32/8 heads with 160 tokens 53.8 -> 49.5; the 400-request
 // tree in the reference's lists 63.2 -> 61.1.
 __device__ __forceinline__ const Stage1Args& args_again() {
-  auto p = (const __attribute__((address_space(4))) Stage1Args*)__builtin_amdgcn_kernarg_segment_ptr();
+  auto p = (const __attribute__((address_space(4))) Stage1Args*)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() + kFirstBytes);
 #ifdef __HIP_DEVICE_COMPILE__
   asm volatile("" : "+s"(p));
 #endif
@@ -1751,10 +1770,10 @@ __device__ __forceinline__ void narrow_pass(const Stage1Args& a, char* smem, con
 // slots): wave w of the vnode takes the tiles w, w + share, ..., and the shares are merged
 // through LDS.  `slot` is the wave's index in the block; a wave without a vnode (exists ==
 // false) only keeps the block's barriers company.  More rows than a pass holds take several passes.
-// ALONE: the block serves no other vnode.
+// ALONE: the block serves no other vnode.  `index`: the vnode's in the narrow range; `records`: Stage1Args::narrow_table.
 template <typename E, int D, bool GATHERED, bool ALONE>
-__device__ __forceinline__ void narrow_item(const Stage1Args& a, char* smem, int slot, int share, bool exists,
-                                            int vnode, int kvh) {
+__device__ __forceinline__ void narrow_item(const Stage1Args& a, const int32_t* records, char* smem, int slot, int share, bool exists,
+                                            int index, int kvh) {
   using N = NarrowGeom<D>;
   static_assert(N::kGroups == 2, "passes of two row groups, then of one");
   VnodeView vn{0, 0, 0, 0};
@@ -1764,8 +1783,8 @@ __device__ __forceinline__ void narrow_item(const Stage1Args& a, char* smem, int
   p.w = slot & (share - 1);
   p.xchg = (unsigned)(slot - p.w) * N::kLds;
   p.rec = 0;
-  p.inlined = !GATHERED && a.narrow_table != nullptr;   // launch uniform
-  if (p.inlined && exists) p.rec = a.narrow_table[(int64_t)(vnode - a.narrow_begin) * kNarrowRecord + lane_here()];
+  p.inlined = !GATHERED && records != nullptr;   // launch uniform
+  if (p.inlined && exists) p.rec = records[(int64_t)index * kNarrowRecord + lane_here()];
   // (what does not depend on the record, while it is on its way)
   NarrowStream<D, GATHERED> rows(a, smem, (unsigned)slot * N::kLds, kvh, p.w, share);
   asm volatile("" : "+s"(rows.kbase), "+s"(rows.vbase), "+s"(rows.k_stride), "+s"(rows.v_stride));
@@ -1775,7 +1794,7 @@ __device__ __forceinline__ void narrow_item(const Stage1Args& a, char* smem, int
     vn.q_off = __builtin_amdgcn_readlane(p.rec, 2);
     vn.q_len = __builtin_amdgcn_readlane(p.rec, 3);
   } else if (exists) {
-    vn = uniform(load_vnode<GATHERED>(a, vnode));
+    vn = uniform(load_vnode<GATHERED>(a, a.narrow_begin + index));
   }
   // (complete for the compiler on every path: a wait for it behind the first direct loads would be a wait for those)
   asm volatile("" : "+v"(p.rec));
@@ -1815,12 +1834,11 @@ __device__ __forceinline__ void narrow_item(const Stage1Args& a, char* smem, int
 // waves: the footprint of one LDS tile per wave instead of a wide block's ring, so that more of
 // these latency-bound waves share a compute unit.
 template <typename E, int D, bool GATHERED>
-__global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 2) stage1_narrow_kernel(Stage1Args a) {
+__global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 2) stage1_narrow_kernel(const int32_t* records, int hkv, unsigned hkv_mul, unsigned hkv_shift, Stage1Args a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int local_vnode = a.by_hkv(blockIdx.x);
-  narrow_item<E, D, GATHERED, true>(a, smem, wave, a.narrow_share, true, a.narrow_begin + local_vnode,
-                              blockIdx.x - local_vnode * a.hkv);
+  const int index = Divisor{hkv_mul, hkv_shift}(blockIdx.x);
+  narrow_item<E, D, GATHERED, true>(a, records, smem, wave, a.narrow_share, true, index, blockIdx.x - index * hkv);
 }
 
 // Whole paths (small launches; see ft_decode_programs): every request is in one vnode, whose run is the request's whole path,
@@ -1836,8 +1854,7 @@ __global__ void __launch_bounds__(kWideBlock, D > 128 ? 1 : 2) stage1_narrow_ker
 // the rounding leaves over is contracted too, a third of a microsecond, and only the output's rounding is left (2.08e-4).
 template <int D> constexpr int kPathWaves = FT_PATH_WAVES(D);
 struct PathArgs {
-  Stage1Args s;                  // (first: args_again() reads it at the start of the arguments)
-  const int32_t* wave_records;   // kPathWaves records of kNarrowRecord ints per vnode
+  Stage1Args s;
   char* o;
   int64_t oo0, oo1;
 };
@@ -1867,12 +1884,12 @@ __device__ __forceinline__ void path_pass(const PathArgs& d, char* smem, const V
   write_merged_shares<D, NG, kPathWaves<D>>(a, xchg, vn, kvh, row0, rows.tile0, out);
 }
 template <typename E, int D>
-__global__ void __launch_bounds__(kWave * kPathWaves<D>, D <= 128 ? 2 : 1) stage1_paths_kernel(PathArgs d) {
+__global__ void __launch_bounds__(kWave * kPathWaves<D>, D <= 128 ? 2 : 1) stage1_paths_kernel(const int32_t* wave_records, int hkv, unsigned hkv_mul, unsigned hkv_shift, PathArgs d) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   const Stage1Args& a = d.s;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int vnode = a.by_hkv(blockIdx.x), kvh = (int)blockIdx.x - vnode * a.hkv;
-  int rec = d.wave_records[((int64_t)vnode * kPathWaves<D> + wave) * kNarrowRecord + lane_here()];
+  const int vnode = Divisor{hkv_mul, hkv_shift}(blockIdx.x), kvh = (int)blockIdx.x - vnode * hkv;
+  int rec = wave_records[((int64_t)vnode * kPathWaves<D> + wave) * kNarrowRecord + lane_here()];
   NarrowStream<D, false> rows(a, smem, (unsigned)wave * NarrowGeom<D>::kLds, kvh, wave, kPathWaves<D>);
   asm volatile("" : "+s"(rows.kbase), "+s"(rows.vbase), "+s"(rows.k_stride), "+s"(rows.v_stride));
   VnodeView vn;
@@ -2000,17 +2017,17 @@ __device__ __forceinline__ void wide_vnode_of_rank(const Stage1Args& a, char* sm
 // The wide vnodes of one block program for one kv head (kv head fastest among the blocks: the eight blocks of a program
 // land on the eight XCDs, and a head's K/V only ever enters one XCD's L2), one after the other.
 template <typename E, int D, bool AGAIN>
-__device__ __forceinline__ void program_block(const Stage1Args& a, char* smem, int program, int kvh) {
-  const PlanInts table = plan_ints(a.prog_table) + 4 * (int64_t)program;
+__device__ __forceinline__ void program_block(const Stage1Args& a, const First& f, char* smem, int program, int kvh) {
+  const PlanInts table = plan_ints(f.prog_table) + 4 * (int64_t)program;
   const int first = table[0], end = table[1];
   RowStream<D, false> rows(a, smem, kvh);
   RecordRequests requests;
   VnodeView vn{0, 0, 0, 0};
   bool listed = false;
-  const bool record = a.prog_records != nullptr;   // launch uniform
+  const bool record = f.prog_records != nullptr;   // launch uniform
   if (record) {
     // table entry and record in one round trip
-    const int32_t* at = a.prog_records + (int64_t)program * kProgRecord;
+    const int32_t* at = f.prog_records + (int64_t)program * kProgRecord;
     const PlanInts head = plan_ints(at);
     vn = VnodeView{head[2], head[3], head[1], (int64_t)head[0]};
     listed = head[4] != 0;
@@ -2061,16 +2078,15 @@ constexpr int kLists = 0, kPrograms = 1, kEmbedding = 2;
 // 168, 110.4 with the 171 that an earlier form took by itself); programs came out slower under the limit.
 constexpr int fused_waves(int D, int mode) { return D > 128 ? 1 : D == 128 || mode != kLists ? 2 : 3; }
 template <typename E, int D, bool GATHERED, int MODE>
-__device__ __forceinline__ void fused_block(const Stage1Args& a, char* smem) {
-  const int wide_blocks = MODE != kLists ? a.num_programs * a.hkv : a.vnode_count * a.wide_chunks * a.hkv;
-  const int narrow_index = (int)blockIdx.x - wide_blocks;
+__device__ __forceinline__ void fused_block(const Stage1Args& a, const First& f, char* smem) {
+  const int narrow_index = (int)blockIdx.x - f.wide_blocks;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // (512-byte rows: most trees gain 1 to 3 % by it, but 32 requests of 64/8 heads of 256 on 15 thousand tokens lose,
   // 121.1 -> 123.3 us.)
   constexpr bool kAgain = D <= 128;
   if (narrow_index < 0) {
     if constexpr (MODE == kLists) {
-      const int slot_of_all = a.by_hkv(blockIdx.x), kvh = (int)blockIdx.x - slot_of_all * a.hkv;
+      const int slot_of_all = f.by_hkv(blockIdx.x), kvh = (int)blockIdx.x - slot_of_all * f.hkv;
       const int rank = a.by_chunks(slot_of_all);
       // Launch slot s of a rank serves chunk (s + rank / 2) % chunks.  Consecutive
       // blocks of one kv head go round robin to the four shader engines of an XCD, strictly in
@@ -2084,49 +2100,49 @@ __device__ __forceinline__ void fused_block(const Stage1Args& a, char* smem) {
       RowStream<D, GATHERED> rows(b, smem, kvh);
       wide_block<E, D, GATHERED>(b, smem, vn, kvh, chunk, chunks, rows, false, RecordRequests());
     } else if constexpr (MODE == kPrograms) {
-      const int program = a.by_hkv(blockIdx.x);
-      program_block<E, D, kAgain>(a, smem, program, (int)blockIdx.x - program * a.hkv);
+      const int program = f.by_hkv(blockIdx.x);
+      program_block<E, D, kAgain>(a, f, smem, program, (int)blockIdx.x - program * f.hkv);
     } else {
       // A program's narrow vnodes, one wave each, before its wide ones (a negative count) or after them: of the
       // two blocks that share a compute unit one starts with its narrow vnodes and the other ends with them, so that
       // the memory-bound narrow vnodes of one run under the arithmetic-bound wide vnodes of the other.
-      const int program = a.by_hkv(blockIdx.x), kvh = (int)blockIdx.x - program * a.hkv;
-      const PlanInts table = plan_ints(a.prog_table) + 4 * (int64_t)program;
+      const int program = f.by_hkv(blockIdx.x), kvh = (int)blockIdx.x - program * f.hkv;
+      const PlanInts table = plan_ints(f.prog_table) + 4 * (int64_t)program;
       const int first = table[2], count = table[3];
       // (one call each, in either order, so that the kernel holds one copy of the code)
 #pragma unroll 1
       for (int turn = 0; turn < 2; ++turn) {
         if ((turn == 0) == (count < 0)) {
           for (int v = first + wave; v < first + abs(count); v += kWideWaves)
-            narrow_item<E, D, GATHERED, false>(kAgain ? args_again() : a, smem, wave, 1, true, a.narrow_begin + v, kvh);
+            narrow_item<E, D, GATHERED, false>(kAgain ? args_again() : a, f.narrow_table, smem, wave, 1, true, v, kvh);
           __syncthreads();  // the waves' tiles become the ring of the next wide vnode
         } else {
-          program_block<E, D, kAgain>(a, smem, program, kvh);
+          program_block<E, D, kAgain>(a, f, smem, program, kvh);
         }
       }
     }
   } else {
     // trailing blocks: an item per wave, or per `share` waves; a wave that shares no vnode and has none is done
-    const int share = a.narrow_share, log_share = share >> 1;   // 1, 2, 4 -> 0, 1, 2
-    const int end = a.narrow_count * a.hkv;
-    const int item = trailing_item((narrow_index * kWideWaves + wave) >> log_share, MODE == kEmbedding ? a.narrow_in_programs * a.hkv : 0, end);
+    const int share = f.narrow_share, log_share = share >> 1;   // 1, 2, 4 -> 0, 1, 2
+    const int end = f.narrow_items;
+    const int item = trailing_item((narrow_index * kWideWaves + wave) >> log_share, MODE == kEmbedding ? a.narrow_in_programs * f.hkv : 0, end);
     if (item < end || share > 1) {
-      const int vnode = a.by_hkv(item);
-      narrow_item<E, D, GATHERED, false>(kAgain ? args_again() : a, smem, wave, share, item < end, a.narrow_begin + vnode, item - vnode * a.hkv);
+      const int index = f.by_hkv(item);
+      narrow_item<E, D, GATHERED, false>(kAgain ? args_again() : a, f.narrow_table, smem, wave, share, item < end, index, item - index * f.hkv);
     }
   }
 }
 
 template <typename E, int D, bool GATHERED, bool PROGRAMS>
-__global__ void __launch_bounds__(kWideBlock, fused_waves(D, PROGRAMS ? kPrograms : kLists)) stage1_fused_kernel(Stage1Args a) {
+__global__ void __launch_bounds__(kWideBlock, fused_waves(D, PROGRAMS ? kPrograms : kLists)) stage1_fused_kernel(FT_FIRST_PARAMETERS, Stage1Args a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  fused_block<E, D, GATHERED, PROGRAMS ? kPrograms : kLists>(a, smem);
+  fused_block<E, D, GATHERED, PROGRAMS ? kPrograms : kLists>(a, FT_FIRST, smem);
 }
 
 template <typename E, int D>
-__global__ void __launch_bounds__(kWideBlock, fused_waves(D, kEmbedding)) stage1_embedding_kernel(Stage1Args a) {
+__global__ void __launch_bounds__(kWideBlock, fused_waves(D, kEmbedding)) stage1_embedding_kernel(FT_FIRST_PARAMETERS, Stage1Args a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  fused_block<E, D, false, kEmbedding>(a, smem);
+  fused_block<E, D, false, kEmbedding>(a, FT_FIRST, smem);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2454,7 +2470,7 @@ template <typename F> __device__ __forceinline__ void with_count(int n, F f) {
 // of a short prompt 7.96 -> 7.62 us, 16 of 32/32 heads 14.17 -> 13.54, 64 on a shared prefix 25.4 -> 24.6, 111 ragged requests
 // of 64-dim heads 12.55 -> 12.4, 64 of 16/1 heads of 256 17.44 -> 17.18).
 template <typename E, int D, int LISTS>
-__global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
+__global__ void __launch_bounds__(kBlock) stage2_kernel(const int32_t* records, Stage2Args a) {
   using G = MergeGeom<D>;
   typedef typename G::Vec Vec;
   constexpr bool SPLIT = LISTS != kWholeLists;
@@ -2469,15 +2485,15 @@ __global__ void __launch_bounds__(kBlock) stage2_kernel(Stage2Args a) {
   int n, first = 0, row0 = 0, recorded = 0;
   bool in_record = false;                                   // block uniform: the list is in the request's record
   const int32_t* list = nullptr;
-  if (a.nsplit > 0) {
-    n = a.nsplit;
-    row0 = req * a.nsplit;
-  } else if (a.req_table) {                                 // launch uniform
-    const int32_t* rec = a.req_table + (int64_t)req * kReqRecord;
+  if (records) {                                            // launch uniform
+    const int32_t* rec = records + (int64_t)req * kReqRecord;
     recorded = rec[2 + min(c, kReqRecEntries - 1)];         // (in one round trip with the length)
     n = plan_ints(rec)[0];
     list = a.req_entries + plan_ints(rec)[1];
     in_record = n <= kReqRecEntries;
+  } else if (a.nsplit > 0) {
+    n = a.nsplit;
+    row0 = req * a.nsplit;
   } else {
     n = plan_ints(a.req_lens)[req];
     list = a.req_entries + plan_ints(a.req_offs)[req];
@@ -2673,7 +2689,7 @@ int launch_stage1_fused(const Stage1Args& a0, hipStream_t stream) {
   constexpr size_t kWideLds = (size_t)WideGeom<D>::kLds;
   constexpr size_t kNarrowLds = (size_t)kWideWaves * NarrowGeom<D>::kLds;
   constexpr size_t lds = kWideLds > kNarrowLds ? kWideLds : kNarrowLds;
-  void (*kern)(Stage1Args) = nullptr;
+  void (*kern)(FT_FIRST_PARAMETERS, Stage1Args) = nullptr;
   if constexpr (MODE == kEmbedding) kern = stage1_embedding_kernel<E, D>;
   else kern = stage1_fused_kernel<E, D, GATHERED, MODE == kPrograms>;
   // (raising the dynamic LDS limit is idempotent: two threads that both find the flag clear both raise it)
@@ -2704,7 +2720,8 @@ int launch_stage1_fused(const Stage1Args& a0, hipStream_t stream) {
   const int64_t blocks = wide_blocks + narrow_blocks;
   if (blocks == 0) return FT_OK;
   if (blocks > INT32_MAX) return FT_ERR_ARGUMENT;
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, 1, 1), dim3(kWideBlock, 1, 1), lds, stream, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, 1, 1), dim3(kWideBlock, 1, 1), lds, stream, a.prog_table, a.prog_records, a.narrow_table,
+                     (int)wide_blocks, a.hkv, a.by_hkv.mul, a.by_hkv.shift, a.narrow_share, a.narrow_count * a.hkv, a);
   return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
 }
 
@@ -2728,12 +2745,13 @@ int launch_stage1_narrow(const Stage1Args& a0, hipStream_t stream) {
     }
     configured.store(true, std::memory_order_release);
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, 1, 1), dim3(kWave * a.narrow_share, 1, 1), lds, stream, a);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, 1, 1), dim3(kWave * a.narrow_share, 1, 1), lds, stream, a.narrow_table, a.hkv, a.by_hkv.mul,
+                     a.by_hkv.shift, a);
   return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
 }
 
 template <typename E, int D>
-int launch_stage1_paths_d(const PathArgs& d, hipStream_t stream) {
+int launch_stage1_paths_d(const PathArgs& d, const int32_t* wave_records, hipStream_t stream) {
   const int64_t blocks = (int64_t)d.s.narrow_count * d.s.hkv;
   if (blocks == 0) return FT_OK;
   if (blocks > INT32_MAX) return FT_ERR_ARGUMENT;
@@ -2749,16 +2767,17 @@ int launch_stage1_paths_d(const PathArgs& d, hipStream_t stream) {
     }
     configured.store(true, std::memory_order_release);
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, 1, 1), dim3(kWave * kPathWaves<D>, 1, 1), lds, stream, d);
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks, 1, 1), dim3(kWave * kPathWaves<D>, 1, 1), lds, stream, wave_records, d.s.hkv,
+                     d.s.by_hkv.mul, d.s.by_hkv.shift, d);
   return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
 }
-int launch_stage1_paths(const PathArgs& a, int head_dim, int dtype, hipStream_t stream) {
+int launch_stage1_paths(const PathArgs& a, const int32_t* wave_records, int head_dim, int dtype, hipStream_t stream) {
 #define FT_DISPATCH_D(E)                                         \
   switch (head_dim) {                                            \
-    case 32: return launch_stage1_paths_d<E, 32>(a, stream);     \
-    case 64: return launch_stage1_paths_d<E, 64>(a, stream);     \
-    case 128: return launch_stage1_paths_d<E, 128>(a, stream);   \
-    case 256: return launch_stage1_paths_d<E, 256>(a, stream);   \
+    case 32: return launch_stage1_paths_d<E, 32>(a, wave_records, stream);     \
+    case 64: return launch_stage1_paths_d<E, 64>(a, wave_records, stream);     \
+    case 128: return launch_stage1_paths_d<E, 128>(a, wave_records, stream);   \
+    case 256: return launch_stage1_paths_d<E, 256>(a, wave_records, stream);   \
     default: return FT_ERR_HEAD_DIM;                             \
   }
   if (dtype == FT_DTYPE_F16) { FT_DISPATCH_D(F16) }
@@ -2831,9 +2850,10 @@ int launch_stage2_inst(const Stage2Args& a0, hipStream_t stream) {
   constexpr int kLeast = D <= 32 ? 16 : D <= 128 ? 8 : 4;
   if ((1 << a.log_groups) < kLeast) a.log_groups = 0;
   const dim3 grid((unsigned)a.batch, (unsigned)std::max(blocks_per_request(kHeads, a.log_splits), a.log_groups ? blocks_per_request(kLaneGroups, a.log_groups) : 0), 1);
-  if (a.log_groups > 0) hipLaunchKernelGGL((stage2_kernel<E, D, kLongLists>), grid, dim3(kBlock, 1, 1), 0, stream, a);
-  else if (a.log_splits > 0) hipLaunchKernelGGL((stage2_kernel<E, D, kSplitLists>), grid, dim3(kBlock, 1, 1), 0, stream, a);
-  else hipLaunchKernelGGL((stage2_kernel<E, D, kWholeLists>), grid, dim3(kBlock, 1, 1), 0, stream, a);
+  const int32_t* records = a.nsplit > 0 ? nullptr : a.req_table;
+  if (a.log_groups > 0) hipLaunchKernelGGL((stage2_kernel<E, D, kLongLists>), grid, dim3(kBlock, 1, 1), 0, stream, records, a);
+  else if (a.log_splits > 0) hipLaunchKernelGGL((stage2_kernel<E, D, kSplitLists>), grid, dim3(kBlock, 1, 1), 0, stream, records, a);
+  else hipLaunchKernelGGL((stage2_kernel<E, D, kWholeLists>), grid, dim3(kBlock, 1, 1), 0, stream, records, a);
   return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
 }
 
@@ -3170,9 +3190,8 @@ int ft_decode_programs(const void* q, const void* k, const void* v, void* o,
     if (!range_ok(phase_node_offsets[1], phase_node_nums[1], num_kv_heads)) return FT_ERR_ARGUMENT;
     if (!aligned16(o) || (oo0 | oo1) % 4 != 0) return FT_ERR_ALIGNMENT;
     d.s.narrow_begin = phase_node_offsets[1]; d.s.narrow_count = phase_node_nums[1];
-    d.wave_records = prog_records;
     d.o = static_cast<char*>(o); d.oo0 = oo0; d.oo1 = oo1;
-    return launch_stage1_paths(d, head_dim, dtype, stream);
+    return launch_stage1_paths(d, prog_records, head_dim, dtype, stream);
   }
   if (int rc = ft_stage1_programs(q, k, v, sq0, sq1, sk0, sk1, sv0, sv1, vnode_to_kv_entries, vnode_to_kv_offs,
                                   vnode_to_kv_lens, vnode_to_q_entries, vnode_to_q_offs, vnode_to_q_lens, mid_o, so0,

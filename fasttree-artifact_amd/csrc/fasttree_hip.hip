@@ -990,9 +990,11 @@ template <int D> struct VOperands {
 // row's soft-max reference has to move (see kSlack) needs no exchange between the four lanes that
 // share the row: each compares its own eight scores, and only when some lane of the wave finds one
 // too large are the maxima exchanged and the accumulators rescaled.  REST: what rounding the probabilities to the
-// storage type leaves over goes to `rest`.
-template <typename E, int D, int NQ, bool REST = false>
-__device__ __forceinline__ void tile_softmax(f32x4 (&s)[2][NQ], int valid, float sc, WaveState<D, NQ>& st, u32x4 (&pf)[NQ], u32x4* rest = nullptr) {
+// storage type leaves over goes to `rest` (kRestAsked: where `asked`, which is uniform).
+constexpr int kNoRest = 0, kRest = 1, kRestAsked = 2;
+template <typename E, int D, int NQ, int REST = kNoRest>
+__device__ __forceinline__ void tile_softmax(f32x4 (&s)[2][NQ], int valid, float sc, WaveState<D, NQ>& st, u32x4 (&pf)[NQ], u32x4* rest = nullptr,
+                                             bool asked = true) {
   if (valid < kTileTokens) {  // wave uniform
     asm volatile("" ::: "memory");  // keeps this a branch: as selects it would run on every tile
     const int c = lane_here() >> 4;
@@ -1033,15 +1035,17 @@ __device__ __forceinline__ void tile_softmax(f32x4 (&s)[2][NQ], int valid, float
     for (int j = 0; j < 8; ++j) x[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j >> 2][qb][j & 3], sc, neg_m));
     st.l[qb] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
     pf[qb] = u32x4{E::pack2(x[0], x[1]), E::pack2(x[2], x[3]), E::pack2(x[4], x[5]), E::pack2(x[6], x[7])};
-    if constexpr (REST)
+    if constexpr (REST != kNoRest)
+      if (asked)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) rest[qb][j] = E::pack2_rest(x[2 * j], x[2 * j + 1], pf[qb][j]);
+        for (int j = 0; j < 4; ++j) rest[qb][j] = E::pack2_rest(x[2 * j], x[2 * j + 1], pf[qb][j]);
   }
 }
 
 // O^T += V^T P^T; `v` holds the operands of the first dim blocks.  read_all(): as in tile_scores; rest: as in tile_softmax.
-template <typename E, int D, int NQ, bool REST = false, typename F = Nothing>
-__device__ __forceinline__ void tile_pv(unsigned vb, VOperands<D>& v, const u32x4 (&pf)[NQ], WaveState<D, NQ>& st, F read_all = F(), const u32x4* rest = nullptr) {
+template <typename E, int D, int NQ, int REST = kNoRest, typename F = Nothing>
+__device__ __forceinline__ void tile_pv(unsigned vb, VOperands<D>& v, const u32x4 (&pf)[NQ], WaveState<D, NQ>& st, F read_all = F(), const u32x4* rest = nullptr,
+                                        bool asked = true) {
   constexpr int DB = D / 16, VB = VOperands<D>::kBatch;
 #pragma unroll
   for (int d0 = 0; d0 < DB; d0 += VB) {
@@ -1051,11 +1055,12 @@ __device__ __forceinline__ void tile_pv(unsigned vb, VOperands<D>& v, const u32x
     for (int db = 0; db < VB; ++db)
 #pragma unroll
       for (int qb = 0; qb < NQ; ++qb) st.o[qb][d0 + db] = E::mfma(v.f[db], pf[qb], st.o[qb][d0 + db]);
-    if constexpr (REST)
+    if constexpr (REST != kNoRest)
+      if (asked)
 #pragma unroll
-      for (int db = 0; db < VB; ++db)
+        for (int db = 0; db < VB; ++db)
 #pragma unroll
-        for (int qb = 0; qb < NQ; ++qb) st.o[qb][d0 + db] = E::mfma(v.f[db], rest[qb], st.o[qb][d0 + db]);
+          for (int qb = 0; qb < NQ; ++qb) st.o[qb][d0 + db] = E::mfma(v.f[db], rest[qb], st.o[qb][d0 + db]);
   }
 }
 
@@ -1539,7 +1544,7 @@ template <int D, bool GATHERED> struct NarrowStream {
 // One wave's share of a narrow vnode for the NG 16-row groups from row0.  The caller has opened the run and asked for
 // the wave's first indices, and for its first rows too if `started`.  `rec` is the lane's int of the vnode's record when
 // `inlined` (else unused).
-template <typename E, int D, int NG, bool GATHERED, bool REST = false>
+template <typename E, int D, int NG, bool GATHERED, int REST>
 __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeView& vn, NarrowStream<D, GATHERED>& rows, bool started,
                                               int kvh, int row0, WaveState<D, NG>& st, int rec, bool inlined) {
   using N = NarrowGeom<D>;
@@ -1630,16 +1635,17 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
         next_k();
       }
       u32x4 rest[NG];
-      tile_softmax<E, D, NG, REST>(sc, vn.kv_len - tile * kTileTokens, a.scale_log2, st, pf, rest);
+      const bool asked = REST == kRest || !inlined;
+      tile_softmax<E, D, NG, REST>(sc, vn.kv_len - tile * kTileTokens, a.scale_log2, st, pf, rest, asked);
       // V landed; the next K and indices may be in flight
       if (indices) wait_direct_loads<N::kLoads + 1>();
       else if (more) wait_direct_loads<N::kLoads>();
       else wait_direct_loads<0>();
       v.request(la.v, 0);
       if constexpr (kEarly) {
-        tile_pv<E, D, NG, REST>(la.v, v, pf, st, next_v, rest);
+        tile_pv<E, D, NG, REST>(la.v, v, pf, st, next_v, rest, asked);
       } else {
-        tile_pv<E, D, NG, REST>(la.v, v, pf, st, Nothing(), rest);
+        tile_pv<E, D, NG, REST>(la.v, v, pf, st, Nothing(), rest, asked);
         next_v();
       }
     }
@@ -1745,11 +1751,11 @@ struct NarrowPass {
   bool inlined, started;
   unsigned xchg;      // byte offset of the areas of the waves that share the vnode in the block's LDS segment
 };
-template <typename E, int D, int NG, bool GATHERED>
+template <typename E, int D, int NG, bool GATHERED, int REST>
 __device__ __forceinline__ void narrow_pass(const Stage1Args& a, char* smem, const VnodeView& vn, NarrowStream<D, GATHERED>& stream, const NarrowPass& p) {
   WaveState<D, NG> st;
   const bool rows = p.row0 < vn.q_len * a.g;
-  if (rows) narrow_attend<E, D, NG, GATHERED>(a, vn, stream, p.started, p.kvh, p.row0, st, p.rec, p.inlined);
+  if (rows) narrow_attend<E, D, NG, GATHERED, REST>(a, vn, stream, p.started, p.kvh, p.row0, st, p.rec, p.inlined);
   else reset_state<D, NG>(st);
   float* xchg = reinterpret_cast<float*>(smem + p.xchg);
   // (rows of less than 256 bytes keep the pairwise merge: with the other one the kernel for narrow vnodes alone takes 131
@@ -1771,7 +1777,7 @@ __device__ __forceinline__ void narrow_pass(const Stage1Args& a, char* smem, con
 // through LDS.  `slot` is the wave's index in the block; a wave without a vnode (exists ==
 // false) only keeps the block's barriers company.  More rows than a pass holds take several passes.
 // ALONE: the block serves no other vnode.  `index`: the vnode's in the narrow range; `records`: Stage1Args::narrow_table.
-template <typename E, int D, bool GATHERED, bool ALONE>
+template <typename E, int D, bool GATHERED, bool ALONE, int REST = kNoRest>
 __device__ __forceinline__ void narrow_item(const Stage1Args& a, const int32_t* records, char* smem, int slot, int share, bool exists,
                                             int index, int kvh) {
   using N = NarrowGeom<D>;
@@ -1824,8 +1830,8 @@ __device__ __forceinline__ void narrow_item(const Stage1Args& a, const int32_t* 
       if (!p.started || rows.pairs()) rows.issue_indices(0, rows.tile0);   // (the second tile's indices too)
       if (!rows.pairs()) rows.issue_indices(1, rows.tile0 + rows.stride);
     }
-    if (groups - done >= 2) narrow_pass<E, D, 2, GATHERED>(a, smem, vn, rows, p);
-    else narrow_pass<E, D, 1, GATHERED>(a, smem, vn, rows, p);
+    if (groups - done >= 2) narrow_pass<E, D, 2, GATHERED, REST>(a, smem, vn, rows, p);
+    else narrow_pass<E, D, 1, GATHERED, REST>(a, smem, vn, rows, p);
     if (share > 1) __syncthreads();  // the exchange area is the staging area of the next pass
   }
 }
@@ -1876,7 +1882,7 @@ __device__ __forceinline__ void path_pass(const PathArgs& d, char* smem, const V
   const Stage1Args& a = d.s;
   static_assert(SharedState<D, NG>::kFloats * kWave * 4 <= NarrowGeom<D>::kLds, "a wave's state fits its LDS area");
   WaveState<D, NG> st;
-  narrow_attend<E, D, NG, false, true>(a, vn, rows, true, kvh, row0, st, rec, true);
+  narrow_attend<E, D, NG, false, kRest>(a, vn, rows, true, kvh, row0, st, rec, true);
   float* xchg = reinterpret_cast<float*>(smem);
   SharedState<D, NG>::put(xchg + rows.tile0 * (NarrowGeom<D>::kLds / 4), st);
   __syncthreads();
@@ -2128,7 +2134,11 @@ __device__ __forceinline__ void fused_block(const Stage1Args& a, const First& f,
     const int item = trailing_item((narrow_index * kWideWaves + wave) >> log_share, MODE == kEmbedding ? a.narrow_in_programs * f.hkv : 0, end);
     if (item < end || share > 1) {
       const int index = f.by_hkv(item);
-      narrow_item<E, D, GATHERED, false>(kAgain ? args_again() : a, f.narrow_table, smem, wave, share, item < end, index, item - index * f.hkv);
+      // (Vnodes without records beside programs are a serving plan's, where a request's prompt and generated tokens may be one
+      // vnode: a maximum, whose probability is 1, the fewer, and more rounded.  128 requests of 2746 tokens, against 64 bits:
+      // 2.890e-4 apart, 2.895e-4 as one, 2.842e-4 with what rounding leaves over (fp16); 120 of 1242 2.275e-3, 2.282e-3 and
+      // 2.173e-3 (bf16); 0 to .1 us.)
+      narrow_item<E, D, GATHERED, false, MODE == kPrograms ? kRestAsked : kNoRest>(kAgain ? args_again() : a, f.narrow_table, smem, wave, share, item < end, index, item - index * f.hkv);
     }
   }
 }

@@ -2622,8 +2622,9 @@ struct StoreArgs {
 };
 
 // A block serves one token (or, of many heads, a part of it), a thread 16 bytes of its K row and the same 16 bytes of
-// its V row.  A token whose slot lies outside the pool is skipped.  Bound by memory round trips and by the translation of
-// addresses in pools that nothing has touched since the last forward: the rows are asked for beside the slot.
+// its V row.  A token whose slot lies outside the pool is skipped.  Bound by the launch and by memory round trips, and so the
+// rows are asked for beside the slot (128 tokens into pools that nothing has touched since the last forward 4 to 4.7 us; touching
+// their pages ahead of the slots changes nothing).
 constexpr int kStoreBlock = 256;
 __global__ void __launch_bounds__(kStoreBlock) store_kv_kernel(StoreArgs a) {
   const int token = blockIdx.x, i = blockIdx.y * blockDim.x + threadIdx.x;

@@ -164,6 +164,13 @@ class LaunchPhases(list):
     num_cus = None
     block_slots = None
 
+    def __setattr__(self, name, value):
+        # A caller that edits the lists in place drops or replaces the records of the narrow vnodes, which repeat them; those
+        # of the waves repeat them as well, and go with them.
+        if name == "narrow_table" and self.wave_records is not None:
+            super().__setattr__("wave_records", None)
+        super().__setattr__(name, value)
+
 
 @dataclass
 class LaunchSchedule:

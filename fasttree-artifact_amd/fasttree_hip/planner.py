@@ -585,7 +585,7 @@ def _place_arranged(plan, kv_entries, num_qo_heads, head_dim, device, buffers):
         nums.narrow_table = part["narrow_table"]
     if head_dim >= 32 and launch_schedule.USE_REQUEST_RECORDS:
         nums.req_table = part["req_table"]
-    if plan.where.get("wave_records", (0, 0))[1] > 0:
+    if plan.where.get("wave_records", (0, 0))[1] > 0 and launch_schedule.USE_NARROW_RECORDS:
         nums.wave_records = part["wave_records"]
     return (part["kv_entries"] if kv_entries is None else kv_entries, part["kv_offs"], part["kv_lens"], part["q_entries"], part["q_offs"],
             part["q_lens"], part["req_entries"], part["req_offs"], part["req_lens"],

@@ -132,3 +132,16 @@ def test_whole_paths_need_room_in_the_slot_list(short_by):
                                          device="cpu", launch_order=True, num_cus=256, buffers=buffers)
     assert (aux[11].wave_records is None) == bool(short_by)
     assert aux[0].numel() == (384 + 4 * 24 + 32 if short_by else paths) and aux[11].modelled_us is not None
+
+
+def test_wave_records_go_with_the_records_they_repeat():
+    """A caller that edits the lists in place drops or replaces ``narrow_table``: the plan is then one in two launches."""
+    from fasttree_hip import _lib
+    from fasttree_hip.decode import _narrow_in_programs
+    from fasttree_hip.launch_schedule import LaunchPhases
+    for value in (None, torch.zeros(64, dtype=torch.int32)):
+        phases = LaunchPhases([0, 4])
+        phases.narrow_table, phases.wave_records = torch.zeros(64, dtype=torch.int32), torch.zeros(512, dtype=torch.int32)
+        assert _narrow_in_programs(phases) == _lib.FT_WHOLE_PATHS
+        phases.narrow_table = value
+        assert phases.wave_records is None and _narrow_in_programs(phases) == 0 and phases.narrow_table is value

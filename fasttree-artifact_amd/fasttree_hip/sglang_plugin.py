@@ -162,6 +162,14 @@ def _requests_per_radix_node(batch) -> Dict[object, List[int]]:
     return reqs_of
 
 
+def rows_reachable(table, named, count, ends) -> bool:
+    """Whether a plan made as if request r had row r of the token table can be moved to the rows that the requests have
+    with 32-bit offsets: a row is ``named`` for each of ``count`` requests, no run ``ends`` past its row, and no row of
+    the table, whichever the requests have, begins or ends past 32 bits."""
+    stride = table.stride(0)
+    return named.dim() == 1 and named.shape[0] >= count and max(ends, default=0) <= stride and stride * max(count, table.shape[0]) < 2**31
+
+
 def prepare_for_fasttree_meta(batch, fasttree_metadata: FastTreeMetadata):
     """Plans one decode batch (schedule.py:12-277) and binds the metadata to it.
 
@@ -174,7 +182,14 @@ def prepare_for_fasttree_meta(batch, fasttree_metadata: FastTreeMetadata):
     query tile list (schedule.py:137-141), and parallelism counts KV *tiles*, not splits
     (schedule.py:113).
     """
-    meta = fasttree_metadata
+    # (rows that the table does not have come to light with the plan's copies: such a plan is made, or refused, again with the
+    # rows at hand)
+    if not _plan_batch(batch, fasttree_metadata):
+        _plan_batch(batch, fasttree_metadata, ask_for_rows=True)
+
+
+def _plan_batch(batch, meta, ask_for_rows=False) -> bool:
+    """What :func:`prepare_for_fasttree_meta` does; False: the batch names rows that the token table does not have."""
     root = batch.tree_cache.root_node
     reqs_of = _requests_per_radix_node(batch)
 
@@ -269,7 +284,8 @@ def prepare_for_fasttree_meta(batch, fasttree_metadata: FastTreeMetadata):
     meta.phase_kv_tile_sizes = kv_tiles
 
     kv_offs, kv_lens, q_entries, q_offs, q_lens = [], [], [], [], []
-    stride = batch.req_to_token_pool.req_to_token.stride(0)
+    token_table = batch.req_to_token_pool.req_to_token
+    stride = token_table.stride(0)
 
     def emit(kv_start, length, members, q_tile, kv_split, n_q):
         # one copy of the member list per KV split, cut into query tiles
@@ -288,11 +304,12 @@ def prepare_for_fasttree_meta(batch, fasttree_metadata: FastTreeMetadata):
     on_gpu = torch.device(meta.device).type == "cuda"
     # Asking for the rows that the requests have in the token table waits for the forwards that are queued, and the device
     # then idles for the rest of the plan (128 requests: 0.9 ms).  So the plan is made as if request r had row r, and the device
-    # moves its offsets to the rows.  (Where a run would leave its row, or numbers 32 bits, the rows are asked for.)
+    # moves its offsets to the rows; what is waited for is the plan's copies, when it is made.  (Where a run would leave its row,
+    # or offsets 32 bits, the rows are asked for.)
     count, at = len(batch.reqs), batch.req_pool_indices
     ends = [off + length for nq, length, off in zip(n_reqs, seqlens, start_of) if nq > 0]
     ends += [len(req.origin_input_ids) + len(req.output_ids) + 1 for req in batch.reqs]
-    moved = on_gpu and at.device == meta.vnode_to_kv_offs.device and max(ends, default=0) <= stride and stride * count < 2**31
+    moved = not ask_for_rows and on_gpu and at.device == meta.vnode_to_kv_offs.device and rows_reachable(token_table, at, count, ends)
     rows = range(count) if moved else at.cpu()
     for i, (node, nq, length, off) in enumerate(zip(order, n_reqs, seqlens, start_of)):
         if nq == 0:
@@ -373,6 +390,8 @@ def prepare_for_fasttree_meta(batch, fasttree_metadata: FastTreeMetadata):
         offs = meta.vnode_to_kv_offs[: len(lists[0])]
         shift = (at[:count].to(torch.int32) - torch.arange(count, device=at.device, dtype=torch.int32)) * stride
         offs += shift[offs // stride]
+        named = torch.empty(count, dtype=at.dtype, pin_memory=True)
+        named.copy_(at[:count], non_blocking=True)
     upload(meta.vnode_to_kv_lens, lists[1])
     upload(meta.vnode_to_q_offs, lists[2])
     upload(meta.vnode_to_q_lens, lists[3])
@@ -390,8 +409,11 @@ def prepare_for_fasttree_meta(batch, fasttree_metadata: FastTreeMetadata):
         meta.req_last_vnodes = [ends_of[(end, rid)] for rid, end in enumerate(tail_ends)]
     # a server may plan on one stream and decode on another
     planner.wait_for_copies(meta.device)
+    if moved and count > 0 and not (0 <= int(named.min()) and int(named.max()) < token_table.shape[0]):
+        return False
 
     batch.fasttree_metadata = meta
+    return True
 
 
 def prepare_for_fasttree_step(batch, fasttree_metadata: FastTreeMetadata):

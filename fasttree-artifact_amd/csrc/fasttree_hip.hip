@@ -2619,22 +2619,39 @@ struct StoreArgs {
   int64_t num_slots;
   int hkv, chunks;             // chunks = 16-byte pieces per (token, head) row
   Divisor by_chunks;
+  int tokens, per_block;       // of launches whose blocks serve several tokens
+  Divisor by_pieces;           // of a token
 };
 
-// A block serves one token (or, of many heads, a part of it), a thread 16 bytes of its K row and the same 16 bytes of
-// its V row.  A token whose slot lies outside the pool is skipped.  Bound by the launch and by memory round trips, and so the
+// A thread moves 16 bytes of a K row and the same 16 bytes of the V row.  A token whose slot lies outside the pool is skipped.
+// A block serves one token (or, of many heads, a part of it); of tokens that are less than a wave's pieces each (SEVERAL) it
+// serves as many as it has threads for, or most lanes of the launch move nothing: 65536 tokens of one 64-dim head 5.3 us so,
+// 16.8 by a wave each, 8192 tokens 2.7 and 3.5, of one 128-dim head 8.8 and 17.0.
+// Bound by the launch and by memory round trips, and so the
 // rows are asked for beside the slot (128 tokens into pools that nothing has touched since the last forward 4 to 4.7 us; touching
 // their pages ahead of the slots changes nothing).
 constexpr int kStoreBlock = 256;
-__global__ void __launch_bounds__(kStoreBlock) store_kv_kernel(StoreArgs a) {
-  const int token = blockIdx.x, i = blockIdx.y * blockDim.x + threadIdx.x;
-  if (i >= a.hkv * a.chunks) return;
+template <bool SEVERAL> __global__ void __launch_bounds__(kStoreBlock) store_kv_kernel(StoreArgs a) {
+  int64_t token = blockIdx.x;
+  int i = blockIdx.y * blockDim.x + threadIdx.x;
+  if constexpr (SEVERAL) {
+    const int at = a.by_pieces(i);
+    token = token * a.per_block + at;
+    i -= at * a.hkv * a.chunks;
+    if (at >= a.per_block || token >= a.tokens) return;
+  } else {
+    if (i >= a.hkv * a.chunks) return;
+  }
   const int head = a.by_chunks(i), chunk = i - head * a.chunks;
   const u32x4 kx = *reinterpret_cast<const u32x4*>(a.k_new + 2 * (token * a.kn0 + head * a.kn1) + 16 * chunk);
   const u32x4 vx = *reinterpret_cast<const u32x4*>(a.v_new + 2 * (token * a.vn0 + head * a.vn1) + 16 * chunk);
-  const PlanInts loc = plan_ints(static_cast<const int32_t*>(a.loc));
-  const int64_t slot = a.loc_is_int64 ? (int64_t)(((uint64_t)(unsigned)loc[2 * (int64_t)token + 1] << 32) | (unsigned)loc[2 * (int64_t)token])
-                                      : (int64_t)loc[token];
+  int64_t slot;
+  if constexpr (SEVERAL) {
+    slot = a.loc_is_int64 ? static_cast<const int64_t*>(a.loc)[token] : (int64_t) static_cast<const int32_t*>(a.loc)[token];
+  } else {
+    const PlanInts loc = plan_ints(static_cast<const int32_t*>(a.loc));
+    slot = a.loc_is_int64 ? (int64_t)(((uint64_t)(unsigned)loc[2 * token + 1] << 32) | (unsigned)loc[2 * token]) : (int64_t)loc[token];
+  }
   if (slot < 0 || slot >= a.num_slots) return;
   *reinterpret_cast<u32x4*>(a.k_pool + 2 * (slot * a.sk0 + head * a.sk1) + 16 * chunk) = kx;
   *reinterpret_cast<u32x4*>(a.v_pool + 2 * (slot * a.sv0 + head * a.sv1) + 16 * chunk) = vx;
@@ -3389,8 +3406,16 @@ int ft_store_kv(const void* k_new, const void* v_new, int64_t kn0, int64_t kn1, 
   a.num_slots = num_slots; a.hkv = num_kv_heads; a.chunks = head_dim / 8;
   a.by_chunks = divisor(a.chunks);
   const int pieces = num_kv_heads * a.chunks, threads = std::min(kStoreBlock, (pieces + kWave - 1) / kWave * kWave);
-  hipLaunchKernelGGL(store_kv_kernel, dim3((unsigned)num_tokens, (unsigned)((pieces + threads - 1) / threads), 1), dim3((unsigned)threads, 1, 1), 0,
-                     stream, a);
+  if (pieces < kWave) {
+    a.tokens = num_tokens;
+    a.per_block = kStoreBlock / pieces;
+    a.by_pieces = divisor(pieces);
+    const int64_t blocks = ((int64_t)num_tokens + a.per_block - 1) / a.per_block;
+    hipLaunchKernelGGL((store_kv_kernel<true>), dim3((unsigned)blocks, 1, 1), dim3(kStoreBlock, 1, 1), 0, stream, a);
+  } else {
+    hipLaunchKernelGGL((store_kv_kernel<false>), dim3((unsigned)num_tokens, (unsigned)((pieces + threads - 1) / threads), 1),
+                       dim3((unsigned)threads, 1, 1), 0, stream, a);
+  }
   return hipGetLastError() == hipSuccess ? FT_OK : FT_ERR_LAUNCH;
 }
 

@@ -2540,7 +2540,8 @@ __global__ void __launch_bounds__(kBlock) stage2_kernel(const int32_t* records, 
     int row;
     if (in_record) {
       row = SPLIT && first > 0 ? lane_value(recorded, lane - c + ((first + c) & (kListRow - 1))) : recorded;
-      row = c < held ? row : row_lane<0>(row);
+      const int first_row = row_lane<0>(row);          // (moved by all lanes: in an arm of the choice the source lane would be off)
+      row = c < held ? row : first_row;
     } else {
       const int i = first + i0 + min(c, held - 1);
       row = a.nsplit > 0 ? row0 + i : list[i];

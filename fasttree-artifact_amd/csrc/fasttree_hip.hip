@@ -62,6 +62,8 @@ struct F16 {
     const h2 v = __builtin_bit_cast(h2, packed);
     return pack2(__builtin_fmaf((float)v[0], -1.f, lo), __builtin_fmaf((float)v[1], -1.f, hi));   // (one mixed instruction each)
   }
+  // the lower (i = 0) or upper of a packed pair
+  static __device__ __forceinline__ float of_pair(unsigned packed, int i) { return (float)__builtin_bit_cast(_Float16, (unsigned short)(packed >> (16 * i))); }
   // acc + lo + hi of a packed pair, in fp32
   static __device__ __forceinline__ float add_pair(unsigned packed, float acc) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -85,6 +87,7 @@ struct BF16 {
   static __device__ __forceinline__ unsigned pack2_rest(float lo, float hi, unsigned packed) {
     return pack2(lo - __builtin_bit_cast(float, packed << 16), hi - __builtin_bit_cast(float, packed & 0xffff0000u));
   }
+  static __device__ __forceinline__ float of_pair(unsigned packed, int i) { return __builtin_bit_cast(float, i ? packed & 0xffff0000u : packed << 16); }
   static __device__ __forceinline__ float add_pair(unsigned packed, float acc) {
     typedef __bf16 b2 __attribute__((ext_vector_type(2)));
     const b2 one = {(__bf16)1.f, (__bf16)1.f};
@@ -990,11 +993,9 @@ template <int D> struct VOperands {
 // row's soft-max reference has to move (see kSlack) needs no exchange between the four lanes that
 // share the row: each compares its own eight scores, and only when some lane of the wave finds one
 // too large are the maxima exchanged and the accumulators rescaled.  REST: what rounding the probabilities to the
-// storage type leaves over goes to `rest` (kRestAsked: where `asked`, which is uniform).
-constexpr int kNoRest = 0, kRest = 1, kRestAsked = 2;
-template <typename E, int D, int NQ, int REST = kNoRest>
-__device__ __forceinline__ void tile_softmax(f32x4 (&s)[2][NQ], int valid, float sc, WaveState<D, NQ>& st, u32x4 (&pf)[NQ], u32x4* rest = nullptr,
-                                             bool asked = true) {
+// storage type leaves over goes to `rest`.
+template <typename E, int D, int NQ, bool REST = false>
+__device__ __forceinline__ void tile_softmax(f32x4 (&s)[2][NQ], int valid, float sc, WaveState<D, NQ>& st, u32x4 (&pf)[NQ], u32x4* rest = nullptr) {
   if (valid < kTileTokens) {  // wave uniform
     asm volatile("" ::: "memory");  // keeps this a branch: as selects it would run on every tile
     const int c = lane_here() >> 4;
@@ -1035,17 +1036,15 @@ __device__ __forceinline__ void tile_softmax(f32x4 (&s)[2][NQ], int valid, float
     for (int j = 0; j < 8; ++j) x[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[j >> 2][qb][j & 3], sc, neg_m));
     st.l[qb] += ((x[0] + x[1]) + (x[2] + x[3])) + ((x[4] + x[5]) + (x[6] + x[7]));
     pf[qb] = u32x4{E::pack2(x[0], x[1]), E::pack2(x[2], x[3]), E::pack2(x[4], x[5]), E::pack2(x[6], x[7])};
-    if constexpr (REST != kNoRest)
-      if (asked)
+    if constexpr (REST)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) rest[qb][j] = E::pack2_rest(x[2 * j], x[2 * j + 1], pf[qb][j]);
+      for (int j = 0; j < 4; ++j) rest[qb][j] = E::pack2_rest(x[2 * j], x[2 * j + 1], pf[qb][j]);
   }
 }
 
 // O^T += V^T P^T; `v` holds the operands of the first dim blocks.  read_all(): as in tile_scores; rest: as in tile_softmax.
-template <typename E, int D, int NQ, int REST = kNoRest, typename F = Nothing>
-__device__ __forceinline__ void tile_pv(unsigned vb, VOperands<D>& v, const u32x4 (&pf)[NQ], WaveState<D, NQ>& st, F read_all = F(), const u32x4* rest = nullptr,
-                                        bool asked = true) {
+template <typename E, int D, int NQ, bool REST = false, typename F = Nothing>
+__device__ __forceinline__ void tile_pv(unsigned vb, VOperands<D>& v, const u32x4 (&pf)[NQ], WaveState<D, NQ>& st, F read_all = F(), const u32x4* rest = nullptr) {
   constexpr int DB = D / 16, VB = VOperands<D>::kBatch;
 #pragma unroll
   for (int d0 = 0; d0 < DB; d0 += VB) {
@@ -1055,12 +1054,11 @@ __device__ __forceinline__ void tile_pv(unsigned vb, VOperands<D>& v, const u32x
     for (int db = 0; db < VB; ++db)
 #pragma unroll
       for (int qb = 0; qb < NQ; ++qb) st.o[qb][d0 + db] = E::mfma(v.f[db], pf[qb], st.o[qb][d0 + db]);
-    if constexpr (REST != kNoRest)
-      if (asked)
+    if constexpr (REST)
 #pragma unroll
-        for (int db = 0; db < VB; ++db)
+      for (int db = 0; db < VB; ++db)
 #pragma unroll
-          for (int qb = 0; qb < NQ; ++qb) st.o[qb][d0 + db] = E::mfma(v.f[db], rest[qb], st.o[qb][d0 + db]);
+        for (int qb = 0; qb < NQ; ++qb) st.o[qb][d0 + db] = E::mfma(v.f[db], rest[qb], st.o[qb][d0 + db]);
   }
 }
 
@@ -1546,7 +1544,11 @@ template <int D, bool GATHERED> struct NarrowStream {
 // One wave's share of a narrow vnode for the NG 16-row groups from row0.  The caller has opened the run and asked for
 // the wave's first indices, and for its first rows too if `started`.  `rec` is the lane's int of the vnode's record when
 // `inlined` (else unused).
-template <typename E, int D, int NG, bool GATHERED, int REST>
+//
+// REST: what rounding the probabilities leaves over is contracted as well.  Such a remainder is 0, or below it, where its
+// probability is not, and an infinite V value then makes NaN of the infinity that the sum is.  So a caller that finds NaN takes the
+// sums again without REST (in code that is never fetched otherwise).
+template <typename E, int D, int NG, bool GATHERED, bool REST>
 __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeView& vn, NarrowStream<D, GATHERED>& rows, bool started,
                                               int kvh, int row0, WaveState<D, NG>& st, int rec, bool inlined) {
   using N = NarrowGeom<D>;
@@ -1637,17 +1639,16 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
         next_k();
       }
       u32x4 rest[NG];
-      const bool asked = REST == kRest || !inlined;
-      tile_softmax<E, D, NG, REST>(sc, vn.kv_len - tile * kTileTokens, a.scale_log2, st, pf, rest, asked);
+      tile_softmax<E, D, NG, REST>(sc, vn.kv_len - tile * kTileTokens, a.scale_log2, st, pf, rest);
       // V landed; the next K and indices may be in flight
       if (indices) wait_direct_loads<N::kLoads + 1>();
       else if (more) wait_direct_loads<N::kLoads>();
       else wait_direct_loads<0>();
       v.request(la.v, 0);
       if constexpr (kEarly) {
-        tile_pv<E, D, NG, REST>(la.v, v, pf, st, next_v, rest, asked);
+        tile_pv<E, D, NG, REST>(la.v, v, pf, st, next_v, rest);
       } else {
-        tile_pv<E, D, NG, REST>(la.v, v, pf, st, Nothing(), rest, asked);
+        tile_pv<E, D, NG, REST>(la.v, v, pf, st, Nothing(), rest);
         next_v();
       }
     }
@@ -1655,6 +1656,24 @@ __device__ __forceinline__ void narrow_attend(const Stage1Args& a, const VnodeVi
     reset_state<D, NG>(st);
   }
   finish_state<D, NG>(st);
+}
+
+// Whether there is NaN in what the wave holds (a maximum of three numbers is an instruction, and NaN where one of them is).
+template <int D, int NG> __device__ __forceinline__ bool holds_nan(const WaveState<D, NG>& st) {
+  f32x4 most = st.o[0][0];
+#pragma unroll
+  for (int i = 1; i < NG * (D / 16); ++i) most = __builtin_elementwise_maximum(most, st.o[i / (D / 16)][i % (D / 16)]);
+  const float all = __builtin_elementwise_maximum(__builtin_elementwise_maximum(most[0], most[1]), __builtin_elementwise_maximum(most[2], most[3]));
+  return __builtin_amdgcn_ballot_w64(!(all == all)) != 0;
+}
+template <typename E, int D, int NG, bool GATHERED>
+__device__ __forceinline__ void walk_again(const Stage1Args& a, const VnodeView& vn, NarrowStream<D, GATHERED>& rows, int kvh, int row0,
+                                           WaveState<D, NG>& st, int rec, bool inlined) {
+  wave_lds_fence();
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): what the wave has written to its area lies there before rows land on it
+  rows.issue_indices(0, rows.tile0);
+  if (!rows.pairs()) rows.issue_indices(1, rows.tile0 + rows.stride);
+  narrow_attend<E, D, NG, GATHERED, false>(a, vn, rows, false, kvh, row0, st, rec, inlined);
 }
 
 // Merge of the `share` waves of one narrow vnode (same rows, interleaved tiles) into the first of
@@ -1676,8 +1695,9 @@ __device__ __forceinline__ void merge_shares(float* xchg, WaveState<D, NG>& st, 
 // The merged rows of a narrow vnode from the states of the SHARE waves that served it, in LDS at xchg: this wave, the
 // w-th, merges and writes its part of the dims of every row.  `more` is given the rows
 // too: request(ri), called by every lane of the wave, names the vnode's ri-th request; write(req, head, dim, x) has in x the
-// dims dim .. dim + 3 of that request's row.
+// dims dim .. dim + 3 of that request's row; sum_again(), where kSumsAgain, is given what a lane merged of a dim block that holds NaN.
 struct WriteNoMore {
+  static constexpr bool kSumsAgain = false;
   __device__ __forceinline__ int request(int) const { return 0; }
   __device__ __forceinline__ void write(int, int, int, const f32x4&) const {}
 };
@@ -1714,10 +1734,11 @@ __device__ __forceinline__ void write_merged_shares(const Stage1Args& a, const f
 #pragma unroll
       for (int db = 0; db < kParts; ++db) sum[db] += o_of[i][db] * weight;
     }
-    const float inv = l > 0.f ? 1.f / l : 0.f;
     const int r = min(row0 + 16 * qb + p, vn.q_len * a.g - 1), ri = a.by_g(r), head = kvh * a.g + r - ri * a.g;
     const int req = more.request(ri);
-    if (row0 + 16 * qb + p <= r) {
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    auto write = [&] {
+      if (row0 + 16 * qb + p > r) return;
       const int64_t row = vn.q_off + ri;
       float* dst = a.mid_o + row * a.so0 + (int64_t)head * a.so1 + 4 * c + 16 * w * kParts;
 #pragma unroll
@@ -1726,6 +1747,18 @@ __device__ __forceinline__ void write_merged_shares(const Stage1Args& a, const f
         more.write(req, head, 4 * c + 16 * (w * kParts + db), sum[db] * inv);
       }
       if (w == 0 && c == 0) a.mid_lse[row * a.sl0 + head] = l > 0.f ? (__builtin_amdgcn_logf(l) + m) * kLn2 : -INFINITY;
+    };
+    write();
+    if constexpr (F::kSumsAgain) {
+      f32x4 all = sum[0];
+#pragma unroll
+      for (int db = 1; db < kParts; ++db) all += sum[db];
+      const float one = (all[0] + all[1]) + (all[2] + all[3]);
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!(one == one)) != 0, 0)) {
+#pragma unroll
+        for (int db = 0; db < kParts; ++db) more.sum_again(kvh, req, head, 16 * (w * kParts + db), m, sum[db]);
+        write();
+      }
     }
   }
 }
@@ -1753,12 +1786,17 @@ struct NarrowPass {
   bool inlined, started;
   unsigned xchg;      // byte offset of the areas of the waves that share the vnode in the block's LDS segment
 };
-template <typename E, int D, int NG, bool GATHERED, int REST>
+template <typename E, int D, int NG, bool GATHERED, bool REST>
 __device__ __forceinline__ void narrow_pass(const Stage1Args& a, char* smem, const VnodeView& vn, NarrowStream<D, GATHERED>& stream, const NarrowPass& p) {
   WaveState<D, NG> st;
   const bool rows = p.row0 < vn.q_len * a.g;
-  if (rows) narrow_attend<E, D, NG, GATHERED, REST>(a, vn, stream, p.started, p.kvh, p.row0, st, p.rec, p.inlined);
-  else reset_state<D, NG>(st);
+  if (rows) {
+    narrow_attend<E, D, NG, GATHERED, REST>(a, vn, stream, p.started, p.kvh, p.row0, st, p.rec, p.inlined);
+    if constexpr (REST)
+      if (__builtin_expect(holds_nan<D, NG>(st), 0)) walk_again<E, D, NG, GATHERED>(a, vn, stream, p.kvh, p.row0, st, p.rec, p.inlined);
+  } else {
+    reset_state<D, NG>(st);
+  }
   float* xchg = reinterpret_cast<float*>(smem + p.xchg);
   // (rows of less than 256 bytes keep the pairwise merge: with the other one the kernel for narrow vnodes alone takes 131
   // registers instead of 126, three waves per SIMD instead of four, and 269 requests of 64/8 heads of 64 83.1 us instead
@@ -1779,7 +1817,7 @@ __device__ __forceinline__ void narrow_pass(const Stage1Args& a, char* smem, con
 // through LDS.  `slot` is the wave's index in the block; a wave without a vnode (exists ==
 // false) only keeps the block's barriers company.  More rows than a pass holds take several passes.
 // ALONE: the block serves no other vnode.  `index`: the vnode's in the narrow range; `records`: Stage1Args::narrow_table.
-template <typename E, int D, bool GATHERED, bool ALONE, int REST = kNoRest>
+template <typename E, int D, bool GATHERED, bool ALONE, bool REST = false>
 __device__ __forceinline__ void narrow_item(const Stage1Args& a, const int32_t* records, char* smem, int slot, int share, bool exists,
                                             int index, int kvh) {
   using N = NarrowGeom<D>;
@@ -1866,7 +1904,15 @@ struct PathArgs {
   char* o;
   int64_t oo0, oo1;
 };
-template <typename E> struct WriteOutput {
+constexpr int kPathFirstBytes = 24;      // of stage1_paths_kernel's arguments ahead of PathArgs
+__device__ __forceinline__ const PathArgs& path_args_again() {   // (see args_again)
+  auto p = (const __attribute__((address_space(4))) PathArgs*)((const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr() + kPathFirstBytes);
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" : "+s"(p));
+#endif
+  return *(const PathArgs*)p;
+}
+template <typename E, int D> struct WriteOutput {
   const PathArgs& d;
   int q_off, rec;
   bool recorded;                 // wave uniform: the vnode's requests are in the record
@@ -1874,6 +1920,39 @@ template <typename E> struct WriteOutput {
     int req = lane_value(rec, 4 + (ri & (kNarrowRecRequests - 1)));
     if (!recorded) req = d.s.q_entries[q_off + ri];
     return req;
+  }
+  // A wave that finds NaN in the 16 dims from `dim` on (see narrow_attend) sums them again from the rows in memory, relative to the
+  // merged maximum m: slow, but small, and of no concern to the block's other waves (looking at the states ahead of the merge takes
+  // .1 us a call, so does letting the block's waves agree on walking the tiles again).
+  // Lane (r16, c) takes every fourth token for row r16; `sum` is of the dims dim + 4 c .. + 3.
+  static constexpr bool kSumsAgain = true;
+  __device__ __forceinline__ void sum_again(int kvh, int req, int head, int dim, float m, f32x4& sum) const {
+    const PathArgs& d = path_args_again();
+    int again = rec;
+    asm volatile("" : "+v"(again));
+    const int c = lane_here() >> 4, kv_len = __builtin_amdgcn_readlane(again, 1);
+    const int32_t* slots = d.s.kv_entries + __builtin_amdgcn_readlane(again, 0);
+    const u32x4* q = reinterpret_cast<const u32x4*>(d.s.q + 2 * ((int64_t)req * d.s.sq0 + (int64_t)head * d.s.sq1));
+    float acc[16] = {};
+#pragma unroll 1
+    for (int t = c; t < kv_len; t += 4) {
+      const int64_t slot = slots[t];
+      const u32x4* k = reinterpret_cast<const u32x4*>(d.s.k + 2 * (slot * d.s.sk0 + (int64_t)kvh * d.s.sk1));
+      const u32x4* v = reinterpret_cast<const u32x4*>(d.s.v + 2 * (slot * d.s.sv0 + (int64_t)kvh * d.s.sv1 + dim));
+      float s = 0.f;
+#pragma unroll 4
+      for (int i = 0; i < D / 8; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s = __builtin_fmaf(E::of_pair(q[i][e >> 1], e & 1), E::of_pair(k[i][e >> 1], e & 1), s);
+      const float x = __builtin_amdgcn_exp2f(__builtin_fmaf(s, d.s.scale_log2, -m));
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[e] = __builtin_fmaf(x, E::of_pair(v[e >> 3][(e >> 1) & 3], e & 1), acc[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const float of_all = xor32_sum(xor16_sum(acc[e]));
+      sum[e & 3] = c == e >> 2 ? of_all : sum[e & 3];
+    }
   }
   __device__ __forceinline__ void write(int req, int head, int dim, const f32x4& x) const {
     *reinterpret_cast<u32x2*>(d.o + 2 * ((int64_t)req * d.oo0 + (int64_t)head * d.oo1 + dim)) = u32x2{E::pack2(x[0], x[1]), E::pack2(x[2], x[3])};
@@ -1884,11 +1963,11 @@ __device__ __forceinline__ void path_pass(const PathArgs& d, char* smem, const V
   const Stage1Args& a = d.s;
   static_assert(SharedState<D, NG>::kFloats * kWave * 4 <= NarrowGeom<D>::kLds, "a wave's state fits its LDS area");
   WaveState<D, NG> st;
-  narrow_attend<E, D, NG, false, kRest>(a, vn, rows, true, kvh, row0, st, rec, true);
+  narrow_attend<E, D, NG, false, true>(a, vn, rows, true, kvh, row0, st, rec, true);
   float* xchg = reinterpret_cast<float*>(smem);
   SharedState<D, NG>::put(xchg + rows.tile0 * (NarrowGeom<D>::kLds / 4), st);
   __syncthreads();
-  const WriteOutput<E> out{d, vn.q_off, rec, vn.q_len <= kNarrowRecRequests};
+  const WriteOutput<E, D> out{d, vn.q_off, rec, vn.q_len <= kNarrowRecRequests};
   write_merged_shares<D, NG, kPathWaves<D>>(a, xchg, vn, kvh, row0, rows.tile0, out);
 }
 template <typename E, int D>
@@ -2068,7 +2147,7 @@ static_assert(trailing_item(INT32_MAX - 10, 9, INT32_MAX) == INT32_MAX - 1 && tr
 // How a fused launch gets its wide vnodes: as the planner's list; as block programs (Stage1Args::prog_table); as
 // block programs that also serve narrow vnodes (Stage1Args::narrow_in_programs).  A kernel for each: one holds no code
 // that its launches do not run.
-constexpr int kLists = 0, kPrograms = 1, kEmbedding = 2;
+constexpr int kLists = 0, kPrograms = 1, kEmbedding = 2, kServing = 3;
 
 // What bounds the start of a block is the fetch of its instructions, which every launch begins with an empty
 // cache for: with one loop over both kinds of work, compiler-made divisions and the program's record handed round
@@ -2107,7 +2186,7 @@ __device__ __forceinline__ void fused_block(const Stage1Args& a, const First& f,
       const Stage1Args& b = kAgain ? args_again() : a;
       RowStream<D, GATHERED> rows(b, smem, kvh);
       wide_block<E, D, GATHERED>(b, smem, vn, kvh, chunk, chunks, rows, false, RecordRequests());
-    } else if constexpr (MODE == kPrograms) {
+    } else if constexpr (MODE != kEmbedding) {
       const int program = f.by_hkv(blockIdx.x);
       program_block<E, D, kAgain>(a, f, smem, program, (int)blockIdx.x - program * f.hkv);
     } else {
@@ -2140,7 +2219,7 @@ __device__ __forceinline__ void fused_block(const Stage1Args& a, const First& f,
       // vnode: a maximum, whose probability is 1, the fewer, and more rounded.  128 requests of 2746 tokens, against 64 bits:
       // 2.890e-4 apart, 2.895e-4 as one, 2.842e-4 with what rounding leaves over (fp16); 120 of 1242 2.275e-3, 2.282e-3 and
       // 2.173e-3 (bf16); 0 to .1 us.)
-      narrow_item<E, D, GATHERED, false, MODE == kPrograms ? kRestAsked : kNoRest>(kAgain ? args_again() : a, f.narrow_table, smem, wave, share, item < end, index, item - index * f.hkv);
+      narrow_item<E, D, GATHERED, false, MODE == kServing>(kAgain ? args_again() : a, f.narrow_table, smem, wave, share, item < end, index, item - index * f.hkv);
     }
   }
 }
@@ -2155,6 +2234,15 @@ template <typename E, int D>
 __global__ void __launch_bounds__(kWideBlock, fused_waves(D, kEmbedding)) stage1_embedding_kernel(FT_FIRST_PARAMETERS, Stage1Args a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   fused_block<E, D, false, kEmbedding>(a, FT_FIRST, smem);
+}
+
+// Programs, and narrow vnodes without records, whose remainders are contracted: a kernel of its own, for that code beside every launch
+// of programs costs the others up to 2 % (with it and the second walk 16.4 -> 16.8 us for 64 of 16/1 heads of 256, the
+// 400-request tree 58.7 -> 59.1; without either 57.8).
+template <typename E, int D>
+__global__ void __launch_bounds__(kWideBlock, fused_waves(D, kServing)) stage1_serving_kernel(FT_FIRST_PARAMETERS, Stage1Args a) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  fused_block<E, D, false, kServing>(a, FT_FIRST, smem);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2722,6 +2810,7 @@ int launch_stage1_fused(const Stage1Args& a0, hipStream_t stream) {
   constexpr size_t lds = kWideLds > kNarrowLds ? kWideLds : kNarrowLds;
   void (*kern)(FT_FIRST_PARAMETERS, Stage1Args) = nullptr;
   if constexpr (MODE == kEmbedding) kern = stage1_embedding_kernel<E, D>;
+  else if constexpr (MODE == kServing) kern = stage1_serving_kernel<E, D>;
   else kern = stage1_fused_kernel<E, D, GATHERED, MODE == kPrograms>;
   // (raising the dynamic LDS limit is idempotent: two threads that both find the flag clear both raise it)
   static std::atomic<bool> configured_on[kMaxDevices];
@@ -2836,6 +2925,7 @@ int launch_stage1_d(const Stage1Args& a, hipStream_t stream) {
     if (a.vnode_count == 0 && !a.prog_table) return launch_stage1_narrow<E, D, GATHERED>(a, stream);
     if constexpr (!GATHERED) {
       if (a.prog_table && a.narrow_in_programs > 0) return launch_stage1_fused<E, D, false, kEmbedding>(a, stream);
+      if (a.prog_table && !a.narrow_table) return launch_stage1_fused<E, D, false, kServing>(a, stream);
       if (a.prog_table) return launch_stage1_fused<E, D, false, kPrograms>(a, stream);
     }
     return launch_stage1_fused<E, D, GATHERED, kLists>(a, stream);

@@ -145,3 +145,34 @@ def test_wave_records_go_with_the_records_they_repeat():
         assert _narrow_in_programs(phases) == _lib.FT_WHOLE_PATHS
         phases.narrow_table = value
         assert phases.wave_records is None and _narrow_in_programs(phases) == 0 and phases.narrow_table is value
+
+
+def _infinite_values(v, slots, d):
+    """A copy of ``v`` with infinities in single dims of the tokens at ``slots``: dim 1 of the first +inf, dim 2 of the second -inf, dim
+    d - 1 both; and those dims."""
+    v = v.clone()
+    v[slots[0], :, 1] = v[slots[0], :, d - 1] = float("inf")
+    v[slots[1], :, 2] = v[slots[1], :, d - 1] = float("-inf")
+    return v, [1, 2, d - 1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,group,heads,dtype", [(128, 4, 8, torch.float16), (128, 20, 2, torch.bfloat16), (64, 3, 8, torch.float16),
+                                                 (32, 1, 4, torch.bfloat16), (256, 16, 1, torch.float16)])
+@pytest.mark.parametrize("at", [(0, 1), (40, 3), (70, 95)])
+def test_infinite_values_stay_infinite(at, d, group, heads, dtype, device):
+    """An infinity among the values of a prompt's tokens is one in the outputs of that dim (and of two of either sign, NaN); the other
+    dims are what they are without it."""
+    print(f"\n[gpu case] whole paths with infinite values at {at}, {group * heads}/{heads} heads of {d}, {dtype}", flush=True)
+    tree, inp, aux, rest = _plan([1, 3], [100, 28], group, heads, d, dtype, device, seed=d)
+    assert aux[11].wave_records is not None
+    o = torch.full_like(inp.Q, float("nan"))
+    v, dims = _infinite_values(inp.V_pool, [int(inp.slot_map[i]) for i in at], d)
+    fasttree_decode(inp.Q, inp.K_pool, v, o, *aux, *rest)
+    assert bool((o[..., 1] == float("inf")).all()) and bool((o[..., 2] == float("-inf")).all()) and bool(torch.isnan(o[..., d - 1]).all())
+    o[..., dims] = 0
+    v[:, :, dims] = 0
+    plain = inp.V_pool
+    inp.V_pool = v
+    _dense_check(tree, inp, o, "the other dims", dtype=dtype)
+    inp.V_pool = plain

@@ -38,7 +38,12 @@ enum {
 /* Arranges vnode lists.  kv_offs / kv_lens / q_offs / q_lens: one entry per vnode (any order);
  * q_entries: the request of every scratch row; kv_entries: the flat slot list the offsets refer to, or
  * NULL (no records are built then).  group: query heads per KV head.  num_cus: the device's compute
- * units.  *modelled_us: what the model expects of the first-stage launch. */
+ * units.  *modelled_us: what the model expects of the first-stage launch.
+ *
+ * Without kv_entries, from head_dim 32 on and beside programs, short vnodes of one run that adjoin may come back as one.  Such
+ * lists are for ft_decode_programs / ft_decode_static with the program table and no narrow_table, which contract what rounding the
+ * probabilities leaves over; ft_decode serves them too, and rounds slightly more of them than of the lists that went in (against
+ * 64 bits 2.895e-4 where 2.890e-4). */
 int ft_schedule_create(int64_t num_vnodes, const int32_t* kv_offs, const int32_t* kv_lens, const int32_t* q_offs,
                        const int32_t* q_lens, int64_t num_rows, const int32_t* q_entries, int64_t num_kv_entries,
                        const int32_t* kv_entries, int batch_size, int group, int num_kv_heads, int head_dim, int num_cus,

@@ -117,6 +117,8 @@ struct Narrow {
 struct Machine {
   int cus, heads, group, head_dim;
   int units() const { return std::max(1, cus / heads); }   // compute units per KV head
+  int block_slots() const { return (head_dim <= 128 ? kBlocksPerCu : 1) * cus; }   // blocks the device holds at a time
+  int64_t wave_slots() const { return (int64_t)block_slots() * kWavesPerBlock; }
 };
 
 int rows_per_block(int head_dim) { return head_dim <= 128 ? 192 : 128; }
@@ -361,6 +363,33 @@ struct NarrowLoad {
   double bytes_us;    // at the memory's rate
 };
 
+// Passes over its run that a narrow vnode takes (one of a 16-row group costs less than one of two: at 512-byte rows about half).
+double passes(const Narrow& v, const Machine& m) {
+  const int64_t rows = (int64_t)v.n * m.group;
+  return rows <= 16 ? (m.head_dim <= 128 ? 0.8 : 0.55) : (double)ceil_div(rows, kWaveRows);
+}
+
+NarrowLoad narrow_load(const std::vector<Narrow>& narrow, const Machine& m, double bytes_us) {
+  NarrowLoad load{0, 0, bytes_us};
+  // the launcher lets 2 or 4 waves share a vnode while that leaves a quarter of the wave slots free
+  const int64_t items = (int64_t)narrow.size() * m.heads;
+  int share = 1;
+  while (share < kWavesPerBlock && 4 * items * 2 * share <= 3 * m.wave_slots()) share *= 2;
+  for (const Narrow& v : narrow) {
+    const double us = kNarrowStart + kNarrowStep * std::max(0.6, m.head_dim / 128.0) * ceil_div(ceil_div(v.tokens, kTile), share) * passes(v, m) + (share > 1 ? kNarrowShare : 0.0);
+    load.block_us += us * m.heads * share / kWavesPerBlock;
+    load.longest_us = std::max(load.longest_us, us);
+  }
+  return load;
+}
+
+// The time that reading the runs' rows takes.
+double read_us(const std::vector<Run>& runs, const Machine& m) {
+  double bytes = 0;
+  for (const Run& r : runs) bytes += 4.0 * m.head_dim * r.tokens * m.heads;
+  return bytes / kBytesPerUs * 256 / m.cus;
+}
+
 std::vector<Piece> cut_runs(const std::vector<Run>& wide, const Machine& m, const Cut& cut) {
   std::vector<Piece> pieces;
   for (const Run& r : wide) {
@@ -562,11 +591,8 @@ struct Launch {
 constexpr double kNone = 1e30;
 Launch solve(const std::vector<Run>& runs, const Machine& m, int narrow_rows, int wave_rows, double bound = kNone) {
   const int block_rows = rows_per_block(m.head_dim);
-  const int slots = (m.head_dim <= 128 ? kBlocksPerCu : 1) * m.cus;      // blocks the device holds at a time
-  const int64_t wave_slots = (int64_t)slots * kWavesPerBlock;
-  double bytes = 0;
-  for (const Run& r : runs) bytes += 4.0 * m.head_dim * r.tokens * m.heads;
-  const double bytes_us = bytes / kBytesPerUs * 256 / m.cus;
+  const int slots = m.block_slots();
+  const double bytes_us = read_us(runs, m);
   std::vector<Run> wide;
   Launch out;
   std::vector<Narrow>& narrow = out.narrow;
@@ -602,28 +628,11 @@ Launch solve(const std::vector<Run>& runs, const Machine& m, int narrow_rows, in
     }
     wide.swap(kept);
   }
-  narrow = cut_long(std::move(narrow), m.group, m.heads, wave_slots);
-  // (a pass of one 16-row group costs less than one of two: at 512-byte rows about half)
-  auto passes = [&](const Narrow& v) {
-    const int64_t rows = (int64_t)v.n * m.group;
-    return rows <= 16 ? (m.head_dim <= 128 ? 0.8 : 0.55) : (double)ceil_div(rows, kWaveRows);
-  };
+  narrow = cut_long(std::move(narrow), m.group, m.heads, m.wave_slots());
   std::stable_sort(narrow.begin(), narrow.end(), [&](const Narrow& a, const Narrow& b) {
-    return ceil_div(a.tokens, kTile) * passes(a) > ceil_div(b.tokens, kTile) * passes(b);
+    return ceil_div(a.tokens, kTile) * passes(a, m) > ceil_div(b.tokens, kTile) * passes(b, m);
   });
-  NarrowLoad load{0, 0, 0};
-  {
-    // the launcher lets 2 or 4 waves share a vnode while that leaves a quarter of the wave slots free
-    const int64_t items = (int64_t)narrow.size() * m.heads;
-    int share = 1;
-    while (share < kWavesPerBlock && 4 * items * 2 * share <= 3 * wave_slots) share *= 2;
-    for (const Narrow& v : narrow) {
-      const double us = kNarrowStart + kNarrowStep * std::max(0.6, m.head_dim / 128.0) * ceil_div(ceil_div(v.tokens, kTile), share) * passes(v) + (share > 1 ? kNarrowShare : 0.0);
-      load.block_us += us * m.heads * share / kWavesPerBlock;
-      load.longest_us = std::max(load.longest_us, us);
-    }
-    load.bytes_us = bytes_us;
-  }
+  const NarrowLoad load = narrow_load(narrow, m, bytes_us);
   Layout& best = out.layout;
   Cut& chosen = out.chosen;
   double& score = out.score;
@@ -784,8 +793,7 @@ int finish(Launch& best, const std::vector<Run>& runs, const Machine& m, int bat
     for (int i : program) placed += (double)best.layout.pieces[i].n * best.layout.pieces[i].tokens;
   if (placed != pairs(runs, [](const Run& r) { return r.tokens; })) return FT_SCHEDULE_ERR_INCOMPLETE;
   build(m, batch, best.layout, best.narrow, kv_entries, s);
-  const int slots = (m.head_dim <= 128 ? kBlocksPerCu : 1) * m.cus;
-  s.arrays[FT_SCHEDULE_COUNTS][3] = best.programs ? best.chosen.row_slots * m.cus : slots;
+  s.arrays[FT_SCHEDULE_COUNTS][3] = best.programs ? best.chosen.row_slots * m.cus : m.block_slots();
   if (modelled_us) *modelled_us = best.layout.total_us + kLaunch;
   return FT_SCHEDULE_OK;
 }
@@ -812,7 +820,13 @@ int ft_schedule_create(int64_t num_vnodes, const int32_t* kv_offs, const int32_t
     Launch launch = best_launch(runs, m);
     // (records of narrow vnodes are made where the slots are known; without them the kernel of programs contracts what rounding leaves
     // over.  Head_dim 16 has no such kernel, and vnodes that are joined would round more: 2.044e-4 of P where 2.036e-4.)
-    if (!kv_entries && m.head_dim >= 32 && !launch.layout.programs.empty()) launch.narrow = join_short(launch.narrow, (int64_t)launch.layout.programs.size(), m.heads, (int64_t)(m.head_dim <= 128 ? kBlocksPerCu : 1) * m.cus * kWavesPerBlock);
+    if (!kv_entries && m.head_dim >= 32 && !launch.layout.programs.empty()) {
+      std::vector<Narrow> joined = join_short(launch.narrow, (int64_t)launch.layout.programs.size(), m.heads, m.wave_slots());
+      if (joined.size() < launch.narrow.size()) {
+        launch.narrow = std::move(joined);
+        place(launch.layout, m, launch.chosen, narrow_load(launch.narrow, m, read_us(runs, m)));   // (the same programs, and what they take beside these)
+      }
+    }
     if (int rc = finish(launch, runs, m, batch_size, kv_entries, *s, modelled_us)) return rc;
     *out = s.release();
     return FT_SCHEDULE_OK;

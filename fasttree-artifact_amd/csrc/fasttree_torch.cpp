@@ -114,6 +114,8 @@ struct Unlocked {
 struct PlanTables {
   const int32_t *prog_table = nullptr, *narrow_table = nullptr, *prog_records = nullptr, *req_table = nullptr;
   int num_programs = 0, narrow_in_programs = 0;
+  const int32_t* wave_records = nullptr;   // of a plan of whole paths
+  int64_t wave_ints = 0;
 };
 
 struct Held {   // a new reference that is dropped at the end of the scope
@@ -130,6 +132,14 @@ PyObject* attribute_or_null(PyObject* o, PyObject* name) {
     PyErr_Clear();
   }
   return a;
+}
+// The records of a plan of whole paths (launch_schedule.whole_paths asks the same).
+void find_wave_records(PyObject* phases, PlanTables& t) {
+  Held records(attribute_or_null(phases, g_wave_records));
+  if (!records.o || records.o == Py_None) return;
+  const at::Tensor& r = tensor(records.o);
+  t.wave_records = static_cast<const int32_t*>(r.data_ptr());
+  t.wave_ints = r.numel();
 }
 // (the plan's list keeps the tensor alive past this call)
 const int32_t* table_address(PyObject* phases, PyObject* name) {
@@ -152,9 +162,8 @@ PlanTables plan_tables(PyObject* phases) {
     t.prog_records = table_address(phases, g_prog_records);
     t.num_programs = count_of(phases, g_num_programs);
     t.narrow_in_programs = count_of(phases, g_narrow_in_programs);
-  } else if (const int32_t* records = table_address(phases, g_wave_records)) {   // a plan of whole paths
-    t.prog_records = records;
-    t.narrow_in_programs = FT_WHOLE_PATHS;
+  } else {
+    find_wave_records(phases, t);
   }
   return t;
 }
@@ -189,13 +198,18 @@ int decode_call(const at::Tensor& q, const Rows& qr, const at::Tensor& k, const 
     refuse("q, k, v and o must share one dtype");
   if (mid_o.scalar_type() != at::kFloat || mid_lse.scalar_type() != at::kFloat) refuse("mid_o and mid_lse must be float32");
 
-  const PlanTables plan = plan_tables(phase_nums);
+  PlanTables plan = plan_tables(phase_nums);
   const Pair nums = int32_pair(phase_nums), offs = int32_pair(phase_offs);
   const double scale = PyFloat_AsDouble(sm_scale);
   if (scale == -1.0 && PyErr_Occurred()) throw PyFailure{};
   const int d = (int)qr.dim, dtype = dtype_code(q);
   const ft_stream_t stream = stream_of(q);
   const int heads_kv = (int)k.size(1);
+  // (laid out for other rows, as for a plan made for another head_dim, they are not for this call)
+  if (plan.wave_records && plan.wave_ints == (int64_t)64 * FT_PATH_WAVES(d) * nums.v[1]) {
+    plan.prog_records = plan.wave_records;
+    plan.narrow_in_programs = FT_WHOLE_PATHS;
+  }
   if ((plan.prog_table || plan.narrow_table) && d >= 32) {
     Unlocked unlocked;
     // the launch was arranged as block programs (launch_schedule.block_programs)

@@ -13,6 +13,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+from .launch_schedule import whole_paths
 
 _DTYPES = {torch.float16: _lib.FT_DTYPE_F16, torch.bfloat16: _lib.FT_DTYPE_BF16}
 
@@ -34,17 +35,17 @@ def _narrow_table_ptr(phase_node_nums):
     return table.data_ptr() if table is not None else None
 
 
-def _narrow_in_programs(phase_node_nums):
+def _narrow_in_programs(phase_node_nums, head_dim=None):
     """The decode call's argument of that name: FT_WHOLE_PATHS for a plan of whole paths."""
     if getattr(phase_node_nums, "prog_table", None) is not None:
         return int(getattr(phase_node_nums, "narrow_in_programs", 0))
-    return _lib.FT_WHOLE_PATHS if getattr(phase_node_nums, "wave_records", None) is not None else 0
+    return _lib.FT_WHOLE_PATHS if whole_paths(phase_node_nums, head_dim) else 0
 
 
-def _prog_records_ptr(phase_node_nums, paths=False):
-    """Device pointer of the records of the block programs a launch-order plan carries (with ``paths``, or of the waves
-    of a plan of whole paths), or None."""
-    if paths and _narrow_in_programs(phase_node_nums) == _lib.FT_WHOLE_PATHS:
+def _prog_records_ptr(phase_node_nums, narrow_in_programs=0):
+    """Device pointer of the records of the block programs a launch-order plan carries (or, for a call of whole paths, of
+    the waves), or None."""
+    if narrow_in_programs == _lib.FT_WHOLE_PATHS:
         return phase_node_nums.wave_records.data_ptr()
     table = getattr(phase_node_nums, "prog_records", None)
     return table.data_ptr() if table is not None and getattr(phase_node_nums, "prog_table", None) is not None else None
@@ -116,6 +117,7 @@ def fasttree_decode_static(q, k_buffer, v_buffer, o, vnode_to_kv_entries, vnode_
         raise _lib.FastTreeLibraryError("q, k, v and o must share one dtype")
     lib = _lib.load()
     programs = getattr(phase_node_nums, "prog_table", None)
+    narrow_in_programs = _narrow_in_programs(phase_node_nums, q.shape[-1])
     rc = lib.ft_decode_static(
         q.data_ptr(), k_buffer.data_ptr(), v_buffer.data_ptr(), o.data_ptr(),
         q.stride(0), q.stride(1), k_buffer.stride(0), k_buffer.stride(1),
@@ -127,7 +129,7 @@ def fasttree_decode_static(q, k_buffer, v_buffer, o, vnode_to_kv_entries, vnode_
         _lib.int32_pair(phase_node_nums), _lib.int32_pair(phase_node_offsets),
         programs.data_ptr() if programs is not None else None,
         int(getattr(phase_node_nums, "num_programs", 0)) if programs is not None else 0,
-        _narrow_in_programs(phase_node_nums), _narrow_table_ptr(phase_node_nums), _prog_records_ptr(phase_node_nums, paths=True),
+        narrow_in_programs, _narrow_table_ptr(phase_node_nums), _prog_records_ptr(phase_node_nums, narrow_in_programs),
         _req_table_ptr(phase_node_nums),
         q.shape[0], q.shape[1], k_buffer.shape[1], q.shape[-1],
         float(sm_scale), _dtype_code(q), _stream_handle(q),

@@ -172,6 +172,13 @@ class LaunchPhases(list):
         super().__setattr__(name, value)
 
 
+def whole_paths(phases, head_dim=None):
+    """Whether the phase list is of a plan of whole paths whose records are laid out for calls of ``head_dim`` (None: any); any other call takes the plan's lists, in two launches.  The compiled binding asks the same."""
+    records = getattr(phases, "wave_records", None)
+    if records is None:
+        return False
+    return head_dim is None or records.numel() == 64 * (8 if head_dim <= 128 else 4) * int(phases[1])
+
 @dataclass
 class LaunchSchedule:
     kv_offs: np.ndarray

@@ -176,3 +176,20 @@ def test_infinite_values_stay_infinite(at, d, group, heads, dtype, device):
     inp.V_pool = v
     _dense_check(tree, inp, o, "the other dims", dtype=dtype)
     inp.V_pool = plain
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("planned,decoded", [(256, 128), (256, 32), (64, 256), (128, 64)])
+def test_plans_made_for_another_head_size(planned, decoded, device):
+    """A model with two head sizes decodes both on one plan (the waves' records are laid out for one number of waves a block)."""
+    print(f"\n[gpu case] plan for head_dim {planned}, call of {decoded}", flush=True)
+    tree, plain, aux, rest = _plan([1, 6], [70, 20], 4, 4, planned, torch.float16, device)
+    assert aux[11].wave_records is not None
+    inp = make_decode_inputs(tree, 16, 4, decoded, device=device, dtype=torch.float16, seed=4, shuffle_slots=True)
+    order = torch.as_tensor(plain.slot_map).argsort()      # the plan's slots -> positions -> these pools' rows
+    k, v = (x[torch.as_tensor(inp.slot_map)[order].to(device)].contiguous() for x in (inp.K_pool, inp.V_pool))
+    width = max(planned, decoded)
+    mid_o, mid_lse = torch.empty(aux[3].numel(), 16, width, device=device), torch.empty(aux[3].numel(), 16, device=device)
+    o = torch.full_like(inp.Q, float("nan"))
+    fasttree_decode(inp.Q, k, v, o, *aux[:9], mid_o, mid_lse, *aux[11:], *rest[:2], 1.0 / math.sqrt(decoded))
+    _dense_check(tree, inp, o, f"head_dim {decoded} on a plan for {planned}")

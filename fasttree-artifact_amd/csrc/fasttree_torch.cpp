@@ -22,7 +22,7 @@ namespace {
 
 PyObject* g_library_error = nullptr;   // fasttree_hip._lib.FastTreeLibraryError
 // attribute names of a launch-order plan's phase list, interned once
-PyObject *g_prog_table, *g_narrow_table, *g_prog_records, *g_req_table, *g_num_programs, *g_narrow_in_programs, *g_wave_records;
+PyObject *g_prog_table, *g_narrow_table, *g_prog_records, *g_req_table, *g_num_programs, *g_narrow_in_programs, *g_wave_records, *g_records_version;
 
 // what decode_layer reads from a FastTreeMetadata, in the order of the decode call's arguments
 constexpr int kMetaAttributes = 14;
@@ -114,7 +114,7 @@ struct Unlocked {
 struct PlanTables {
   const int32_t *prog_table = nullptr, *narrow_table = nullptr, *prog_records = nullptr, *req_table = nullptr;
   int num_programs = 0, narrow_in_programs = 0;
-  const int32_t* wave_records = nullptr;   // of a plan of whole paths
+  const int32_t* wave_records = nullptr;   // of a plan of whole paths whose lists nobody has written to
   int64_t wave_ints = 0;
 };
 
@@ -133,10 +133,14 @@ PyObject* attribute_or_null(PyObject* o, PyObject* name) {
   }
   return a;
 }
-// The records of a plan of whole paths (launch_schedule.whole_paths asks the same).
+// The records of a plan of whole paths, if they still say what its lists do (launch_schedule.whole_paths asks the same).
 void find_wave_records(PyObject* phases, PlanTables& t) {
   Held records(attribute_or_null(phases, g_wave_records));
   if (!records.o || records.o == Py_None) return;
+  Held narrow(attribute_or_null(phases, g_narrow_table)), version(attribute_or_null(phases, g_records_version));
+  if (!narrow.o || narrow.o == Py_None || !version.o || version.o == Py_None) return;
+  const at::Tensor& table = tensor(narrow.o);
+  if (table.is_inference() || (int64_t)table._version() != integer(version.o)) return;
   const at::Tensor& r = tensor(records.o);
   t.wave_records = static_cast<const int32_t*>(r.data_ptr());
   t.wave_ints = r.numel();
@@ -335,7 +339,7 @@ PyMODINIT_FUNC PyInit__torch_binding(void) {
   struct { PyObject** at; const char* name; } names[] = {
       {&g_prog_table, "prog_table"}, {&g_narrow_table, "narrow_table"}, {&g_prog_records, "prog_records"},
       {&g_req_table, "req_table"}, {&g_num_programs, "num_programs"}, {&g_narrow_in_programs, "narrow_in_programs"},
-      {&g_wave_records, "wave_records"}};
+      {&g_wave_records, "wave_records"}, {&g_records_version, "records_version"}};
   for (auto& n : names)
     if (!(*n.at = PyUnicode_InternFromString(n.name))) return nullptr;
   for (int i = 0; i < kMetaAttributes; ++i)

@@ -159,23 +159,37 @@ class LaunchPhases(list):
     #: int32 device tensor, 64 entries per wave of every vnode, of a plan of whole paths (include/fasttree_hip.h,
     #: FT_WHOLE_PATHS), whose decode call is one launch; None for every other plan
     wave_records = None
+    #: how often ``narrow_table`` had been written to when ``wave_records`` was set (:func:`times_written`)
+    records_version = None
     #: what the schedule's model expects the first-stage launch to take, and the machine it was laid out for
     modelled_us = None
     num_cus = None
     block_slots = None
 
     def __setattr__(self, name, value):
-        # A caller that edits the lists in place drops or replaces the records of the narrow vnodes, which repeat them; those
-        # of the waves repeat them as well, and go with them.
+        # A caller that edits the lists in place drops, replaces or rewrites the records of the narrow vnodes, which repeat them;
+        # those of the waves repeat them as well, and go with them (or are not looked at: :func:`whole_paths`).
         if name == "narrow_table" and self.wave_records is not None:
             super().__setattr__("wave_records", None)
         super().__setattr__(name, value)
+        if name == "wave_records":
+            super().__setattr__("records_version", times_written(self.narrow_table))
+
+
+def times_written(table):
+    """The count of in-place writes to a tensor (or to what it shares memory with) that torch keeps; None without a tensor, or
+    where torch keeps none (tensors made in inference mode)."""
+    return None if table is None or table.is_inference() else table._version
 
 
 def whole_paths(phases, head_dim=None):
-    """Whether the phase list is of a plan of whole paths whose records are laid out for calls of ``head_dim`` (None: any); any other call takes the plan's lists, in two launches.  The compiled binding asks the same."""
+    """Whether the phase list is of a plan of whole paths whose records still say what its lists do, and are laid out for calls of
+    ``head_dim`` (None: any); any other call takes the plan's lists, in two launches.  The compiled binding asks the same."""
     records = getattr(phases, "wave_records", None)
     if records is None:
+        return False
+    written = times_written(getattr(phases, "narrow_table", None))
+    if written is None or written != getattr(phases, "records_version", None):
         return False
     return head_dim is None or records.numel() == 64 * (8 if head_dim <= 128 else 4) * int(phases[1])
 
@@ -867,7 +881,8 @@ class _PackedTensor:
     def __call__(self, n):
         import torch
 
-        self.tensor = torch.empty(n, dtype=torch.int32, pin_memory=self.pin)
+        with torch.inference_mode(False):   # (a tensor whose writes are counted)
+            self.tensor = torch.empty(n, dtype=torch.int32, pin_memory=self.pin)
         return self.tensor.numpy()
 
 

@@ -461,7 +461,8 @@ class PlanBuffers:
         import torch
 
         def ints(n):
-            return torch.empty(int(n), dtype=torch.int32, device=device)
+            with torch.inference_mode(False):   # (tensors whose writes are counted: launch_schedule.times_written)
+                return torch.empty(int(n), dtype=torch.int32, device=device)
 
         self.device = device
         self.vnode_to_kv_entries = ints(max_kv_entries)
@@ -562,6 +563,8 @@ def _scratch(rows, num_qo_heads, head_dim, device, buffers):
 def _place_arranged(plan, kv_entries, num_qo_heads, head_dim, device, buffers):
     """The decode call's arguments for a :class:`launch_schedule.Arranged` plan; ``kv_entries``: the flat
     slot list on the device, or None where it is part of the plan."""
+    import torch
+
     from . import launch_schedule
     from .launch_schedule import LaunchPhases
 
@@ -571,7 +574,8 @@ def _place_arranged(plan, kv_entries, num_qo_heads, head_dim, device, buffers):
         wait_for_copies(buffers.device)
     else:
         # one copy for the whole plan; the arrays are views of it
-        whole = plan.packed.to(device)
+        with torch.inference_mode(False):
+            whole = plan.packed.to(device)
         part = {name: whole[lo: lo + n] for name, (lo, n) in plan.where.items()}
     nums = LaunchPhases([plan.n_wide, plan.n_narrow])
     nums.modelled_us, nums.num_cus, nums.block_slots = plan.modelled_us, plan.num_cus, plan.block_slots

@@ -178,6 +178,53 @@ def test_infinite_values_stay_infinite(at, d, group, heads, dtype, device):
     inp.V_pool = plain
 
 
+@pytest.mark.parametrize("inference", [False, True])
+@pytest.mark.parametrize("in_buffers", [False, True])
+def test_written_records_are_two_launches(in_buffers, inference):
+    """A caller that writes into the narrow vnodes' records has the waves' records left alone from there on; one that decodes rows of
+    another size than the plan was made for, for that call."""
+    from fasttree_hip import _lib
+    from fasttree_hip.decode import _narrow_in_programs
+    from fasttree_hip.kv_tree import assign_requests, kv_prefix_sums
+    with torch.inference_mode(inference):
+        buffers = PlanBuffers(32, 128, 8192, 256, 256, 64, device="cpu") if in_buffers else None
+        tree = nodes_from_rows(generate_tree([1, 4], [384, 24]))
+        params = FastTreeParams()
+        params.set_q_tile_sizes([16, 4])
+        params.set_kv_tile_sizes([32, 32])
+        params.set_kv_group_num(4)
+        aux, _ = fasttree_preparation(tree, kv_prefix_sums(tree), assign_requests(tree), 32, 8, 128, [1024, 256], [256, 1024], [256, 256], params,
+                                      device="cpu", launch_order=True, num_cus=256, buffers=buffers)
+        assert [_narrow_in_programs(aux[11], d) for d in (32, 64, 128, 256)] == [_lib.FT_WHOLE_PATHS] * 3 + [0]
+        aux[11].narrow_table.view(-1, 64)[:, 1] -= 1
+        assert _narrow_in_programs(aux[11], 128) == 0 and _narrow_in_programs(aux[11]) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("static", [False, True])
+@pytest.mark.parametrize("in_buffers", [False, True])
+def test_shortened_runs_are_decoded_as_they_are(in_buffers, static, device):
+    """Lists and narrow vnodes' records rewritten in place: the last two tokens of every path are not attended any more."""
+    print(f"\n[gpu case] whole paths shortened in place, buffers {in_buffers}, static {static}", flush=True)
+    buffers = PlanBuffers(32, 128, 8192, 256, 256, 64) if in_buffers else None
+    tree, inp, aux, rest = _plan([1, 3], [100, 28], 4, 8, 128, torch.float16, device, buffers=buffers)
+
+    def decode():
+        o = torch.full_like(inp.Q, float("nan"))
+        if static:
+            fasttree_decode_static(inp.Q, inp.K_pool, inp.V_pool, o, *aux[:9], aux[11], aux[12], rest[2])
+        else:
+            fasttree_decode(inp.Q, inp.K_pool, inp.V_pool, o, *aux, *rest)
+        return o
+
+    assert aux[11].wave_records is not None
+    _dense_check(tree, inp, decode(), "as planned")
+    aux[2].sub_(2)
+    aux[11].narrow_table.view(-1, 64)[:, 1] -= 2
+    inp.path_tokens = [p[:-2] for p in inp.path_tokens]
+    _dense_check(tree, inp, decode(), "shortened")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("planned,decoded", [(256, 128), (256, 32), (64, 256), (128, 64)])
 def test_plans_made_for_another_head_size(planned, decoded, device):

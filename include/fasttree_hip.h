@@ -165,7 +165,8 @@ int ft_decode(const void* q, const void* k, const void* v, void* o,
  * (vnode, KV head) is a block of FT_PATH_WAVES(head_dim) waves, which take every FT_PATH_WAVES-th 32-token tile of the
  * run.  prog_records holds FT_PATH_WAVES records per vnode of the second range, laid out as narrow_table's, the w-th
  * with the slots of the run's w-th tile (vnode_to_kv_entries[kv_off + min(32 w + t, kv_len - 1)]).  The lists are otherwise
- * those of a complete plan.
+ * those of a complete plan.  A vnode may have any number of requests (ft_schedule_tree makes vnodes of up to 32 query rows, what
+ * one pass of a block serves; more take several passes over the run).
  */
 #define FT_WHOLE_PATHS (-1)
 #define FT_PATH_WAVES(head_dim) ((head_dim) <= 128 ? 8 : 4)

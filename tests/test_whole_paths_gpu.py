@@ -240,3 +240,71 @@ def test_plans_made_for_another_head_size(planned, decoded, device):
     o = torch.full_like(inp.Q, float("nan"))
     fasttree_decode(inp.Q, k, v, o, *aux[:9], mid_o, mid_lse, *aux[11:], *rest[:2], 1.0 / math.sqrt(decoded))
     _dense_check(tree, inp, o, f"head_dim {decoded} on a plan for {planned}")
+
+
+def _several_a_leaf(per_leaf, lens, group, planned_group, heads, d, dtype, device):
+    """A prompt of lens[0] tokens and leaves of lens[1] that per_leaf[i] requests end at (numbered across the leaves in turn), planned for
+    ``planned_group`` query heads per KV head and to be decoded with ``group``."""
+    from types import SimpleNamespace
+
+    tree = nodes_from_rows(generate_tree([1, len(per_leaf)], lens))
+    inp = make_decode_inputs(tree, group * heads, heads, d, device=device, dtype=dtype, seed=len(per_leaf) + d, shuffle_slots=True)
+    left, of_leaf, batch = list(per_leaf), [[] for _ in per_leaf], sum(per_leaf)
+    paths = []
+    while any(left):
+        for i, n in enumerate(left):
+            if n > 0:
+                of_leaf[i].append(len(paths))
+                paths.append(inp.path_tokens[i])
+                left[i] -= 1
+    tree[0].requests = list(range(batch))
+    for node, requests in zip(tree[1:], of_leaf):
+        node.requests = requests
+    q = torch.randn(batch, group * heads, d, generator=torch.Generator().manual_seed(d)).to(dtype).to(device)
+    inp = SimpleNamespace(Q=q, K_pool=inp.K_pool, V_pool=inp.V_pool, KV_ptrs=inp.KV_ptrs, slot_map=inp.slot_map, path_tokens=paths, batch_size=batch)
+    params = FastTreeParams()
+    params.set_q_tile_sizes([max(1, 64 // planned_group), max(1, 16 // planned_group)])
+    params.set_kv_tile_sizes([32, 32])
+    params.set_kv_group_num(planned_group)
+    aux, _ = fasttree_preparation(tree, inp.KV_ptrs, batch, planned_group * heads, heads, d, [1024, 256], [256, 1024], [256, 256], params,
+                                  device=device, kv_slot_map=inp.slot_map, launch_order=True, num_cus=256)
+    return tree, inp, aux, (list(params.TSQs), list(params.TSKs), 1.0 / math.sqrt(d))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("per_leaf,planned_group,group", [([3, 1, 2], 4, 4), ([16, 2], 1, 1), ([17, 16], 1, 1), ([32, 5], 1, 1), ([8, 3], 4, 4),
+                                                          ([8, 7], 4, 16), ([32, 17], 1, 3)])
+@pytest.mark.parametrize("d,heads", [(128, 4), (64, 3), (256, 2)])
+def test_leaves_of_several_requests(per_leaf, planned_group, group, d, heads, device):
+    """Every request of a leaf gets its own output: a few, as many as a record names and more, one and two row groups; and, on a plan made
+    for fewer query heads per KV head, more rows than the two groups of a pass."""
+    print(f"\n[gpu case] leaves of {per_leaf} requests, group {group} on a plan for {planned_group}, head_dim {d}", flush=True)
+    tree, inp, aux, rest = _several_a_leaf(per_leaf, [90, 45], group, planned_group, heads, d, torch.float16, device)
+    assert aux[11].wave_records is not None and list(aux[11]) == [0, len(per_leaf)] and sorted(aux[5].tolist()) == sorted(per_leaf)
+    rows = inp.batch_size
+    mid_o, mid_lse = torch.empty(rows, group * heads, d, device=device), torch.empty(rows, group * heads, device=device)
+    o = torch.full_like(inp.Q, float("nan"))
+    fasttree_decode(inp.Q, inp.K_pool, inp.V_pool, o, *aux[:9], mid_o, mid_lse, *aux[11:], *rest)
+    _dense_check(tree, inp, o, f"leaves of {per_leaf} requests")
+    two = torch.empty_like(o)
+    fasttree_decode_stage2(*aux[6:9], mid_o, mid_lse, two)
+    assert torch.equal(two, o), "the merge of one partial result is the rounded result"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,group,heads", [(128, 16, 1), (64, 3, 8), (256, 16, 1)])
+def test_paths_of_two_tokens_in_bf16(d, group, heads, device):
+    """What rounding the probabilities leaves over is contracted too, so only the output's rounding is left: 2^-8 of a value that has 8
+    significant bits.  The remainders are rounded likewise (2^-8 of 2^-8 of a probability), the rest is fp32."""
+    print(f"\n[gpu case] whole paths of two tokens, {group * heads}/{heads} heads of {d}, bf16", flush=True)
+    tree, inp, aux, rest = _plan([1, 3], [1, 1], group, heads, d, torch.bfloat16, device, seed=2)
+    assert aux[11].wave_records is not None
+    o = torch.full_like(inp.Q, float("nan"))
+    fasttree_decode(inp.Q, inp.K_pool, inp.V_pool, o, *aux, *rest)
+    for r, path in enumerate(inp.path_tokens):
+        k, v = (x[torch.as_tensor(path).to(device)].double().cpu() for x in (inp.K_pool, inp.V_pool))
+        q = inp.Q[r].double().cpu().view(heads, group, d)
+        p = torch.softmax(torch.einsum("hgd,thd->hgt", q, k) * rest[2], -1)
+        want, most = torch.einsum("hgt,thd->hgd", p, v), torch.einsum("hgt,thd->hgd", p, v.abs())
+        error = (o[r].double().cpu().view(heads, group, d) - want).abs()
+        assert bool((error <= want.abs() * 2 ** -8 + most * 2 ** -16 + 1e-5).all()), (r, error.max())

@@ -89,6 +89,12 @@ constexpr double kClearlyBetter = 0.95, kClearlyUs = 1.5;
 // unit has a block.  Whole calls of head_dim 128, whole paths and otherwise, us: 4 requests of 32/8 heads with 80 tokens each
 // 4.3 and 6.5, 408 tokens 6.4 and 7.5, 924 tokens 8.4 and 7.7 (not taken), 1524 tokens 10.5 and 8.4; 31 with 300 tokens 6.5 and
 // 9.6, with 1100 11.4 and 11.2; 240 of 16/1 heads with 288 tokens 7.0 and 9.4, with 1100 12.1 and 17.3.
+//
+// A block has its unit to itself at 256- and 512-byte rows, so past a block per unit a second round begins there: 33 requests of 300
+// tokens 9.6 and 8.5, of 408 tokens 11.1 and 8.6, 9 of 32/32 heads 9.5 and 7.9, 65 of 16/4 heads of 256 17.3 and 14.0, 257 of 16/1
+// heads 10.4 and 10.2.  The rule is drawn one block short of that: just a block per unit (32 of 32/8 heads) would still be
+// shorter, 6.0 and 8.5 (408 tokens 6.8 and 8.2, 8 of 32/32 5.7 and 7.8, 256 of 16/1 of 256 11.6 and 18.9).  Of rows of 128 bytes a unit
+// holds two blocks, and whole paths would go on being shorter: 33 of 64-dim heads 5.5 and 7.4, 64 5.9 and 8.0, 96 8.0 and 9.9.
 constexpr double kPathStart = 3.8, kPathRound = 1.1, kPathShared = 0.43;
 
 struct Run {
@@ -319,6 +325,10 @@ std::vector<Narrow> cut_long(std::vector<Narrow> in, int group, int heads, int64
 // First stage, us: 128 requests of 128 + 58 tokens beside 32 programs per KV head 30.5 -> 29.3, 128 of 100 + 60 beside as many
 // 27.3 -> 24.4, 120 of 30 + 70 21.0 -> 18.5.  Not taken where all fit in as they are (64 of 160 + 140 + 90 beside 12 programs 23.2
 // -> 25.4), nor where not all of them do even so (192 of 120 + 18 32.6 either way).
+// Around the last wave slot the gain is a matter of a few hundredths either way.  Whole calls of eight groups on 2560 tokens beside
+// 24 programs, apart and as one: of 128 + 58 tokens 128 requests 36.1 and 35.1, 144 40.1 and 39.9, 160 (the slots are just filled)
+// 41.6 and 40.8, and past the line 168 42.0 and 41.4, 192 45.7 and 43.7; of 100 + 60 tokens 128 33.9 and 33.3, 144 36.6 and 37.5,
+// 160 38.0 and 38.6, past it 176 39.4 and 40.0, 192 42.7 and 41.4.
 std::vector<Narrow> join_short(const std::vector<Narrow>& in, int64_t programs, int heads, int64_t wave_slots) {
   auto fit = [&](const std::vector<Narrow>& v) { return ((int64_t)v.size() + programs * kWavesPerBlock) * heads <= wave_slots; };
   if (fit(in)) return in;
